@@ -19,12 +19,11 @@
 namespace mifdtd {
 
 struct BInst {
-    SGeom g;          // whole instance: i0 = 0, nquads = nx*ny*nz_pitch/4
+    SGeom g;          // whole instance: i0 = 0
     SFields F;
     SCpml cp;
-    SSrc se, sh;      // E / H sources with tval unset
+    SAux ae, ah;      // E / H sources (tval unset) and probes (out unset; slot = column in a probe row)
     int tv_e[kSMaxSrc], tv_h[kSMaxSrc];  // column of each source's value in a tvals row
-    SProbe pe, ph;    // probes with out unset; slot = column in a probe row
 };
 
 // Renumber instance-local block b so each XCD takes R consecutive blocks in turn.
@@ -52,21 +51,16 @@ __global__ __launch_bounds__(SB) void k_batch(const BInst *__restrict__ inst, co
         else hi = mid;
     }
     const BInst &I = inst[lo];
-    const float *tab = I.F.lut;
     const unsigned nb = first_block[lo + 1] - first_block[lo];
-    const unsigned f = xcd_rows(b - first_block[lo], nb, remap_rows) * SB + threadIdx.x;
-    if (f >= I.g.nquads) return;
-    SSrc src = EHALF ? I.se : I.sh;
-#pragma unroll
-    for (int m = 0; m < kSMaxSrc; ++m)
-        if (m < src.n) src.tval[m] = tv_row[EHALF ? I.tv_e[m] : I.tv_h[m]];
-    SProbe prb = EHALF ? I.pe : I.ph;
-    prb.out = probe_row;
+    RowAt r;
+    if (!slab_quad(I.g, xcd_rows(b - first_block[lo], nb, remap_rows), r)) return;
     if (EHALF)
-        e_quad<CM, PML>(I.g, f, I.F.e[0], I.F.e[1], I.F.e[2], I.F.e[3], I.F.e[4], I.F.e[5], I.F.ce[0], I.F.ce[1],
-                        I.F.ce[2], I.cp, src, prb, I.F.cm[0], I.F.cm[1], I.F.cm[2], tab);
+        e_quad_at<CM, PML>(I.g, r.i, r.j, r.k0, r.next, I.F.e[0], I.F.e[1], I.F.e[2], I.F.e[0], I.F.e[1], I.F.e[2],
+                           I.F.e[3], I.F.e[4], I.F.e[5], I.F.ce[0], I.F.ce[1], I.F.ce[2], I.cp, I.ae, I.F.cm[0],
+                           I.F.cm[1], I.F.cm[2], I.F.lut, nullptr, nullptr, probe_row, tv_row, I.tv_e);
     else
-        h_quad<PML>(I.g, f, I.F.e[0], I.F.e[1], I.F.e[2], I.F.e[3], I.F.e[4], I.F.e[5], I.cp, src, prb);
+        h_quad_at<PML>(I.g, r.i, r.j, r.k0, r.prev, I.F.e[0], I.F.e[1], I.F.e[2], I.F.e[3], I.F.e[4], I.F.e[5],
+                       I.F.e[3], I.F.e[4], I.F.e[5], I.cp, I.ah, nullptr, probe_row, tv_row, I.tv_h);
 }
 
 }  // namespace mifdtd
@@ -117,10 +111,8 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
         B.g.ny = ny;
         B.g.nzp = nzp;
         B.g.nz = nz;
-        B.g.Q = (unsigned)(nzp / 4);
         B.g.i0 = 0;
-        B.g.nquads = (unsigned)((unsigned long long)nx * ny * (nzp / 4));
-        B.g.remap = 0;
+        B.g.m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)(nzp / 4), nz, d.npml);
         for (int c = 0; c < 6; c++) B.F.e[c] = d.e[c];
         for (int c = 0; c < 3; c++) B.F.ce[c] = d.ce[c];
         if (tbl) {
@@ -160,7 +152,7 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
             if (c < 0 || c > 5 || bx[0] < 0 || bx[2] < 0 || bx[4] < 0 || bx[1] >= nx || bx[3] >= ny || bx[5] >= nzp ||
                 bx[0] > bx[1] || bx[2] > bx[3] || bx[4] > bx[5])
                 return fail(MIFDTD_EINVAL, "instance %d: source %d outside the grid", n, s);
-            SSrc &X = c < 3 ? B.se : B.sh;
+            SSrc &X = c < 3 ? B.ae.src : B.ah.src;
             int *tv = c < 3 ? B.tv_e : B.tv_h;
             const int m = X.n++;
             X.comp[m] = c;
@@ -182,7 +174,7 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
             const int c = d.probe_comp[q];
             if (c < 0 || c > 5 || p[0] < 0 || p[0] >= nx || p[1] < 0 || p[1] >= ny || p[2] < 0 || p[2] >= nzp)
                 return fail(MIFDTD_EINVAL, "instance %d: probe %d outside the grid", n, q);
-            SProbe &P = c < 3 ? B.pe : B.ph;
+            SProbe &P = c < 3 ? B.ae.prb : B.ah.prb;
             const int m = P.n++;
             P.comp[m] = c;
             P.i[m] = p[0];
@@ -191,8 +183,10 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
             P.slot[m] = tprobe + q;
         }
         tprobe += d.nprobe;
+        aux_box(B.ae);
+        aux_box(B.ah);
         first[n] = (unsigned)blocks;
-        blocks += (B.g.nquads + SB - 1) / SB;
+        blocks += (row_quads_blocks(B.g.m) + kStripes - 1) / kStripes * kStripes;  // block % 8 is the stripe
         if (blocks >= (1ull << 31)) return fail(MIFDTD_ERANGE, "batch exceeds 2^31 blocks");
     }
     first[ninst] = (unsigned)blocks;

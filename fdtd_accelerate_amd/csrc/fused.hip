@@ -557,16 +557,6 @@ __device__ __forceinline__ Q4 lds_q(const float *p, unsigned l4)
     return Q4{{t.x, t.y, t.z, t.w}};
 }
 
-// Whole-wave lane shifts (DPP wave_shl:1 / wave_shr:1 of the 64-lane wave): lane i takes
-// lane i+1's (next) or lane i-1's (prev) value; the lane at the end takes 0.
-__device__ __forceinline__ float lane_next(float x)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float lane_prev(float x)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, false));
-}
 __device__ __forceinline__ float lane_at(float x, int l)
 {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
@@ -998,7 +988,7 @@ __global__ __launch_bounds__(768) void k_fused2(
 
 // CE: CEM as in the sweep (kCeTable reads the 3 x 256 table from global memory).
 template <int CEM, int FEAT>
-__global__ __launch_bounds__(256) void k_shell_e(SGeom g, ShellBoxes sb, unsigned total, const float *ex, const float *ey,
+__global__ __launch_bounds__(256) void k_shell_e(SAux, SGeom g, ShellBoxes sb, unsigned total, const float *ex, const float *ey,
                                                  const float *ez, float *oex, float *oey, float *oez,
                                                  const float *__restrict__ hx, const float *__restrict__ hy,
                                                  const float *__restrict__ hz, const float *__restrict__ cex,
@@ -1006,28 +996,31 @@ __global__ __launch_bounds__(256) void k_shell_e(SGeom g, ShellBoxes sb, unsigne
                                                  const unsigned char *__restrict__ mx,
                                                  const unsigned char *__restrict__ my,
                                                  const unsigned char *__restrict__ mz, const float *__restrict__ lut,
-                                                 SCpml cp, SSrc src, SProbe prb, SDrude dr, STfsf tfe)
+                                                 SCpml cp, SDrude dr, STfsf tfe)
 {
     const float *tab = lut;  // read from global memory (L1/L2 resident)
     const unsigned f = blockIdx.x * 256u + threadIdx.x;
     if (f >= total) return;
     int i, j, k0;
-    shell_quad(sb, f, i, j, k0);
-    e_quad_at<CEM, true, FEAT>(g, i, j, k0, ex, ey, ez, oex, oey, oez, hx, hy, hz, cex, cey, cez, cp, src, prb, mx, my,
-                               mz, tab, &dr, &tfe);
+    bool next, prev;
+    shell_quad(sb, f, i, j, k0, next, prev);
+    e_quad_at<CEM, true, FEAT>(g, i, j, k0, next && (threadIdx.x & 63) < 63, ex, ey, ez, oex, oey, oez, hx, hy, hz,
+                               cex, cey, cez, cp, first_kernel_arg<SAux>(), mx, my, mz, tab, &dr, &tfe);
 }
 
 template <bool TF>
-__global__ __launch_bounds__(256) void k_shell_h(SGeom g, ShellBoxes sb, unsigned total, const float *__restrict__ oex,
+__global__ __launch_bounds__(256) void k_shell_h(SAux, SGeom g, ShellBoxes sb, unsigned total, const float *__restrict__ oex,
                                                  const float *__restrict__ oey, const float *__restrict__ oez,
                                                  const float *hx, const float *hy, const float *hz, float *ohx,
-                                                 float *ohy, float *ohz, SCpml cp, SSrc src, SProbe prb, STfsf tfh)
+                                                 float *ohy, float *ohz, SCpml cp, STfsf tfh)
 {
     const unsigned f = blockIdx.x * 256u + threadIdx.x;
     if (f >= total) return;
     int i, j, k0;
-    shell_quad(sb, f, i, j, k0);
-    h_quad_at<true>(g, i, j, k0, oex, oey, oez, hx, hy, hz, ohx, ohy, ohz, cp, src, prb, TF ? &tfh : nullptr);
+    bool next, prev;
+    shell_quad(sb, f, i, j, k0, next, prev);
+    h_quad_at<true>(g, i, j, k0, prev && (threadIdx.x & 63) > 0, oex, oey, oez, hx, hy, hz, ohx, ohy, ohz, cp,
+                    first_kernel_arg<SAux>(), TF ? &tfh : nullptr);
 }
 
 }  // namespace mifdtd
@@ -1354,26 +1347,27 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
     int nsweeps = 0;  // sweep launches so far (event pairs used)
 
     // the sources' time values and probe rows of step s
-    auto step_tables = [&](int s, FSrc &fs, SSrc &ss, FProbe &fp, SProbe &sp) {
+    auto step_tables = [&](int s, FSrc &fs, FProbe &fp, SAux &ss) {
         fs = src;
-        ss = ssrc;
+        ss.src = ssrc;
         fp = prb;
-        sp = sprb;
-        for (int n = 0; n < src.n; n++) ss.tval[n] = fs.tval[n] = tvals[(size_t)s * src.n + n];
-        sp.out = fp.out = d->nprobe ? probe_series + (size_t)s * d->nprobe : nullptr;
+        ss.prb = sprb;
+        for (int n = 0; n < src.n; n++) ss.src.tval[n] = fs.tval[n] = tvals[(size_t)s * src.n + n];
+        ss.prb.out = fp.out = d->nprobe ? probe_series + (size_t)s * d->nprobe : nullptr;
+        aux_box(ss);
     };
     // shell E pass over boxes b: E from ei (H from hi) to eo, psi E from pe to pe_out
     auto shell_e = [&](const ShellBoxes &b, unsigned long long tot, const float *const *ei, const float *const *hi,
-                       float *const *eo, float *pe, float *pe_out, const SSrc &ss, const SProbe &sp, int fe) -> int {
+                       float *const *eo, float *pe, float *pe_out, const SAux &ss, int fe) -> int {
         SCpml c = scp;
         c.pe = pe;
         c.pe_out = pe_out;
         const unsigned nbk = (unsigned)((tot + 255) / 256);
         if (!nbk) return 0;
 #define MIFDTD_SHELL_E_LAUNCH(CEV, FV)                                                                            \
-    k_shell_e<CEV, FV><<<nbk, 256, 0, st>>>(sg, b, (unsigned)tot, ei[0], ei[1], ei[2], eo[0], eo[1], eo[2], hi[3],    \
+    k_shell_e<CEV, FV><<<nbk, 256, 0, st>>>(ss, sg, b, (unsigned)tot, ei[0], ei[1], ei[2], eo[0], eo[1], eo[2], hi[3],    \
                                             hi[4], hi[5], d->ce[0], d->ce[1], d->ce[2], d->ce_mat[0], d->ce_mat[1],  \
-                                            d->ce_mat[2], d->ce_lut, c, ss, sp, sdr, tfe)
+                                            d->ce_mat[2], d->ce_lut, c, sdr, tfe)
         if (cem == kCeTable) MIFDTD_BY_FEAT(MIFDTD_SHELL_E_LAUNCH, kCeTable, fe);
         else if (cem == kCeArrays) MIFDTD_BY_FEAT(MIFDTD_SHELL_E_LAUNCH, kCeArrays, fe);
         else MIFDTD_BY_FEAT(MIFDTD_SHELL_E_LAUNCH, kCeConst, fe);
@@ -1383,15 +1377,15 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
     };
     // shell H pass over boxes b: H from hi to ho with the new E of en (psi H in place)
     auto shell_h = [&](const ShellBoxes &b, unsigned long long tot, const float *const *en, const float *const *hi,
-                       float *const *ho, const SSrc &ss, const SProbe &sp) -> int {
+                       float *const *ho, const SAux &ss) -> int {
         const unsigned nbk = (unsigned)((tot + 255) / 256);
         if (!nbk) return 0;
         if (tfsf)
-            k_shell_h<true><<<nbk, 256, 0, st>>>(sg, b, (unsigned)tot, en[0], en[1], en[2], hi[3], hi[4], hi[5], ho[3],
-                                                 ho[4], ho[5], scp, ss, sp, tfh);
+            k_shell_h<true><<<nbk, 256, 0, st>>>(ss, sg, b, (unsigned)tot, en[0], en[1], en[2], hi[3], hi[4], hi[5], ho[3],
+                                                 ho[4], ho[5], scp, tfh);
         else
-            k_shell_h<false><<<nbk, 256, 0, st>>>(sg, b, (unsigned)tot, en[0], en[1], en[2], hi[3], hi[4], hi[5], ho[3],
-                                                  ho[4], ho[5], scp, ss, sp, tfh);
+            k_shell_h<false><<<nbk, 256, 0, st>>>(ss, sg, b, (unsigned)tot, en[0], en[1], en[2], hi[3], hi[4], hi[5], ho[3],
+                                                  ho[4], ho[5], scp, tfh);
         MIFDTD_CHECK_LAUNCH("CPML shell H launch");
         return 0;
     };
@@ -1420,14 +1414,13 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
     // (step s+1).
     for (; pairs && s + 2 <= nsteps; s += 2) {
         FSrc fs1, fs2;
-        SSrc ss1, ss2;
+        SAux ss1, ss2;
         FProbe fp1, fp2;
-        SProbe sp1, sp2;
-        step_tables(s, fs1, ss1, fp1, sp1);
-        step_tables(s + 1, fs2, ss2, fp2, sp2);
-        if (int rc = shell_e(sb2[2], tot2[2], in, in, mid, pin, pout, ss1, sp1, 0)) return rc;
-        if (int rc = shell_h(sb2[1], tot2[1], mid, in, mid, ss1, sp1)) return rc;
-        if (int rc = shell_e(sb2[0], tot2[0], mid, mid, out, pout, pout, ss2, sp2, 0)) return rc;
+        step_tables(s, fs1, fp1, ss1);
+        step_tables(s + 1, fs2, fp2, ss2);
+        if (int rc = shell_e(sb2[2], tot2[2], in, in, mid, pin, pout, ss1, 0)) return rc;
+        if (int rc = shell_h(sb2[1], tot2[1], mid, in, mid, ss1)) return rc;
+        if (int rc = shell_e(sb2[0], tot2[0], mid, mid, out, pout, pout, ss2, 0)) return rc;
         mark(0);
 #define MIFDTD_FUSED2_LAUNCH(CEV)                                                                                   \
     k_fused2<CEV><<<g2.nblocks, nthr2, lds2, st>>>(g2, in[0], in[1], in[2], in[3], in[4], in[5], mid[0], mid[1],    \
@@ -1441,23 +1434,22 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
         mark(1);
         ++nsweeps;
         MIFDTD_CHECK_LAUNCH("two-step sweep launch");
-        if (int rc = shell_h(sb2[0], tot2[0], out, mid, out, ss2, sp2)) return rc;
+        if (int rc = shell_h(sb2[0], tot2[0], out, mid, out, ss2)) return rc;
         swap_sets();
         ++swaps;
     }
     // single steps: shell E, the one-step sweep, shell H
     for (; s < nsteps; s++) {
         FSrc fs;
-        SSrc ss;
+        SAux ss;
         FProbe fp;
-        SProbe sp;
-        step_tables(s, fs, ss, fp, sp);
+        step_tables(s, fs, fp, ss);
         if (tfsf)  // the incident line's E half: the E patches of this step read its H
             if (int rc = mifdtd_tfsf_line(d->tfsf_line_e, d->tfsf_line_h, d->tfsf_abc, d->tfsf_line_n, 1, d->tfsf_src[s],
                                           stream))
                 return rc;
         if (shell_on)
-            if (int rc = shell_e(sb, total, in, in, out, pin, pout, ss, sp, feat)) return rc;
+            if (int rc = shell_e(sb, total, in, in, out, pin, pout, ss, feat)) return rc;
         if (sweep) {
             mark(0);
 #define MIFDTD_FUSED_LAUNCH_W(CEV, FV, W)                                                                            \
@@ -1487,7 +1479,7 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
             if (int rc = mifdtd_pbc(out[c1], out[c2], nx, ny, nzp, pad, a, 1, stream)) return rc;
         }
         if (shell_on)
-            if (int rc = shell_h(sb, total, out, in, out, ss, sp)) return rc;
+            if (int rc = shell_h(sb, total, out, in, out, ss)) return rc;
         for (int q = 0; q < d->npbc; q++) {  // periodic H copies
             const int a = d->pbc_axes[q];
             const int c1 = a == 0 ? 4 : 3, c2 = a == 2 ? 4 : 5;

@@ -42,7 +42,8 @@ struct ShellBoxes {
     unsigned start[kMaxShellBoxes + 1];
 };
 
-__host__ __device__ __forceinline__ void shell_quad(const ShellBoxes &s, unsigned f, int &i, int &j, int &k0)
+__host__ __device__ __forceinline__ void shell_quad(const ShellBoxes &s, unsigned f, int &i, int &j, int &k0,
+                                                    bool &next, bool &prev)
 {
     int b = 0;
     while (b + 1 < s.n && f >= s.start[b + 1]) ++b;
@@ -61,6 +62,14 @@ __host__ __device__ __forceinline__ void shell_quad(const ShellBoxes &s, unsigne
     i = s.i0[b] + (ii ? a : o);
     j = s.j0[b] + (ii ? o : a) + wrap;
     k0 = 4 * (qq - wrap * s.Q);
+    next = q + 1 < nq;  // the next thread's quad follows in memory (across a seam's row end too)
+    prev = q > 0;
+}
+
+__host__ __device__ __forceinline__ void shell_quad(const ShellBoxes &s, unsigned f, int &i, int &j, int &k0)
+{
+    bool next, prev;
+    shell_quad(s, f, i, j, k0, next, prev);
 }
 
 // Appends the box (planes [i0,i1), rows [j0,j1), quads [q0,q1)) to sb unless it is empty.

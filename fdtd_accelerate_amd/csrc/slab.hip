@@ -14,22 +14,25 @@
 
 namespace mifdtd {
 
-// CM: CeMode (kCeTable: CE from the material indices and the 3 x 256 table).
+// CM: CeMode (kCeTable: CE from the material indices and the 3 x 256 table).  The
+// sources and probes (first argument) are read only by the waves near them.
 template <int CM, bool PML>
-__global__ __launch_bounds__(SB) void k_slab_e(SGeom g, SFields F, SCpml cp, SSrc src, SProbe prb)
+__global__ __launch_bounds__(SB) void k_slab_e(SAux, SGeom g, SFields F, SCpml cp)
 {
-    const float *tab = F.lut;
-    const unsigned f = (g.remap ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * SB + threadIdx.x;
-    if (f < g.nquads)
-        e_quad<CM, PML>(g, f, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], F.ce[0], F.ce[1], F.ce[2], cp, src, prb,
-                        F.cm[0], F.cm[1], F.cm[2], tab);
+    RowAt r;
+    if (!slab_quad(g, blockIdx.x, r)) return;
+    e_quad_at<CM, PML>(g, r.i, r.j, r.k0, r.next, F.e[0], F.e[1], F.e[2], F.e[0], F.e[1], F.e[2], F.e[3], F.e[4],
+                       F.e[5], F.ce[0], F.ce[1], F.ce[2], cp, first_kernel_arg<SAux>(), F.cm[0], F.cm[1], F.cm[2],
+                       F.lut);
 }
 
 template <bool PML>
-__global__ __launch_bounds__(SB) void k_slab_h(SGeom g, SFields F, SCpml cp, SSrc src, SProbe prb)
+__global__ __launch_bounds__(SB) void k_slab_h(SAux, SGeom g, SFields F, SCpml cp)
 {
-    const unsigned f = (g.remap ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * SB + threadIdx.x;
-    if (f < g.nquads) h_quad<PML>(g, f, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], cp, src, prb);
+    RowAt r;
+    if (!slab_quad(g, blockIdx.x, r)) return;
+    h_quad_at<PML>(g, r.i, r.j, r.k0, r.prev, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], F.e[3], F.e[4], F.e[5],
+                   cp, first_kernel_arg<SAux>());
 }
 
 }  // namespace mifdtd
@@ -131,22 +134,19 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
         F.lut = d->ce_lut;
     }
     const int ns = (nx + S - 1) / S;
-    // Small slabs: give each XCD a contiguous run of rows (j+-1 reuse in its L2).
-    const int remap = S <= 8;
     auto geom = [&](int sl) {
         SGeom g;
         g.nx = nx;
         g.ny = ny;
         g.nzp = nzp;
         g.nz = nz;
-        g.Q = Q;
         g.i0 = sl * S;
-        g.nquads = (unsigned)(plane_q * (unsigned long long)(nx - g.i0 < S ? nx - g.i0 : S));
-        g.remap = remap;
+        g.m = row_quads((unsigned)(nx - g.i0 < S ? nx - g.i0 : S), (unsigned)ny, Q, nz, pml ? d->npml : 0);
         return g;
     };
-    auto sources = [&](int step, bool e_half) {
-        SSrc X{};
+    auto tables = [&](const SProbe &P, int step, bool e_half) {
+        SAux A{};
+        SSrc &X = A.src;
         for (int n = 0; n < d->nsrc; n++) {
             if ((d->src_comp[n] < 3) != e_half) continue;
             const int *b = d->src_box[n];
@@ -163,31 +163,28 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
             X.ow[m] = d->src_overwrite[n];
             X.tval[m] = tvals[(size_t)step * d->nsrc + n];
         }
-        return X;
-    };
-    auto probes = [&](const SProbe &P, int step) {
-        SProbe X = P;
-        X.out = d->nprobe ? probe_series + (size_t)step * d->nprobe : nullptr;
-        return X;
+        A.prb = P;
+        A.prb.out = d->nprobe ? probe_series + (size_t)step * d->nprobe : nullptr;
+        aux_box(A);
+        return A;
     };
     for (int n = 0; n < nsteps; n++) {
-        const SSrc se = sources(n, true), sh = sources(n, false);
-        const SProbe pen = probes(pe, n), phn = probes(ph, n);
+        const SAux ae = tables(pe, n, true), ah = tables(ph, n, false);
         for (int sl = 0; sl < ns; sl++) {
             const SGeom g = geom(sl);
-            const unsigned grid = (g.nquads + SB - 1) / SB;
+            const unsigned grid = (unsigned)row_quads_blocks(g.m);
 #define MIFDTD_SLAB_E(CM)                                                   \
     do {                                                                    \
-        if (pml) k_slab_e<CM, true><<<grid, SB, 0, st>>>(g, F, cp, se, pen);  \
-        else k_slab_e<CM, false><<<grid, SB, 0, st>>>(g, F, cp, se, pen);    \
+        if (pml) k_slab_e<CM, true><<<grid, SB, 0, st>>>(ae, g, F, cp);  \
+        else k_slab_e<CM, false><<<grid, SB, 0, st>>>(ae, g, F, cp);    \
     } while (0)
             if (cem == kCeTable) MIFDTD_SLAB_E(kCeTable);
             else if (cem == kCeArrays) MIFDTD_SLAB_E(kCeArrays);
             else MIFDTD_SLAB_E(kCeConst);
 #undef MIFDTD_SLAB_E
             MIFDTD_CHECK_LAUNCH("slab E launch");
-            if (pml) k_slab_h<true><<<grid, SB, 0, st>>>(g, F, cp, sh, phn);
-            else k_slab_h<false><<<grid, SB, 0, st>>>(g, F, cp, sh, phn);
+            if (pml) k_slab_h<true><<<grid, SB, 0, st>>>(ah, g, F, cp);
+            else k_slab_h<false><<<grid, SB, 0, st>>>(ah, g, F, cp);
             MIFDTD_CHECK_LAUNCH("slab H launch");
         }
     }

@@ -5,6 +5,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "row_quads.hpp"
 
 namespace mifdtd {
 
@@ -162,19 +163,9 @@ __device__ __forceinline__ unsigned tfsf_mask(const STfsf &t, int ia, int ib, in
 
 struct SGeom {
     int nx, ny, nzp, nz;
-    unsigned Q;        // quads per row
     int i0;            // first plane of the slab
-    unsigned nquads;   // quads in the slab
-    int remap;         // deal the slab's blocks to XCDs in contiguous runs
+    RowQuads m;        // thread -> quad order over the slab's rows (whole-grid passes)
 };
-
-// Blocks are dealt round-robin to the 8 XCDs; renumber them so that each XCD runs a
-// contiguous run of rows and the j-1 / j+1 rows a block reads sit in its own L2.
-__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb)
-{
-    if (nb & 7u) return b;
-    return (b & 7u) * (nb >> 3) + (b >> 3);
-}
 
 __device__ __forceinline__ int sslab_e(int q, int n_e, int npml, int &side, int &p)
 {
@@ -193,11 +184,13 @@ __device__ __forceinline__ int sslab_h(int q, int n_e, int npml, int &side, int 
     return -1;
 }
 
-__device__ __forceinline__ void sapply_src(const SSrc &s, int c, int i, int j, int k0, Q4 &v)
+// Source n's value of the step is s.tval[n], or tv_row[tv[n]] where tv_row is given.
+__device__ __forceinline__ void sapply_src(const SSrc &s, int c, int i, int j, int k0, Q4 &v,
+                                           const float *tv_row = nullptr, const int *tv = nullptr)
 {
-#pragma unroll
-    for (int n = 0; n < kSMaxSrc; ++n) {
-        if (n < s.n && s.comp[n] == c && i >= s.i0[n] && i <= s.i1[n] && j >= s.j0[n] && j <= s.j1[n] &&
+#pragma unroll 1
+    for (int n = 0; n < s.n; ++n) {
+        if (s.comp[n] == c && i >= s.i0[n] && i <= s.i1[n] && j >= s.j0[n] && j <= s.j1[n] &&
             k0 + 3 >= s.k0[n] && k0 <= s.k1[n]) {
             const int lj = s.j1[n] - s.j0[n] + 1, lk = s.k1[n] - s.k0[n] + 1;
 #pragma unroll
@@ -206,7 +199,7 @@ __device__ __forceinline__ void sapply_src(const SSrc &s, int c, int i, int j, i
                 if (k >= s.k0[n] && k <= s.k1[n]) {
                     const float w = s.sv[n] ? s.sv[n][((size_t)(i - s.i0[n]) * lj + (j - s.j0[n])) * lk + (k - s.k0[n])]
                                             : s.svs[n];
-                    const float add = s.tval[n] * w;
+                    const float add = (tv_row ? tv_row[tv[n]] : s.tval[n]) * w;
                     v.v[l] = s.ow[n] ? add : v.v[l] + add;
                 }
             }
@@ -214,22 +207,33 @@ __device__ __forceinline__ void sapply_src(const SSrc &s, int c, int i, int j, i
     }
 }
 
-__device__ __forceinline__ void sprobe(const SProbe &p, int c, int i, int j, int k0, const Q4 &v)
+// row: the step's probe row (p.out where it is null).
+__device__ __forceinline__ void sprobe(const SProbe &p, int c, int i, int j, int k0, const Q4 &v, float *row = nullptr)
 {
-#pragma unroll
-    for (int n = 0; n < kSMaxProbe; ++n) {
-        if (n < p.n && p.comp[n] == c && p.i[n] == i && p.j[n] == j) {
+    float *out = row ? row : p.out;
+#pragma unroll 1
+    for (int n = 0; n < p.n; ++n) {
+        if (p.comp[n] == c && p.i[n] == i && p.j[n] == j) {
 #pragma unroll
             for (int l = 0; l < 4; ++l)
-                if (p.k[n] == k0 + l) p.out[p.slot[n]] = v.v[l];
+                if (p.k[n] == k0 + l) out[p.slot[n]] = v.v[l];
         }
     }
 }
 
-// Both passes are written load-all / compute / store-all: every global load of a quad
-// (fields, neighbours, CE, psi) is issued before the first store, so a wave pays one
-// memory round trip even on CPML cells (psi pointers may alias the fields as far as the
-// compiler knows, so a load placed after a field store would wait for it).
+// The kernel's first argument, read where it is used: tables that few waves consult
+// (sources, probes) passed as an ordinary argument are loaded into scalar registers at the
+// kernel's start (54 of them spilled to vector lanes in the E pass).
+template <class T>
+__device__ __forceinline__ const T &first_kernel_arg()
+{
+    return *(const T *)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// Both passes issue the quad's core loads (fields, neighbours, CE) and the psi of its
+// first x or y face together, then compute; the psi of a second face (the edges along z)
+// and of the z faces follow after the core update.  That keeps the passes at 6 waves per
+// SIMD; holding all six psi quads across the update took 120 VGPRs, 4 waves per SIMD.
 
 // How CE reaches the E update: the constant 0.5, three float arrays, or three uint8
 // material-index arrays into a 3 x 256 float table (same float values, so the products
@@ -249,21 +253,68 @@ __device__ __forceinline__ Q4 ce_from_table(const unsigned char *__restrict__ m,
     return q;
 }
 
+// Whole-wave lane shifts (DPP wave_shl:1 / wave_shr:1): lane i takes lane i+1's (next) or
+// lane i-1's (prev) value; the lane at the end takes 0.
+__device__ __forceinline__ float lane_next(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_prev(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, false));
+}
+
+// Sources and probes of one half step with the box [lo, hi] (quads: cells k rounded down
+// and up) around all of them: waves outside the box skip the tables.
+struct SAux {
+    int i0, i1, j0, j1, k0, k1;  // i0 > i1: none
+    SSrc src;
+    SProbe prb;
+    __device__ __forceinline__ bool near(int i, int j, int q0) const
+    {
+        return i >= i0 && i <= i1 && j >= j0 && j <= j1 && q0 + 3 >= k0 && q0 <= k1;
+    }
+};
+
+inline void aux_cover(SAux &a, int i0, int i1, int j0, int j1, int k0, int k1)
+{
+    const bool first = a.i0 > a.i1;
+    a.i0 = first || i0 < a.i0 ? i0 : a.i0;
+    a.i1 = first || i1 > a.i1 ? i1 : a.i1;
+    a.j0 = first || j0 < a.j0 ? j0 : a.j0;
+    a.j1 = first || j1 > a.j1 ? j1 : a.j1;
+    a.k0 = first || k0 < a.k0 ? k0 : a.k0;
+    a.k1 = first || k1 > a.k1 ? k1 : a.k1;
+}
+
+// The box around src's and prb's cells.
+inline void aux_box(SAux &a)
+{
+    a.i0 = 1;
+    a.i1 = 0;
+    for (int n = 0; n < a.src.n; ++n)
+        aux_cover(a, a.src.i0[n], a.src.i1[n], a.src.j0[n], a.src.j1[n], a.src.k0[n], a.src.k1[n]);
+    for (int n = 0; n < a.prb.n; ++n)
+        aux_cover(a, a.prb.i[n], a.prb.i[n], a.prb.j[n], a.prb.j[n], a.prb.k[n], a.prb.k[n]);
+}
+
 // E pass on the quad (i, j, k0..k0+3): reads E from exi.. and writes it to exo.. (the
 // same arrays for an in-place update, the next-step buffers for a ping-pong one); psi E
 // is read from cp.pe and written to cp.pe_out.  CE: CM = 0 the constant 0.5, 1 the float
 // arrays cex.., 2 the uint8 material indices mx.. into tab ([3][256] floats, the same
-// values as the arrays, so the products are identical).
+// values as the arrays, so the products are identical).  next: the next lane holds the
+// quad at k0+4 (else this lane loads its k0+4 neighbours itself).
 constexpr int kFeatDrude = 1, kFeatTfsf = 2;  // optional E-pass features (template bits)
 
 template <int CM, bool PML, int FEAT = 0>
 __device__ __forceinline__ void e_quad_at(
-    const SGeom &g, int i, int j, int k0, const float *exi, const float *eyi, const float *ezi, float *exo,
+    const SGeom &g, int i, int j, int k0, bool next, const float *exi, const float *eyi, const float *ezi, float *exo,
     float *eyo, float *ezo, const float *__restrict__ hx, const float *__restrict__ hy, const float *__restrict__ hz,
     const float *__restrict__ cex, const float *__restrict__ cey, const float *__restrict__ cez,
-    const SCpml &cp, const SSrc &src, const SProbe &prb, const unsigned char *__restrict__ mx = nullptr,
+    const SCpml &cp, const SAux &aux, const unsigned char *__restrict__ mx = nullptr,
     const unsigned char *__restrict__ my = nullptr, const unsigned char *__restrict__ mz = nullptr,
-    const float *tab = nullptr, const SDrude *dr = nullptr, const STfsf *tf = nullptr)
+    const float *tab = nullptr, const SDrude *dr = nullptr, const STfsf *tf = nullptr, float *prow = nullptr,
+    const float *tv_row = nullptr, const int *tv = nullptr)
 {
     constexpr bool DR = (FEAT & kFeatDrude) != 0;
     constexpr bool TF = (FEAT & kFeatTfsf) != 0;
@@ -281,59 +332,50 @@ __device__ __forceinline__ void e_quad_at(
     const Q4 c2 = CM == 2 ? ce_from_table(mz + id, tab + 512) : CM ? ld4(cez + id) : splat4(0.5f);
     const Q4 hzU = jy ? ld4(hz + id + nzp) : z4;   // hz(j+1)
     const Q4 hxU = jy ? ld4(hx + id + nzp) : z4;   // hx(j+1)
-    const float hyn = jy ? hy[id + 4] : 0.f;       // hy(k0+4): next quad / next row start
     const Q4 hzN = ix ? ld4(hz + id + sx) : z4;    // hz(i+1)
     const Q4 hyN = ix ? ld4(hy + id + sx) : z4;    // hy(i+1)
-    const float hxn = ix ? hx[id + 4] : 0.f;       // hx(k0+4)
+    // hy, hx at k0+4: the next quad / next row's start
+    float hyn = 0.f, hxn = 0.f;
+    if (!next) {
+        if (jy) hyn = hy[id + 4];
+        if (ix) hxn = hx[id + 4];
+    }
 
     const int npml = PML ? cp.npml : 0;
     int xs = 0, xp = 0, ys = 0, yp = 0, xt = -1, yt = -1;
-    Q4 px1 = z4, px2 = z4, py1 = z4, py2 = z4;
-    size_t ox1 = 0, ox2 = 0, oy1 = 0, oy2 = 0;  // psi offsets of the x / y face quads
-    float pz1[4] = {0.f, 0.f, 0.f, 0.f}, pz2[4] = {0.f, 0.f, 0.f, 0.f};
-    int zt[4] = {-1, -1, -1, -1};
-    bool anyz = false;
+    Q4 p1 = z4, p2 = z4;   // psi of the x face, or of the y face where there is no x face
+    size_t o1 = 0, o2 = 0;
     if (PML) {
         xt = (cp.axes & 1) ? sslab_e(i, nx, npml, xs, xp) : -1;  // x slab planes are all < nx-1
-        if (xt > 0) {
-            const size_t o = ((size_t)xp * ny + j) * nzp + k0;
-            ox1 = cp.off(xs, 0) + o;
-            ox2 = cp.off(xs, 1) + o;
-            px1 = ld4(cp.pe + ox1);
-            px2 = ld4(cp.pe + ox2);
-        }
         yt = (cp.axes & 2) ? sslab_e(j, ny, npml, ys, yp) : -1;  // y slab rows are all < ny-1
-        if (yt > 0) {
-            const size_t o = ((size_t)i * npml + yp) * nzp + k0;
-            oy1 = cp.off(2 + ys, 0) + o;
-            oy2 = cp.off(2 + ys, 1) + o;
-            py1 = ld4(cp.pe + oy1);
-            py2 = ld4(cp.pe + oy2);
-        }
-        if ((cp.axes & 4) && (k0 < npml || k0 + 3 >= nz - 1 - npml)) {
-            const size_t o = ((size_t)i * ny + j) * npml;
-#pragma unroll
-            for (int l = 0; l < 4; ++l) {
-                int zs, zp;
-                zt[l] = sslab_e(k0 + l, nz, npml, zs, zp);
-                if (zt[l] > 0) {
-                    const float *q = cp.pe + cp.off(4 + zs, 0) + o + zp;  // psi2 sits sZ after psi1
-                    pz1[l] = q[0];
-                    pz2[l] = q[cp.sZ];
-                    anyz = true;
-                }
-            }
+        if (xt > 0 || yt > 0) {
+            const size_t o = xt > 0 ? ((size_t)xp * ny + j) * nzp + k0 : ((size_t)i * npml + yp) * nzp + k0;
+            const int f = xt > 0 ? xs : 2 + ys;
+            o1 = cp.off(f, 0) + o;
+            o2 = cp.off(f, 1) + o;
+            p1 = ld4(cp.pe + o1);
+            p2 = ld4(cp.pe + o2);
         }
     }
 
     // -------------------------------------------------------------- compute
     // ex: += cex*((hz[j+1]-hz) - (hy[k+1]-hy)) ; CPML + y psi2 (hz), - z psi1 (hy)
+    // ey: += cey*((hx[k+1]-hx) - (hz[i+1]-hz)) ; CPML - x psi1 (hz), + z psi2 (hx)
+    // ez: += cez*((hy[i+1]-hy) - (hx[j+1]-hx)) ; CPML + x psi2 (hy), - y psi1 (hx)
+    const float y3 = lane_next(hy0.v[0]), x3 = lane_next(hx0.v[0]);  // every lane of the wave takes part
+    if (next) {
+        hyn = y3;
+        hxn = x3;
+    }
     // Drude box: J' of the three components (rows inside the box)
     const bool drow = DR && dr->row_in(i, j);
     Q4 jn0 = z4, jn1 = z4, jn2 = z4;
-    float y1[4];
+    float y1[4], x1[4];
 #pragma unroll
-    for (int l = 0; l < 4; ++l) y1[l] = l < 3 ? hy0.v[l + 1] : hyn;
+    for (int l = 0; l < 4; ++l) {
+        y1[l] = l < 3 ? hy0.v[l + 1] : hyn;
+        x1[l] = l < 3 ? hx0.v[l + 1] : hxn;
+    }
     if (jy) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
@@ -341,32 +383,6 @@ __device__ __forceinline__ void e_quad_at(
             e0.v[l] = (k0 + l < nz - 1) ? v : v * 0.f;
         }
     }
-    if (drow) drude_quad(*dr, 0, i, j, k0, c0, e0, jn0);
-    if (jy) {
-        if (PML) {
-            if (yt > 0) {
-                const float b = cp.bE[yt], a = cp.aE[yt];
-#pragma unroll
-                for (int l = 0; l < 4; ++l)
-                    if (k0 + l < nz - 1) {
-                        const float tt = b * py2.v[l] + a * (hzU.v[l] - hz0.v[l]);
-                        py2.v[l] = tt;
-                        e0.v[l] = e0.v[l] + c0.v[l] * tt;
-                    }
-            }
-#pragma unroll
-            for (int l = 0; l < 4; ++l)
-                if (zt[l] > 0) {
-                    const float tt = cp.bE[zt[l]] * pz1[l] + cp.aE[zt[l]] * (y1[l] - hy0.v[l]);
-                    pz1[l] = tt;
-                    e0.v[l] = e0.v[l] - c0.v[l] * tt;
-                }
-        }
-    }
-    // ey: += cey*((hx[k+1]-hx) - (hz[i+1]-hz)) ; CPML - x psi1 (hz), + z psi2 (hx)
-    float x1[4];
-#pragma unroll
-    for (int l = 0; l < 4; ++l) x1[l] = l < 3 ? hx0.v[l + 1] : hxn;
     if (ix) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
@@ -374,29 +390,6 @@ __device__ __forceinline__ void e_quad_at(
             e1.v[l] = (k0 + l < nz - 1) ? v : v * 0.f;
         }
     }
-    if (drow) drude_quad(*dr, 1, i, j, k0, c1, e1, jn1);
-    if (ix) {
-        if (PML) {
-            if (xt > 0) {
-                const float b = cp.bE[xt], a = cp.aE[xt];
-#pragma unroll
-                for (int l = 0; l < 4; ++l)
-                    if (k0 + l < nz - 1) {
-                        const float tt = b * px1.v[l] + a * (hzN.v[l] - hz0.v[l]);
-                        px1.v[l] = tt;
-                        e1.v[l] = e1.v[l] - c1.v[l] * tt;
-                    }
-            }
-#pragma unroll
-            for (int l = 0; l < 4; ++l)
-                if (zt[l] > 0) {
-                    const float tt = cp.bE[zt[l]] * pz2[l] + cp.aE[zt[l]] * (x1[l] - hx0.v[l]);
-                    pz2[l] = tt;
-                    e1.v[l] = e1.v[l] + c1.v[l] * tt;
-                }
-        }
-    }
-    // ez: += cez*((hy[i+1]-hy) - (hx[j+1]-hx)) ; CPML + x psi2 (hy), - y psi1 (hx)
     if (ix && jy) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
@@ -404,34 +397,90 @@ __device__ __forceinline__ void e_quad_at(
             e2.v[l] = (k0 + l < nz) ? v : v * 0.f;
         }
     }
-    if (drow) drude_quad(*dr, 2, i, j, k0, c2, e2, jn2);
-    if (ix && jy) {
-        if (PML) {
-            if (xt > 0) {
-                const float b = cp.bE[xt], a = cp.aE[xt];
+    if (drow) {
+        drude_quad(*dr, 0, i, j, k0, c0, e0, jn0);
+        drude_quad(*dr, 1, i, j, k0, c1, e1, jn1);
+        drude_quad(*dr, 2, i, j, k0, c2, e2, jn2);
+    }
+    if (PML) {
+        if (xt > 0) {  // psi1: ey, psi2: ez
+            const float b = cp.bE[xt], a = cp.aE[xt];
+#pragma unroll
+            for (int l = 0; l < 4; ++l)
+                if (k0 + l < nz - 1) {
+                    const float tt = b * p1.v[l] + a * (hzN.v[l] - hz0.v[l]);
+                    p1.v[l] = tt;
+                    e1.v[l] = e1.v[l] - c1.v[l] * tt;
+                }
+            if (jy) {
 #pragma unroll
                 for (int l = 0; l < 4; ++l)
                     if (k0 + l < nz) {
-                        const float tt = b * px2.v[l] + a * (hyN.v[l] - hy0.v[l]);
-                        px2.v[l] = tt;
+                        const float tt = b * p2.v[l] + a * (hyN.v[l] - hy0.v[l]);
+                        p2.v[l] = tt;
                         e2.v[l] = e2.v[l] + c2.v[l] * tt;
                     }
             }
-            if (yt > 0) {
-                const float b = cp.bE[yt], a = cp.aE[yt];
+            st4(cp.pe_out + o1, p1);
+            st4(cp.pe_out + o2, p2);
+        }
+        if (yt > 0) {  // psi1: ez, psi2: ex
+            if (xt > 0) {
+                const size_t o = ((size_t)i * npml + yp) * nzp + k0;
+                o1 = cp.off(2 + ys, 0) + o;
+                o2 = cp.off(2 + ys, 1) + o;
+                p1 = ld4(cp.pe + o1);
+                p2 = ld4(cp.pe + o2);
+            }
+            const float b = cp.bE[yt], a = cp.aE[yt];
+#pragma unroll
+            for (int l = 0; l < 4; ++l)
+                if (k0 + l < nz - 1) {
+                    const float tt = b * p2.v[l] + a * (hzU.v[l] - hz0.v[l]);
+                    p2.v[l] = tt;
+                    e0.v[l] = e0.v[l] + c0.v[l] * tt;
+                }
+            if (ix) {
 #pragma unroll
                 for (int l = 0; l < 4; ++l)
                     if (k0 + l < nz) {
-                        const float tt = b * py1.v[l] + a * (hxU.v[l] - hx0.v[l]);
-                        py1.v[l] = tt;
+                        const float tt = b * p1.v[l] + a * (hxU.v[l] - hx0.v[l]);
+                        p1.v[l] = tt;
                         e2.v[l] = e2.v[l] - c2.v[l] * tt;
                     }
             }
+            st4(cp.pe_out + o1, p1);
+            st4(cp.pe_out + o2, p2);
+        }
+        if ((cp.axes & 4) && (k0 < npml || (k0 + 3 >= nz - 1 - npml && k0 < nz - 1))) {  // psi1: ex, psi2: ey
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                int zs, zp;
+                const int zt = sslab_e(k0 + l, nz, npml, zs, zp);
+                if (zt > 0) {
+                    const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
+                    const float b = cp.bE[zt], a = cp.aE[zt];
+                    const float q1 = cp.pe[o], q2 = cp.pe[o + cp.sZ];
+                    if (jy) {
+                        const float tt = b * q1 + a * (y1[l] - hy0.v[l]);
+                        cp.pe_out[o] = tt;
+                        e0.v[l] = e0.v[l] - c0.v[l] * tt;
+                    }
+                    if (ix) {
+                        const float tt = b * q2 + a * (x1[l] - hx0.v[l]);
+                        cp.pe_out[o + cp.sZ] = tt;
+                        e1.v[l] = e1.v[l] + c1.v[l] * tt;
+                    }
+                }
+            }
         }
     }
-    sapply_src(src, 0, i, j, k0, e0);
-    sapply_src(src, 1, i, j, k0, e1);
-    sapply_src(src, 2, i, j, k0, e2);
+    const bool near = aux.near(i, j, k0);
+    if (near) {
+        sapply_src(aux.src, 0, i, j, k0, e0, tv_row, tv);
+        sapply_src(aux.src, 1, i, j, k0, e1, tv_row, tv);
+        sapply_src(aux.src, 2, i, j, k0, e2, tv_row, tv);
+    }
     if (TF) tfsf_quad(*tf, 0, i, j, k0, e0, e1, e2);
 
     // --------------------------------------------------------------- stores
@@ -444,58 +493,22 @@ __device__ __forceinline__ void e_quad_at(
         drude_store(*dr, 1, i, j, k0, jn1);
         drude_store(*dr, 2, i, j, k0, jn2);
     }
-    if (PML) {
-        if (xt > 0) {
-            st4(cp.pe_out + ox1, px1);
-            st4(cp.pe_out + ox2, px2);
-        }
-        if (yt > 0) {
-            st4(cp.pe_out + oy1, py1);
-            st4(cp.pe_out + oy2, py2);
-        }
-        if (anyz) {
-#pragma unroll
-            for (int l = 0; l < 4; ++l)
-                if (zt[l] > 0) {
-                    int zs, zp;
-                    sslab_e(k0 + l, nz, npml, zs, zp);
-                    float *q = cp.pe_out + cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
-                    if (jy) q[0] = pz1[l];
-                    if (ix) q[cp.sZ] = pz2[l];
-                }
-        }
+    if (near) {
+        sprobe(aux.prb, 0, i, j, k0, e0, prow);
+        sprobe(aux.prb, 1, i, j, k0, e1, prow);
+        sprobe(aux.prb, 2, i, j, k0, e2, prow);
     }
-    sprobe(prb, 0, i, j, k0, e0);
-    sprobe(prb, 1, i, j, k0, e1);
-    sprobe(prb, 2, i, j, k0, e2);
-}
-
-// E pass on quad f of the slab described by g (in place); CE as in e_quad_at (CM = 2:
-// the material indices mx.. into tab).
-template <int CM, bool PML>
-__device__ __forceinline__ void e_quad(
-    const SGeom &g, unsigned f, float *ex, float *ey, float *ez,
-    const float *__restrict__ hx, const float *__restrict__ hy, const float *__restrict__ hz,
-    const float *__restrict__ cex, const float *__restrict__ cey, const float *__restrict__ cez,
-    const SCpml &cp, const SSrc &src, const SProbe &prb, const unsigned char *__restrict__ mx = nullptr,
-    const unsigned char *__restrict__ my = nullptr, const unsigned char *__restrict__ mz = nullptr,
-    const float *tab = nullptr)
-{
-    const unsigned row = f / g.Q;
-    const int k0 = (int)(f - row * g.Q) * 4;
-    const int di = (int)(row / (unsigned)g.ny);
-    const int j = (int)row - di * g.ny;
-    e_quad_at<CM, PML>(g, g.i0 + di, j, k0, ex, ey, ez, ex, ey, ez, hx, hy, hz, cex, cey, cez, cp, src, prb, mx, my,
-                       mz, tab);
 }
 
 // H pass on the quad (i, j, k0..k0+3): reads H from hxi.. and writes it to hxo.. (the
-// same arrays for an in-place update); psi H is updated in place (cp.ph).
+// same arrays for an in-place update); psi H is updated in place (cp.ph).  prev: the
+// previous lane holds the quad at k0-4.
 template <bool PML>
 __device__ __forceinline__ void h_quad_at(
-    const SGeom &g, int i, int j, int k0, const float *__restrict__ ex, const float *__restrict__ ey,
+    const SGeom &g, int i, int j, int k0, bool prev, const float *__restrict__ ex, const float *__restrict__ ey,
     const float *__restrict__ ez, const float *hxi, const float *hyi, const float *hzi, float *hxo, float *hyo,
-    float *hzo, const SCpml &cp, const SSrc &src, const SProbe &prb, const STfsf *tf = nullptr)
+    float *hzo, const SCpml &cp, const SAux &aux, const STfsf *tf = nullptr, float *prow = nullptr,
+    const float *tv_row = nullptr, const int *tv = nullptr)
 {
     const int nx = g.nx, ny = g.ny, nzp = g.nzp, nz = g.nz;
     (void)nx;
@@ -509,60 +522,47 @@ __device__ __forceinline__ void h_quad_at(
     Q4 h0 = ld4(hxi + id), h1 = ld4(hyi + id), h2 = ld4(hzi + id);
     const Q4 ezD = jp ? ld4(ez + id - nzp) : z4;   // ez(j-1)
     const Q4 exD = jp ? ld4(ex + id - nzp) : z4;   // ex(j-1)
-    const float eyp = jp ? ey[id - 1] : 0.f;       // ey(k0-1): previous quad / previous row end
     const Q4 ezB = ip ? ld4(ez + id - sx) : z4;    // ez(i-1)
     const Q4 eyB = ip ? ld4(ey + id - sx) : z4;    // ey(i-1)
-    const float exp_ = ip ? ex[id - 1] : 0.f;      // ex(k0-1)
+    // ey, ex at k0-1: the previous quad / previous row's end
+    float eyp = 0.f, exp_ = 0.f;
+    if (!prev) {
+        if (jp) eyp = ey[id - 1];
+        if (ip) exp_ = ex[id - 1];
+    }
 
     const int npml = PML ? cp.npml : 0;
     int xs = 0, xp = 0, ys = 0, yp = 0, xt = -1, yt = -1;
-    Q4 px1 = z4, px2 = z4, py1 = z4, py2 = z4;
-    float *ppx1 = nullptr, *ppx2 = nullptr, *ppy1 = nullptr, *ppy2 = nullptr;
-    float pz1[4] = {0.f, 0.f, 0.f, 0.f}, pz2[4] = {0.f, 0.f, 0.f, 0.f};
-    int zt[4] = {-1, -1, -1, -1};
-    bool anyz = false;
+    Q4 p1 = z4, p2 = z4;   // psi of the x face, or of the y face where there is no x face
+    size_t o1 = 0, o2 = 0;
     if (PML) {
         xt = ip && (cp.axes & 1) ? sslab_h(i, nx, npml, xs, xp) : -1;  // plane 0 is the wall
-        if (xt > 0) {
-            const size_t o = ((size_t)xp * ny + j) * nzp + k0;
-            ppx1 = cp.ph + cp.off(xs, 0) + o;
-            ppx2 = cp.ph + cp.off(xs, 1) + o;
-            px1 = ld4(ppx1);
-            px2 = ld4(ppx2);
-        }
         yt = jp && (cp.axes & 2) ? sslab_h(j, ny, npml, ys, yp) : -1;  // row 0 is the wall
-        if (yt > 0) {
-            const size_t o = ((size_t)i * npml + yp) * nzp + k0;
-            ppy1 = cp.ph + cp.off(2 + ys, 0) + o;
-            ppy2 = cp.ph + cp.off(2 + ys, 1) + o;
-            py1 = ld4(ppy1);
-            py2 = ld4(ppy2);
-        }
-        if ((cp.axes & 4) && (k0 < npml || k0 + 3 >= nz - npml)) {
-            const size_t o = ((size_t)i * ny + j) * npml;
-#pragma unroll
-            for (int l = 0; l < 4; ++l) {
-                int zs, zp;
-                const int k = k0 + l;
-                zt[l] = k > 0 ? sslab_h(k, nz, npml, zs, zp) : -1;  // k = 0 is the wall
-                if (zt[l] > 0) {
-                    const float *q = cp.ph + cp.off(4 + zs, 0) + o + zp;
-                    pz1[l] = q[0];
-                    pz2[l] = q[cp.sZ];
-                    anyz = true;
-                }
-            }
+        if (xt > 0 || yt > 0) {
+            const size_t o = xt > 0 ? ((size_t)xp * ny + j) * nzp + k0 : ((size_t)i * npml + yp) * nzp + k0;
+            const int f = xt > 0 ? xs : 2 + ys;
+            o1 = cp.off(f, 0) + o;
+            o2 = cp.off(f, 1) + o;
+            p1 = ld4(cp.ph + o1);
+            p2 = ld4(cp.ph + o2);
         }
     }
 
     // -------------------------------------------------------------- compute
+    // hx: j>0 ; -= 0.5*((ez - ez[j-1]) - (ey - ey[k-1])) ; CPML - y psi2 (ez), + z psi1 (ey)
+    // hy: i>0 ; -= 0.5*((ex - ex[k-1]) - (ez - ez[i-1])) ; CPML + x psi1 (ez), - z psi2 (ex)
+    // hz: i, j>0 ; -= 0.5*((ey - ey[i-1]) - (ex - ex[j-1])) ; CPML - x psi2 (ey), + y psi1 (ex)
+    const float y3 = lane_prev(ey0.v[3]), x3 = lane_prev(ex0.v[3]);  // every lane of the wave takes part
+    if (prev) {
+        eyp = y3;
+        exp_ = x3;
+    }
     float ym[4], xm[4];
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
         ym[l] = l > 0 ? ey0.v[l - 1] : eyp;
         xm[l] = l > 0 ? ex0.v[l - 1] : exp_;
     }
-    // hx: j>0 ; -= 0.5*((ez - ez[j-1]) - (ey - ey[k-1])) ; CPML - y psi2 (ez), + z psi1 (ey)
     if (jp) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
@@ -570,135 +570,135 @@ __device__ __forceinline__ void h_quad_at(
             const int k = k0 + l;
             h0.v[l] = (k > 0 && k < nz) ? v : v * 0.f;
         }
-        if (PML) {
-            if (yt > 0) {
-                const float b = cp.bH[yt], a = cp.aH[yt];
-#pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const int k = k0 + l;
-                    if (k > 0 && k < nz) {
-                        const float tt = b * py2.v[l] + a * (ez0.v[l] - ezD.v[l]);
-                        py2.v[l] = tt;
-                        h0.v[l] = h0.v[l] - 0.5f * tt;
-                    }
-                }
-            }
-#pragma unroll
-            for (int l = 0; l < 4; ++l)
-                if (zt[l] > 0) {
-                    const float tt = cp.bH[zt[l]] * pz1[l] + cp.aH[zt[l]] * (ey0.v[l] - ym[l]);
-                    pz1[l] = tt;
-                    h0.v[l] = h0.v[l] + 0.5f * tt;
-                }
-        }
     }
     if (ip) {
-        // hy: -= 0.5*((ex - ex[k-1]) - (ez - ez[i-1])) ; CPML + x psi1 (ez), - z psi2 (ex)
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             const float v = h1.v[l] - 0.5f * ((ex0.v[l] - xm[l]) - (ez0.v[l] - ezB.v[l]));
             const int k = k0 + l;
             h1.v[l] = (k > 0 && k < nz) ? v : v * 0.f;
         }
-        if (PML) {
-            if (xt > 0) {
-                const float b = cp.bH[xt], a = cp.aH[xt];
+    }
+    if (ip && jp) {
 #pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const int k = k0 + l;
-                    if (k > 0 && k < nz) {
-                        const float tt = b * px1.v[l] + a * (ez0.v[l] - ezB.v[l]);
-                        px1.v[l] = tt;
-                        h1.v[l] = h1.v[l] + 0.5f * tt;
-                    }
-                }
-            }
-#pragma unroll
-            for (int l = 0; l < 4; ++l)
-                if (zt[l] > 0) {
-                    const float tt = cp.bH[zt[l]] * pz2[l] + cp.aH[zt[l]] * (ex0.v[l] - xm[l]);
-                    pz2[l] = tt;
-                    h1.v[l] = h1.v[l] - 0.5f * tt;
-                }
+        for (int l = 0; l < 4; ++l) {
+            const float v = h2.v[l] - 0.5f * ((ey0.v[l] - eyB.v[l]) - (ex0.v[l] - exD.v[l]));
+            h2.v[l] = (k0 + l < nz) ? v : v * 0.f;
         }
-        // hz: j>0 ; -= 0.5*((ey - ey[i-1]) - (ex - ex[j-1])) ; CPML - x psi2 (ey), + y psi1 (ex)
-        if (jp) {
+    }
+    if (PML) {
+        if (xt > 0) {  // psi1: hy, psi2: hz
+            const float b = cp.bH[xt], a = cp.aH[xt];
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                const float v = h2.v[l] - 0.5f * ((ey0.v[l] - eyB.v[l]) - (ex0.v[l] - exD.v[l]));
-                h2.v[l] = (k0 + l < nz) ? v : v * 0.f;
-            }
-            if (PML) {
-                if (xt > 0) {
-                    const float b = cp.bH[xt], a = cp.aH[xt];
-#pragma unroll
-                    for (int l = 0; l < 4; ++l)
-                        if (k0 + l < nz) {
-                            const float tt = b * px2.v[l] + a * (ey0.v[l] - eyB.v[l]);
-                            px2.v[l] = tt;
-                            h2.v[l] = h2.v[l] - 0.5f * tt;
-                        }
+                const int k = k0 + l;
+                if (k > 0 && k < nz) {
+                    const float tt = b * p1.v[l] + a * (ez0.v[l] - ezB.v[l]);
+                    p1.v[l] = tt;
+                    h1.v[l] = h1.v[l] + 0.5f * tt;
                 }
-                if (yt > 0) {
-                    const float b = cp.bH[yt], a = cp.aH[yt];
+            }
+            if (jp) {
 #pragma unroll
-                    for (int l = 0; l < 4; ++l)
-                        if (k0 + l < nz) {
-                            const float tt = b * py1.v[l] + a * (ex0.v[l] - exD.v[l]);
-                            py1.v[l] = tt;
-                            h2.v[l] = h2.v[l] + 0.5f * tt;
-                        }
+                for (int l = 0; l < 4; ++l)
+                    if (k0 + l < nz) {
+                        const float tt = b * p2.v[l] + a * (ey0.v[l] - eyB.v[l]);
+                        p2.v[l] = tt;
+                        h2.v[l] = h2.v[l] - 0.5f * tt;
+                    }
+            }
+            st4(cp.ph + o1, p1);
+            st4(cp.ph + o2, p2);
+        }
+        if (yt > 0) {  // psi1: hz, psi2: hx
+            if (xt > 0) {
+                const size_t o = ((size_t)i * npml + yp) * nzp + k0;
+                o1 = cp.off(2 + ys, 0) + o;
+                o2 = cp.off(2 + ys, 1) + o;
+                p1 = ld4(cp.ph + o1);
+                p2 = ld4(cp.ph + o2);
+            }
+            const float b = cp.bH[yt], a = cp.aH[yt];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                const int k = k0 + l;
+                if (k > 0 && k < nz) {
+                    const float tt = b * p2.v[l] + a * (ez0.v[l] - ezD.v[l]);
+                    p2.v[l] = tt;
+                    h0.v[l] = h0.v[l] - 0.5f * tt;
+                }
+            }
+            if (ip) {
+#pragma unroll
+                for (int l = 0; l < 4; ++l)
+                    if (k0 + l < nz) {
+                        const float tt = b * p1.v[l] + a * (ex0.v[l] - exD.v[l]);
+                        p1.v[l] = tt;
+                        h2.v[l] = h2.v[l] + 0.5f * tt;
+                    }
+            }
+            st4(cp.ph + o1, p1);
+            st4(cp.ph + o2, p2);
+        }
+        if ((cp.axes & 4) && (k0 < npml || (k0 + 3 >= nz - npml && k0 < nz))) {  // psi1: hx, psi2: hy
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                int zs, zp;
+                const int k = k0 + l;
+                const int zt = k > 0 ? sslab_h(k, nz, npml, zs, zp) : -1;  // k = 0 is the wall
+                if (zt > 0) {
+                    const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
+                    const float b = cp.bH[zt], a = cp.aH[zt];
+                    const float q1 = cp.ph[o], q2 = cp.ph[o + cp.sZ];
+                    if (jp) {
+                        const float tt = b * q1 + a * (ey0.v[l] - ym[l]);
+                        cp.ph[o] = tt;
+                        h0.v[l] = h0.v[l] + 0.5f * tt;
+                    }
+                    if (ip) {
+                        const float tt = b * q2 + a * (ex0.v[l] - xm[l]);
+                        cp.ph[o + cp.sZ] = tt;
+                        h1.v[l] = h1.v[l] - 0.5f * tt;
+                    }
                 }
             }
         }
     }
-    sapply_src(src, 3, i, j, k0, h0);
-    sapply_src(src, 4, i, j, k0, h1);
-    sapply_src(src, 5, i, j, k0, h2);
+    const bool near = aux.near(i, j, k0);
+    if (near) {
+        sapply_src(aux.src, 3, i, j, k0, h0, tv_row, tv);
+        sapply_src(aux.src, 4, i, j, k0, h1, tv_row, tv);
+        sapply_src(aux.src, 5, i, j, k0, h2, tv_row, tv);
+    }
     if (tf) tfsf_quad(*tf, 3, i, j, k0, h0, h1, h2);
 
     // --------------------------------------------------------------- stores
     st4(hxo + id, h0);
     st4(hyo + id, h1);
     st4(hzo + id, h2);
-    if (PML) {
-        if (xt > 0) {
-            st4(ppx1, px1);
-            st4(ppx2, px2);
-        }
-        if (yt > 0) {
-            st4(ppy1, py1);
-            st4(ppy2, py2);
-        }
-        if (anyz) {
-            const size_t o = ((size_t)i * ny + j) * npml;
-#pragma unroll
-            for (int l = 0; l < 4; ++l)
-                if (zt[l] > 0) {
-                    int zs, zp;
-                    sslab_h(k0 + l, nz, npml, zs, zp);
-                    float *q = cp.ph + cp.off(4 + zs, 0) + o + zp;
-                    if (jp) q[0] = pz1[l];
-                    if (ip) q[cp.sZ] = pz2[l];
-                }
-        }
+    if (near) {
+        sprobe(aux.prb, 3, i, j, k0, h0, prow);
+        sprobe(aux.prb, 4, i, j, k0, h1, prow);
+        sprobe(aux.prb, 5, i, j, k0, h2, prow);
     }
-    sprobe(prb, 3, i, j, k0, h0);
-    sprobe(prb, 4, i, j, k0, h1);
-    sprobe(prb, 5, i, j, k0, h2);
 }
 
-// H pass on quad f of the slab described by g (in place).
-template <bool PML>
-__device__ __forceinline__ void h_quad(
-    const SGeom &g, unsigned f, const float *__restrict__ ex, const float *__restrict__ ey, const float *__restrict__ ez,
-    float *hx, float *hy, float *hz, const SCpml &cp, const SSrc &src, const SProbe &prb)
+// Cells of this thread in the whole-grid passes; false for an idle thread.
+struct RowAt {
+    int i, j, k0;
+    bool next, prev;
+};
+
+__device__ __forceinline__ bool slab_quad(const SGeom &g, unsigned b, RowAt &r)
 {
-    const unsigned row = f / g.Q;
-    const int k0 = (int)(f - row * g.Q) * 4;
-    const int di = (int)(row / (unsigned)g.ny);
-    const int j = (int)row - di * g.ny;
-    h_quad_at<PML>(g, g.i0 + di, j, k0, ex, ey, ez, hx, hy, hz, hx, hy, hz, cp, src, prb);
+    const QuadAt a = row_quad(g.m, b, threadIdx.x);
+    const int lane = threadIdx.x & 63;
+    r.i = g.i0 + a.i;
+    r.j = a.j;
+    r.k0 = 4 * a.q;
+    r.next = a.next && lane < 63;
+    r.prev = a.prev && lane > 0;
+    return a.active;
 }
 
 struct SFields {
