@@ -1,12 +1,14 @@
 // Batched whole-step engine: many independent Yee + CPML simulations of uneven sizes
-// advanced together, two launches per step for the whole batch (E pass of every
-// instance, then H pass of every instance).
+// advanced together, two launches per step for each group of instances (E pass of every
+// instance of the group, then H pass).
 //
 // A launch's blocks are the concatenation of each instance's blocks (instance order);
 // block b finds its instance by binary search in the block-prefix table and runs the
 // same per-quad E/H update as the slab engine (core + CPML + sources + probes), so small
-// instances no longer leave the GPU idle between launches and a batch of N instances
-// costs 2 launches per step instead of 2N.  Per-instance descriptors live in device
+// instances do not leave the GPU idle between launches.  The instances do not depend on
+// each other, so a run takes one group after the other through all of its steps: a
+// group's fields stay in the last-level cache from one half step to the next (kGroupBytes),
+// where the whole batch at once streams from HBM.  Per-instance descriptors live in device
 // memory (built once by mifdtd_batch_create); the per-step source values and probe
 // outputs are rows of device arrays indexed by the step.  Optionally the launches of a
 // run are captured once into a hipGraph and replayed as one graph launch.
@@ -18,6 +20,12 @@
 
 namespace mifdtd {
 
+// Working set of a launch group: as much as stays in the 256 MiB last-level cache from one
+// half step to the next.  64 uneven cubes of 64 to 192 cells (5.2 GB), 40 steps, ms per
+// step: 16 MiB 3.01, 64 MiB 2.91, 128 MiB 2.83, 160 MiB 2.79, 200 MiB 2.72, 256 MiB 2.83,
+// 400 MiB 3.48, one launch for the whole batch 3.63.
+constexpr size_t kGroupBytes = (size_t)200 << 20;
+
 struct BInst {
     SGeom g;          // whole instance: i0 = 0
     SFields F;
@@ -26,7 +34,8 @@ struct BInst {
     int tv_e[kSMaxSrc], tv_h[kSMaxSrc];  // column of each source's value in a tvals row
 };
 
-// Renumber instance-local block b so each XCD takes R consecutive blocks in turn.
+// Renumber instance-local block b so each XCD takes R consecutive blocks in turn (R = 0: the
+// row order's own stripes, one per XCD; 64 uneven cubes: 2.72 ms per step, R = 16 3.26).
 __device__ __forceinline__ unsigned xcd_rows(unsigned b, unsigned nb, unsigned R)
 {
     if (R == 0) return b;
@@ -40,11 +49,11 @@ __device__ __forceinline__ unsigned xcd_rows(unsigned b, unsigned nb, unsigned R
 // CM: CeMode of the E pass (kCeTable: the instance's material indices and table).
 template <int CM, bool PML, bool EHALF>
 __global__ __launch_bounds__(SB) void k_batch(const BInst *__restrict__ inst, const unsigned *__restrict__ first_block,
-                                             int ninst, const float *__restrict__ tv_row, float *probe_row,
-                                             unsigned remap_rows)
+                                             int inst0, int inst1, unsigned block0, const float *__restrict__ tv_row,
+                                             float *probe_row, unsigned remap_rows)
 {
-    const unsigned b = blockIdx.x;
-    int lo = 0, hi = ninst;  // first_block[lo] <= b < first_block[hi]
+    const unsigned b = block0 + blockIdx.x;
+    int lo = inst0, hi = inst1;  // first_block[lo] <= b < first_block[hi]
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         if (first_block[mid] <= b) lo = mid;
@@ -67,6 +76,12 @@ __global__ __launch_bounds__(SB) void k_batch(const BInst *__restrict__ inst, co
 
 using namespace mifdtd;
 
+// Consecutive instances that one launch advances.
+struct BGroup {
+    int i0, i1;            // instances [i0, i1)
+    unsigned b0, nblocks;  // their blocks
+};
+
 // What the launches of a batch need besides the device descriptors.
 struct BMeta {
     int ninst = 0;
@@ -74,6 +89,7 @@ struct BMeta {
     bool pml = false;
     unsigned total_blocks = 0;
     int total_src = 0, total_probe = 0;
+    std::vector<BGroup> groups;  // launch groups, in instance order
 };
 
 // Validate the instances and fill h[0..ninst) and first[0..ninst] (host arrays).
@@ -87,6 +103,8 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
     int batch_npml = 0;  // the one npml of the shared 2*(npml+1)-entry tables
     int tsrc = 0, tprobe = 0;
     unsigned long long blocks = 0;
+    size_t group_bytes = 0;
+    m.groups.clear();
     for (int n = 0; n < ninst; n++) {
         const mifdtd_instance &d = inst[n];
         const int nx = d.nx, ny = d.ny, nzp = d.nz_pitch, pad = d.pad;
@@ -188,6 +206,15 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
         first[n] = (unsigned)blocks;
         blocks += (row_quads_blocks(B.g.m) + kStripes - 1) / kStripes * kStripes;  // block % 8 is the stripe
         if (blocks >= (1ull << 31)) return fail(MIFDTD_ERANGE, "batch exceeds 2^31 blocks");
+        const size_t bytes = (size_t)nx * ny * nzp * (24 + (tbl ? 3 : hc ? 12 : 0)) +
+                             (d.npml > 0 ? 32 * (B.cp.sX + B.cp.sY + B.cp.sZ) : 0);
+        if (m.groups.empty() || group_bytes + bytes > kGroupBytes) {
+            m.groups.push_back({n, n, first[n], 0});
+            group_bytes = 0;
+        }
+        group_bytes += bytes;
+        m.groups.back().i1 = n + 1;
+        m.groups.back().nblocks = (unsigned)blocks - m.groups.back().b0;
     }
     first[ninst] = (unsigned)blocks;
     m.ninst = ninst;
@@ -202,26 +229,27 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
 static int batch_launches(const BMeta &b, const BInst *d_inst, const unsigned *d_first, int nsteps, const float *tvals,
                           float *probe_series, unsigned R, hipStream_t st)
 {
-    const unsigned grid = b.total_blocks;
-    for (int s = 0; s < nsteps; s++) {
-        const float *tv = b.total_src ? tvals + (size_t)s * b.total_src : nullptr;
-        float *pr = b.total_probe ? probe_series + (size_t)s * b.total_probe : nullptr;
+    for (const BGroup &gr : b.groups) {
+        for (int s = 0; s < nsteps; s++) {
+            const float *tv = b.total_src ? tvals + (size_t)s * b.total_src : nullptr;
+            float *pr = b.total_probe ? probe_series + (size_t)s * b.total_probe : nullptr;
 #define MIFDTD_BATCH_LAUNCH(CM, PML, EH) \
-    k_batch<CM, PML, EH><<<grid, SB, 0, st>>>(d_inst, d_first, b.ninst, tv, pr, R)
+    k_batch<CM, PML, EH><<<gr.nblocks, SB, 0, st>>>(d_inst, d_first, gr.i0, gr.i1, gr.b0, tv, pr, R)
 #define MIFDTD_BATCH_E(CM)                                   \
     do {                                                     \
         if (b.pml) MIFDTD_BATCH_LAUNCH(CM, true, true);      \
         else MIFDTD_BATCH_LAUNCH(CM, false, true);           \
     } while (0)
-        if (b.cem == kCeTable) MIFDTD_BATCH_E(kCeTable);
-        else if (b.cem == kCeArrays) MIFDTD_BATCH_E(kCeArrays);
-        else MIFDTD_BATCH_E(kCeConst);
-        MIFDTD_CHECK_LAUNCH("batch E launch");
-        if (b.pml) MIFDTD_BATCH_LAUNCH(kCeConst, true, false);
-        else MIFDTD_BATCH_LAUNCH(kCeConst, false, false);
+            if (b.cem == kCeTable) MIFDTD_BATCH_E(kCeTable);
+            else if (b.cem == kCeArrays) MIFDTD_BATCH_E(kCeArrays);
+            else MIFDTD_BATCH_E(kCeConst);
+            MIFDTD_CHECK_LAUNCH("batch E launch");
+            if (b.pml) MIFDTD_BATCH_LAUNCH(kCeConst, true, false);
+            else MIFDTD_BATCH_LAUNCH(kCeConst, false, false);
 #undef MIFDTD_BATCH_E
-        MIFDTD_CHECK_LAUNCH("batch H launch");
+            MIFDTD_CHECK_LAUNCH("batch H launch");
 #undef MIFDTD_BATCH_LAUNCH
+        }
     }
     return 0;
 }

@@ -420,7 +420,7 @@ int mifdtd_batch_sizes(const mifdtd_batch *b, int *total_src, int *total_probe,
  * probe_series: DEVICE (nsteps, total_probe).  use_graph != 0 captures the run's
  * launches into one hipGraph and launches it (needs a non-null stream; the call then
  * returns after the graph completed).  remap_rows > 0 deals each instance's blocks to
- * the 8 XCDs in runs of remap_rows consecutive blocks. */
+ * the 8 XCDs in runs of remap_rows consecutive blocks (0: a stripe of every plane per XCD). */
 int mifdtd_batch_run(mifdtd_batch *b, int nsteps, const float *tvals, float *probe_series,
                      int use_graph, int remap_rows, mifdtd_stream_t stream);
 int mifdtd_batch_destroy(mifdtd_batch *b);

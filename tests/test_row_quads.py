@@ -61,3 +61,19 @@ def test_slab_rows_equal_inplace(ns, npml, ce):
     if npml:
         assert torch.equal(a.cpml.psiE_buf.view(torch.int32), b.cpml.psiE_buf.view(torch.int32))
         assert torch.equal(a.cpml.psiH_buf.view(torch.int32), b.cpml.psiH_buf.view(torch.int32))
+
+
+@pytest.mark.gpu
+def test_batch_groups_equal_single_runs():
+    """Instances that fill more than one launch group (200 MiB of working set each) end as
+    the same simulations run alone."""
+    from fdtd_accelerate_amd.batch import BatchedYee
+    shapes = [(150, 141, 150), (60, 50, 40), (131, 160, 170), (40, 90, 33)]
+    pairs = [_pair(ns, 8, "float") for ns in shapes]
+    bt = BatchedYee([b for _, b in pairs])
+    series = bt.run(3)
+    for (a, b), rb in zip(pairs, series):
+        assert a.run(3).tobytes() == rb.tobytes()
+        for x, y in zip(a.fields.ehs, b.fields.ehs):
+            assert torch.equal(x.view(torch.int32), y.view(torch.int32))
+    bt.close()
