@@ -24,7 +24,8 @@
 // (on the zero initial state it is a no-op).  Two launches per step.  Sources do not
 // depend on the state (no adjoint).
 
-#include "common.hpp"
+#include "row_quads.hpp"
+#include "step_quad.hpp"
 
 namespace mifdtd {
 
@@ -67,11 +68,6 @@ __device__ __forceinline__ bool valid_e(int c, int i, int j, int k, const AGeom 
 {
     return in_grid(i, j, k, g) && e_row(c, i, j, g.nx, g.ny) && e_lane(c, k, g.nz);
 }
-__device__ __forceinline__ bool valid_h(int c, int i, int j, int k, const AGeom &g)
-{
-    return in_grid(i, j, k, g) && h_row(c, i, j) && h_lane(c, k, g.nz);
-}
-
 // CPML slab lookup along one axis: returns the table entry (>0) of coordinate q, or -1,
 // and the slab side / depth p.  E planes: front p -> p+1, back n-1-npml+p -> npml+1+p;
 // H planes: front p -> p+1, back n-npml+p -> npml+2+p.
@@ -101,15 +97,6 @@ __device__ __forceinline__ int tab_h(int q, int n, int npml, int &sd, int &p)
 __device__ __forceinline__ bool near_a(int q, int n, int npml) { return q < npml || q >= n - npml - 1; }
 __device__ __forceinline__ bool near_c(int q, int n, int npml) { return q <= npml || q >= n - 1 - npml; }
 
-// Cell (i, j, k) of flat index n (< 2^32: the launch checks it).
-__device__ __forceinline__ void decode(unsigned n, const AGeom &g, int &i, int &j, int &k)
-{
-    const unsigned r = n / (unsigned)g.nzp;
-    k = (int)(n - r * (unsigned)g.nzp);
-    i = (int)(r / (unsigned)g.ny);
-    j = (int)(r - (unsigned)i * (unsigned)g.ny);
-}
-
 // packed psi index of cell (i, j, k) on face (axis, side) at depth p
 __device__ __forceinline__ size_t psi_at(const AGeom &g, int axis, int sd, int p, int c, int i, int j, int k)
 {
@@ -121,45 +108,99 @@ __device__ __forceinline__ size_t psi_at(const AGeom &g, int axis, int sd, int p
     return g.off(f, c) + r;
 }
 
-// ------------------------------------------------------------------- pass A helpers
-// t_H at H cell (i,j,k) of component hc for the face (axis), psi comp pc and sign:
-// t = lpsiH + sgn*0.5*lH, or 0 when that H cell is not a valid slab cell of the face.
-__device__ __forceinline__ float tH(const AGeom &g, const float *__restrict__ lH, const float *__restrict__ lpH,
-                                    int axis, int pc, int hc, float sgn, int i, int j, int k, float &a_out,
-                                    const float *__restrict__ aH)
+// ------------------------------------------------------------------ the two passes
+// One lane per quad of 4 z cells in the whole-grid passes' thread order (row_quads.hpp:
+// a stripe of every plane per XCD, z-slab quads in waves of their own).  A quad's
+// neighbour rows, planes and cells are loaded (or taken from the next lane) once and serve
+// the curl and the CPML terms of all three axes; the psi of an axis is loaded only by the
+// rows and quads it reaches.  With a thread per cell the passes ran 7 scalar gathers per
+// component and re-derived every neighbour's validity: 160^3 cells, CPML 10, 75.5 + 110.6
+// us; now 41.0 + 61.0.  The bound is the traffic behind the L2s (84 B per cell and step and
+// the psi).
+__device__ __forceinline__ Q4 keep_cells(const Q4 &q, int k0, int lo, int hi)  // lanes lo <= k < hi, else 0
 {
-    a_out = 0.f;
-    if (!valid_h(hc, i, j, k, g)) return 0.f;
-    const int q = axis == 0 ? i : axis == 1 ? j : k;
+    Q4 r;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) r.v[l] = (k0 + l >= lo && k0 + l < hi) ? q.v[l] : 0.f;
+    return r;
+}
+
+__device__ __forceinline__ Q4 scale4(const float *__restrict__ ce, size_t id, const Q4 &q)
+{
+    const Q4 c = ce ? ld4u(ce + id) : splat4(0.5f);
+    Q4 r;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) r.v[l] = c.v[l] * q.v[l];
+    return r;
+}
+
+// H (E) slab entry and psi offset of coordinate q along an axis; t <= 0: not in a slab.
+struct Entry {
+    int t;
+    size_t o1, o2;  // psi1, psi2 of cell (i, j, k) (x, y faces: of the quad's first cell)
+};
+
+template <bool E>
+__device__ __forceinline__ Entry entry(const AGeom &g, int axis, int q, int i, int j, int k)
+{
     const int n = axis == 0 ? g.nx : axis == 1 ? g.ny : g.nz;
     int sd, p;
-    const int t = tab_h(q, n, g.npml, sd, p);
-    if (t < 0) return 0.f;
-    a_out = aH[t];
-    return lpH[psi_at(g, axis, sd, p, pc, i, j, k)] + sgn * 0.5f * lH[cidx(i, j, k, g)];
+    Entry e;
+    e.t = E ? tab_e(q, n, g.npml, sd, p) : tab_h(q, n, g.npml, sd, p);
+    e.o1 = e.o2 = 0;
+    if (e.t > 0) {
+        e.o1 = psi_at(g, axis, sd, p, 0, i, j, k);
+        e.o2 = psi_at(g, axis, sd, p, 1, i, j, k);
+    }
+    return e;
 }
 
-// Dt^T(a t) at E cell q along the axis: a(q) t(q) - a(q+1) t(q+1)
-__device__ __forceinline__ float dtT(const AGeom &g, const float *lH, const float *lpH, const float *aH, int axis,
-                                     int pc, int hc, float sgn, int i, int j, int k)
+// psi' = b * (psi + s) of one face's quad: s1, s2 the terms, c1, c2 the cells [lo, hi) they hold.
+__device__ __forceinline__ void psi_step(float *lp, const Entry &e, float b, bool row1, const Q4 &s1, int lo1, int hi1,
+                                         bool row2, const Q4 &s2, int lo2, int hi2, int k0, const Q4 &q1, const Q4 &q2)
 {
-    float a0, a1;
-    const float t0 = tH(g, lH, lpH, axis, pc, hc, sgn, i, j, k, a0, aH);
-    const float t1 = tH(g, lH, lpH, axis, pc, hc, sgn, i + (axis == 0), j + (axis == 1), k + (axis == 2), a1, aH);
-    return a0 * t0 - a1 * t1;
+    Q4 r1 = q1, r2 = q2;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const int k = k0 + l;
+        if (row1 && k >= lo1 && k < hi1) r1.v[l] = b * (q1.v[l] + s1.v[l]);
+        if (row2 && k >= lo2 && k < hi2) r2.v[l] = b * (q2.v[l] + s2.v[l]);
+    }
+    st4u(lp + e.o1, r1);
+    st4u(lp + e.o2, r2);
 }
 
-__device__ __forceinline__ float lhv(const AGeom &g, const float *__restrict__ l, int c, int i, int j, int k)
+__device__ __forceinline__ Q4 neg4(const Q4 &q)
 {
-    return valid_h(c, i, j, k, g) ? l[cidx(i, j, k, g)] : 0.f;
+    return Q4{{-q.v[0], -q.v[1], -q.v[2], -q.v[3]}};
+}
+__device__ __forceinline__ Q4 half4(const Q4 &q, float s)
+{
+    return Q4{{s * q.v[0], s * q.v[1], s * q.v[2], s * q.v[3]}};
 }
 
-__device__ __forceinline__ void pass_d_cell(const AGeom &g, int i, int j, int k, size_t n, const float *const LE[3],
-                                            const float *const CE[3], float *lpE, const float *bE);
-__device__ __forceinline__ void pass_b_cell(const AGeom &g, int i, int j, int k, size_t n, const float *const LH[3],
-                                            float *lpH, const float *bH);
+// a * (psi + s) on the cells [lo, hi) of a valid row in the slab, else 0.
+__device__ __forceinline__ Q4 psi_term(bool on, float a, const Q4 &psi, const Q4 &s, int k0, int lo, int hi)
+{
+    Q4 r;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const int k = k0 + l;
+        r.v[l] = on && k >= lo && k < hi ? a * (psi.v[l] + s.v[l]) : 0.f;
+    }
+    return r;
+}
 
-__global__ __launch_bounds__(AB) void k_adj_a(AGeom g, float *__restrict__ lex, float *__restrict__ ley,
+__device__ __forceinline__ void add_diff(Q4 &v, const Q4 &p, const Q4 &m)
+{
+#pragma unroll
+    for (int l = 0; l < 4; ++l) v.v[l] += p.v[l] - m.v[l];
+}
+
+__device__ __forceinline__ Q4 psi_ld(bool on, const float *lp, size_t o) { return on ? ld4u(lp + o) : splat4(0.f); }
+
+// Pass A (and D of the later step) on one quad.
+__global__ __launch_bounds__(AB) void k_adj_a(AGeom g, RowQuads m, float *__restrict__ lex, float *__restrict__ ley,
                                               float *__restrict__ lez, float *__restrict__ lhx,
                                               float *__restrict__ lhy, float *__restrict__ lhz,
                                               const float *__restrict__ lpH, const float *__restrict__ aH,
@@ -168,111 +209,130 @@ __global__ __launch_bounds__(AB) void k_adj_a(AGeom g, float *__restrict__ lex, 
                                               const float *__restrict__ cez, float *__restrict__ lpE,
                                               const float *__restrict__ bE)
 {
-    const unsigned n = blockIdx.x * AB + threadIdx.x;
-    if (n >= g.ncell) return;
-    int i, j, k;
-    decode(n, g, i, j, k);
-    const size_t id = (size_t)n;
-    const bool nx_ = g.npml > 0 && near_a(i, g.nx, g.npml), ny_ = g.npml > 0 && near_a(j, g.ny, g.npml),
-               nz_ = g.npml > 0 && near_a(k, g.nz, g.npml);
-    if (nx_ || ny_ || nz_) {  // pass D of the later step, on this cell (reads lE before A changes it)
-        const float *LEd[3] = {lex, ley, lez};
-        const float *CEd[3] = {cex, cey, cez};
-        pass_d_cell(g, i, j, k, id, LEd, CEd, lpE, bE);
+    const QuadAt at = row_quad(m, blockIdx.x, threadIdx.x);
+    if (!at.active) return;
+    const int i = at.i, j = at.j, k0 = 4 * at.q;
+    const bool next = at.next && (threadIdx.x & 63) < 63;
+    const int nz = g.nz;
+    const size_t id = cidx(i, j, k0, g), sj = (size_t)g.nzp, si = (size_t)g.ny * g.nzp;
+    const bool ip = i > 0, jp = j > 0, ix = i + 1 < g.nx, jy = j + 1 < g.ny;
+    const Q4 z4 = splat4(0.f);
+    // H valid cells: hx rows j > 0, hy planes i > 0 (0 < k < nz); hz i, j > 0 (k < nz)
+    const Q4 hx0 = jp ? keep_cells(ld4u(lhx + id), k0, 1, nz) : z4;
+    const Q4 hy0 = ip ? keep_cells(ld4u(lhy + id), k0, 1, nz) : z4;
+    const Q4 hz0 = ip && jp ? keep_cells(ld4u(lhz + id), k0, 0, nz) : z4;
+    const Q4 hxU = jy ? keep_cells(ld4u(lhx + id + sj), k0, 1, nz) : z4;
+    const Q4 hzU = jy && ip ? keep_cells(ld4u(lhz + id + sj), k0, 0, nz) : z4;
+    const Q4 hyN = ix ? keep_cells(ld4u(lhy + id + si), k0, 1, nz) : z4;
+    const Q4 hzN = ix && jp ? keep_cells(ld4u(lhz + id + si), k0, 0, nz) : z4;
+    Q4 vx = ld4u(lex + id), vy = ld4u(ley + id), vz = ld4u(lez + id);
+    float hx4 = 0.f, hy4 = 0.f;  // at k0 + 4
+    if (!next && k0 + 4 < nz) {
+        if (jp) hx4 = lhx[id + 4];
+        if (ip) hy4 = lhy[id + 4];
     }
-    const float *LH[3] = {lhx, lhy, lhz};
+    const float hxs = lane_next(hx0.v[0]), hys = lane_next(hy0.v[0]);  // every lane takes part
+    if (next) {
+        hx4 = hxs;
+        hy4 = hys;
+    }
+    const bool nx_ = g.npml > 0 && near_a(i, g.nx, g.npml), ny_ = g.npml > 0 && near_a(j, g.ny, g.npml),
+               nz_ = g.npml > 0 && (k0 < g.npml || k0 + 3 >= nz - g.npml - 1);
+    const Q4 ex0 = vx, ey0 = vy, ez0 = vz;
     // -0.5*K(lH valid):  ex: (z[j+1]-z) - (y[k+1]-y);  ey: (x[k+1]-x) - (z[i+1]-z);
     //                     ez: (y[i+1]-y) - (x[j+1]-x)
-    float ax = 0.f, ay = 0.f, az = 0.f;
-    ax = (lhv(g, LH[2], 2, i, j + 1, k) - lhv(g, LH[2], 2, i, j, k)) - (lhv(g, LH[1], 1, i, j, k + 1) - lhv(g, LH[1], 1, i, j, k));
-    ay = (lhv(g, LH[0], 0, i, j, k + 1) - lhv(g, LH[0], 0, i, j, k)) - (lhv(g, LH[2], 2, i + 1, j, k) - lhv(g, LH[2], 2, i, j, k));
-    az = (lhv(g, LH[1], 1, i + 1, j, k) - lhv(g, LH[1], 1, i, j, k)) - (lhv(g, LH[0], 0, i, j + 1, k) - lhv(g, LH[0], 0, i, j, k));
-    float vx = lex[id] - 0.5f * ax, vy = ley[id] - 0.5f * ay, vz = lez[id] - 0.5f * az;
-    if (nx_) {  // x: psi1 -> hy from ez (+), psi2 -> hz from ey (-)
-        vz += dtT(g, lhy, lpH, aH, 0, 0, 1, +1.f, i, j, k);
-        vy += dtT(g, lhz, lpH, aH, 0, 1, 2, -1.f, i, j, k);
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const float y1 = l < 3 ? hy0.v[l + 1] : hy4, x1 = l < 3 ? hx0.v[l + 1] : hx4;
+        vx.v[l] = vx.v[l] - 0.5f * ((hzU.v[l] - hz0.v[l]) - (y1 - hy0.v[l]));
+        vy.v[l] = vy.v[l] - 0.5f * ((x1 - hx0.v[l]) - (hzN.v[l] - hz0.v[l]));
+        vz.v[l] = vz.v[l] - 0.5f * ((hyN.v[l] - hy0.v[l]) - (hxU.v[l] - hx0.v[l]));
     }
-    if (ny_) {  // y: psi1 -> hz from ex (+), psi2 -> hx from ez (-)
-        vx += dtT(g, lhz, lpH, aH, 1, 0, 2, +1.f, i, j, k);
-        vz += dtT(g, lhx, lpH, aH, 1, 1, 0, -1.f, i, j, k);
+    if (nx_) {
+        const Entry d = entry<true>(g, 0, i, i, j, k0), t0 = entry<false>(g, 0, i, i, j, k0),
+                    t1 = entry<false>(g, 0, i + 1, i + 1, j, k0);
+        const bool on0 = t0.t > 0 && ip, on1 = t1.t > 0 && ix;
+        const Q4 q1 = psi_ld(d.t > 0, lpE, d.o1), q2 = psi_ld(d.t > 0, lpE, d.o2);
+        const Q4 r1 = psi_ld(on0, lpH, t0.o1), r2 = psi_ld(on0, lpH, t0.o2);
+        const Q4 s1 = psi_ld(on1, lpH, t1.o1), s2 = psi_ld(on1, lpH, t1.o2);
+        if (d.t > 0)  // D: psi1 ey (-), psi2 ez (+)
+            psi_step(lpE, d, bE[d.t], true, neg4(scale4(cey, id, ey0)), 0, nz - 1, jy, scale4(cez, id, ez0), 0, nz, k0,
+                     q1, q2);
+        const float a0 = on0 ? aH[t0.t] : 0.f, a1 = on1 ? aH[t1.t] : 0.f;
+        // psi1 -> hy from ez (+), psi2 -> hz from ey (-)
+        add_diff(vz, psi_term(on0, a0, r1, half4(hy0, 0.5f), k0, 1, nz), psi_term(on1, a1, s1, half4(hyN, 0.5f), k0, 1, nz));
+        add_diff(vy, psi_term(on0 && jp, a0, r2, half4(hz0, -0.5f), k0, 0, nz),
+                 psi_term(on1 && jp, a1, s2, half4(hzN, -0.5f), k0, 0, nz));
     }
-    if (nz_) {  // z: psi1 -> hx from ey (+), psi2 -> hy from ex (-)
-        vy += dtT(g, lhx, lpH, aH, 2, 0, 0, +1.f, i, j, k);
-        vx += dtT(g, lhy, lpH, aH, 2, 1, 1, -1.f, i, j, k);
+    if (ny_) {
+        const Entry d = entry<true>(g, 1, j, i, j, k0), t0 = entry<false>(g, 1, j, i, j, k0),
+                    t1 = entry<false>(g, 1, j + 1, i, j + 1, k0);
+        const bool on0 = t0.t > 0 && jp, on1 = t1.t > 0 && jy;
+        const Q4 q1 = psi_ld(d.t > 0, lpE, d.o1), q2 = psi_ld(d.t > 0, lpE, d.o2);
+        const Q4 r1 = psi_ld(on0, lpH, t0.o1), r2 = psi_ld(on0, lpH, t0.o2);
+        const Q4 s1 = psi_ld(on1, lpH, t1.o1), s2 = psi_ld(on1, lpH, t1.o2);
+        if (d.t > 0)  // D: psi1 ez (-), psi2 ex (+)
+            psi_step(lpE, d, bE[d.t], ix, neg4(scale4(cez, id, ez0)), 0, nz, true, scale4(cex, id, ex0), 0, nz - 1, k0,
+                     q1, q2);
+        const float a0 = on0 ? aH[t0.t] : 0.f, a1 = on1 ? aH[t1.t] : 0.f;
+        // psi1 -> hz from ex (+), psi2 -> hx from ez (-)
+        add_diff(vx, psi_term(on0 && ip, a0, r1, half4(hz0, 0.5f), k0, 0, nz),
+                 psi_term(on1 && ip, a1, s1, half4(hzU, 0.5f), k0, 0, nz));
+        add_diff(vz, psi_term(on0, a0, r2, half4(hx0, -0.5f), k0, 1, nz), psi_term(on1, a1, s2, half4(hxU, -0.5f), k0, 1, nz));
+    }
+    if (nz_) {
+        // D: psi1 ex (-), psi2 ey (+)
+        const Q4 gx = scale4(cex, id, ex0), gy = scale4(cey, id, ey0);
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const Entry d = entry<true>(g, 2, k0 + l, i, j, k0 + l);
+            if (d.t > 0) {
+                const float b = bE[d.t];
+                if (jy) lpE[d.o1] = b * (lpE[d.o1] - gx.v[l]);
+                if (ix) lpE[d.o2] = b * (lpE[d.o2] + gy.v[l]);
+            }
+        }
+        // a t of cells k0 .. k0+4: psi1 -> hx from ey (+), psi2 -> hy from ex (-)
+        float t1[5], t2[5];
+#pragma unroll
+        for (int l = 0; l < 5; ++l) {
+            const int k = k0 + l;
+            t1[l] = t2[l] = 0.f;
+            const int kk = k < g.nzp ? k : 0;
+            const Entry t = entry<false>(g, 2, kk, i, j, kk);
+            if (k > 0 && k < nz && t.t > 0) {
+                const float a = aH[t.t];
+                if (jp) t1[l] = a * (lpH[t.o1] + 0.5f * (l < 4 ? hx0.v[l & 3] : hx4));
+                if (ip) t2[l] = a * (lpH[t.o2] - 0.5f * (l < 4 ? hy0.v[l & 3] : hy4));
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+            if (near_a(k0 + l, nz, g.npml)) {
+                vy.v[l] += t1[l] - t1[l + 1];
+                vx.v[l] += t2[l] - t2[l + 1];
+            }
     }
     if (eplane && i == iplane) {
-        const size_t pid = (size_t)j * g.nzp + k;
-        const size_t ps = (size_t)g.ny * g.nzp;
-        vx += 2.f * eplane[pid];
-        vy += 2.f * eplane[ps + pid];
-        vz += 2.f * eplane[2 * ps + pid];
-    }
-    lex[id] = vx;
-    ley[id] = vy;
-    lez[id] = vz;
-    // H masked lanes: H' does not depend on H there
-    for (int c = 0; c < 3; ++c)
-        if (h_row(c, i, j) && !h_lane(c, k, g.nz)) (c == 0 ? lhx : c == 1 ? lhy : lhz)[id] = 0.f;
-}
-
-// Pass B on one cell: lpsiH = b_H * (lpsiH + sgn*0.5*lH) on its valid H slab entries.
-__device__ __forceinline__ void pass_b_cell(const AGeom &g, int i, int j, int k, size_t n, const float *const LH[3],
-                                            float *lpH, const float *bH)
-{
-    // (axis, psi comp) -> (H comp, sign)
-    const int hcs[3][2] = {{1, 2}, {2, 0}, {0, 1}};
-    const float sg[2] = {+1.f, -1.f};
+        const size_t pid = (size_t)j * g.nzp + k0, ps = (size_t)g.ny * g.nzp;
+        const Q4 px = ld4u(eplane + pid), py = ld4u(eplane + ps + pid), pz = ld4u(eplane + 2 * ps + pid);
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        const int q = ax == 0 ? i : ax == 1 ? j : k;
-        const int nn = ax == 0 ? g.nx : ax == 1 ? g.ny : g.nz;
-        int sd, p;
-        const int t = tab_h(q, nn, g.npml, sd, p);
-        if (t < 0) continue;
-#pragma unroll
-        for (int pc = 0; pc < 2; ++pc) {
-            const int hc = hcs[ax][pc];
-            if (!valid_h(hc, i, j, k, g)) continue;
-            const size_t pi = psi_at(g, ax, sd, p, pc, i, j, k);
-            lpH[pi] = bH[t] * (lpH[pi] + sg[pc] * 0.5f * LH[hc][n]);
+        for (int l = 0; l < 4; ++l) {
+            vx.v[l] += 2.f * px.v[l];
+            vy.v[l] += 2.f * py.v[l];
+            vz.v[l] += 2.f * pz.v[l];
         }
     }
-}
-
-// ------------------------------------------------------------------- pass C helpers
-__device__ __forceinline__ float gev(const AGeom &g, const float *__restrict__ l, const float *__restrict__ ce, int c,
-                                     int i, int j, int k)
-{
-    if (!valid_e(c, i, j, k, g)) return 0.f;
-    const size_t q = cidx(i, j, k, g);
-    return (ce ? ce[q] : 0.5f) * l[q];
-}
-
-// t_E at E cell (i,j,k): lpsiE + sgn*CE*lE on valid E slab cells of the face, else 0.
-__device__ __forceinline__ float tE(const AGeom &g, const float *__restrict__ lE, const float *__restrict__ ce,
-                                    const float *__restrict__ lpE, int axis, int pc, int ec, float sgn, int i, int j,
-                                    int k, float &a_out, const float *__restrict__ aE)
-{
-    a_out = 0.f;
-    if (!valid_e(ec, i, j, k, g)) return 0.f;
-    const int q = axis == 0 ? i : axis == 1 ? j : k;
-    const int n = axis == 0 ? g.nx : axis == 1 ? g.ny : g.nz;
-    int sd, p;
-    const int t = tab_e(q, n, g.npml, sd, p);
-    if (t < 0) return 0.f;
-    a_out = aE[t];
-    const size_t c = cidx(i, j, k, g);
-    return lpE[psi_at(g, axis, sd, p, pc, i, j, k)] + sgn * (ce ? ce[c] : 0.5f) * lE[c];
-}
-
-// D^T(a t) at H cell q along the axis: a(q-1) t(q-1) - a(q) t(q)
-__device__ __forceinline__ float dT(const AGeom &g, const float *lE, const float *ce, const float *lpE,
-                                    const float *aE, int axis, int pc, int ec, float sgn, int i, int j, int k)
-{
-    float am, a0;
-    const float tm = tE(g, lE, ce, lpE, axis, pc, ec, sgn, i - (axis == 0), j - (axis == 1), k - (axis == 2), am, aE);
-    const float t0 = tE(g, lE, ce, lpE, axis, pc, ec, sgn, i, j, k, a0, aE);
-    return am * tm - a0 * t0;
+    st4u(lex + id, vx);
+    st4u(ley + id, vy);
+    st4u(lez + id, vz);
+    // H masked lanes: H' does not depend on H there
+    if (k0 == 0 || k0 + 3 >= nz) {
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+            for (int c = 0; c < 3; ++c)
+                if (h_row(c, i, j) && !h_lane(c, k0 + l, nz)) (c == 0 ? lhx : c == 1 ? lhy : lhz)[id + l] = 0.f;
+    }
 }
 
 struct ADesign {
@@ -281,7 +341,33 @@ struct ADesign {
     double *grad;                // (3, di, dj, dk) accumulated dJ/dCE
 };
 
-__global__ __launch_bounds__(AB) void k_adj_c(AGeom g, float *__restrict__ lex, float *__restrict__ ley,
+struct __attribute__((packed, aligned(8))) D2u {  // two doubles at any 8-byte aligned address
+    double x, y;
+};
+
+// grad += lE * curl of one component on the quad's cells inside the box (q: box index of
+// the quad's first cell).
+__device__ __forceinline__ void grad_quad(const ADesign &dz, size_t q, int dk, const Q4 &e, int k0, int hi)
+{
+    if (dk >= 0 && dk + 3 < dz.dk && k0 + 3 < hi && (q & 3u) == 0) {
+        const Q4 c = ld4u(dz.curl + q);
+        D2u *p = reinterpret_cast<D2u *>(dz.grad + q);
+        D2u a = p[0], b = p[1];
+        a.x += (double)e.v[0] * (double)c.v[0];
+        a.y += (double)e.v[1] * (double)c.v[1];
+        b.x += (double)e.v[2] * (double)c.v[2];
+        b.y += (double)e.v[3] * (double)c.v[3];
+        p[0] = a;
+        p[1] = b;
+        return;
+    }
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+        if (dk + l >= 0 && dk + l < dz.dk && k0 + l < hi) dz.grad[q + l] += (double)e.v[l] * (double)dz.curl[q + l];
+}
+
+// Pass C (and B) on one quad.
+__global__ __launch_bounds__(AB) void k_adj_c(AGeom g, RowQuads m, float *__restrict__ lex, float *__restrict__ ley,
                                               float *__restrict__ lez, float *__restrict__ lhx,
                                               float *__restrict__ lhy, float *__restrict__ lhz,
                                               const float *__restrict__ cex, const float *__restrict__ cey,
@@ -289,76 +375,125 @@ __global__ __launch_bounds__(AB) void k_adj_c(AGeom g, float *__restrict__ lex, 
                                               const float *__restrict__ aE, ADesign dz,
                                               float *__restrict__ lpH, const float *__restrict__ bH)
 {
-    const unsigned n = blockIdx.x * AB + threadIdx.x;
-    if (n >= g.ncell) return;
-    int i, j, k;
-    decode(n, g, i, j, k);
-    const size_t id = (size_t)n;
-    const bool nx_ = g.npml > 0 && near_c(i, g.nx, g.npml), ny_ = g.npml > 0 && near_c(j, g.ny, g.npml),
-               nz_ = g.npml > 0 && near_c(k, g.nz, g.npml);
-    if (nx_ || ny_ || nz_) {  // pass B on this cell (reads lH before C changes it)
-        const float *LHb[3] = {lhx, lhy, lhz};
-        pass_b_cell(g, i, j, k, id, LHb, lpH, bH);
+    const QuadAt at = row_quad(m, blockIdx.x, threadIdx.x);
+    if (!at.active) return;
+    const int i = at.i, j = at.j, k0 = 4 * at.q;
+    const bool prev = at.prev && (threadIdx.x & 63) > 0;
+    const int nz = g.nz;
+    const size_t id = cidx(i, j, k0, g), sj = (size_t)g.nzp, si = (size_t)g.ny * g.nzp;
+    const bool ip = i > 0, jp = j > 0, ix = i + 1 < g.nx, jy = j + 1 < g.ny;
+    const Q4 z4 = splat4(0.f);
+    const Q4 ex0 = ld4u(lex + id), ey0 = ld4u(ley + id), ez0 = ld4u(lez + id);
+    Q4 vx = ld4u(lhx + id), vy = ld4u(lhy + id), vz = ld4u(lhz + id);
+    // CE*lE on valid E cells: ex rows j < ny-1, ey planes i < nx-1 (k < nz-1); ez both (k < nz)
+    const Q4 gx0 = jy ? keep_cells(scale4(cex, id, ex0), k0, 0, nz - 1) : z4;
+    const Q4 gy0 = ix ? keep_cells(scale4(cey, id, ey0), k0, 0, nz - 1) : z4;
+    const Q4 gz0 = ix && jy ? keep_cells(scale4(cez, id, ez0), k0, 0, nz) : z4;
+    const Q4 gxD = jp ? keep_cells(scale4(cex, id - sj, ld4u(lex + id - sj)), k0, 0, nz - 1) : z4;
+    const Q4 gzD = jp && ix ? keep_cells(scale4(cez, id - sj, ld4u(lez + id - sj)), k0, 0, nz) : z4;
+    const Q4 gyB = ip ? keep_cells(scale4(cey, id - si, ld4u(ley + id - si)), k0, 0, nz - 1) : z4;
+    const Q4 gzB = ip && jy ? keep_cells(scale4(cez, id - si, ld4u(lez + id - si)), k0, 0, nz) : z4;
+    float gxm = 0.f, gym = 0.f;  // at k0 - 1
+    if (!prev && k0 > 0 && k0 - 1 < nz - 1) {
+        if (jy) gxm = (cex ? cex[id - 1] : 0.5f) * lex[id - 1];
+        if (ix) gym = (cey ? cey[id - 1] : 0.5f) * ley[id - 1];
     }
-    const float *LE[3] = {lex, ley, lez};
-    const float *CE[3] = {cex, cey, cez};
+    const float gxs = lane_prev(gx0.v[3]), gys = lane_prev(gy0.v[3]);  // every lane takes part
+    if (prev) {
+        gxm = gxs;
+        gym = gys;
+    }
+    const bool nx_ = g.npml > 0 && near_c(i, g.nx, g.npml), ny_ = g.npml > 0 && near_c(j, g.ny, g.npml),
+               nz_ = g.npml > 0 && (k0 <= g.npml || k0 + 3 >= nz - 1 - g.npml);
+    const Q4 hx0 = vx, hy0 = vy, hz0 = vz;
     // Kt(CE*lE valid): hx: (z - z[j-1]) - (y - y[k-1]); hy: (x - x[k-1]) - (z - z[i-1]);
     //                  hz: (y - y[i-1]) - (x - x[j-1])
-    const float bx = (gev(g, LE[2], CE[2], 2, i, j, k) - gev(g, LE[2], CE[2], 2, i, j - 1, k)) -
-                     (gev(g, LE[1], CE[1], 1, i, j, k) - gev(g, LE[1], CE[1], 1, i, j, k - 1));
-    const float by = (gev(g, LE[0], CE[0], 0, i, j, k) - gev(g, LE[0], CE[0], 0, i, j, k - 1)) -
-                     (gev(g, LE[2], CE[2], 2, i, j, k) - gev(g, LE[2], CE[2], 2, i - 1, j, k));
-    const float bz = (gev(g, LE[1], CE[1], 1, i, j, k) - gev(g, LE[1], CE[1], 1, i - 1, j, k)) -
-                     (gev(g, LE[0], CE[0], 0, i, j, k) - gev(g, LE[0], CE[0], 0, i, j - 1, k));
-    float vx = lhx[id] + bx, vy = lhy[id] + by, vz = lhz[id] + bz;
-    if (nx_) {  // x: psi1 -> ey from hz (-CE), psi2 -> ez from hy (+CE)
-        vz += dT(g, ley, cey, lpE, aE, 0, 0, 1, -1.f, i, j, k);
-        vy += dT(g, lez, cez, lpE, aE, 0, 1, 2, +1.f, i, j, k);
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const float xm = l > 0 ? gx0.v[l - 1] : gxm, ym = l > 0 ? gy0.v[l - 1] : gym;
+        vx.v[l] = vx.v[l] + ((gz0.v[l] - gzD.v[l]) - (gy0.v[l] - ym));
+        vy.v[l] = vy.v[l] + ((gx0.v[l] - xm) - (gz0.v[l] - gzB.v[l]));
+        vz.v[l] = vz.v[l] + ((gy0.v[l] - gyB.v[l]) - (gx0.v[l] - gxD.v[l]));
     }
-    if (ny_) {  // y: psi1 -> ez from hx (-), psi2 -> ex from hz (+)
-        vx += dT(g, lez, cez, lpE, aE, 1, 0, 2, -1.f, i, j, k);
-        vz += dT(g, lex, cex, lpE, aE, 1, 1, 0, +1.f, i, j, k);
+    if (nx_) {
+        const Entry d = entry<false>(g, 0, i, i, j, k0), tm = entry<true>(g, 0, i - 1, i - 1, j, k0),
+                    t0 = entry<true>(g, 0, i, i, j, k0);
+        const bool on = d.t > 0 && ip, onm = tm.t > 0, on0 = t0.t > 0;
+        const Q4 q1 = psi_ld(on, lpH, d.o1), q2 = psi_ld(on, lpH, d.o2);
+        const Q4 r1 = psi_ld(onm, lpE, tm.o1), r2 = psi_ld(onm, lpE, tm.o2);
+        const Q4 s1 = psi_ld(on0, lpE, t0.o1), s2 = psi_ld(on0, lpE, t0.o2);
+        if (on)  // B: psi1 hy (+), psi2 hz (-)
+            psi_step(lpH, d, bH[d.t], true, half4(hy0, 0.5f), 1, nz, jp, half4(hz0, -0.5f), 0, nz, k0, q1, q2);
+        const float am = onm ? aE[tm.t] : 0.f, a0 = on0 ? aE[t0.t] : 0.f;
+        // psi1 -> ey from hz (-CE), psi2 -> ez from hy (+CE)
+        add_diff(vz, psi_term(onm, am, r1, neg4(gyB), k0, 0, nz - 1), psi_term(on0, a0, s1, neg4(gy0), k0, 0, nz - 1));
+        add_diff(vy, psi_term(onm && jy, am, r2, gzB, k0, 0, nz), psi_term(on0 && jy, a0, s2, gz0, k0, 0, nz));
     }
-    if (nz_) {  // z: psi1 -> ex from hy (-), psi2 -> ey from hx (+)
-        vy += dT(g, lex, cex, lpE, aE, 2, 0, 0, -1.f, i, j, k);
-        vx += dT(g, ley, cey, lpE, aE, 2, 1, 1, +1.f, i, j, k);
+    if (ny_) {
+        const Entry d = entry<false>(g, 1, j, i, j, k0), tm = entry<true>(g, 1, j - 1, i, j - 1, k0),
+                    t0 = entry<true>(g, 1, j, i, j, k0);
+        const bool on = d.t > 0 && jp, onm = tm.t > 0, on0 = t0.t > 0;
+        const Q4 q1 = psi_ld(on, lpH, d.o1), q2 = psi_ld(on, lpH, d.o2);
+        const Q4 r1 = psi_ld(onm, lpE, tm.o1), r2 = psi_ld(onm, lpE, tm.o2);
+        const Q4 s1 = psi_ld(on0, lpE, t0.o1), s2 = psi_ld(on0, lpE, t0.o2);
+        if (on)  // B: psi1 hz (+), psi2 hx (-)
+            psi_step(lpH, d, bH[d.t], ip, half4(hz0, 0.5f), 0, nz, true, half4(hx0, -0.5f), 1, nz, k0, q1, q2);
+        const float am = onm ? aE[tm.t] : 0.f, a0 = on0 ? aE[t0.t] : 0.f;
+        // psi1 -> ez from hx (-), psi2 -> ex from hz (+)
+        add_diff(vx, psi_term(onm && ix, am, r1, neg4(gzD), k0, 0, nz), psi_term(on0 && ix, a0, s1, neg4(gz0), k0, 0, nz));
+        add_diff(vz, psi_term(onm, am, r2, gxD, k0, 0, nz - 1), psi_term(on0, a0, s2, gx0, k0, 0, nz - 1));
     }
-    lhx[id] = vx;
-    lhy[id] = vy;
-    lhz[id] = vz;
+    if (nz_) {
+        // B: psi1 hx (+), psi2 hy (-)
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const int k = k0 + l;
+            const Entry d = entry<false>(g, 2, k, i, j, k);
+            if (d.t > 0 && k > 0) {
+                const float b = bH[d.t];
+                if (jp) lpH[d.o1] = b * (lpH[d.o1] + 0.5f * hx0.v[l]);
+                if (ip) lpH[d.o2] = b * (lpH[d.o2] - 0.5f * hy0.v[l]);
+            }
+        }
+        // a t of cells k0-1 .. k0+3: psi1 -> ex from hy (-), psi2 -> ey from hx (+)
+        float t1[5], t2[5];
+#pragma unroll
+        for (int l = 0; l < 5; ++l) {
+            const int k = k0 - 1 + l;
+            t1[l] = t2[l] = 0.f;
+            const int kk = k > 0 ? k : 0;
+            const Entry t = entry<true>(g, 2, kk, i, j, kk);
+            if (k >= 0 && k < nz - 1 && t.t > 0) {
+                const float a = aE[t.t];
+                if (jy) t1[l] = a * (lpE[t.o1] - (l > 0 ? gx0.v[(l + 3) & 3] : gxm));
+                if (ix) t2[l] = a * (lpE[t.o2] + (l > 0 ? gy0.v[(l + 3) & 3] : gym));
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+            if (near_c(k0 + l, nz, g.npml)) {
+                vy.v[l] += t1[l] - t1[l + 1];
+                vx.v[l] += t2[l] - t2[l + 1];
+            }
+    }
+    st4u(lhx + id, vx);
+    st4u(lhy + id, vy);
+    st4u(lhz + id, vz);
     // gradient of the CE of the design box: lE * (K H_prev)
-    const int di = i - dz.i0, dj = j - dz.j0, dk = k - dz.k0;
-    if (dz.grad && di >= 0 && di < dz.di && dj >= 0 && dj < dz.dj && dk >= 0 && dk < dz.dk) {
-        const size_t q = ((size_t)di * dz.dj + dj) * dz.dk + dk;
+    const int di = i - dz.i0, dj = j - dz.j0, dk = k0 - dz.k0;
+    if (dz.grad && di >= 0 && di < dz.di && dj >= 0 && dj < dz.dj && dk + 3 >= 0 && dk < dz.dk) {
+        const size_t q = (((size_t)di * dz.dj + dj) * dz.dk) + dk;  // dk may be -3..-1: cells before the box are skipped
         const size_t s = (size_t)dz.di * dz.dj * dz.dk;
-        for (int c = 0; c < 3; ++c)
-            if (valid_e(c, i, j, k, g)) dz.grad[c * s + q] += (double)LE[c][id] * (double)dz.curl[c * s + q];
+        if (jy) grad_quad(dz, q, dk, ex0, k0, nz - 1);
+        if (ix) grad_quad(dz, q + s, dk, ey0, k0, nz - 1);
+        if (ix && jy) grad_quad(dz, q + 2 * s, dk, ez0, k0, nz);
     }
     // E masked lanes: E' does not depend on E there
-    for (int c = 0; c < 3; ++c)
-        if (e_row(c, i, j, g.nx, g.ny) && !e_lane(c, k, g.nz)) (c == 0 ? lex : c == 1 ? ley : lez)[id] = 0.f;
-}
-
-// Pass D on one cell: lpsiE = b_E * (lpsiE + sgn*CE*lE) on its valid E slab entries.
-__device__ __forceinline__ void pass_d_cell(const AGeom &g, int i, int j, int k, size_t n, const float *const LE[3],
-                                            const float *const CE[3], float *lpE, const float *bE)
-{
-    const int ecs[3][2] = {{1, 2}, {2, 0}, {0, 1}};
-    const float sg[2] = {-1.f, +1.f};
+    if (k0 + 3 >= nz - 1) {
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        const int q = ax == 0 ? i : ax == 1 ? j : k;
-        const int nn = ax == 0 ? g.nx : ax == 1 ? g.ny : g.nz;
-        int sd, p;
-        const int t = tab_e(q, nn, g.npml, sd, p);
-        if (t < 0) continue;
-#pragma unroll
-        for (int pc = 0; pc < 2; ++pc) {
-            const int ec = ecs[ax][pc];
-            if (!valid_e(ec, i, j, k, g)) continue;
-            const size_t pi = psi_at(g, ax, sd, p, pc, i, j, k);
-            lpE[pi] = bE[t] * (lpE[pi] + sg[pc] * (CE[ec] ? CE[ec][n] : 0.5f) * LE[ec][n]);
-        }
+        for (int l = 0; l < 4; ++l)
+            for (int c = 0; c < 3; ++c)
+                if (e_row(c, i, j, g.nx, g.ny) && !e_lane(c, k0 + l, nz)) (c == 0 ? lex : c == 1 ? ley : lez)[id + l] = 0.f;
     }
 }
 
@@ -453,12 +588,13 @@ int mifdtd_adjoint_step(int nx, int ny, int nz_pitch, int pad, float *const lam[
         dz.grad = grad;
     }
     if (g.ncell > 0xffffffffull - AB) return fail(MIFDTD_ERANGE, "grid of %llu cells: at most 2^32 - %d", g.ncell, AB);
-    const unsigned grid = (unsigned)((g.ncell + AB - 1) / AB);
+    const RowQuads m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)(nz_pitch / 4), g.nz, npml, npml + 1);
+    const unsigned grid = (unsigned)row_quads_blocks(m);
     hipStream_t st = to_stream(stream);
-    k_adj_a<<<grid, AB, 0, st>>>(g, lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], lpsiH, aH, eplane, iplane, c0, c1,
+    k_adj_a<<<grid, AB, 0, st>>>(g, m, lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], lpsiH, aH, eplane, iplane, c0, c1,
                                  c2, lpsiE, bE);
     MIFDTD_CHECK_LAUNCH("adjoint pass A");
-    k_adj_c<<<grid, AB, 0, st>>>(g, lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], c0, c1, c2, lpsiE, aE, dz, lpsiH,
+    k_adj_c<<<grid, AB, 0, st>>>(g, m, lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], c0, c1, c2, lpsiE, aE, dz, lpsiH,
                                  bH);
     MIFDTD_CHECK_LAUNCH("adjoint pass C");
     return 0;

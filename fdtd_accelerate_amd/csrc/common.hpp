@@ -51,6 +51,22 @@ __device__ __forceinline__ void st4(float *__restrict__ p, const Q4 &q)
     *reinterpret_cast<float4 *>(p) = make_float4(q.v[0], q.v[1], q.v[2], q.v[3]);
 }
 
+// The same at any 4-byte aligned address (one 16-byte access too: gfx950 takes them unaligned).
+struct __attribute__((packed, aligned(4))) F4u {
+    float x, y, z, w;
+};
+
+__device__ __forceinline__ Q4 ld4u(const float *__restrict__ p)
+{
+    const F4u t = *reinterpret_cast<const F4u *>(p);
+    return Q4{{t.x, t.y, t.z, t.w}};
+}
+
+__device__ __forceinline__ void st4u(float *__restrict__ p, const Q4 &q)
+{
+    *reinterpret_cast<F4u *>(p) = F4u{q.v[0], q.v[1], q.v[2], q.v[3]};
+}
+
 __device__ __forceinline__ Q4 splat4(float x)
 {
     Q4 q;

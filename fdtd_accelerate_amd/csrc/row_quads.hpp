@@ -98,15 +98,16 @@ inline void stripe_rows(RowQuads &m, unsigned ny, int npml)
 
 // The order for `planes` planes of ny rows of Q quads (nz cells, npml-cell z slabs; npml =
 // 0: none).  The E slabs are [0, npml) and [nz-1-npml, nz-1), the H slabs [0, npml) and
-// [nz-npml, nz): one order serves both.
-inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml)
+// [nz-npml, nz): one order serves both.  front: cells at the front that count as slab cells
+// (the adjoint passes reach one cell further).
+inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, int front = 0)
 {
     RowQuads m;
     m.Q = Q;
     m.planes = planes;
     m.ns = ny >= kStripeMinRows ? kStripes : 1;
     stripe_rows(m, ny, npml);
-    m.zf = npml > 0 ? (unsigned)((npml + 3) / 4) : 0u;
+    m.zf = npml > 0 ? (unsigned)(((front > npml ? front : npml) + 3) / 4) : 0u;
     m.zb = npml > 0 ? (unsigned)((nz - 1 - npml) / 4) : Q;
     if (m.zf >= m.zb) {  // every quad may hold a slab cell: one run
         m.zf = 0;
