@@ -7,14 +7,15 @@
 // were read before, by blocks of the same L2.
 //
 // Groups: the quads of R consecutive rows of a stripe are taken by a whole number of
-// 256-thread blocks: first the quads with no cell of a z CPML slab, row after row, then
-// those of the z slabs.  A row of 64 to 256 cells is 16 to 64 quads, so with quads in plain
-// row order every wave holds some z-slab lanes and issues the z slab's psi loads,
-// arithmetic and stores for a few lanes; grouped, they fill waves of their own (at 160
-// cells and npml 10: 6 of 40 quads a row, 2 of 10 waves instead of all).  R is the smallest
-// group that leaves next to no idle thread.  Quads next to each other in a run are next to
-// each other in memory too, so a lane finds its k+4 (k-1) neighbour in the next (previous)
-// lane except at a run's end.
+// 256-thread blocks: first the lines (8 quads) with no cell of a z CPML slab, row after row,
+// then those at the rows' ends with the z slabs.  A row of 64 to 256 cells is 16 to 64
+// quads, so with quads in plain row order every wave holds some z-slab lanes and issues the
+// z slab's psi loads, arithmetic and stores for a few lanes.  Runs cut within a line make
+// two waves fetch it: whole step at 256^3 / 320^3 / 448^3, CPML 10-12, cut at the slab 321 /
+// 557 / 1565 us, at lines 302 / 511 / 1455, plain row order 307 / 519 / 1360; 128^3 38.0 /
+// 37.1 / 39.2.  R is the smallest group that leaves next to no idle thread.  Quads next to
+// each other in a run are next to each other in memory too, so a lane finds its k+4 (k-1)
+// neighbour in the next (previous) lane except at a run's end.
 #pragma once
 
 #include "common.hpp"
@@ -31,6 +32,8 @@ struct RowQuads {
     unsigned planes;
     unsigned ns;        // stripes: 8, or 1 for planes of few rows
     unsigned jx[9];     // first row of each stripe, and ny
+    unsigned m_b;       // ceil(2^32 / bpg), 0: divide (grids of more than 2^32 / bpg blocks)
+    unsigned m_s[8];    // the same of each stripe's rows per plane
 };
 
 struct QuadAt {
@@ -45,13 +48,25 @@ constexpr unsigned kStripes = 8;       // one per XCD
 // 28.4 / 33.3.
 constexpr unsigned kStripeMinRows = 72;
 
+// n / d by d's reciprocal r = ceil(2^32 / d) where n * d < 2^32 (then exact), by division
+// where r is 0.  Block indices are uniform: a division costs the wave some 20 instructions.
+__host__ __device__ __forceinline__ unsigned div_by(unsigned n, unsigned d, unsigned r)
+{
+    return r ? (unsigned)(((unsigned long long)n * r) >> 32) : n / d;
+}
+inline unsigned reciprocal(unsigned long long n_max, unsigned d)
+{
+    if (d < 2 || n_max * d >= (1ull << 32)) return 0u;
+    return (unsigned)(((1ull << 32) + d - 1) / d);
+}
+
 // Quad of thread t of block b.
 __host__ __device__ __forceinline__ QuadAt row_quad(const RowQuads &m, unsigned b, unsigned t)
 {
-    const unsigned x = b % m.ns, bs = b / m.ns;
+    const unsigned x = m.ns == kStripes ? b & (kStripes - 1) : 0u, bs = m.ns == kStripes ? b / kStripes : b;
     const unsigned jx = m.jx[x], S = m.jx[x + 1] - jx;  // the stripe's rows [jx, jx+S)
     const unsigned nrows = m.planes * S;
-    const unsigned grp = bs / m.bpg, part = bs - grp * m.bpg;
+    const unsigned grp = div_by(bs, m.bpg, m.m_b), part = bs - grp * m.bpg;
     const unsigned row0 = grp * m.R;
     const unsigned rows = row0 >= nrows ? 0u : nrows - row0 < m.R ? nrows - row0 : m.R;
     const unsigned r = part * 256u + t;
@@ -68,7 +83,7 @@ __host__ __device__ __forceinline__ QuadAt row_quad(const RowQuads &m, unsigned 
     a.q = (int)(in ? m.zf + pos : z);
     a.next = pos + 1 < len && (in || pos + 1 != m.zf);
     a.prev = pos > 0 && (in || pos != m.zf);
-    unsigned i = row0 / S, j = row0 - i * S + rr;
+    unsigned i = div_by(row0, S, m.m_s[x]), j = row0 - i * S + rr;
     while (j >= S) {  // at most R / S steps
         j -= S;
         ++i;
@@ -78,14 +93,18 @@ __host__ __device__ __forceinline__ QuadAt row_quad(const RowQuads &m, unsigned 
     return a;
 }
 
+constexpr unsigned kEqualRows = 512;
+
 // The stripes' rows: equal shares of the rows' cost, a row of a y slab (psi read and
 // written) costing 1.3 rows.  With equal row counts the first and the last XCD, which hold
-// the y slabs, end last: 96^3 / 160^3 / 192^3 cells, CPML 10, E + H pass 25.3 / 75.6 / 153.0
-// us; with 1.3, 24.3 / 74.2 / 148.5.
+// the y slabs, end last: 160^3 / 192^3 / 256^3 cells, CPML 10, E + H pass 71.2 / 113.8 /
+// 318.9 us; with 1.3, 69.6 / 107.8 / 302.7.  Planes of kEqualRows rows and more take equal
+// stripes: the 4th-order step at 512^3 10.86 ms against 11.10 (256^3 1.47 / 1.44).
 inline void stripe_rows(RowQuads &m, unsigned ny, int npml)
 {
     const unsigned slab = npml > 0 ? (unsigned)npml : 0u;
-    auto cost = [&](unsigned j) { return j < slab || j >= ny - slab ? 13u : 10u; };
+    const unsigned slab_cost = ny >= kEqualRows ? 10u : 13u;
+    auto cost = [&](unsigned j) { return j < slab || j >= ny - slab ? slab_cost : 10u; };
     unsigned total = 0;
     for (unsigned j = 0; j < ny; ++j) total += cost(j);
     unsigned x = 0, sum = 0;
@@ -94,6 +113,14 @@ inline void stripe_rows(RowQuads &m, unsigned ny, int npml)
         sum += cost(j);
     }
     while (x <= 8) m.jx[x++] = ny;
+}
+
+// Blocks of a pass (a multiple of the stripes; the stripes' own counts differ by a row a plane).
+inline unsigned long long row_quads_blocks(const RowQuads &m)
+{
+    unsigned long long S = 0;
+    for (unsigned x = 0; x < m.ns; ++x) S = m.jx[x + 1] - m.jx[x] > S ? m.jx[x + 1] - m.jx[x] : S;
+    return (m.planes * S + m.R - 1) / m.R * m.bpg * m.ns;
 }
 
 // The order for `planes` planes of ny rows of Q quads (nz cells, npml-cell z slabs; npml =
@@ -109,6 +136,10 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     stripe_rows(m, ny, npml);
     m.zf = npml > 0 ? (unsigned)(((front > npml ? front : npml) + 3) / 4) : 0u;
     m.zb = npml > 0 ? (unsigned)((nz - 1 - npml) / 4) : Q;
+    if (npml > 0) {  // whole 128-byte lines (8 quads) on either side of a run's end
+        m.zf = (m.zf + 7) / 8 * 8;
+        m.zb = m.zb / 8 * 8;
+    }
     if (m.zf >= m.zb) {  // every quad may hold a slab cell: one run
         m.zf = 0;
         m.zb = 0;
@@ -131,15 +162,12 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     m.bpg = (best * Q + 255) / 256;
     m.m_in = m.nin ? (unsigned)(((1ull << 31) + m.nin - 1) / m.nin) : 0u;
     m.m_z = m.nzq ? (unsigned)(((1ull << 31) + m.nzq - 1) / m.nzq) : 0u;
+    m.m_b = reciprocal(row_quads_blocks(m) + kStripes, m.bpg);
+    for (unsigned x = 0; x < 8; ++x) {
+        const unsigned S = m.jx[x + 1] - m.jx[x];
+        m.m_s[x] = reciprocal((unsigned long long)planes * S + 64 * m.R, S);
+    }
     return m;
-}
-
-// Blocks of a pass (a multiple of the stripes; the stripes' own counts differ by a row a plane).
-inline unsigned long long row_quads_blocks(const RowQuads &m)
-{
-    unsigned long long S = 0;
-    for (unsigned x = 0; x < m.ns; ++x) S = m.jx[x + 1] - m.jx[x] > S ? m.jx[x + 1] - m.jx[x] : S;
-    return (m.planes * S + m.R - 1) / m.R * m.bpg * m.ns;
 }
 
 }  // namespace mifdtd

@@ -298,6 +298,23 @@ inline void aux_box(SAux &a)
         aux_cover(a, a.prb.i[n], a.prb.i[n], a.prb.j[n], a.prb.j[n], a.prb.k[n], a.prb.k[n]);
 }
 
+// z-face psi and table entries of a quad's cells, loaded ahead of the update: loads that
+// follow the previous cell's psi store are four memory round trips in a row.
+struct ZFace {
+    float q1[4], q2[4], b[4], a[4];
+    // cell l: psi1 at p (psi2 s2 after it) and table entry t, where the cell is in the slab (t > 0)
+    __device__ __forceinline__ void load(int l, int t, const float *psi, size_t off, size_t s2, const float *tb,
+                                         const float *ta)
+    {
+        const size_t o = t > 0 ? off : 0;
+        const int e = t > 0 ? t : 0;
+        q1[l] = psi[o];
+        q2[l] = psi[o + s2];
+        b[l] = tb[e];
+        a[l] = ta[e];
+    }
+};
+
 // E pass on the quad (i, j, k0..k0+3): reads E from exi.. and writes it to exo.. (the
 // same arrays for an in-place update, the next-step buffers for a ping-pong one); psi E
 // is read from cp.pe and written to cp.pe_out.  CE: CM = 0 the constant 0.5, 1 the float
@@ -344,17 +361,32 @@ __device__ __forceinline__ void e_quad_at(
     const int npml = PML ? cp.npml : 0;
     int xs = 0, xp = 0, ys = 0, yp = 0, xt = -1, yt = -1;
     Q4 p1 = z4, p2 = z4;   // psi of the x face, or of the y face where there is no x face
+    float pb = 0.f, pa = 0.f;
     size_t o1 = 0, o2 = 0;
+    ZFace z;
+    bool zq = false;
     if (PML) {
         xt = (cp.axes & 1) ? sslab_e(i, nx, npml, xs, xp) : -1;  // x slab planes are all < nx-1
         yt = (cp.axes & 2) ? sslab_e(j, ny, npml, ys, yp) : -1;  // y slab rows are all < ny-1
         if (xt > 0 || yt > 0) {
             const size_t o = xt > 0 ? ((size_t)xp * ny + j) * nzp + k0 : ((size_t)i * npml + yp) * nzp + k0;
             const int f = xt > 0 ? xs : 2 + ys;
+            const int t = xt > 0 ? xt : yt;
             o1 = cp.off(f, 0) + o;
             o2 = cp.off(f, 1) + o;
             p1 = ld4(cp.pe + o1);
             p2 = ld4(cp.pe + o2);
+            pb = cp.bE[t];
+            pa = cp.aE[t];
+        }
+        zq = (cp.axes & 4) && (k0 < npml || (k0 + 3 >= nz - 1 - npml && k0 < nz - 1));
+        if (zq) {
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                int zs, zp;
+                const int t = sslab_e(k0 + l, nz, npml, zs, zp);
+                z.load(l, t, cp.pe, cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp, cp.sZ, cp.bE, cp.aE);
+            }
         }
     }
 
@@ -404,7 +436,7 @@ __device__ __forceinline__ void e_quad_at(
     }
     if (PML) {
         if (xt > 0) {  // psi1: ey, psi2: ez
-            const float b = cp.bE[xt], a = cp.aE[xt];
+            const float b = pb, a = pa;
 #pragma unroll
             for (int l = 0; l < 4; ++l)
                 if (k0 + l < nz - 1) {
@@ -431,8 +463,10 @@ __device__ __forceinline__ void e_quad_at(
                 o2 = cp.off(2 + ys, 1) + o;
                 p1 = ld4(cp.pe + o1);
                 p2 = ld4(cp.pe + o2);
+                pb = cp.bE[yt];
+                pa = cp.aE[yt];
             }
-            const float b = cp.bE[yt], a = cp.aE[yt];
+            const float b = pb, a = pa;
 #pragma unroll
             for (int l = 0; l < 4; ++l)
                 if (k0 + l < nz - 1) {
@@ -452,25 +486,21 @@ __device__ __forceinline__ void e_quad_at(
             st4(cp.pe_out + o1, p1);
             st4(cp.pe_out + o2, p2);
         }
-        if ((cp.axes & 4) && (k0 < npml || (k0 + 3 >= nz - 1 - npml && k0 < nz - 1))) {  // psi1: ex, psi2: ey
+        if (zq) {  // psi1: ex, psi2: ey
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 int zs, zp;
-                const int zt = sslab_e(k0 + l, nz, npml, zs, zp);
-                if (zt > 0) {
-                    const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
-                    const float b = cp.bE[zt], a = cp.aE[zt];
-                    const float q1 = cp.pe[o], q2 = cp.pe[o + cp.sZ];
-                    if (jy) {
-                        const float tt = b * q1 + a * (y1[l] - hy0.v[l]);
-                        cp.pe_out[o] = tt;
-                        e0.v[l] = e0.v[l] - c0.v[l] * tt;
-                    }
-                    if (ix) {
-                        const float tt = b * q2 + a * (x1[l] - hx0.v[l]);
-                        cp.pe_out[o + cp.sZ] = tt;
-                        e1.v[l] = e1.v[l] + c1.v[l] * tt;
-                    }
+                const bool on = sslab_e(k0 + l, nz, npml, zs, zp) > 0;
+                const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
+                if (on && jy) {
+                    const float tt = z.b[l] * z.q1[l] + z.a[l] * (y1[l] - hy0.v[l]);
+                    cp.pe_out[o] = tt;
+                    e0.v[l] = e0.v[l] - c0.v[l] * tt;
+                }
+                if (on && ix) {
+                    const float tt = z.b[l] * z.q2[l] + z.a[l] * (x1[l] - hx0.v[l]);
+                    cp.pe_out[o + cp.sZ] = tt;
+                    e1.v[l] = e1.v[l] + c1.v[l] * tt;
                 }
             }
         }
@@ -534,17 +564,33 @@ __device__ __forceinline__ void h_quad_at(
     const int npml = PML ? cp.npml : 0;
     int xs = 0, xp = 0, ys = 0, yp = 0, xt = -1, yt = -1;
     Q4 p1 = z4, p2 = z4;   // psi of the x face, or of the y face where there is no x face
+    float pb = 0.f, pa = 0.f;
     size_t o1 = 0, o2 = 0;
+    ZFace z;
+    bool zq = false;
     if (PML) {
         xt = ip && (cp.axes & 1) ? sslab_h(i, nx, npml, xs, xp) : -1;  // plane 0 is the wall
         yt = jp && (cp.axes & 2) ? sslab_h(j, ny, npml, ys, yp) : -1;  // row 0 is the wall
         if (xt > 0 || yt > 0) {
             const size_t o = xt > 0 ? ((size_t)xp * ny + j) * nzp + k0 : ((size_t)i * npml + yp) * nzp + k0;
             const int f = xt > 0 ? xs : 2 + ys;
+            const int t = xt > 0 ? xt : yt;
             o1 = cp.off(f, 0) + o;
             o2 = cp.off(f, 1) + o;
             p1 = ld4(cp.ph + o1);
             p2 = ld4(cp.ph + o2);
+            pb = cp.bH[t];
+            pa = cp.aH[t];
+        }
+        zq = (cp.axes & 4) && (k0 < npml || (k0 + 3 >= nz - npml && k0 < nz));
+        if (zq) {
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                int zs, zp;
+                const int t = sslab_h(k0 + l, nz, npml, zs, zp);
+                z.load(l, k0 + l > 0 ? t : -1, cp.ph, cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp, cp.sZ, cp.bH,
+                       cp.aH);  // k = 0 is the wall
+            }
         }
     }
 
@@ -588,7 +634,7 @@ __device__ __forceinline__ void h_quad_at(
     }
     if (PML) {
         if (xt > 0) {  // psi1: hy, psi2: hz
-            const float b = cp.bH[xt], a = cp.aH[xt];
+            const float b = pb, a = pa;
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 const int k = k0 + l;
@@ -617,8 +663,10 @@ __device__ __forceinline__ void h_quad_at(
                 o2 = cp.off(2 + ys, 1) + o;
                 p1 = ld4(cp.ph + o1);
                 p2 = ld4(cp.ph + o2);
+                pb = cp.bH[yt];
+                pa = cp.aH[yt];
             }
-            const float b = cp.bH[yt], a = cp.aH[yt];
+            const float b = pb, a = pa;
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 const int k = k0 + l;
@@ -640,26 +688,21 @@ __device__ __forceinline__ void h_quad_at(
             st4(cp.ph + o1, p1);
             st4(cp.ph + o2, p2);
         }
-        if ((cp.axes & 4) && (k0 < npml || (k0 + 3 >= nz - npml && k0 < nz))) {  // psi1: hx, psi2: hy
+        if (zq) {  // psi1: hx, psi2: hy
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 int zs, zp;
-                const int k = k0 + l;
-                const int zt = k > 0 ? sslab_h(k, nz, npml, zs, zp) : -1;  // k = 0 is the wall
-                if (zt > 0) {
-                    const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
-                    const float b = cp.bH[zt], a = cp.aH[zt];
-                    const float q1 = cp.ph[o], q2 = cp.ph[o + cp.sZ];
-                    if (jp) {
-                        const float tt = b * q1 + a * (ey0.v[l] - ym[l]);
-                        cp.ph[o] = tt;
-                        h0.v[l] = h0.v[l] + 0.5f * tt;
-                    }
-                    if (ip) {
-                        const float tt = b * q2 + a * (ex0.v[l] - xm[l]);
-                        cp.ph[o + cp.sZ] = tt;
-                        h1.v[l] = h1.v[l] - 0.5f * tt;
-                    }
+                const bool on = sslab_h(k0 + l, nz, npml, zs, zp) > 0 && k0 + l > 0;
+                const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
+                if (on && jp) {
+                    const float tt = z.b[l] * z.q1[l] + z.a[l] * (ey0.v[l] - ym[l]);
+                    cp.ph[o] = tt;
+                    h0.v[l] = h0.v[l] + 0.5f * tt;
+                }
+                if (on && ip) {
+                    const float tt = z.b[l] * z.q2[l] + z.a[l] * (ex0.v[l] - xm[l]);
+                    cp.ph[o + cp.sZ] = tt;
+                    h1.v[l] = h1.v[l] - 0.5f * tt;
                 }
             }
         }
