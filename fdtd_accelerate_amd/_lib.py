@@ -73,6 +73,17 @@ class DesignBox(ctypes.Structure):
     _fields_ = [("i0", _I), ("j0", _I), ("k0", _I), ("di", _I), ("dj", _I), ("dk", _I)]
 
 
+class S4Desc(ctypes.Structure):
+    """``mifdtd_s4_desc`` (include/mifdtd.h)."""
+    _fields_ = [
+        ("nx", _I), ("ny", _I), ("nz", _I), ("e", _P * 6), ("ce", _P * 3), ("ce0", _F), ("ce_mat", _P * 3), ("ce_lut", _P),
+        ("ch", _P * 3), ("ch0", _F), ("cl", _F * 5), ("dl", _F * 4), ("cpml_e", CpmlHalf * 4), ("cpml_h", CpmlHalf * 5),
+        ("nsrc", _I), ("src_comp", _I * MAX_SRC), ("src_box", (_I * 6) * MAX_SRC), ("src_sv", _P * MAX_SRC),
+        ("src_svs", _F * MAX_SRC),
+        ("nprobe", _I), ("probe_comp", _I * MAX_PROBE), ("probe_ijk", (_I * 3) * MAX_PROBE),
+    ]
+
+
 # name -> (restype, argtypes)
 _SIGS = {
     "mifdtd_last_error": (ctypes.c_char_p, []),
@@ -117,6 +128,7 @@ _SIGS = {
     "mifdtd_s4_update_h": (_I, [_I] * 3 + [_F] + [_P] * 9 + [_F, _P]),
     "mifdtd_s4_update_e": (_I, [_I] * 3 + [_F] + [_P] * 9 + [_F, _P]),
     "mifdtd_s4_update_e_lut": (_I, [_I] * 3 + [_F] + [_P] * 10 + [_P]),
+    "mifdtd_s4_run": (_I, [ctypes.POINTER(S4Desc), _I, _P, _P, _P]),
     "mifdtd_s4_cpml_e": (_I, [_I] * 3 + [ctypes.POINTER(CpmlHalf), _F] + [_P] * 9 + [_F, _P]),
     "mifdtd_s4_cpml_h": (_I, [_I] * 3 + [ctypes.POINTER(CpmlHalf), _F] + [_P] * 9 + [_F, _P]),
 }

@@ -4,7 +4,7 @@
 // no padding.
 //
 // A lane per x-quad (4 consecutive x cells of one (j, k) row; nx must be a multiple of
-// 4), work-groups marching z (below).  Per-cell arithmetic keeps the reference's
+// 4).  Per-cell arithmetic keeps the reference's
 // evaluation order:
 //   H: h -= (cl*ch) * (27*(((a0 - a1) - b0) + b1) - (((a2 - a3) - b2) + b3))
 //   E: e += (dl*ce) * (27*(((a0 - a1) - b0) + b1) - (((a2 - a3) - b2) + b3))
@@ -12,70 +12,65 @@
 // Guards (which cells each stage writes) follow dielectric.c:30-42,77-89 including its
 // i < nx-1, j < ny-1, k < nz-1 loop bounds.
 
-#include "common.hpp"
+#include "row_quads.hpp"
+#include "step_quad.hpp"
 
 namespace mifdtd {
 
 constexpr int S4B = 256;
-constexpr int kS4Rows = 8;     // owned rows per work-group of the z-marching stages (T+3 waves)
-constexpr int kS4Planes = 32;  // planes per z chunk
 
-// ------------------------------------------------------------------ z-marching stages
-// The stage updates with the neighbour rows and planes read once per work-group:
-// a work-group owns one x segment of 64 quads (a lane per quad) of T rows [j0, j0+T) and
-// marches the planes of a z chunk [k0, k1).  Wave w holds row j0-1+w (E stage) or
-// j0-2+w (H stage), so that the T owned rows have the y halo rows (E: j-1, j+1, j+2;
-// H: j-2, j-1, j+1) as waves of the same work-group; per plane each wave publishes the
-// two components its neighbours need (E: hz, hx; H: ez, ex) in LDS (double-buffered, one
-// barrier per plane).  The z neighbours (E: hy, hx at k-1 .. k+2; H: ey, ex at k-2 ..
-// k+1) stay in a four-plane register window per owned lane, and the x neighbours come
-// from the adjacent lanes (the segment's edge lanes load theirs).  Arithmetic and
-// guards are those of the header above, so the values equal the reference's.
-struct S4ZGeom {
+// ------------------------------------------------------------------ stage kernels
+// A lane per x-quad in the whole-grid thread order (row_quads.hpp with z as the planes and
+// x as the cells: a stripe of every plane's rows per XCD, x-slab quads in waves of their
+// own).  One pass updates E (or H) of a stage with its CPML, sources and probes, so each
+// array is read and written once per stage; the y and z neighbour rows (three of each) are
+// L2 hits of the stripe.  The bound is the traffic behind the L2s.  Against a marching
+// work-group per 8 rows x 32 planes with separate CPML launches (which left most of the
+// chip idle on small grids: 36 work-groups at 132 x 90 x 75), per step with CPML 10: 64^3
+// 627 -> 68 us, 132 x 90 x 75 732 -> 115, 200^3 1081 -> 552, 400 x 300 x 200 2789 -> 2067,
+// 512^3 10.99 -> 10.86 ms.  The contiguous-axis faces cost most of what CPML costs (512^3:
+// none 10.2, y and z 10.3, x 11.0 ms).
+struct S4Geom {
     int nx, ny, nz;
-    int Qx;   // quads per x row
-    int nxs;  // x segments of 64 quads per row
-    int T;    // owned rows per work-group
-    int nyt;  // row tiles
-    int cz;   // planes per z chunk
-    int nzc;  // z chunks
+    RowQuads m;
+};
+
+// CPML of one half: psi1/psi2 of face 2*axis + side (null: off), tables of the stage.
+struct S4Cpml {
+    int npml;
+    float *psi1[6], *psi2[6];
+    const float *b, *a;
 };
 
 // x neighbours of this lane's quad q of f (x = i0 .. i0+3): f[i0-2], f[i0-1], f[i0+4],
-// f[i0+5], zero outside the row.  Called by every lane of the wave (shuffles).
+// f[i0+5], zero outside the row.  Called by every lane of the wave (lane shifts).
 struct XN {
     float m2, m1, p4, p5;
 };
 
-__device__ __forceinline__ XN xneigh(const float *f, size_t id, const Q4 &q, int lane, int qi, int Qx)
+__device__ __forceinline__ XN xneigh(const float *f, size_t id, const Q4 &q, int i0, int nx, bool prev, bool next)
 {
     XN n;
-    n.m2 = __shfl_up(q.v[2], 1);
-    n.m1 = __shfl_up(q.v[3], 1);
-    n.p4 = __shfl_down(q.v[0], 1);
-    n.p5 = __shfl_down(q.v[1], 1);
-    if (lane == 0) {
-        n.m2 = qi > 0 ? f[id - 2] : 0.f;
-        n.m1 = qi > 0 ? f[id - 1] : 0.f;
+    n.m2 = lane_prev(q.v[2]);
+    n.m1 = lane_prev(q.v[3]);
+    n.p4 = lane_next(q.v[0]);
+    n.p5 = lane_next(q.v[1]);
+    if (!prev) {
+        const float2 t = i0 > 0 ? *reinterpret_cast<const float2 *>(f + id - 2) : make_float2(0.f, 0.f);
+        n.m2 = t.x;
+        n.m1 = t.y;
     }
-    if (qi + 1 >= Qx) {
-        n.p4 = n.p5 = 0.f;
-    } else if (lane == 63) {
-        n.p4 = f[id + 4];
-        n.p5 = f[id + 5];
+    if (!next) {
+        const float2 t = i0 + 4 < nx ? *reinterpret_cast<const float2 *>(f + id + 4) : make_float2(0.f, 0.f);
+        n.p4 = t.x;
+        n.p5 = t.y;
     }
     return n;
 }
 
-__device__ __forceinline__ Q4 lds4(const float *p) { return Q4{{p[0], p[1], p[2], p[3]}}; }
-
-__device__ __forceinline__ void put4(float *p, const Q4 &q)
-{
-    *reinterpret_cast<float4 *>(p) = make_float4(q.v[0], q.v[1], q.v[2], q.v[3]);
-}
-
 // CE of the E stage: the constant ce0, three float arrays, or three uint8 material-index
-// arrays into a 3 x 256 table of the float values (staged in LDS; the same products).
+// arrays into a 3 x 256 table of the float values (the same products; the table stays in
+// the caches).
 enum S4Ce { kS4CeConst = 0, kS4CeArrays = 1, kS4CeTable = 2 };
 
 template <int CEM>
@@ -83,228 +78,360 @@ __device__ __forceinline__ Q4 s4_ce(const float *c, const unsigned char *m, cons
 {
     if (CEM == kS4CeConst) return splat4(ce0);
     if (CEM == kS4CeArrays) return ld4(c + id);
-    const uchar4 t = *reinterpret_cast<const uchar4 *>(m + id);
-    return Q4{{tab[t.x], tab[t.y], tab[t.z], tab[t.w]}};
+    return ce_from_table(m + id, tab);
 }
 
-template <int CEM>
-__global__ __launch_bounds__(1024) void k_s4_e_zm(S4ZGeom g, float dl, float *__restrict__ ex, float *__restrict__ ey,
-                                                  float *__restrict__ ez, const float *__restrict__ hx,
-                                                  const float *__restrict__ hy, const float *__restrict__ hz,
-                                                  const float *__restrict__ cx, const float *__restrict__ cy,
-                                                  const float *__restrict__ cz, float ce0,
-                                                  const unsigned char *__restrict__ mx,
-                                                  const unsigned char *__restrict__ my,
-                                                  const unsigned char *__restrict__ mz, const float *__restrict__ lut)
+// The 4th-order difference at one cell: 27 (p1 - p0) - (p2 - m1).
+__device__ __forceinline__ float diff4(float m1, float p0, float p1, float p2) { return 27.f * (p1 - p0) - (p2 - m1); }
+
+struct S4Half {
+    float w;     // stage weight
+    float b, a;  // table entry
+};
+
+// psi' = b psi + a d of one cell, and f -/+= w c psi'.
+__device__ __forceinline__ void s4_psi_cell(const S4Half &h, float &psi, float d, float c, float &f, bool minus)
 {
-    extern __shared__ float zl[];  // [2][T+3][2][256]: hz, hx of plane k, rows j0-1 .. j0+T+1; [768] CE table
-    const int T = g.T;
-    float *tab = zl + (size_t)2 * (T + 3) * 512;
-    if (CEM == kS4CeTable) {
-        for (int t = threadIdx.x; t < 768; t += blockDim.x) tab[t] = lut[t];
-        __syncthreads();
-    }
-    unsigned b = blockIdx.x;
-    const int xs = (int)(b % (unsigned)g.nxs);
-    b /= (unsigned)g.nxs;
-    const int yt = (int)(b % (unsigned)g.nyt);
-    const int zc = (int)(b / (unsigned)g.nyt);
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
-    const int j0 = yt * T, k0 = zc * g.cz, k1 = min(nz, k0 + g.cz);
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int j = j0 - 1 + w;
-    const int qi = xs * 64 + lane;
-    const bool qact = qi < g.Qx;
-    const int i0 = 4 * (qact ? qi : g.Qx - 1);  // inactive lanes address the row's last quad
-    const bool rowok = j >= 0 && j < ny;
-    const size_t sz = (size_t)nx * ny;
-    const size_t rowoff = (size_t)(rowok ? j : 0) * nx + i0;
-    const bool own = w >= 1 && w <= T && j < ny;
-    const float c27 = 27.f;
-    const Q4 z4 = splat4(0.f);
-    Q4 hyw[4], hxw[4];  // planes k-1 .. k+2 of this lane's quad (owned rows)
-    if (own) {
+    const float tt = h.b * psi + h.a * d;
+    psi = tt;
+    if (minus) f -= h.w * c * tt;
+    else f += h.w * c * tt;
+}
+
+// A quad's cells in an x face.  The slabs are more than a quad apart (nx >= 2 npml + 4), so
+// a quad meets one side only: its cells' psi and table entries are consecutive.
+struct S4FaceX {
+    float *p1, *p2;  // psi1, psi2 of cell l = 0 (which may lie outside the slab)
+    int t0;          // its table entry
+    int lo, hi;      // cells l in [lo, hi) are in the slab and written by the stage
+    float q1[4], q2[4], b[4], a[4];
+    // slab planes [s0, s0+p) with entries from t; the stage writes [w0, w1); row = p*(j + ny*k)
+    __device__ __forceinline__ void load(const S4Cpml &cp, int side, int i0, int s0, int t, int w0, int w1, size_t row)
+    {
+        float *f1 = side ? cp.psi1[1] : cp.psi1[0], *f2 = side ? cp.psi2[1] : cp.psi2[0];
+        lo = max(max(s0, w0) - i0, 0);
+        hi = f1 ? min(min(s0 + cp.npml, w1) - i0, 4) : 0;
+        const ptrdiff_t o = (ptrdiff_t)row + (i0 - s0);
+        p1 = f1 + o;
+        p2 = f2 + o;
+        t0 = t + (i0 - s0);
+        const float *pb = cp.b + t0, *pa = cp.a + t0;
+        // all loads before any store: a load that follows the previous cell's psi store is a
+        // memory round trip of its own
 #pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            const int kk = k0 - 1 + m;
-            const bool in = kk >= 0 && kk < nz;
-            hyw[m] = in ? ld4(hy + (size_t)kk * sz + rowoff) : z4;
-            hxw[m] = in ? ld4(hx + (size_t)kk * sz + rowoff) : z4;
+        for (int l = 0; l < 4; ++l) {
+            q1[l] = q2[l] = b[l] = a[l] = 0.f;
+            if (l >= lo && l < hi) {
+                q1[l] = p1[l];
+                q2[l] = p2[l];
+                b[l] = pb[l];
+                a[l] = pa[l];
+            }
         }
     }
-    for (int k = k0; k < k1; ++k) {
-        float *buf = zl + (size_t)((k - k0) & 1) * (T + 3) * 512;
-        const size_t idk = (size_t)k * sz + rowoff;
-        const Q4 hzk = rowok ? ld4(hz + idk) : z4;
-        Q4 hxk, e0, e1, e2, c0, c1, c2;
-        if (own) {
-            const bool in2 = k + 2 < nz;
-            hyw[3] = in2 ? ld4(hy + idk + 2 * sz) : z4;
-            hxw[3] = in2 ? ld4(hx + idk + 2 * sz) : z4;
-            hxk = hxw[1];
-            e0 = ld4(ex + idk);
-            e1 = ld4(ey + idk);
-            e2 = ld4(ez + idk);
-            c0 = s4_ce<CEM>(cx, mx, tab, idk, ce0);
-            c1 = s4_ce<CEM>(cy, my, tab + 256, idk, ce0);
-            c2 = s4_ce<CEM>(cz, mz, tab + 512, idk, ce0);
-        } else {
-            hxk = rowok ? ld4(hx + idk) : z4;
-        }
-        put4(buf + (size_t)(w * 2) * 256 + 4 * lane, hzk);
-        put4(buf + (size_t)(w * 2 + 1) * 256 + 4 * lane, hxk);
-        XN nz_{}, ny_{};
-        if (own) {
-            nz_ = xneigh(hz, idk, hzk, lane, qi, g.Qx);
-            ny_ = xneigh(hy, idk, hyw[1], lane, qi, g.Qx);
-        }
-        __syncthreads();
-        if (own && qact && j <= ny - 2 && k <= nz - 2) {
-            const bool rx = j > 0 && j < ny - 2 && k > 0 && k < nz - 2;
-            const bool ry = k > 0 && k < nz - 2;
-            const bool rz = j > 0 && j < ny - 2;
-            const Q4 hzjm = lds4(buf + (size_t)((w - 1) * 2) * 256 + 4 * lane);
-            const Q4 hzjp = lds4(buf + (size_t)((w + 1) * 2) * 256 + 4 * lane);
-            const Q4 hzj2 = lds4(buf + (size_t)((w + 2) * 2) * 256 + 4 * lane);
-            const Q4 hxjm = lds4(buf + (size_t)((w - 1) * 2 + 1) * 256 + 4 * lane);
-            const Q4 hxjp = lds4(buf + (size_t)((w + 1) * 2 + 1) * 256 + 4 * lane);
-            const Q4 hxj2 = lds4(buf + (size_t)((w + 2) * 2 + 1) * 256 + 4 * lane);
-            // x windows f[i0-2 .. i0+5] of hz and hy at plane k
-            const float wz[8] = {nz_.m2, nz_.m1, hzk.v[0], hzk.v[1], hzk.v[2], hzk.v[3], nz_.p4, nz_.p5};
-            const float wy[8] = {ny_.m2, ny_.m1, hyw[1].v[0], hyw[1].v[1], hyw[1].v[2], hyw[1].v[3], ny_.p4, ny_.p5};
-            const int ib = 4 * qi;
+};
+
+template <int CEM, bool PML>
+__global__ __launch_bounds__(S4B) void k_s4_e(SAux, S4Geom g, S4Cpml cp, float dl, float *__restrict__ ex,
+                                              float *__restrict__ ey, float *__restrict__ ez,
+                                              const float *__restrict__ hx, const float *__restrict__ hy,
+                                              const float *__restrict__ hz, const float *__restrict__ cx,
+                                              const float *__restrict__ cy, const float *__restrict__ cz, float ce0,
+                                              const unsigned char *__restrict__ mx, const unsigned char *__restrict__ my,
+                                              const unsigned char *__restrict__ mz, const float *__restrict__ lut)
+{
+    const QuadAt at = row_quad(g.m, blockIdx.x, threadIdx.x);
+    if (!at.active) return;
+    const int k = at.i, j = at.j, i0 = 4 * at.q;
+    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const int lane = threadIdx.x & 63;
+    const size_t sy = (size_t)nx, sz = (size_t)nx * ny;
+    const size_t id = (size_t)k * sz + (size_t)j * sy + i0;
+    const Q4 z4 = splat4(0.f);
+    // cells written: i, j, k <= n-2 and, off the component's own axis, 1 .. n-3
+    const bool rows = j <= ny - 2 && k <= nz - 2;
+    const bool jin = rows && j > 0 && j < ny - 2, kin = rows && k > 0 && k < nz - 2;
+    const bool rx = jin && kin, ry = kin, rz = jin;
+
+    const Q4 hx0 = ld4(hx + id), hy0 = ld4(hy + id), hz0 = ld4(hz + id);
+    Q4 e0 = ld4(ex + id), e1 = ld4(ey + id), e2 = ld4(ez + id);
+    const Q4 c0 = s4_ce<CEM>(cx, mx, lut, id, ce0);
+    const Q4 c1 = s4_ce<CEM>(cy, my, lut + 256, id, ce0);
+    const Q4 c2 = s4_ce<CEM>(cz, mz, lut + 512, id, ce0);
+    Q4 hzm = z4, hzp = z4, hz2 = z4, hxm = z4, hxp = z4, hx2 = z4;  // rows j-1, j+1, j+2
+    if (jin) {
+        hzm = ld4(hz + id - sy);
+        hzp = ld4(hz + id + sy);
+        hz2 = ld4(hz + id + 2 * sy);
+        hxm = ld4(hx + id - sy);
+        hxp = ld4(hx + id + sy);
+        hx2 = ld4(hx + id + 2 * sy);
+    }
+    Q4 hyM = z4, hyP = z4, hyQ = z4, hxM = z4, hxP = z4, hxQ = z4;  // planes k-1, k+1, k+2
+    if (kin) {
+        hyM = ld4(hy + id - sz);
+        hyP = ld4(hy + id + sz);
+        hyQ = ld4(hy + id + 2 * sz);
+        hxM = ld4(hx + id - sz);
+        hxP = ld4(hx + id + sz);
+        hxQ = ld4(hx + id + 2 * sz);
+    }
+    const bool prev = at.prev && lane > 0, next = at.next && lane < 63;
+    const XN nz_ = xneigh(hz, id, hz0, i0, nx, prev, next), ny_ = xneigh(hy, id, hy0, i0, nx, prev, next);
+    // x windows f[i0-2 .. i0+5]
+    const float wz[8] = {nz_.m2, nz_.m1, hz0.v[0], hz0.v[1], hz0.v[2], hz0.v[3], nz_.p4, nz_.p5};
+    const float wy[8] = {ny_.m2, ny_.m1, hy0.v[0], hy0.v[1], hy0.v[2], hy0.v[3], ny_.p4, ny_.p5};
+    const float c27 = 27.f;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const int i = i0 + l;
+        const bool in = i > 0 && i < nx - 2;
+        if (rx && i <= nx - 2)
+            e0.v[l] += dl * c0.v[l] * (c27 * (hzp.v[l] - hz0.v[l] - hyP.v[l] + hy0.v[l])
+                                       - (hz2.v[l] - hzm.v[l] - hyQ.v[l] + hyM.v[l]));
+        if (ry && in)
+            e1.v[l] += dl * c1.v[l] * (c27 * (hxP.v[l] - hx0.v[l] - wz[l + 3] + hz0.v[l])
+                                       - (hxQ.v[l] - hxM.v[l] - wz[l + 4] + wz[l + 1]));
+        if (rz && in)
+            e2.v[l] += dl * c2.v[l] * (c27 * (wy[l + 3] - hy0.v[l] - hxp.v[l] + hx0.v[l])
+                                       - (wy[l + 4] - wy[l + 1] - hx2.v[l] + hxm.v[l]));
+    }
+    if (PML && rows) {
+        const int p = cp.npml;
+        int sdy, qy, sdz, qz;
+        const int ty = jin ? sslab_e(j, ny, p, sdy, qy) : -1, tz = kin ? sslab_e(k, nz, p, sdz, qz) : -1;
+        // the y and z faces' differences now: their rows and planes are not held any longer
+        Q4 dy1 = z4, dy2 = z4, dz1 = z4, dz2 = z4;
+        if (ty > 0) {
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                const int i = ib + l;
-                if (i > nx - 2) continue;
-                if (rx)
-                    e0.v[l] += dl * c0.v[l] * (c27 * (hzjp.v[l] - hzk.v[l] - hyw[2].v[l] + hyw[1].v[l])
-                                               - (hzj2.v[l] - hzjm.v[l] - hyw[3].v[l] + hyw[0].v[l]));
-                if (i > 0 && i < nx - 2 && ry)
-                    e1.v[l] += dl * c1.v[l] * (c27 * (hxw[2].v[l] - hxw[1].v[l] - wz[l + 3] + hzk.v[l])
-                                               - (hxw[3].v[l] - hxw[0].v[l] - wz[l + 4] + wz[l + 1]));
-                if (i > 0 && i < nx - 2 && rz)
-                    e2.v[l] += dl * c2.v[l] * (c27 * (wy[l + 3] - hyw[1].v[l] - hxjp.v[l] + hxw[1].v[l])
-                                               - (wy[l + 4] - wy[l + 1] - hxj2.v[l] + hxjm.v[l]));
+                dy1.v[l] = diff4(hxm.v[l], hx0.v[l], hxp.v[l], hx2.v[l]);
+                dy2.v[l] = diff4(hzm.v[l], hz0.v[l], hzp.v[l], hz2.v[l]);
             }
-            if (rx) st4(ex + idk, e0);
-            if (ry) st4(ey + idk, e1);
-            if (rz) st4(ez + idk, e2);
         }
-        if (own) {
+        if (tz > 0) {
 #pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                hyw[m] = hyw[m + 1];
-                hxw[m] = hxw[m + 1];
+            for (int l = 0; l < 4; ++l) {
+                dz1.v[l] = diff4(hyM.v[l], hy0.v[l], hyP.v[l], hyQ.v[l]);
+                dz2.v[l] = diff4(hxM.v[l], hx0.v[l], hxP.v[l], hxQ.v[l]);
             }
         }
+        // x faces: psi1 -> ey from hz (-), psi2 -> ez from hy (+)
+        if (i0 < p || i0 + 3 >= nx - 1 - p) {
+            S4FaceX fx;
+            const int side = i0 + 3 >= nx - 1 - p;
+            fx.load(cp, side, i0, side ? nx - 1 - p : 0, side ? p + 1 : 1, 1, nx - 2, (size_t)p * ((size_t)j + (size_t)ny * k));
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                if (l < fx.lo || l >= fx.hi) continue;
+                const S4Half h{dl, fx.b[l], fx.a[l]};
+                if (ry) {
+                    s4_psi_cell(h, fx.q1[l], diff4(wz[l + 1], wz[l + 2], wz[l + 3], wz[l + 4]), c1.v[l], e1.v[l], true);
+                    fx.p1[l] = fx.q1[l];
+                }
+                if (rz) {
+                    s4_psi_cell(h, fx.q2[l], diff4(wy[l + 1], wy[l + 2], wy[l + 3], wy[l + 4]), c2.v[l], e2.v[l], false);
+                    fx.p2[l] = fx.q2[l];
+                }
+            }
+        }
+        // y faces: psi1 -> ez from hx (-), psi2 -> ex from hz (+)
+        if (ty > 0) {
+            float *p1 = sdy ? cp.psi1[3] : cp.psi1[2], *p2 = sdy ? cp.psi2[3] : cp.psi2[2];
+            if (p1) {
+                const size_t n = (size_t)i0 + sy * ((size_t)qy + (size_t)p * k);
+                const S4Half h{dl, cp.b[ty], cp.a[ty]};
+                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+#pragma unroll
+                for (int l = 0; l < 4; ++l) {
+                    const int i = i0 + l;
+                    if (i > 0 && i < nx - 2) s4_psi_cell(h, s1.v[l], dy1.v[l], c2.v[l], e2.v[l], true);
+                    if (rx && i <= nx - 2) s4_psi_cell(h, s2.v[l], dy2.v[l], c0.v[l], e0.v[l], false);
+                }
+                st4u(p1 + n, s1);
+                st4u(p2 + n, s2);
+            }
+        }
+        // z faces: psi1 -> ex from hy (-), psi2 -> ey from hx (+)
+        if (tz > 0) {
+            float *p1 = sdz ? cp.psi1[5] : cp.psi1[4], *p2 = sdz ? cp.psi2[5] : cp.psi2[4];
+            if (p1) {
+                const size_t n = (size_t)i0 + sy * ((size_t)j + (size_t)ny * qz);
+                const S4Half h{dl, cp.b[tz], cp.a[tz]};
+                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+#pragma unroll
+                for (int l = 0; l < 4; ++l) {
+                    const int i = i0 + l;
+                    if (rx && i <= nx - 2) s4_psi_cell(h, s1.v[l], dz1.v[l], c0.v[l], e0.v[l], true);
+                    if (i > 0 && i < nx - 2) s4_psi_cell(h, s2.v[l], dz2.v[l], c1.v[l], e1.v[l], false);
+                }
+                st4u(p1 + n, s1);
+                st4u(p2 + n, s2);
+            }
+        }
+    }
+    const SAux &aux = first_kernel_arg<SAux>();
+    const bool near = aux.near(k, j, i0);
+    if (near) {
+        sapply_src(aux.src, 0, k, j, i0, e0);
+        sapply_src(aux.src, 1, k, j, i0, e1);
+        sapply_src(aux.src, 2, k, j, i0, e2);
+    }
+    st4(ex + id, e0);
+    st4(ey + id, e1);
+    st4(ez + id, e2);
+    if (near) {
+        sprobe(aux.prb, 0, k, j, i0, e0);
+        sprobe(aux.prb, 1, k, j, i0, e1);
+        sprobe(aux.prb, 2, k, j, i0, e2);
     }
 }
 
-template <bool HC>
-__global__ __launch_bounds__(1024) void k_s4_h_zm(S4ZGeom g, float cl, const float *__restrict__ ex,
-                                                  const float *__restrict__ ey, const float *__restrict__ ez,
-                                                  float *__restrict__ hx, float *__restrict__ hy, float *__restrict__ hz,
-                                                  const float *__restrict__ cx, const float *__restrict__ cy,
-                                                  const float *__restrict__ cz, float ch0)
+template <bool HC, bool PML>
+__global__ __launch_bounds__(S4B) void k_s4_h(SAux, S4Geom g, S4Cpml cp, float cl, const float *__restrict__ ex,
+                                              const float *__restrict__ ey, const float *__restrict__ ez,
+                                              float *__restrict__ hx, float *__restrict__ hy, float *__restrict__ hz,
+                                              const float *__restrict__ cx, const float *__restrict__ cy,
+                                              const float *__restrict__ cz, float ch0)
 {
-    extern __shared__ float zl[];  // [2][T+3][2][256]: ez, ex of plane k, rows j0-2 .. j0+T
-    const int T = g.T;
-    unsigned b = blockIdx.x;
-    const int xs = (int)(b % (unsigned)g.nxs);
-    b /= (unsigned)g.nxs;
-    const int yt = (int)(b % (unsigned)g.nyt);
-    const int zc = (int)(b / (unsigned)g.nyt);
+    const QuadAt at = row_quad(g.m, blockIdx.x, threadIdx.x);
+    if (!at.active) return;
+    const int k = at.i, j = at.j, i0 = 4 * at.q;
     const int nx = g.nx, ny = g.ny, nz = g.nz;
-    const int j0 = yt * T, k0 = zc * g.cz, k1 = min(nz, k0 + g.cz);
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int j = j0 - 2 + w;
-    const int qi = xs * 64 + lane;
-    const bool qact = qi < g.Qx;
-    const int i0 = 4 * (qact ? qi : g.Qx - 1);
-    const bool rowok = j >= 0 && j < ny;
-    const size_t sz = (size_t)nx * ny;
-    const size_t rowoff = (size_t)(rowok ? j : 0) * nx + i0;
-    const bool own = w >= 2 && w <= T + 1 && j < ny;
-    const float c27 = 27.f;
+    const size_t sy = (size_t)nx, sz = (size_t)nx * ny;
+    const size_t id = (size_t)k * sz + (size_t)j * sy + i0;
     const Q4 z4 = splat4(0.f);
-    Q4 eyw[4], exw[4];  // planes k-2 .. k+1 of this lane's quad (owned rows)
-    if (own) {
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            const int kk = k0 - 2 + m;
-            const bool in = kk >= 0 && kk < nz;
-            eyw[m] = in ? ld4(ey + (size_t)kk * sz + rowoff) : z4;
-            exw[m] = in ? ld4(ex + (size_t)kk * sz + rowoff) : z4;
-        }
+    // cells written: i, j, k <= n-2 and, off the component's own axis, 2 .. n-2
+    const bool rows = j <= ny - 2 && k <= nz - 2;
+    const bool jin = rows && j > 1, kin = rows && k > 1;
+    const bool rx = jin && kin, ry = kin, rz = jin;
+
+    const Q4 ex0 = ld4(ex + id), ey0 = ld4(ey + id), ez0 = ld4(ez + id);
+    Q4 h0 = ld4(hx + id), h1 = ld4(hy + id), h2 = ld4(hz + id);
+    const Q4 c0 = HC ? ld4(cx + id) : splat4(ch0);
+    const Q4 c1 = HC ? ld4(cy + id) : splat4(ch0);
+    const Q4 c2 = HC ? ld4(cz + id) : splat4(ch0);
+    Q4 ez2 = z4, ezm = z4, ezp = z4, ex2 = z4, exm = z4, exp = z4;  // rows j-2, j-1, j+1
+    if (jin) {
+        ez2 = ld4(ez + id - 2 * sy);
+        ezm = ld4(ez + id - sy);
+        ezp = ld4(ez + id + sy);
+        ex2 = ld4(ex + id - 2 * sy);
+        exm = ld4(ex + id - sy);
+        exp = ld4(ex + id + sy);
     }
-    for (int k = k0; k < k1; ++k) {
-        float *buf = zl + (size_t)((k - k0) & 1) * (T + 3) * 512;
-        const size_t idk = (size_t)k * sz + rowoff;
-        const Q4 ezk = rowok ? ld4(ez + idk) : z4;
-        Q4 exk, h0, h1, h2, c0, c1, c2;
-        if (own) {
-            const bool in1 = k + 1 < nz;
-            eyw[3] = in1 ? ld4(ey + idk + sz) : z4;
-            exw[3] = in1 ? ld4(ex + idk + sz) : z4;
-            exk = exw[2];
-            h0 = ld4(hx + idk);
-            h1 = ld4(hy + idk);
-            h2 = ld4(hz + idk);
-            c0 = HC ? ld4(cx + idk) : splat4(ch0);
-            c1 = HC ? ld4(cy + idk) : splat4(ch0);
-            c2 = HC ? ld4(cz + idk) : splat4(ch0);
-        } else {
-            exk = rowok ? ld4(ex + idk) : z4;
-        }
-        put4(buf + (size_t)(w * 2) * 256 + 4 * lane, ezk);
-        put4(buf + (size_t)(w * 2 + 1) * 256 + 4 * lane, exk);
-        XN nz_{}, ny_{};
-        if (own) {
-            nz_ = xneigh(ez, idk, ezk, lane, qi, g.Qx);
-            ny_ = xneigh(ey, idk, eyw[2], lane, qi, g.Qx);
-        }
-        __syncthreads();
-        if (own && qact && j <= ny - 2 && k <= nz - 2) {
-            const bool rx = j > 1 && k > 1;
-            const bool ry = k > 1;
-            const bool rz = j > 1;
-            const Q4 ezjm = lds4(buf + (size_t)((w - 1) * 2) * 256 + 4 * lane);
-            const Q4 ezjp = lds4(buf + (size_t)((w + 1) * 2) * 256 + 4 * lane);
-            const Q4 ezj2 = lds4(buf + (size_t)((w - 2) * 2) * 256 + 4 * lane);
-            const Q4 exjm = lds4(buf + (size_t)((w - 1) * 2 + 1) * 256 + 4 * lane);
-            const Q4 exjp = lds4(buf + (size_t)((w + 1) * 2 + 1) * 256 + 4 * lane);
-            const Q4 exj2 = lds4(buf + (size_t)((w - 2) * 2 + 1) * 256 + 4 * lane);
-            const float wz[8] = {nz_.m2, nz_.m1, ezk.v[0], ezk.v[1], ezk.v[2], ezk.v[3], nz_.p4, nz_.p5};
-            const float wy[8] = {ny_.m2, ny_.m1, eyw[2].v[0], eyw[2].v[1], eyw[2].v[2], eyw[2].v[3], ny_.p4, ny_.p5};
-            const int ib = 4 * qi;
+    Q4 eyQ = z4, eyM = z4, eyP = z4, exQ = z4, exM = z4, exP = z4;  // planes k-2, k-1, k+1
+    if (kin) {
+        eyQ = ld4(ey + id - 2 * sz);
+        eyM = ld4(ey + id - sz);
+        eyP = ld4(ey + id + sz);
+        exQ = ld4(ex + id - 2 * sz);
+        exM = ld4(ex + id - sz);
+        exP = ld4(ex + id + sz);
+    }
+    const bool prev = at.prev && lane > 0, next = at.next && lane < 63;
+    const XN nz_ = xneigh(ez, id, ez0, i0, nx, prev, next), ny_ = xneigh(ey, id, ey0, i0, nx, prev, next);
+    const float wz[8] = {nz_.m2, nz_.m1, ez0.v[0], ez0.v[1], ez0.v[2], ez0.v[3], nz_.p4, nz_.p5};
+    const float wy[8] = {ny_.m2, ny_.m1, ey0.v[0], ey0.v[1], ey0.v[2], ey0.v[3], ny_.p4, ny_.p5};
+    const float c27 = 27.f;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const int i = i0 + l;
+        const bool in = i > 1 && i <= nx - 2;
+        if (rx && i <= nx - 2)
+            h0.v[l] -= cl * c0.v[l] * (c27 * (ez0.v[l] - ezm.v[l] - ey0.v[l] + eyM.v[l])
+                                       - (ezp.v[l] - ez2.v[l] - eyP.v[l] + eyQ.v[l]));
+        if (ry && in)
+            h1.v[l] -= cl * c1.v[l] * (c27 * (ex0.v[l] - exM.v[l] - ez0.v[l] + wz[l + 1])
+                                       - (exP.v[l] - exQ.v[l] - wz[l + 3] + wz[l]));
+        if (rz && in)
+            h2.v[l] -= cl * c2.v[l] * (c27 * (ey0.v[l] - wy[l + 1] - ex0.v[l] + exm.v[l])
+                                       - (wy[l + 3] - wy[l] - exp.v[l] + ex2.v[l]));
+    }
+    if (PML && rows) {
+        const int p = cp.npml;
+        int sdy, qy, sdz, qz;
+        const int ty = jin ? sslab_h(j, ny, p, sdy, qy) : -1, tz = kin ? sslab_h(k, nz, p, sdz, qz) : -1;
+        // the y and z faces' differences now: their rows and planes are not held any longer
+        Q4 dy1 = z4, dy2 = z4, dz1 = z4, dz2 = z4;
+        if (ty > 0) {
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                const int i = ib + l;
-                if (i > nx - 2) continue;
-                if (rx && j < ny - 1 && k < nz - 1)
-                    h0.v[l] -= cl * c0.v[l] * (c27 * (ezk.v[l] - ezjm.v[l] - eyw[2].v[l] + eyw[1].v[l])
-                                               - (ezjp.v[l] - ezj2.v[l] - eyw[3].v[l] + eyw[0].v[l]));
-                if (i > 1 && ry)
-                    h1.v[l] -= cl * c1.v[l] * (c27 * (exw[2].v[l] - exw[1].v[l] - ezk.v[l] + wz[l + 1])
-                                               - (exw[3].v[l] - exw[0].v[l] - wz[l + 3] + wz[l]));
-                if (i > 1 && rz)
-                    h2.v[l] -= cl * c2.v[l] * (c27 * (eyw[2].v[l] - wy[l + 1] - exw[2].v[l] + exjm.v[l])
-                                               - (wy[l + 3] - wy[l] - exjp.v[l] + exj2.v[l]));
+                dy1.v[l] = diff4(ex2.v[l], exm.v[l], ex0.v[l], exp.v[l]);
+                dy2.v[l] = diff4(ez2.v[l], ezm.v[l], ez0.v[l], ezp.v[l]);
             }
-            if (rx) st4(hx + idk, h0);
-            if (ry) st4(hy + idk, h1);
-            if (rz) st4(hz + idk, h2);
         }
-        if (own) {
+        if (tz > 0) {
 #pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                eyw[m] = eyw[m + 1];
-                exw[m] = exw[m + 1];
+            for (int l = 0; l < 4; ++l) {
+                dz1.v[l] = diff4(eyQ.v[l], eyM.v[l], ey0.v[l], eyP.v[l]);
+                dz2.v[l] = diff4(exQ.v[l], exM.v[l], ex0.v[l], exP.v[l]);
             }
         }
+        // x faces: psi1 -> hy from ez (+), psi2 -> hz from ey (-)
+        if (i0 < p || i0 + 3 >= nx - p) {
+            S4FaceX fx;
+            const int side = i0 + 3 >= nx - p;
+            fx.load(cp, side, i0, side ? nx - p : 0, side ? p + 2 : 1, 2, nx - 1, (size_t)p * ((size_t)j + (size_t)ny * k));
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                if (l < fx.lo || l >= fx.hi) continue;
+                const S4Half h{cl, fx.b[l], fx.a[l]};
+                if (ry) {
+                    s4_psi_cell(h, fx.q1[l], diff4(wz[l], wz[l + 1], wz[l + 2], wz[l + 3]), c1.v[l], h1.v[l], false);
+                    fx.p1[l] = fx.q1[l];
+                }
+                if (rz) {
+                    s4_psi_cell(h, fx.q2[l], diff4(wy[l], wy[l + 1], wy[l + 2], wy[l + 3]), c2.v[l], h2.v[l], true);
+                    fx.p2[l] = fx.q2[l];
+                }
+            }
+        }
+        // y faces: psi1 -> hz from ex (+), psi2 -> hx from ez (-)
+        if (ty > 0) {
+            float *p1 = sdy ? cp.psi1[3] : cp.psi1[2], *p2 = sdy ? cp.psi2[3] : cp.psi2[2];
+            if (p1) {
+                const size_t n = (size_t)i0 + sy * ((size_t)qy + (size_t)p * k);
+                const S4Half h{cl, cp.b[ty], cp.a[ty]};
+                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+#pragma unroll
+                for (int l = 0; l < 4; ++l) {
+                    const int i = i0 + l;
+                    if (i > 1 && i <= nx - 2) s4_psi_cell(h, s1.v[l], dy1.v[l], c2.v[l], h2.v[l], false);
+                    if (rx && i <= nx - 2) s4_psi_cell(h, s2.v[l], dy2.v[l], c0.v[l], h0.v[l], true);
+                }
+                st4u(p1 + n, s1);
+                st4u(p2 + n, s2);
+            }
+        }
+        // z faces: psi1 -> hx from ey (+), psi2 -> hy from ex (-)
+        if (tz > 0) {
+            float *p1 = sdz ? cp.psi1[5] : cp.psi1[4], *p2 = sdz ? cp.psi2[5] : cp.psi2[4];
+            if (p1) {
+                const size_t n = (size_t)i0 + sy * ((size_t)j + (size_t)ny * qz);
+                const S4Half h{cl, cp.b[tz], cp.a[tz]};
+                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+#pragma unroll
+                for (int l = 0; l < 4; ++l) {
+                    const int i = i0 + l;
+                    if (rx && i <= nx - 2) s4_psi_cell(h, s1.v[l], dz1.v[l], c0.v[l], h0.v[l], false);
+                    if (i > 1 && i <= nx - 2) s4_psi_cell(h, s2.v[l], dz2.v[l], c1.v[l], h1.v[l], true);
+                }
+                st4u(p1 + n, s1);
+                st4u(p2 + n, s2);
+            }
+        }
+    }
+    const SAux &aux = first_kernel_arg<SAux>();
+    const bool near = aux.near(k, j, i0);
+    st4(hx + id, h0);
+    st4(hy + id, h1);
+    st4(hz + id, h2);
+    if (near) {
+        sprobe(aux.prb, 3, k, j, i0, h0);
+        sprobe(aux.prb, 4, k, j, i0, h1);
+        sprobe(aux.prb, 5, k, j, i0, h2);
     }
 }
 
@@ -462,20 +589,103 @@ static int s4_check(int nx, int ny, int nz)
     return 0;
 }
 
-static int s4_zgeom(int nx, int ny, int nz, S4ZGeom &z, unsigned &nblocks)
+static S4Geom s4_geom(int nx, int ny, int nz, int npml)
 {
-    z.nx = nx;
-    z.ny = ny;
-    z.nz = nz;
-    z.Qx = nx / 4;
-    z.nxs = (z.Qx + 63) / 64;
-    z.T = kS4Rows;
-    z.nyt = (ny + z.T - 1) / z.T;
-    z.cz = kS4Planes;
-    z.nzc = (nz + z.cz - 1) / z.cz;
-    const unsigned long long nb = (unsigned long long)z.nxs * z.nyt * z.nzc;
-    if (nb >= (1ull << 31)) return fail(MIFDTD_ERANGE, "4th-order grid too large");
-    nblocks = (unsigned)nb;
+    return S4Geom{nx, ny, nz, row_quads((unsigned)nz, (unsigned)ny, (unsigned)(nx / 4), nx, npml)};
+}
+
+static int s4_check_fields(float *const e[6])
+{
+    for (int c = 0; c < 6; c++) {
+        if (!e[c]) return fail(MIFDTD_ENULL, "field pointer is NULL");
+        if (!aligned16(e[c])) return fail(MIFDTD_EALIGN, "field pointer not 16-byte aligned");
+    }
+    return 0;
+}
+
+static int s4_check_coef(const float *c0, const float *c1, const float *c2)
+{
+    if (!(c0 || c1 || c2)) return 0;
+    if (!(c0 && c1 && c2)) return fail(MIFDTD_ENULL, "coefficient arrays must be all set or all NULL");
+    if (!aligned16(c0) || !aligned16(c1) || !aligned16(c2))
+        return fail(MIFDTD_EALIGN, "coefficient pointer not 16-byte aligned");
+    return 0;
+}
+
+static int s4_check_mat(const unsigned char *const m[3], const float *lut)
+{
+    if (!m[0] || !m[1] || !m[2] || !lut) return fail(MIFDTD_ENULL, "material index or table is NULL");
+    for (int c = 0; c < 3; c++)
+        if (reinterpret_cast<uintptr_t>(m[c]) & 3u) return fail(MIFDTD_EALIGN, "material index array not 4-byte aligned");
+    return 0;
+}
+
+static int s4_check_pml(int nx, int ny, int nz, const mifdtd_cpml_half *cp)
+{
+    const int npml = cp->npml;
+    if (npml < 1 || npml > MIFDTD_MAX_NPML) return fail(MIFDTD_EINVAL, "npml %d outside [1,%d]", npml, MIFDTD_MAX_NPML);
+    if (nx < 2 * npml + 4 || ny < 2 * npml + 4 || nz < 2 * npml + 4)
+        return fail(MIFDTD_EINVAL, "4th-order grid (%d,%d,%d) too small for npml %d", nx, ny, nz, npml);
+    if (!cp->b || !cp->a) return fail(MIFDTD_ENULL, "CPML tables are NULL");
+    for (int f = 0; f < 6; f++)
+        if ((cp->psi1[f] == nullptr) != (cp->psi2[f] == nullptr))
+            return fail(MIFDTD_ENULL, "psi1/psi2 of face %d must both be set or both NULL", f);
+    return 0;
+}
+
+static S4Cpml s4_pml(const mifdtd_cpml_half &h)
+{
+    S4Cpml c{};
+    c.npml = h.npml;
+    c.b = h.b;
+    c.a = h.a;
+    for (int f = 0; f < 6; f++) {
+        c.psi1[f] = h.psi1[f];
+        c.psi2[f] = h.psi2[f];
+    }
+    return c;
+}
+
+// One E (H) stage: pml null without CPML.
+static int s4_stage_e(const S4Geom &g, const S4Cpml *pml, const SAux &aux, float dl, float *const e[6], int cem,
+                      const float *const c[3], float ce0, const unsigned char *const m[3], const float *lut, hipStream_t st)
+{
+    const unsigned nb = (unsigned)row_quads_blocks(g.m);
+    const S4Cpml cp = pml ? *pml : S4Cpml{};
+#define MIFDTD_S4_E(CEM, P)                                                                                             \
+    k_s4_e<CEM, P><<<nb, S4B, 0, st>>>(aux, g, cp, dl, e[0], e[1], e[2], e[3], e[4], e[5], c[0], c[1], c[2], ce0, m[0], m[1], \
+                                       m[2], lut)
+    if (cem == kS4CeTable) {
+        if (pml) MIFDTD_S4_E(kS4CeTable, true);
+        else MIFDTD_S4_E(kS4CeTable, false);
+    } else if (cem == kS4CeArrays) {
+        if (pml) MIFDTD_S4_E(kS4CeArrays, true);
+        else MIFDTD_S4_E(kS4CeArrays, false);
+    } else {
+        if (pml) MIFDTD_S4_E(kS4CeConst, true);
+        else MIFDTD_S4_E(kS4CeConst, false);
+    }
+#undef MIFDTD_S4_E
+    MIFDTD_CHECK_LAUNCH("s4 update_e launch");
+    return 0;
+}
+
+static int s4_stage_h(const S4Geom &g, const S4Cpml *pml, const SAux &aux, float cl, float *const e[6],
+                      const float *const c[3], float ch0, hipStream_t st)
+{
+    const unsigned nb = (unsigned)row_quads_blocks(g.m);
+    const S4Cpml cp = pml ? *pml : S4Cpml{};
+#define MIFDTD_S4_H(HC, P) \
+    k_s4_h<HC, P><<<nb, S4B, 0, st>>>(aux, g, cp, cl, e[0], e[1], e[2], e[3], e[4], e[5], c[0], c[1], c[2], ch0)
+    if (c[0]) {
+        if (pml) MIFDTD_S4_H(true, true);
+        else MIFDTD_S4_H(true, false);
+    } else {
+        if (pml) MIFDTD_S4_H(false, true);
+        else MIFDTD_S4_H(false, false);
+    }
+#undef MIFDTD_S4_H
+    MIFDTD_CHECK_LAUNCH("s4 update_h launch");
     return 0;
 }
 
@@ -483,34 +693,16 @@ static int s4_core(bool h_half, int nx, int ny, int nz, float w, float *ex, floa
                    float *hz, const float *c0, const float *c1, const float *c2, float cconst, hipStream_t st)
 {
     if (int rc = s4_check(nx, ny, nz)) return rc;
-    const float *ptrs[6] = {ex, ey, ez, hx, hy, hz};
-    for (const float *p : ptrs) {
-        if (!p) return fail(MIFDTD_ENULL, "field pointer is NULL");
-        if (!aligned16(p)) return fail(MIFDTD_EALIGN, "field pointer not 16-byte aligned");
-    }
-    const bool hc = c0 || c1 || c2;
-    if (hc && !(c0 && c1 && c2)) return fail(MIFDTD_ENULL, "coefficient arrays must be all set or all NULL");
-    if (hc && (!aligned16(c0) || !aligned16(c1) || !aligned16(c2)))
-        return fail(MIFDTD_EALIGN, "coefficient pointer not 16-byte aligned");
-    S4ZGeom z;
-    unsigned nb = 0;
-    if (int rc = s4_zgeom(nx, ny, nz, z, nb)) return rc;
-    const unsigned threads = 64u * (unsigned)(z.T + 3);
-    const size_t lds = sizeof(float) * 2 * (size_t)(z.T + 3) * 512;
-    if (h_half) {
-        if (hc) k_s4_h_zm<true><<<nb, threads, lds, st>>>(z, w, ex, ey, ez, hx, hy, hz, c0, c1, c2, cconst);
-        else k_s4_h_zm<false><<<nb, threads, lds, st>>>(z, w, ex, ey, ez, hx, hy, hz, c0, c1, c2, cconst);
-        MIFDTD_CHECK_LAUNCH("s4 update_h launch");
-    } else {
-        if (hc)
-            k_s4_e_zm<kS4CeArrays><<<nb, threads, lds, st>>>(z, w, ex, ey, ez, hx, hy, hz, c0, c1, c2, cconst,
-                                                                       nullptr, nullptr, nullptr, nullptr);
-        else
-            k_s4_e_zm<kS4CeConst><<<nb, threads, lds, st>>>(z, w, ex, ey, ez, hx, hy, hz, c0, c1, c2, cconst,
-                                                                      nullptr, nullptr, nullptr, nullptr);
-        MIFDTD_CHECK_LAUNCH("s4 update_e launch");
-    }
-    return 0;
+    float *const e[6] = {ex, ey, ez, hx, hy, hz};
+    if (int rc = s4_check_fields(e)) return rc;
+    if (int rc = s4_check_coef(c0, c1, c2)) return rc;
+    const float *const c[3] = {c0, c1, c2};
+    const unsigned char *const m[3] = {nullptr, nullptr, nullptr};
+    const S4Geom g = s4_geom(nx, ny, nz, 0);
+    SAux aux{};
+    aux_box(aux);
+    if (h_half) return s4_stage_h(g, nullptr, aux, w, e, c, cconst, st);
+    return s4_stage_e(g, nullptr, aux, w, e, c0 ? kS4CeArrays : kS4CeConst, c, cconst, m, nullptr, st);
 }
 
 template <int AXIS>
@@ -551,11 +743,7 @@ static int s4_cpml(bool h_half, int nx, int ny, int nz, const mifdtd_cpml_half *
 {
     if (int rc = s4_check(nx, ny, nz)) return rc;
     if (!cp) return fail(MIFDTD_ENULL, "CPML descriptor is NULL");
-    const int npml = cp->npml;
-    if (npml < 1 || npml > MIFDTD_MAX_NPML) return fail(MIFDTD_EINVAL, "npml %d outside [1,%d]", npml, MIFDTD_MAX_NPML);
-    if (nx < 2 * npml + 4 || ny < 2 * npml + 4 || nz < 2 * npml + 4)
-        return fail(MIFDTD_EINVAL, "4th-order grid (%d,%d,%d) too small for npml %d", nx, ny, nz, npml);
-    if (!cp->b || !cp->a) return fail(MIFDTD_ENULL, "CPML tables are NULL");
+    if (int rc = s4_check_pml(nx, ny, nz, cp)) return rc;
     if ((c0 || c1 || c2) && !(c0 && c1 && c2)) return fail(MIFDTD_ENULL, "coefficient arrays must be all set or all NULL");
     if (int rc = s4_cpml_axis<0>(h_half, nx, ny, nz, cp, w, ex, ey, ez, hx, hy, hz, c0, c1, c2, cconst, st)) return rc;
     if (int rc = s4_cpml_axis<1>(h_half, nx, ny, nz, cp, w, ex, ey, ez, hx, hy, hz, c0, c1, c2, cconst, st)) return rc;
@@ -609,23 +797,102 @@ int mifdtd_s4_update_e_lut(int nx, int ny, int nz, float dl, float *ex, float *e
                            const unsigned char *mat_z, const float *lut, mifdtd_stream_t stream)
 {
     if (int rc = s4_check(nx, ny, nz)) return rc;
-    const float *ptrs[6] = {ex, ey, ez, hx, hy, hz};
-    for (const float *p : ptrs) {
-        if (!p) return fail(MIFDTD_ENULL, "field pointer is NULL");
-        if (!aligned16(p)) return fail(MIFDTD_EALIGN, "field pointer not 16-byte aligned");
+    float *const e[6] = {ex, ey, ez, const_cast<float *>(hx), const_cast<float *>(hy), const_cast<float *>(hz)};
+    if (int rc = s4_check_fields(e)) return rc;
+    const unsigned char *const m[3] = {mat_x, mat_y, mat_z};
+    if (int rc = s4_check_mat(m, lut)) return rc;
+    const float *const c[3] = {nullptr, nullptr, nullptr};
+    SAux aux{};
+    aux_box(aux);
+    return s4_stage_e(s4_geom(nx, ny, nz, 0), nullptr, aux, dl, e, kS4CeTable, c, 0.f, m, lut, to_stream(stream));
+}
+
+int mifdtd_s4_run(const mifdtd_s4_desc *d, int nsteps, const float *tvals, float *probe_series, mifdtd_stream_t stream)
+{
+    if (!d) return fail(MIFDTD_ENULL, "step descriptor is NULL");
+    const int nx = d->nx, ny = d->ny, nz = d->nz;
+    if (int rc = s4_check(nx, ny, nz)) return rc;
+    if (nsteps < 0) return fail(MIFDTD_EINVAL, "nsteps < 0");
+    if (int rc = s4_check_fields(d->e)) return rc;
+    if (int rc = s4_check_coef(d->ce[0], d->ce[1], d->ce[2])) return rc;
+    if (int rc = s4_check_coef(d->ch[0], d->ch[1], d->ch[2])) return rc;
+    const bool tbl = d->ce_mat[0] != nullptr;
+    if (tbl)
+        if (int rc = s4_check_mat(d->ce_mat, d->ce_lut)) return rc;
+    const int cem = tbl ? kS4CeTable : d->ce[0] ? kS4CeArrays : kS4CeConst;
+    const bool pml = d->cpml_e[0].npml > 0;
+    S4Cpml pe[4], ph[5];
+    if (pml) {
+        for (int s = 0; s < 9; s++) {
+            const mifdtd_cpml_half &h = s < 4 ? d->cpml_e[s] : d->cpml_h[s - 4];
+            if (h.npml != d->cpml_e[0].npml) return fail(MIFDTD_EINVAL, "the stages' npml differ");
+            if (int rc = s4_check_pml(nx, ny, nz, &h)) return rc;
+            (s < 4 ? pe[s] : ph[s - 4]) = s4_pml(h);
+        }
     }
-    if (!mat_x || !mat_y || !mat_z || !lut) return fail(MIFDTD_ENULL, "material index or table is NULL");
-    const unsigned char *mats[3] = {mat_x, mat_y, mat_z};
-    for (const unsigned char *m : mats)
-        if (reinterpret_cast<uintptr_t>(m) & 3u) return fail(MIFDTD_EALIGN, "material index array not 4-byte aligned");
-    S4ZGeom z;
-    unsigned nb = 0;
-    if (int rc = s4_zgeom(nx, ny, nz, z, nb)) return rc;
-    const unsigned threads = 64u * (unsigned)(z.T + 3);
-    const size_t lds = sizeof(float) * (2 * (size_t)(z.T + 3) * 512 + 768);
-    k_s4_e_zm<kS4CeTable><<<nb, threads, lds, to_stream(stream)>>>(z, dl, ex, ey, ez, hx, hy, hz, nullptr, nullptr,
-                                                                   nullptr, 0.f, mat_x, mat_y, mat_z, lut);
-    MIFDTD_CHECK_LAUNCH("s4 update_e (CE table) launch");
+    if (d->nsrc < 0 || d->nsrc > MIFDTD_FUSED_MAX_SRC) return fail(MIFDTD_EINVAL, "nsrc outside [0,%d]", MIFDTD_FUSED_MAX_SRC);
+    if (d->nprobe < 0 || d->nprobe > MIFDTD_FUSED_MAX_PROBE)
+        return fail(MIFDTD_EINVAL, "nprobe outside [0,%d]", MIFDTD_FUSED_MAX_PROBE);
+    if (d->nsrc && !tvals) return fail(MIFDTD_ENULL, "tvals is NULL");
+    if (d->nprobe && !probe_series) return fail(MIFDTD_ENULL, "probe_series is NULL");
+    // the passes' planes are z and their cells x
+    SSrc src{};
+    src.n = d->nsrc;
+    for (int n = 0; n < d->nsrc; n++) {
+        const int *b = d->src_box[n];
+        if (d->src_comp[n] < 0 || d->src_comp[n] > 2) return fail(MIFDTD_EINVAL, "source %d component %d", n, d->src_comp[n]);
+        if (b[0] < 0 || b[2] < 0 || b[4] < 0 || b[1] >= nx || b[3] >= ny || b[5] >= nz || b[0] > b[1] || b[2] > b[3] ||
+            b[4] > b[5])
+            return fail(MIFDTD_EINVAL, "source box %d outside the grid", n);
+        src.comp[n] = d->src_comp[n];
+        src.i0[n] = b[4];
+        src.i1[n] = b[5];
+        src.j0[n] = b[2];
+        src.j1[n] = b[3];
+        src.k0[n] = b[0];
+        src.k1[n] = b[1];
+        src.sv[n] = d->src_sv[n];
+        src.svs[n] = d->src_svs[n];
+    }
+    SProbe pbe{}, pbh{};
+    for (int n = 0; n < d->nprobe; n++) {
+        const int *p = d->probe_ijk[n], c = d->probe_comp[n];
+        if (c < 0 || c > 5 || p[0] < 0 || p[0] >= nx || p[1] < 0 || p[1] >= ny || p[2] < 0 || p[2] >= nz)
+            return fail(MIFDTD_EINVAL, "probe %d outside the grid", n);
+        SProbe &P = c < 3 ? pbe : pbh;
+        const int m = P.n++;
+        P.comp[m] = c;
+        P.i[m] = p[2];
+        P.j[m] = p[1];
+        P.k[m] = p[0];
+        P.slot[m] = n;
+    }
+    const S4Geom g = s4_geom(nx, ny, nz, pml ? d->cpml_e[0].npml : 0);
+    hipStream_t st = to_stream(stream);
+    for (int t = 0; t < nsteps; t++) {
+        float *row = d->nprobe ? probe_series + (size_t)t * d->nprobe : nullptr;
+        for (int s = 0; s < 5; s++) {
+            SAux ah{};
+            if (s == 4) {  // the H components are final after the closing stage
+                ah.prb = pbh;
+                ah.prb.out = row;
+            }
+            aux_box(ah);
+            if (int rc = s4_stage_h(g, pml ? &ph[s] : nullptr, ah, d->cl[s], d->e, d->ch, d->ch0, st)) return rc;
+            if (s == 4) break;
+            SAux ae{};
+            ae.src = src;
+            for (int n = 0; n < src.n; n++) ae.src.tval[n] = tvals[((size_t)t * 4 + s) * src.n + n];
+            if (s == 3) {
+                ae.prb = pbe;
+                ae.prb.out = row;
+            }
+            aux_box(ae);
+            if (int rc = s4_stage_e(g, pml ? &pe[s] : nullptr, ae, d->dl[s], d->e, cem, d->ce, d->ce0, d->ce_mat,
+                                    d->ce_lut, st))
+                return rc;
+        }
+    }
     return 0;
 }
 

@@ -219,6 +219,49 @@ class S4Sim:
                       p0[2], p1[2], p0[1], p1[1], p0[0], p1[0], tv,
                       None if sv is None else sv.data_ptr(), svs, 0, st)
 
+    def _whole_steps(self, nsteps, buf):
+        """``nsteps`` steps in one call (``mifdtd_s4_run``: every stage with its CPML, sources
+        and probes in one pass); ``buf``: device (nsteps, nprobe) probe buffer or None."""
+        d = _lib.S4Desc()
+        d.nx, d.ny, d.nz = self.nx, self.ny, self.nz
+        for c in range(6):
+            d.e[c] = self.ehs[c].data_ptr()
+        d.ce0 = d.ch0 = self.c0
+        for c in range(3):
+            if self.ce_mat is not None:
+                d.ce_mat[c] = self.ce_mat[c].data_ptr()
+            elif self.ces is not None:
+                d.ce[c] = self.ces[c].data_ptr()
+            if self.chs is not None:
+                d.ch[c] = self.chs[c].data_ptr()
+        if self.ce_mat is not None:
+            d.ce_lut = self.ce_lut.data_ptr()
+        d.cl[:] = self.cl
+        d.dl[:] = self.dl[:4]
+        if self.npml:
+            for s in range(4):
+                d.cpml_e[s] = self._half(self.psiE, *self._tabE[s])
+            for s in range(5):
+                d.cpml_h[s] = self._half(self.psiH, *self._tabH[s])
+        d.nsrc = len(self.sources)
+        tv = np.zeros((max(nsteps, 1), 4, max(len(self.sources), 1)), np.float32)
+        for n, (c, p0, p1, tfunc, sv, svs) in enumerate(self.sources):
+            d.src_comp[n] = c
+            d.src_box[n][:] = (p0[0], p1[0], p0[1], p1[1], p0[2], p1[2])
+            d.src_sv[n] = None if sv is None else sv.data_ptr()
+            d.src_svs[n] = svs
+            for t in range(nsteps):
+                for s in range(4):
+                    tv[t, s, n] = np.float32(tfunc(self.tstep + t + s / 5.0))
+        if buf is not None:
+            d.nprobe = len(self.probe_points)
+            for n, (c, pt) in enumerate(self.probe_points):
+                d.probe_comp[n] = c
+                d.probe_ijk[n][:] = pt
+        _lib.call("mifdtd_s4_run", ctypes.byref(d), nsteps, tv.ctypes.data, None if buf is None else buf.data_ptr(),
+                  _lib.stream_handle(self.stream))
+        self.tstep += nsteps
+
     def step(self, buf=None, t=0, events=None):
         """One step; ``events`` (a pair of timing events) brackets the first E-stage
         kernel on the simulation's stream."""
@@ -235,8 +278,11 @@ class S4Sim:
     def run(self, nsteps):
         nprobe = len(self.probe_points)
         buf = torch.zeros((nsteps, nprobe), dtype=torch.float32, device=self.device) if nprobe else None
-        for t in range(nsteps):
-            self.step(buf, t)
+        if len(self.sources) <= _lib.MAX_SRC and nprobe <= _lib.MAX_PROBE:
+            self._whole_steps(nsteps, buf)
+        else:
+            for t in range(nsteps):
+                self.step(buf, t)
         if buf is None:
             return None
         s = buf.cpu().numpy()

@@ -535,6 +535,38 @@ int mifdtd_s4_cpml_h(int nx, int ny, int nz, const mifdtd_cpml_half *cp, float c
                      const float *chx, const float *chy, const float *chz, float ch0,
                      mifdtd_stream_t stream);
 
+/* nsteps whole steps (S4/PyCUDA/100-base.py:124-141): for s in 0..3 H(cl[s]), E(dl[s]), the
+ * sources; then H(cl[4]), each stage with its CPML in the same pass.  Arrays as in the
+ * stage calls; ce_mat/ce_lut as in mifdtd_s4_update_e_lut (ce is then ignored); NULL ce /
+ * ch mean ce0 / ch0.  cpml_e[s], cpml_h[s]: the stages' tables and the (shared) psi arrays;
+ * npml 0 in all: none.  Sources: E components, inclusive boxes (i0,i1,j0,j1,k0,k1), value
+ * tvals[(t*4 + s)*nsrc + n] (HOST) times src_sv (DEVICE box array, x fastest) or, where
+ * that is NULL, src_svs.  Probes (i,j,k) are recorded at the end of each step into
+ * probe_series (DEVICE, nsteps x nprobe). */
+typedef struct {
+    int nx, ny, nz;
+    float *e[6];
+    const float *ce[3];
+    float ce0;
+    const unsigned char *ce_mat[3];
+    const float *ce_lut;
+    const float *ch[3];
+    float ch0;
+    float cl[5], dl[4];
+    mifdtd_cpml_half cpml_e[4], cpml_h[5];
+    int nsrc;
+    int src_comp[MIFDTD_FUSED_MAX_SRC];
+    int src_box[MIFDTD_FUSED_MAX_SRC][6];
+    const float *src_sv[MIFDTD_FUSED_MAX_SRC];
+    float src_svs[MIFDTD_FUSED_MAX_SRC];
+    int nprobe;
+    int probe_comp[MIFDTD_FUSED_MAX_PROBE];
+    int probe_ijk[MIFDTD_FUSED_MAX_PROBE][3];
+} mifdtd_s4_desc;
+
+int mifdtd_s4_run(const mifdtd_s4_desc *d, int nsteps, const float *tvals, float *probe_series,
+                  mifdtd_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
