@@ -158,7 +158,7 @@ def naive_update_h(ehs, chs, pad: int) -> None:
 
 # --------------------------------------------------------------- reference KEMP core
 def ref_available() -> bool:
-    return os.path.isdir("/root/reference") or os.path.isdir(_REF_DIR)
+    return any(os.path.isdir(d) and os.listdir(d) for d in ("/root/reference", _REF_DIR))
 
 
 def ref_core(dtype, pad: int, split: bool = False):
