@@ -8,8 +8,8 @@ bandwidth on MI355X, less than the per-launch cost of small slabs.)
 
 ``fused_tiles`` returns (rows_per_thread T, planes_per_chunk CX) for a grid: a table of
 measured winners (filled by ``tune_fused``) keyed by (nx, ny, nz_pitch, npml), else a
-heuristic that keeps enough work-groups in flight (>= 4 per CU on 256 CUs) while
-keeping the warm-up plane overhead (1/CX) small.
+rule on the rounds of work-groups over the 256 CUs; ``whole_grid_faster`` says whether a
+grid is too small, or fills the sweep's z segments too little, for a sweep at all.
 """
 from __future__ import annotations
 
@@ -50,12 +50,8 @@ def lds_fits_pairs(T, CX, table):
     return 4 * ((768 if table else 0) + 4 * R * 512 + 4 * (-(-R // 4)) + (CX + 3) * R * 4) + 1024 <= 160 * 1024
 
 
-def heuristic(nx, ny, nzp, npml):
-    """T owned rows per block (y halo overhead 1/T; the block has T+1 waves), CX planes
-    per chunk (seed-plane overhead 1/CX), keeping >= 1024 blocks.  T = 9 measured best
-    at 1024^3 (10.87 ms per sweep against 11.40 for T = 7 and 10.98 for T = 11, CX = 64,
-    interleaved on one MI355X): a smaller halo share outweighs the lower occupancy of
-    one 10-wave work-group per CU."""
+def _halved(nx, ny):
+    """T = 9 rows, CX = 64 planes halved while fewer than 1024 blocks."""
     T = min(9, max(1, ny // 8))
     nrb = -(-ny // T)
     cx = min(nx, 64)
@@ -64,15 +60,37 @@ def heuristic(nx, ny, nzp, npml):
     return T, max(1, cx)
 
 
+def heuristic(nx, ny, nzp, npml, halved=False):
+    """(T, CX): owned rows per block (one halo row each, T+1 waves) and planes per chunk
+    (one seed plane each).  One work-group runs per CU, so a sweep takes whole rounds of
+    256 blocks: the tile with the least rounds * (CX + 2) * (T + 3), the planes and waves of
+    a block with one plane for its start and two waves for the barrier.  Sweep against
+    T = 9 and CX halved until 1024 blocks: 256^3 135 / 143 us, 384^3 563 / 651, 512^3
+    1205-1230 / 1267, 350 x 420 x 500 641 / 694; within 3% of the best of 126 tiles
+    measured at five grids.  ``halved``: that older rule, which a Drude sweep (at most 7
+    rows, two blocks per CU) and a TFSF sweep (13 rows, its z-face rows cost more) keep, and
+    tiles of which the caller gives one number."""
+    if halved:
+        return _halved(nx, ny)
+    edge = 2 * (npml + 1) if npml else 0
+    bx, by = max(1, nx - edge), max(1, ny - edge)
+    best, cost = None, None
+    for T in (13, 11, 9, 8, 7, 6, 5, 4, 3, 2, 1):
+        if T > max(1, by // 2):
+            continue
+        for CX in range(min(bx, 64), min(bx, 8) - 1, -1):
+            rounds = -(-(-(-by // T) * -(-bx // CX)) // N_CU)
+            c = rounds * (CX + 2) * (T + 3)
+            if cost is None or c < cost:
+                best, cost = (T, CX), c
+    return best
+
+
 def heuristic_pairs(nx, ny, nzp, npml):
     """(T, CX) of the two-step sweep: T = 9 owned rows (12 waves, the kernel's launch
     bound; 9.95 ms per step at 1024^3 against 11.8 for T = 5), CX = 64 planes, halved
     while fewer than 1024 blocks."""
-    T = min(9, max(1, ny // 8))
-    nrb = -(-ny // T)
-    cx = min(nx, 64)
-    while cx > 8 and nrb * (-(-nx // cx)) < 1024:
-        cx = -(-cx // 2)
+    T, cx = _halved(nx, ny)
     while cx > 1 and not lds_fits_pairs(T, cx, True):
         cx -= 1
     return T, max(1, cx)
@@ -85,11 +103,36 @@ def fused_pairs(nx, ny, nzp, npml):
     return False
 
 
-def fused_tiles(nx, ny, nzp, npml, pairs=False):
+def fused_tiles(nx, ny, nzp, npml, pairs=False, halved=False):
     if pairs:
         return heuristic_pairs(nx, ny, nzp, npml)
     t = _load().get((nx, ny, nzp, npml))
-    return t if t is not None else heuristic(nx, ny, nzp, npml)
+    return t if t is not None else heuristic(nx, ny, nzp, npml, halved)
+
+
+def fused_tuned(nx, ny, nzp, npml):
+    """Whether ``tune_fused`` measured a tile for this grid."""
+    return (nx, ny, nzp, npml) in _load()
+
+
+def whole_grid_faster(cells, box_cells, fill, face_cells, ce_bytes, tri, drude, tfsf):
+    """Whether a step as two passes over the whole grid is faster than the sweep of the box
+    with its two shell passes.  A cell of the box costs 48 B + CE at 5 TB/s over the filled
+    part of the sweep's 256-cell z segments (a fifth to a quarter more with a plane wave or
+    a Drude box), a shell cell 72 B + CE at 2.9 TB/s, the sweep's launches 20 us more; a
+    cell of the whole-grid passes 72 B + CE, and 32 B of psi in the slabs, at 5.35 TB/s.
+    Measured, sweep / whole grid, CE as indices, CPML 12: 96^3 57 / 22 us, 160^3 85 / 63,
+    224^3 221 / 200, 256^3 277 / 279, 288^3 381 / 407, 320^3 623 / 529, 384^3 970 / 885,
+    448^3 1308 / 1462, 512^3 1707 / 2001; with a plane wave 384^3 1118 / 939, 512^3
+    2065 / 2077; with a Drude box 384^3 1355 / 1063, 512^3 2582 / 2428."""
+    sweep = box_cells * (48 + (2 if tri else ce_bytes)) / 5.0e6 / max(fill, 1e-3)
+    if tfsf:
+        sweep *= 1.22
+    if drude:
+        sweep *= 1.25
+    sweep += (cells - box_cells) * (72 + ce_bytes) / 2.9e6 + 20.0
+    whole = (cells * (72 + ce_bytes) + 32 * face_cells) / 5.35e6 * (1.05 if tfsf else 1.0)
+    return whole < sweep
 
 
 def tune_fused(sim, candidates=((7, 64), (9, 64), (9, 96), (11, 64), (11, 128), (13, 64), (15, 96)), steps=5, save=True):

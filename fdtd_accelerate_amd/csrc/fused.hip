@@ -41,6 +41,7 @@
 #include "common.hpp"
 #include "step_quad.hpp"
 #include "shell_boxes.hpp"
+#include "whole_pass.hpp"
 
 #include <vector>
 
@@ -1356,6 +1357,34 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
         ss.prb.out = fp.out = d->nprobe ? probe_series + (size_t)s * d->nprobe : nullptr;
         aux_box(ss);
     };
+    // the sources and probes of one half step
+    auto half_aux = [](const SAux &a, bool e_half) {
+        SAux h{};
+        for (int n = 0; n < a.src.n; n++) {
+            if ((a.src.comp[n] < 3) != e_half) continue;
+            const int m = h.src.n++;
+            h.src.comp[m] = a.src.comp[n];
+            h.src.i0[m] = a.src.i0[n]; h.src.i1[m] = a.src.i1[n];
+            h.src.j0[m] = a.src.j0[n]; h.src.j1[m] = a.src.j1[n];
+            h.src.k0[m] = a.src.k0[n]; h.src.k1[m] = a.src.k1[n];
+            h.src.ow[m] = a.src.ow[n];
+            h.src.tval[m] = a.src.tval[n];
+            h.src.svs[m] = a.src.svs[n];
+            h.src.sv[m] = a.src.sv[n];
+        }
+        for (int n = 0; n < a.prb.n; n++) {
+            if ((a.prb.comp[n] < 3) != e_half) continue;
+            const int m = h.prb.n++;
+            h.prb.comp[m] = a.prb.comp[n];
+            h.prb.i[m] = a.prb.i[n];
+            h.prb.j[m] = a.prb.j[n];
+            h.prb.k[m] = a.prb.k[n];
+            h.prb.slot[m] = a.prb.slot[n];
+        }
+        h.prb.out = a.prb.out;
+        aux_box(h);
+        return h;
+    };
     // shell E pass over boxes b: E from ei (H from hi) to eo, psi E from pe to pe_out
     auto shell_e = [&](const ShellBoxes &b, unsigned long long tot, const float *const *ei, const float *const *hi,
                        float *const *eo, float *pe, float *pe_out, const SAux &ss, int fe) -> int {
@@ -1392,6 +1421,28 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
     auto mark = [&](int q) {
         if (sweep_ms) (void)hipEventRecord(marks[2 * (size_t)nsweeps + q], st);
     };
+    // periodic copies of one half step (priority after the incident corrections)
+    auto pbc_copies = [&](float *const *e, bool e_half) -> int {
+        const int b = e_half ? 0 : 3;
+        for (int q = 0; q < d->npbc; q++) {
+            const int a = d->pbc_axes[q];
+            const int c1 = b + (a == 0 ? 1 : 0), c2 = b + (a == 2 ? 1 : 2);  // the components tangential to axis a
+            if (int rc = mifdtd_pbc(e[c1], e[c2], nx, ny, nzp, pad, a, e_half ? 1 : 0, stream)) return rc;
+        }
+        return 0;
+    };
+    auto sweep_time = [&]() -> int {
+        float total_ms = 0.f;
+        hipError_t err = hipStreamSynchronize(st);
+        for (int q = 0; err == hipSuccess && q < nsweeps; q++) {
+            float t = 0.f;
+            err = hipEventElapsedTime(&t, marks[2 * (size_t)q], marks[2 * (size_t)q + 1]);
+            total_ms += t;
+        }
+        if (err != hipSuccess) return fail((int)err, "sweep timing events failed");
+        *sweep_ms = nsteps > 0 ? total_ms / nsteps : 0.f;
+        return 0;
+    };
     auto swap_sets = [&]() {
         for (int q = 0; q < 6; q++) { const float *x = in[q]; in[q] = out[q]; out[q] = const_cast<float *>(x); }
         float *tp = pin;
@@ -1403,6 +1454,48 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
             sdr.jout[q] = const_cast<float *>(x);
         }
     };
+    if (d->whole_grid) {  // every step as an E and an H pass over the whole grid, in place
+        if (pairs) return fail(MIFDTD_EINVAL, "whole-grid steps and step pairs exclude each other");
+        WholeGrid w{};
+        w.g = sg;
+        const int zp = (pml_axes & 4) ? d->npml : 0;
+        if ((unsigned long long)nx * ny * Q + SB >= (1ull << 31)) return fail(MIFDTD_ERANGE, "grid too large");
+        w.g.m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, zp, 0, (unsigned)zph / 4);
+        for (int q = 0; q < 6; q++) w.F.e[q] = d->e[q];
+        for (int q = 0; q < 3; q++) {
+            w.F.ce[q] = d->ce[q];
+            w.F.cm[q] = d->ce_mat[q];
+        }
+        w.F.lut = d->ce_lut;
+        w.cp = scp;
+        w.cp.pe = w.cp.pe_out = d->psiE;
+        w.cem = cem;
+        w.st = st;
+        SDrude drw = sdr;
+        for (int q = 0; q < 3; q++) drw.jout[q] = d->drude_j[q];
+        for (int n = 0; n < nsteps; n++) {
+            FSrc fs;
+            SAux ss;
+            FProbe fp;
+            step_tables(n, fs, fp, ss);
+            if (tfsf)
+                if (int rc = mifdtd_tfsf_line(d->tfsf_line_e, d->tfsf_line_h, d->tfsf_abc, d->tfsf_line_n, 1,
+                                              d->tfsf_src[n], stream))
+                    return rc;
+            mark(0);
+            if (int rc = whole_e(w, half_aux(ss, true), drude ? &drw : nullptr, tfsf ? &tfe : nullptr)) return rc;
+            if (int rc = pbc_copies(d->e, true)) return rc;
+            if (int rc = whole_h(w, half_aux(ss, false), tfsf ? &tfh : nullptr)) return rc;
+            mark(1);
+            ++nsweeps;
+            if (int rc = pbc_copies(d->e, false)) return rc;
+            if (tfsf)
+                if (int rc = mifdtd_tfsf_line(d->tfsf_line_e, d->tfsf_line_h, d->tfsf_abc, d->tfsf_line_n, 0, 0.f, stream))
+                    return rc;
+        }
+        if (parity) *parity = 0;
+        return sweep_ms ? sweep_time() : 0;
+    }
     const unsigned nthr = 64u * (unsigned)(T + 1);
     const bool wide = T > kNarrowRows;  // blocks of more than 10 waves: the 1024-thread build
     const unsigned nthr2 = 64u * (unsigned)R2;
@@ -1473,18 +1566,10 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
             ++nsweeps;
             MIFDTD_CHECK_LAUNCH("fused sweep launch");
         }
-        for (int q = 0; q < d->npbc; q++) {  // periodic E copies (priority after the incident corrections)
-            const int a = d->pbc_axes[q];
-            const int c1 = a == 0 ? 1 : 0, c2 = a == 2 ? 1 : 2;  // the E components tangential to axis a
-            if (int rc = mifdtd_pbc(out[c1], out[c2], nx, ny, nzp, pad, a, 1, stream)) return rc;
-        }
+        if (int rc = pbc_copies(out, true)) return rc;
         if (shell_on)
             if (int rc = shell_h(sb, total, out, in, out, ss)) return rc;
-        for (int q = 0; q < d->npbc; q++) {  // periodic H copies
-            const int a = d->pbc_axes[q];
-            const int c1 = a == 0 ? 4 : 3, c2 = a == 2 ? 4 : 5;
-            if (int rc = mifdtd_pbc(out[c1], out[c2], nx, ny, nzp, pad, a, 0, stream)) return rc;
-        }
+        if (int rc = pbc_copies(out, false)) return rc;
         if (tfsf)  // the line's H half (the H patches of this step read its E)
             if (int rc = mifdtd_tfsf_line(d->tfsf_line_e, d->tfsf_line_h, d->tfsf_abc, d->tfsf_line_n, 0, 0.f, stream))
                 return rc;
@@ -1492,18 +1577,7 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
         ++swaps;
     }
     if (parity) *parity = swaps & 1;
-    if (sweep_ms) {
-        float total_ms = 0.f;
-        hipError_t err = hipStreamSynchronize(st);
-        for (int q = 0; err == hipSuccess && q < nsweeps; q++) {
-            float t = 0.f;
-            err = hipEventElapsedTime(&t, marks[2 * (size_t)q], marks[2 * (size_t)q + 1]);
-            total_ms += t;
-        }
-        if (err != hipSuccess) return fail((int)err, "sweep timing events failed");
-        *sweep_ms = nsteps > 0 ? total_ms / nsteps : 0.f;
-    }
-    return 0;
+    return sweep_ms ? sweep_time() : 0;
 }
 
 int mifdtd_fused_run(const mifdtd_fused_desc *d, int nsteps, const float *tvals, float *probe_series,

@@ -126,8 +126,9 @@ inline unsigned long long row_quads_blocks(const RowQuads &m)
 // The order for `planes` planes of ny rows of Q quads (nz cells, npml-cell z slabs; npml =
 // 0: none).  The E slabs are [0, npml) and [nz-1-npml, nz-1), the H slabs [0, npml) and
 // [nz-npml, nz): one order serves both.  front: cells at the front that count as slab cells
-// (the adjoint passes reach one cell further).
-inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, int front = 0)
+// (the adjoint passes reach one cell further).  phase: quads from a 128-byte line to each
+// row's first quad.
+inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, int front = 0, unsigned phase = 0)
 {
     RowQuads m;
     m.Q = Q;
@@ -137,8 +138,8 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     m.zf = npml > 0 ? (unsigned)(((front > npml ? front : npml) + 3) / 4) : 0u;
     m.zb = npml > 0 ? (unsigned)((nz - 1 - npml) / 4) : Q;
     if (npml > 0) {  // whole 128-byte lines (8 quads) on either side of a run's end
-        m.zf = (m.zf + 7) / 8 * 8;
-        m.zb = m.zb / 8 * 8;
+        m.zf = (m.zf + phase + 7) / 8 * 8 - phase;
+        m.zb = m.zb + phase < 8 ? 0 : (m.zb + phase) / 8 * 8 - phase;
     }
     if (m.zf >= m.zb) {  // every quad may hold a slab cell: one run
         m.zf = 0;

@@ -10,9 +10,16 @@
 // E pass) and E of plane i needs H_old of planes i and i+1 (not yet touched: the slab's
 // H pass runs after its E pass, the next slab's later).
 
-#include "step_quad.hpp"
+#include "whole_pass.hpp"
 
 namespace mifdtd {
+
+// The tables of a half step that few waves read, as the kernel's first argument.
+struct SExtra {
+    SAux aux;
+    SDrude dr;
+    STfsf tf;
+};
 
 // CM: CeMode (kCeTable: CE from the material indices and the 3 x 256 table).  The
 // sources and probes (first argument) are read only by the waves near them.
@@ -26,6 +33,18 @@ __global__ __launch_bounds__(SB) void k_slab_e(SAux, SGeom g, SFields F, SCpml c
                        F.lut);
 }
 
+// With a Drude box and / or TFSF patches (FEAT; a grid without CPML has cp.axes 0).
+template <int CM, int FEAT>
+__global__ __launch_bounds__(SB) void k_slab_e_feat(SExtra, SGeom g, SFields F, SCpml cp)
+{
+    RowAt r;
+    if (!slab_quad(g, blockIdx.x, r)) return;
+    const SExtra &x = first_kernel_arg<SExtra>();
+    e_quad_at<CM, true, FEAT>(g, r.i, r.j, r.k0, r.next, F.e[0], F.e[1], F.e[2], F.e[0], F.e[1], F.e[2], F.e[3], F.e[4],
+                              F.e[5], F.ce[0], F.ce[1], F.ce[2], cp, x.aux, F.cm[0], F.cm[1], F.cm[2], F.lut, &x.dr,
+                              &x.tf);
+}
+
 template <bool PML>
 __global__ __launch_bounds__(SB) void k_slab_h(SAux, SGeom g, SFields F, SCpml cp)
 {
@@ -33,6 +52,59 @@ __global__ __launch_bounds__(SB) void k_slab_h(SAux, SGeom g, SFields F, SCpml c
     if (!slab_quad(g, blockIdx.x, r)) return;
     h_quad_at<PML>(g, r.i, r.j, r.k0, r.prev, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], F.e[3], F.e[4], F.e[5],
                    cp, first_kernel_arg<SAux>());
+}
+
+__global__ __launch_bounds__(SB) void k_slab_h_tfsf(SExtra, SGeom g, SFields F, SCpml cp)
+{
+    RowAt r;
+    if (!slab_quad(g, blockIdx.x, r)) return;
+    const SExtra &x = first_kernel_arg<SExtra>();
+    h_quad_at<true>(g, r.i, r.j, r.k0, r.prev, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], F.e[3], F.e[4], F.e[5],
+                    cp, x.aux, &x.tf);
+}
+
+template <int CM>
+static void launch_e(const WholeGrid &w, unsigned grid, const SAux &a, const SDrude *dr, const STfsf *tf)
+{
+    if (!dr && !tf) {
+        if (w.cp.npml > 0) k_slab_e<CM, true><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+        else k_slab_e<CM, false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+        return;
+    }
+    SExtra x{};
+    x.aux = a;
+    if (dr) x.dr = *dr;
+    if (tf) x.tf = *tf;
+    if (dr && tf) k_slab_e_feat<CM, kFeatDrude | kFeatTfsf><<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+    else if (dr) k_slab_e_feat<CM, kFeatDrude><<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+    else k_slab_e_feat<CM, kFeatTfsf><<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+}
+
+int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf)
+{
+    const unsigned grid = (unsigned)row_quads_blocks(w.g.m);
+    if (w.cem == kCeTable) launch_e<kCeTable>(w, grid, a, dr, tf);
+    else if (w.cem == kCeArrays) launch_e<kCeArrays>(w, grid, a, dr, tf);
+    else launch_e<kCeConst>(w, grid, a, dr, tf);
+    MIFDTD_CHECK_LAUNCH("whole-grid E launch");
+    return 0;
+}
+
+int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf)
+{
+    const unsigned grid = (unsigned)row_quads_blocks(w.g.m);
+    if (tf) {
+        SExtra x{};
+        x.aux = a;
+        x.tf = *tf;
+        k_slab_h_tfsf<<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+    } else if (w.cp.npml > 0) {
+        k_slab_h<true><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+    } else {
+        k_slab_h<false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+    }
+    MIFDTD_CHECK_LAUNCH("whole-grid H launch");
+    return 0;
 }
 
 }  // namespace mifdtd
@@ -168,24 +240,17 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
         aux_box(A);
         return A;
     };
+    WholeGrid w{};
+    w.F = F;
+    w.cp = cp;
+    w.cem = cem;
+    w.st = st;
     for (int n = 0; n < nsteps; n++) {
         const SAux ae = tables(pe, n, true), ah = tables(ph, n, false);
         for (int sl = 0; sl < ns; sl++) {
-            const SGeom g = geom(sl);
-            const unsigned grid = (unsigned)row_quads_blocks(g.m);
-#define MIFDTD_SLAB_E(CM)                                                   \
-    do {                                                                    \
-        if (pml) k_slab_e<CM, true><<<grid, SB, 0, st>>>(ae, g, F, cp);  \
-        else k_slab_e<CM, false><<<grid, SB, 0, st>>>(ae, g, F, cp);    \
-    } while (0)
-            if (cem == kCeTable) MIFDTD_SLAB_E(kCeTable);
-            else if (cem == kCeArrays) MIFDTD_SLAB_E(kCeArrays);
-            else MIFDTD_SLAB_E(kCeConst);
-#undef MIFDTD_SLAB_E
-            MIFDTD_CHECK_LAUNCH("slab E launch");
-            if (pml) k_slab_h<true><<<grid, SB, 0, st>>>(ah, g, F, cp);
-            else k_slab_h<false><<<grid, SB, 0, st>>>(ah, g, F, cp);
-            MIFDTD_CHECK_LAUNCH("slab H launch");
+            w.g = geom(sl);
+            if (int rc = whole_e(w, ae, nullptr, nullptr)) return rc;
+            if (int rc = whole_h(w, ah, nullptr)) return rc;
         }
     }
     return 0;

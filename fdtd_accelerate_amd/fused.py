@@ -20,7 +20,8 @@ import torch
 
 from . import _lib
 from . import fields as _fields
-from .autotune import fused_pairs, fused_tiles, lds_fits, lds_fits_pairs, slab_planes
+from .autotune import (fused_pairs, fused_tiles, fused_tuned, lds_fits, lds_fits_pairs, slab_planes,
+                       whole_grid_faster)
 
 _COMP = {"ex": 0, "ey": 1, "ez": 2, "hx": 3, "hy": 4, "hz": 5}
 
@@ -144,7 +145,8 @@ def _check_tfsf_sources(sim, tfsf):
 class FusedStepper:
     kernel_name = "k_fused"
 
-    def __init__(self, sim, rows_per_thread=None, planes_per_chunk=None, step_pairs=None, z_phase=None):
+    def __init__(self, sim, rows_per_thread=None, planes_per_chunk=None, step_pairs=None, z_phase=None,
+                 whole_grid=None):
         from .drude import Drude
         from .pbc import Pbc
         from .tfsf import Tfsf
@@ -203,10 +205,12 @@ class FusedStepper:
             # CE indices (1 B per cell) placed so that the sweep's segments start on lines
             with torch.cuda.stream(f.stream):
                 f.ce_mat = [_offset_copy(m, (-kb) % 128) for m in f.ce_mat]
-        T, CX = fused_tiles(f.nx, f.ny, f.nz_pitch, npml, self.pairs)
+        table = f.ce_mat is not None
+        asked = rows_per_thread is not None or planes_per_chunk is not None
+        T, CX = fused_tiles(f.nx, f.ny, f.nz_pitch, npml, self.pairs,
+                            asked or self.drude is not None or self.tfsf is not None)
         self.T = rows_per_thread or T
         self.CX = planes_per_chunk or CX
-        table = f.ce_mat is not None
         if not lds_fits(self.T, self.CX, table):
             raise ValueError(f"rows_per_thread {self.T} / planes_per_chunk {self.CX} need more than 160 KiB of LDS")
         if self.pairs and not (self.T <= 9 and lds_fits_pairs(self.T, self.CX, table)):
@@ -237,6 +241,23 @@ class FusedStepper:
         self._tri_kb = kb if z_phase else 0
         self.ce_tri = self.ce_tri_lut = self._tri_src = None
         self._build_ce_triples()
+        # whole-grid steps instead of the sweep and its shell, unless a tile was asked for or
+        # measured (tune_fused); a run with sweep timing takes the sweep
+        if whole_grid and self.pairs:
+            raise ValueError("whole-grid steps and step pairs exclude each other")
+        self.whole_grid = bool(whole_grid) if whole_grid is not None else \
+            not (asked or self.pairs or fused_tuned(f.nx, f.ny, f.nz_pitch, npml)) and self._whole_grid_faster()
+
+    def _whole_grid_faster(self):
+        f, cp = self.sim.fields, self.sim.cpml
+        xb, xe, yb, ye, kb, ke = self.sweep_box()
+        zb0 = kb if self.z_phase and self.cpml_axes & 4 else 256 * (kb // 256)
+        fill = (ke - kb) / max(256 * (-(-(ke - zb0) // 256)), 1)
+        cells = f.nx * f.ny * f.nz
+        face = sum(2 * cp.npml * cells // f.ns[a] for a in range(3) if (self.cpml_axes >> a) & 1) if cp else 0
+        ce = 0 if not f.ce_on else 12 if f.ce_mat is None else 3
+        return whole_grid_faster(cells, self.sweep_cells(), fill, face, ce, self.ce_tri is not None,
+                                 self.drude is not None, self.tfsf is not None)
 
     def _build_ce_triples(self):
         """One uint16 index per cell into the distinct (cex, cey, cez) triples of the
@@ -386,6 +407,7 @@ class FusedStepper:
         if tf is not None:  # the line's hard source per step, as Tfsf.update_e computes it
             tsrc = np.array([np.float32(np.sin(tf.wdt * (tf.tstep + k))) for k in range(max(nsteps, 1))], np.float32)
             d.tfsf_src = tsrc.ctypes.data
+        d.whole_grid = int(getattr(self, "whole_grid", False) and not timed)
         parity = ctypes.c_int(0)
         args = (ctypes.byref(d), nsteps, tv.ctypes.data, None if buf is None else buf.data_ptr(),
                 ctypes.byref(parity), _lib.stream_handle(f.stream))

@@ -342,6 +342,10 @@ typedef struct {
     const unsigned short *ce_tri;
     const float *ce_tri_lut;
     int ce_tri_n;
+    /* optional, 1: every step as an E pass and an H pass over the whole grid, in place in
+     * e[], psiE and drude_j (the same values; *parity stays 0, sweep_ms brackets the two
+     * passes) -- the faster form for grids that a sweep does not fill; not with e_mid */
+    int whole_grid;
 } mifdtd_fused_desc;
 #define MIFDTD_FUSED_MAX_CE_TRI 4096
 
