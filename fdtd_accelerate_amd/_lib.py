@@ -106,8 +106,11 @@ _SIGS = {
     "mifdtd_cpml_face_z_h": (_I, [_I] * 6 + [_P] * 8 + [_P]),
     "mifdtd_cpml_e": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 9 + [_P]),
     "mifdtd_cpml_h": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 9 + [_P]),
+    "mifdtd_half_e": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 13 + [_P]),
+    "mifdtd_half_h": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 9 + [_P]),
     "mifdtd_source": (_I, [_P] + [_I] * 9 + [_F, _P, _F, _I, _P]),
     "mifdtd_gather": (_I, [_P, _P, _I, _P, _P]),
+    "mifdtd_record": (_I, [_P, _I, _P, _P]),
     "mifdtd_pbc": (_I, [_P, _P] + [_I] * 6 + [_P]),
     "mifdtd_drude_e": (_I, [_P] * 5 + [_I] * 9 + [_P]),
     "mifdtd_tfsf_line": (_I, [_P, _P, _P, _I, _I, _F, _P]),

@@ -17,6 +17,7 @@ import numpy as np
 import torch
 
 from . import _lib, util
+from .core import Core
 from .fields import Fields
 
 
@@ -154,6 +155,32 @@ class Cpml:
         _lib.call("mifdtd_cpml_h", f.nx, f.ny, f.nz_pitch, f.pad, self._descH, *f.ptrs(f.ehs),
                   *f.ptrs(chs), _lib.stream_handle(f.stream))
 
+    def joins_core(self, core):
+        """Whether ``update_core_e`` / ``update_core_h`` stand for the core's update followed by
+        this CPML's: both are of these classes themselves, on the same fields, with the
+        update methods as defined here (none replaced in a subclass, a class or an instance)."""
+        return (type(core) is Core and type(self) is Cpml and core.mainf is self.mainf
+                and not {"update_e", "update_h"} & (core.__dict__.keys() | self.__dict__.keys())
+                and (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h) == _OWN)
+
+    def update_core_e(self):
+        f = self.mainf
+        ces = f.ces if f.ce_on else (None, None, None)
+        mats = (None,) * 4
+        if f.ce_on and f.ce_mat is not None:
+            mats = (*f.ptrs(f.ce_mat), f.ce_lut.data_ptr())
+        _lib.call("mifdtd_half_e", f.nx, f.ny, f.nz_pitch, f.pad, self._descE, *f.ptrs(f.ehs), *f.ptrs(ces), *mats,
+                  _lib.stream_handle(f.stream))
+
+    def update_core_h(self):
+        f = self.mainf
+        chs = f.chs if f.ch_on else (None, None, None)
+        _lib.call("mifdtd_half_h", f.nx, f.ny, f.nz_pitch, f.pad, self._descH, *f.ptrs(f.ehs), *f.ptrs(chs),
+                  _lib.stream_handle(f.stream))
+
+
+# The update methods that a joined half step stands for (joins_core).
+_OWN = (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h)
 
 _FACE_E = {0: ("ey", "ez", "hy", "hz", 1, 2), 1: ("ex", "ez", "hx", "hz", 0, 2), 2: ("ex", "ey", "hx", "hy", 0, 1)}
 

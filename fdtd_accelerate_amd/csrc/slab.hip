@@ -45,13 +45,14 @@ __global__ __launch_bounds__(SB) void k_slab_e_feat(SExtra, SGeom g, SFields F, 
                               &x.tf);
 }
 
-template <bool PML>
+// CH: F.ce holds the three CH arrays.
+template <bool PML, bool CH>
 __global__ __launch_bounds__(SB) void k_slab_h(SAux, SGeom g, SFields F, SCpml cp)
 {
     RowAt r;
     if (!slab_quad(g, blockIdx.x, r)) return;
-    h_quad_at<PML>(g, r.i, r.j, r.k0, r.prev, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], F.e[3], F.e[4], F.e[5],
-                   cp, first_kernel_arg<SAux>());
+    h_quad_at<PML, CH>(g, r.i, r.j, r.k0, r.prev, F.e[0], F.e[1], F.e[2], F.e[3], F.e[4], F.e[5], F.e[3], F.e[4], F.e[5],
+                       cp, first_kernel_arg<SAux>(), nullptr, nullptr, nullptr, nullptr, F.ce);
 }
 
 __global__ __launch_bounds__(SB) void k_slab_h_tfsf(SExtra, SGeom g, SFields F, SCpml cp)
@@ -90,7 +91,7 @@ int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf
     return 0;
 }
 
-int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf)
+int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *const *ch)
 {
     const unsigned grid = (unsigned)row_quads_blocks(w.g.m);
     if (tf) {
@@ -98,13 +99,32 @@ int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf)
         x.aux = a;
         x.tf = *tf;
         k_slab_h_tfsf<<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+    } else if (ch) {
+        SFields F = w.F;
+        for (int c = 0; c < 3; c++) F.ce[c] = ch[c];
+        if (w.cp.npml > 0) k_slab_h<true, true><<<grid, SB, 0, w.st>>>(a, w.g, F, w.cp);
+        else k_slab_h<false, true><<<grid, SB, 0, w.st>>>(a, w.g, F, w.cp);
     } else if (w.cp.npml > 0) {
-        k_slab_h<true><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+        k_slab_h<true, false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
     } else {
-        k_slab_h<false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+        k_slab_h<false, false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
     }
     MIFDTD_CHECK_LAUNCH("whole-grid H launch");
     return 0;
+}
+
+RowQuads grid_order(int nx, int ny, int nzp, int nz, int npml)
+{
+    thread_local int key[5] = {0, 0, 0, 0, 0};
+    thread_local RowQuads m;
+    const int want[5] = {nx, ny, nzp, nz, npml};
+    bool same = true;
+    for (int n = 0; n < 5; n++) same = same && key[n] == want[n];
+    if (!same) {
+        m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)(nzp / 4), nz, npml);
+        for (int n = 0; n < 5; n++) key[n] = want[n];
+    }
+    return m;
 }
 
 }  // namespace mifdtd

@@ -533,12 +533,13 @@ __device__ __forceinline__ void e_quad_at(
 // H pass on the quad (i, j, k0..k0+3): reads H from hxi.. and writes it to hxo.. (the
 // same arrays for an in-place update); psi H is updated in place (cp.ph).  prev: the
 // previous lane holds the quad at k0-4.
-template <bool PML>
+// CH: the coefficient arrays ch[0..2] in place of the constant 0.5.
+template <bool PML, bool CH = false>
 __device__ __forceinline__ void h_quad_at(
     const SGeom &g, int i, int j, int k0, bool prev, const float *__restrict__ ex, const float *__restrict__ ey,
     const float *__restrict__ ez, const float *hxi, const float *hyi, const float *hzi, float *hxo, float *hyo,
     float *hzo, const SCpml &cp, const SAux &aux, const STfsf *tf = nullptr, float *prow = nullptr,
-    const float *tv_row = nullptr, const int *tv = nullptr)
+    const float *tv_row = nullptr, const int *tv = nullptr, const float *const *ch = nullptr)
 {
     const int nx = g.nx, ny = g.ny, nzp = g.nzp, nz = g.nz;
     (void)nx;
@@ -550,6 +551,9 @@ __device__ __forceinline__ void h_quad_at(
     // ---------------------------------------------------------------- loads
     const Q4 ex0 = ld4(ex + id), ey0 = ld4(ey + id), ez0 = ld4(ez + id);
     Q4 h0 = ld4(hxi + id), h1 = ld4(hyi + id), h2 = ld4(hzi + id);
+    const Q4 c0 = CH ? ld4(ch[0] + id) : splat4(0.5f);
+    const Q4 c1 = CH ? ld4(ch[1] + id) : splat4(0.5f);
+    const Q4 c2 = CH ? ld4(ch[2] + id) : splat4(0.5f);
     const Q4 ezD = jp ? ld4(ez + id - nzp) : z4;   // ez(j-1)
     const Q4 exD = jp ? ld4(ex + id - nzp) : z4;   // ex(j-1)
     const Q4 ezB = ip ? ld4(ez + id - sx) : z4;    // ez(i-1)
@@ -612,7 +616,7 @@ __device__ __forceinline__ void h_quad_at(
     if (jp) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
-            const float v = h0.v[l] - 0.5f * ((ez0.v[l] - ezD.v[l]) - (ey0.v[l] - ym[l]));
+            const float v = h0.v[l] - c0.v[l] * ((ez0.v[l] - ezD.v[l]) - (ey0.v[l] - ym[l]));
             const int k = k0 + l;
             h0.v[l] = (k > 0 && k < nz) ? v : v * 0.f;
         }
@@ -620,7 +624,7 @@ __device__ __forceinline__ void h_quad_at(
     if (ip) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
-            const float v = h1.v[l] - 0.5f * ((ex0.v[l] - xm[l]) - (ez0.v[l] - ezB.v[l]));
+            const float v = h1.v[l] - c1.v[l] * ((ex0.v[l] - xm[l]) - (ez0.v[l] - ezB.v[l]));
             const int k = k0 + l;
             h1.v[l] = (k > 0 && k < nz) ? v : v * 0.f;
         }
@@ -628,7 +632,7 @@ __device__ __forceinline__ void h_quad_at(
     if (ip && jp) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
-            const float v = h2.v[l] - 0.5f * ((ey0.v[l] - eyB.v[l]) - (ex0.v[l] - exD.v[l]));
+            const float v = h2.v[l] - c2.v[l] * ((ey0.v[l] - eyB.v[l]) - (ex0.v[l] - exD.v[l]));
             h2.v[l] = (k0 + l < nz) ? v : v * 0.f;
         }
     }
@@ -641,7 +645,7 @@ __device__ __forceinline__ void h_quad_at(
                 if (k > 0 && k < nz) {
                     const float tt = b * p1.v[l] + a * (ez0.v[l] - ezB.v[l]);
                     p1.v[l] = tt;
-                    h1.v[l] = h1.v[l] + 0.5f * tt;
+                    h1.v[l] = h1.v[l] + c1.v[l] * tt;
                 }
             }
             if (jp) {
@@ -650,7 +654,7 @@ __device__ __forceinline__ void h_quad_at(
                     if (k0 + l < nz) {
                         const float tt = b * p2.v[l] + a * (ey0.v[l] - eyB.v[l]);
                         p2.v[l] = tt;
-                        h2.v[l] = h2.v[l] - 0.5f * tt;
+                        h2.v[l] = h2.v[l] - c2.v[l] * tt;
                     }
             }
             st4(cp.ph + o1, p1);
@@ -673,7 +677,7 @@ __device__ __forceinline__ void h_quad_at(
                 if (k > 0 && k < nz) {
                     const float tt = b * p2.v[l] + a * (ez0.v[l] - ezD.v[l]);
                     p2.v[l] = tt;
-                    h0.v[l] = h0.v[l] - 0.5f * tt;
+                    h0.v[l] = h0.v[l] - c0.v[l] * tt;
                 }
             }
             if (ip) {
@@ -682,7 +686,7 @@ __device__ __forceinline__ void h_quad_at(
                     if (k0 + l < nz) {
                         const float tt = b * p1.v[l] + a * (ex0.v[l] - exD.v[l]);
                         p1.v[l] = tt;
-                        h2.v[l] = h2.v[l] + 0.5f * tt;
+                        h2.v[l] = h2.v[l] + c2.v[l] * tt;
                     }
             }
             st4(cp.ph + o1, p1);
@@ -697,12 +701,12 @@ __device__ __forceinline__ void h_quad_at(
                 if (on && jp) {
                     const float tt = z.b[l] * z.q1[l] + z.a[l] * (ey0.v[l] - ym[l]);
                     cp.ph[o] = tt;
-                    h0.v[l] = h0.v[l] + 0.5f * tt;
+                    h0.v[l] = h0.v[l] + c0.v[l] * tt;
                 }
                 if (on && ip) {
                     const float tt = z.b[l] * z.q2[l] + z.a[l] * (ex0.v[l] - xm[l]);
                     cp.ph[o + cp.sZ] = tt;
-                    h1.v[l] = h1.v[l] - 0.5f * tt;
+                    h1.v[l] = h1.v[l] - c1.v[l] * tt;
                 }
             }
         }

@@ -15,8 +15,20 @@ struct WholeGrid {
     hipStream_t st;
 };
 
-// E pass, then H pass, each in place; dr / tf: null where the step has none.
+// No sources and probes.
+inline SAux no_aux()
+{
+    SAux a{};
+    aux_box(a);
+    return a;
+}
+
+// E pass, then H pass, each in place; dr / tf: null where the step has none; ch: the three
+// CH arrays, null for the constant 0.5 (which a step with tf has).
 int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf);
-int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf);
+int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *const *ch = nullptr);
+
+// row_quads of the whole grid; the last one a thread asked for is kept.
+RowQuads grid_order(int nx, int ny, int nzp, int nz, int npml);
 
 }  // namespace mifdtd

@@ -16,7 +16,7 @@
 #include <cstdarg>
 #include <mutex>
 
-#include "common.hpp"
+#include "whole_pass.hpp"
 
 namespace mifdtd {
 
@@ -116,84 +116,6 @@ __global__ __launch_bounds__(kBlock) void k_update_e(
     }
 }
 
-// update_e with the CE arrays held as per-component uint8 material indices into a
-// 3 x 256 float table (the exact float32 CE values; staged in LDS): 39 instead of 48
-// bytes per cell, same arithmetic and masks as k_update_e<true>.
-__device__ __forceinline__ Q4 lut4(const float *tab, const unsigned char *m)
-{
-    const uchar4 t = *reinterpret_cast<const uchar4 *>(m);
-    Q4 q;
-    q.v[0] = tab[t.x];
-    q.v[1] = tab[t.y];
-    q.v[2] = tab[t.z];
-    q.v[3] = tab[t.w];
-    return q;
-}
-
-__global__ __launch_bounds__(kBlock) void k_update_e_lut(
-    int nx, int ny, int nzp, int nz, unsigned nquads, unsigned Q,
-    float *__restrict__ ex, float *__restrict__ ey, float *__restrict__ ez,
-    const float *__restrict__ hx, const float *__restrict__ hy, const float *__restrict__ hz,
-    const unsigned char *__restrict__ mx, const unsigned char *__restrict__ my, const unsigned char *__restrict__ mz,
-    const float *__restrict__ lut)
-{
-    __shared__ float tab[3 * 256];
-    for (int t = threadIdx.x; t < 3 * 256; t += kBlock) tab[t] = lut[t];
-    __syncthreads();
-    const unsigned f = blockIdx.x * kBlock + threadIdx.x;
-    if (f >= nquads) return;
-    const unsigned row = f / Q;
-    const int k0 = (int)(f - row * Q) * 4;
-    const int i = (int)(row / (unsigned)ny);
-    const int j = (int)row - i * ny;
-    const size_t id = (size_t)row * nzp + k0;
-    const size_t sx = (size_t)ny * nzp;
-
-    const Q4 hx0 = ld4(hx + id), hy0 = ld4(hy + id), hz0 = ld4(hz + id);
-
-    if (j < ny - 1) {
-        const Q4 e = ld4(ex + id);
-        const Q4 c = lut4(tab, mx + id);
-        const Q4 h1 = ld4(hz + id + nzp);
-        const float hyn = hy[id + 4];
-        Q4 r;
-#pragma unroll
-        for (int l = 0; l < 4; l++) {
-            const float h2 = l < 3 ? hy0.v[l + 1] : hyn;
-            const float v = e.v[l] + c.v[l] * ((h1.v[l] - hz0.v[l]) - (h2 - hy0.v[l]));
-            r.v[l] = (k0 + l < nz - 1) ? v : v * 0.f;
-        }
-        st4(ex + id, r);
-    }
-    if (i < nx - 1) {
-        const Q4 e = ld4(ey + id);
-        const Q4 c = lut4(tab + 256, my + id);
-        const Q4 h2 = ld4(hz + id + sx);
-        const float hxn = hx[id + 4];
-        Q4 r;
-#pragma unroll
-        for (int l = 0; l < 4; l++) {
-            const float h1 = l < 3 ? hx0.v[l + 1] : hxn;
-            const float v = e.v[l] + c.v[l] * ((h1 - hx0.v[l]) - (h2.v[l] - hz0.v[l]));
-            r.v[l] = (k0 + l < nz - 1) ? v : v * 0.f;
-        }
-        st4(ey + id, r);
-        if (j < ny - 1) {
-            const Q4 e3 = ld4(ez + id);
-            const Q4 c3 = lut4(tab + 512, mz + id);
-            const Q4 g1 = ld4(hy + id + sx);
-            const Q4 g2 = ld4(hx + id + nzp);
-            Q4 r3;
-#pragma unroll
-            for (int l = 0; l < 4; l++) {
-                const float v = e3.v[l] + c3.v[l] * ((g1.v[l] - hy0.v[l]) - (g2.v[l] - hx0.v[l]));
-                r3.v[l] = (k0 + l < nz) ? v : v * 0.f;
-            }
-            st4(ez + id, r3);
-        }
-    }
-}
-
 template <bool HAS_C>
 __global__ __launch_bounds__(kBlock) void k_update_h(
     int nx, int ny, int nzp, int nz, unsigned q0, unsigned q1, unsigned Q,
@@ -258,37 +180,71 @@ __global__ __launch_bounds__(kBlock) void k_update_h(
     }
 }
 
-// idx0 / nmax: the element range [idx0, nmax) of the split form (nmax < 0: the whole
-// grid); a quad is updated when its first element lies in the range, as the reference's
-// SSE loop does, so idx0 must start a quad.
-static int launch_core(bool e_half, int nx, int ny, int nzp, int pad,
-                       float *ex, float *ey, float *ez, float *hx, float *hy, float *hz,
-                       const float *c0, const float *c1, const float *c2, hipStream_t st,
-                       long long idx0 = 0, long long nmax = -1)
+static int check_fields(const float *const (&ptrs)[6])
 {
-    if (int rc = check_grid(nx, ny, nzp, pad)) return rc;
-    const float *ptrs[6] = {ex, ey, ez, hx, hy, hz};
     for (const float *p : ptrs) {
         if (!p) return fail(MIFDTD_ENULL, "field pointer is NULL");
         if (!aligned16(p)) return fail(MIFDTD_EALIGN, "field pointer %p is not 16-byte aligned", (const void *)p);
     }
-    const bool has_c = c0 || c1 || c2;
-    if (has_c) {
-        if (!(c0 && c1 && c2)) return fail(MIFDTD_ENULL, "coefficient arrays must be all set or all NULL");
-        if (!aligned16(c0) || !aligned16(c1) || !aligned16(c2))
-            return fail(MIFDTD_EALIGN, "coefficient pointer is not 16-byte aligned");
-    }
+    return 0;
+}
+static int check_coeffs(const float *c0, const float *c1, const float *c2)
+{
+    if (!(c0 || c1 || c2)) return 0;
+    if (!(c0 && c1 && c2)) return fail(MIFDTD_ENULL, "coefficient arrays must be all set or all NULL");
+    if (!aligned16(c0) || !aligned16(c1) || !aligned16(c2))
+        return fail(MIFDTD_EALIGN, "coefficient pointer is not 16-byte aligned");
+    return 0;
+}
+
+// The whole grid's half step.  In the whole-grid thread order (row_quads.hpp) the E + H core
+// of a cube ran, against a thread per quad in plain order: 160^3 67.6 -> 53.5 us, 192^3
+// 111 -> 88, 256^3 269 -> 260.
+static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_z, const float *const (&f)[6], hipStream_t st)
+{
+    WholeGrid w{};
+    w.g.nx = nx;
+    w.g.ny = ny;
+    w.g.nzp = nzp;
+    w.g.nz = nz;
+    w.g.m = grid_order(nx, ny, nzp, nz, npml_z);
+    for (int c = 0; c < 6; c++) w.F.e[c] = const_cast<float *>(f[c]);
+    w.cem = kCeConst;
+    w.st = st;
+    return w;
+}
+
+static int launch_core(bool e_half, int nx, int ny, int nzp, int pad, const float *const (&f)[6], const float *c0,
+                       const float *c1, const float *c2, hipStream_t st)
+{
+    if (int rc = check_grid(nx, ny, nzp, pad)) return rc;
+    if (int rc = check_fields(f)) return rc;
+    if (int rc = check_coeffs(c0, c1, c2)) return rc;
+    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, 0, f, st);
+    const float *c[3] = {c0, c1, c2};
+    if (!e_half) return whole_h(w, no_aux(), nullptr, c0 ? c : nullptr);
+    for (int q = 0; q < 3; q++) w.F.ce[q] = c[q];
+    if (c0) w.cem = kCeArrays;
+    return whole_e(w, no_aux(), nullptr, nullptr);
+}
+
+// [idx0, nmax): the element range of the split form; a quad is updated when its first
+// element lies in the range, as the reference's SSE loop does, so idx0 must start a quad.
+static int launch_range(bool e_half, int nx, int ny, int nzp, int pad, const float *const (&f)[6], const float *c0,
+                        const float *c1, const float *c2, hipStream_t st, long long idx0, long long nmax)
+{
+    if (int rc = check_grid(nx, ny, nzp, pad)) return rc;
+    if (int rc = check_fields(f)) return rc;
+    if (int rc = check_coeffs(c0, c1, c2)) return rc;
+    const bool has_c = c0 != nullptr;
+    float *ex = const_cast<float *>(f[0]), *ey = const_cast<float *>(f[1]), *ez = const_cast<float *>(f[2]);
+    float *hx = const_cast<float *>(f[3]), *hy = const_cast<float *>(f[4]), *hz = const_cast<float *>(f[5]);
     const unsigned Q = (unsigned)(nzp / 4);
-    const unsigned nquads = (unsigned)nx * ny * Q;
-    unsigned q0 = 0, q1 = nquads;
-    if (nmax >= 0) {
-        const long long n = 4ll * nquads;
-        if (idx0 < 0 || idx0 > nmax || nmax > n)
-            return fail(MIFDTD_EINVAL, "element range [%lld, %lld) outside the grid's %lld", idx0, nmax, n);
-        if (idx0 % 4) return fail(MIFDTD_EALIGN, "idx0 %lld does not start a 4-element vector", idx0);
-        q0 = (unsigned)(idx0 / 4);
-        q1 = (unsigned)((nmax + 3) / 4);
-    }
+    const long long n = 4ll * nx * ny * Q;
+    if (idx0 < 0 || idx0 > nmax || nmax > n)
+        return fail(MIFDTD_EINVAL, "element range [%lld, %lld) outside the grid's %lld", idx0, nmax, n);
+    if (idx0 % 4) return fail(MIFDTD_EALIGN, "idx0 %lld does not start a 4-element vector", idx0);
+    const unsigned q0 = (unsigned)(idx0 / 4), q1 = (unsigned)((nmax + 3) / 4);
     if (q1 == q0) return 0;
     const unsigned grid = (q1 - q0 + kBlock - 1) / kBlock;
     const int nz = nzp - pad;
@@ -659,6 +615,17 @@ __global__ __launch_bounds__(kBlock) void k_gather(const float *__restrict__ f, 
     if (n < count) out[n] = f[off[n]];
 }
 
+// One value of each of up to kRecord arrays.
+constexpr int kRecord = 32;
+struct RecordAt {
+    const float *p[kRecord];
+};
+__global__ __launch_bounds__(kRecord) void k_record(RecordAt r, int count, float *__restrict__ out)
+{
+    const int n = threadIdx.x;
+    if (n < count) out[n] = *r.p[n];
+}
+
 // ------------------------------------------------------------- periodic boundary
 // Copy plane `src` of two components onto plane `dst` across axis `axis`: element n of
 // the plane is (j, k) of plane i for x (ny * nzp elements, contiguous), (i, k) of row j
@@ -782,8 +749,7 @@ int mifdtd_update_e(int nx, int ny, int nz_pitch, int pad, float *ex, float *ey,
                     const float *hx, const float *hy, const float *hz,
                     const float *cex, const float *cey, const float *cez, mifdtd_stream_t stream)
 {
-    return launch_core(true, nx, ny, nz_pitch, pad, ex, ey, ez, const_cast<float *>(hx), const_cast<float *>(hy),
-                       const_cast<float *>(hz), cex, cey, cez, to_stream(stream));
+    return launch_core(true, nx, ny, nz_pitch, pad, {ex, ey, ez, hx, hy, hz}, cex, cey, cez, to_stream(stream));
 }
 
 int mifdtd_update_e_range(int nx, int ny, int nz_pitch, int pad, long long idx0, long long nmax, float *ex, float *ey,
@@ -791,8 +757,8 @@ int mifdtd_update_e_range(int nx, int ny, int nz_pitch, int pad, long long idx0,
                           const float *cey, const float *cez, mifdtd_stream_t stream)
 {
     if (nmax < 0) return fail(MIFDTD_EINVAL, "nmax %lld < 0", nmax);
-    return launch_core(true, nx, ny, nz_pitch, pad, ex, ey, ez, const_cast<float *>(hx), const_cast<float *>(hy),
-                       const_cast<float *>(hz), cex, cey, cez, to_stream(stream), idx0, nmax);
+    return launch_range(true, nx, ny, nz_pitch, pad, {ex, ey, ez, hx, hy, hz}, cex, cey, cez, to_stream(stream), idx0,
+                        nmax);
 }
 
 int mifdtd_update_h_range(int nx, int ny, int nz_pitch, int pad, long long idx0, long long nmax, const float *ex,
@@ -800,8 +766,16 @@ int mifdtd_update_h_range(int nx, int ny, int nz_pitch, int pad, long long idx0,
                           const float *chy, const float *chz, mifdtd_stream_t stream)
 {
     if (nmax < 0) return fail(MIFDTD_EINVAL, "nmax %lld < 0", nmax);
-    return launch_core(false, nx, ny, nz_pitch, pad, const_cast<float *>(ex), const_cast<float *>(ey),
-                       const_cast<float *>(ez), hx, hy, hz, chx, chy, chz, to_stream(stream), idx0, nmax);
+    return launch_range(false, nx, ny, nz_pitch, pad, {ex, ey, ez, hx, hy, hz}, chx, chy, chz, to_stream(stream), idx0,
+                        nmax);
+}
+
+static int check_mats(const unsigned char *const (&mats)[3], const float *lut)
+{
+    if (!mats[0] || !mats[1] || !mats[2] || !lut) return fail(MIFDTD_ENULL, "material index or table is NULL");
+    for (const unsigned char *m : mats)
+        if (reinterpret_cast<uintptr_t>(m) & 3u) return fail(MIFDTD_EALIGN, "material index array not 4-byte aligned");
+    return 0;
 }
 
 int mifdtd_update_e_lut(int nx, int ny, int nz_pitch, int pad, float *ex, float *ey, float *ez, const float *hx,
@@ -809,30 +783,110 @@ int mifdtd_update_e_lut(int nx, int ny, int nz_pitch, int pad, float *ex, float 
                         const unsigned char *mat_z, const float *lut, mifdtd_stream_t stream)
 {
     if (int rc = check_grid(nx, ny, nz_pitch, pad)) return rc;
-    const float *ptrs[6] = {ex, ey, ez, hx, hy, hz};
-    for (const float *p : ptrs) {
-        if (!p) return fail(MIFDTD_ENULL, "field pointer is NULL");
-        if (!aligned16(p)) return fail(MIFDTD_EALIGN, "field pointer %p is not 16-byte aligned", (const void *)p);
-    }
-    if (!mat_x || !mat_y || !mat_z || !lut) return fail(MIFDTD_ENULL, "material index or table is NULL");
-    const unsigned char *mats[3] = {mat_x, mat_y, mat_z};
-    for (const unsigned char *m : mats)
-        if (reinterpret_cast<uintptr_t>(m) & 3u) return fail(MIFDTD_EALIGN, "material index array not 4-byte aligned");
-    const unsigned Q = (unsigned)(nz_pitch / 4);
-    const unsigned nquads = (unsigned)nx * ny * Q;
-    const unsigned grid = (nquads + kBlock - 1) / kBlock;
-    k_update_e_lut<<<grid, kBlock, 0, to_stream(stream)>>>(nx, ny, nz_pitch, nz_pitch - pad, nquads, Q, ex, ey, ez, hx,
-                                                           hy, hz, mat_x, mat_y, mat_z, lut);
-    MIFDTD_CHECK_LAUNCH("update_e_lut launch");
-    return 0;
+    const float *const f[6] = {ex, ey, ez, hx, hy, hz};
+    if (int rc = check_fields(f)) return rc;
+    const unsigned char *const mats[3] = {mat_x, mat_y, mat_z};
+    if (int rc = check_mats(mats, lut)) return rc;
+    WholeGrid w = whole_grid(nx, ny, nz_pitch, nz_pitch - pad, 0, f, to_stream(stream));
+    for (int c = 0; c < 3; c++) w.F.cm[c] = mats[c];
+    w.F.lut = lut;
+    w.cem = kCeTable;
+    return whole_e(w, no_aux(), nullptr, nullptr);
 }
 
 int mifdtd_update_h(int nx, int ny, int nz_pitch, int pad, const float *ex, const float *ey, const float *ez,
                     float *hx, float *hy, float *hz,
                     const float *chx, const float *chy, const float *chz, mifdtd_stream_t stream)
 {
-    return launch_core(false, nx, ny, nz_pitch, pad, const_cast<float *>(ex), const_cast<float *>(ey),
-                       const_cast<float *>(ez), hx, hy, hz, chx, chy, chz, to_stream(stream));
+    return launch_core(false, nx, ny, nz_pitch, pad, {ex, ey, ez, hx, hy, hz}, chx, chy, chz, to_stream(stream));
+}
+
+// The CPML of one half step for the whole-grid passes: psi packed (MIFDTD_PSI_PACKED: psi1 and
+// psi2 of each face in one buffer) with both faces of an axis or none.  False: not of this form.
+static bool packed_cpml(const mifdtd_cpml_half &h, int nx, int ny, int nzp, bool e_half, SCpml &cp)
+{
+    cp = SCpml{};
+    cp.npml = h.npml;
+    cp.sX = (size_t)h.npml * ny * nzp;
+    cp.sY = (size_t)nx * h.npml * nzp;
+    cp.sZ = (size_t)nx * ny * h.npml;
+    const size_t size[3] = {cp.sX, cp.sY, cp.sZ}, first[3] = {0, 4 * cp.sX, 4 * cp.sX + 4 * cp.sY};
+    uintptr_t base = 0;
+    for (int ax = 0; ax < 3; ax++) {
+        if (!h.psi1[2 * ax] && !h.psi1[2 * ax + 1] && !h.psi2[2 * ax] && !h.psi2[2 * ax + 1]) continue;
+        for (int sd = 0; sd < 2; sd++)
+            for (int c = 0; c < 2; c++) {
+                const uintptr_t p = reinterpret_cast<uintptr_t>((c ? h.psi2 : h.psi1)[2 * ax + sd]);
+                const uintptr_t b = p - sizeof(float) * (first[ax] + (size_t)(2 * sd + c) * size[ax]);
+                if (!p || (cp.axes && b != base)) return false;
+                base = b;
+                cp.axes |= 1 << ax;
+            }
+    }
+    if (!cp.axes || (base & 15u)) return false;
+    float *psi = reinterpret_cast<float *>(base);
+    if (e_half) {
+        cp.pe = cp.pe_out = psi;
+        cp.bE = h.b;
+        cp.aE = h.a;
+    } else {
+        cp.ph = psi;
+        cp.bH = h.b;
+        cp.aH = h.a;
+    }
+    return true;
+}
+
+int mifdtd_half_e(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, float *ex, float *ey, float *ez,
+                  const float *hx, const float *hy, const float *hz, const float *cex, const float *cey,
+                  const float *cez, const unsigned char *mat_x, const unsigned char *mat_y,
+                  const unsigned char *mat_z, const float *lut, mifdtd_stream_t stream)
+{
+    if (!cp) return fail(MIFDTD_ENULL, "cpml descriptor is NULL");
+    if (int rc = check_cpml(nx, ny, nzp, pad, cp->npml, cp->b, cp->a)) return rc;
+    const float *const f[6] = {ex, ey, ez, hx, hy, hz};
+    if (int rc = check_fields(f)) return rc;
+    if (int rc = check_coeffs(cex, cey, cez)) return rc;
+    const unsigned char *const mats[3] = {mat_x, mat_y, mat_z};
+    const bool table = mat_x || mat_y || mat_z || lut;
+    if (table)
+        if (int rc = check_mats(mats, lut)) return rc;
+    SCpml sc;
+    if (!packed_cpml(*cp, nx, ny, nzp, true, sc)) {
+        const int rc = table ? mifdtd_update_e_lut(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, mat_x, mat_y, mat_z, lut, stream)
+                             : mifdtd_update_e(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, cex, cey, cez, stream);
+        return rc ? rc : mifdtd_cpml_e(nx, ny, nzp, pad, cp, ex, ey, ez, hx, hy, hz, cex, cey, cez, stream);
+    }
+    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 4) ? cp->npml : 0, f, to_stream(stream));
+    const float *const ce[3] = {cex, cey, cez};
+    for (int c = 0; c < 3; c++) {
+        w.F.ce[c] = ce[c];
+        w.F.cm[c] = mats[c];
+    }
+    w.F.lut = lut;
+    w.cem = table ? kCeTable : cex ? kCeArrays : kCeConst;
+    w.cp = sc;
+    return whole_e(w, no_aux(), nullptr, nullptr);
+}
+
+int mifdtd_half_h(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, const float *ex, const float *ey,
+                  const float *ez, float *hx, float *hy, float *hz, const float *chx, const float *chy,
+                  const float *chz, mifdtd_stream_t stream)
+{
+    if (!cp) return fail(MIFDTD_ENULL, "cpml descriptor is NULL");
+    if (int rc = check_cpml(nx, ny, nzp, pad, cp->npml, cp->b, cp->a)) return rc;
+    const float *const f[6] = {ex, ey, ez, hx, hy, hz};
+    if (int rc = check_fields(f)) return rc;
+    if (int rc = check_coeffs(chx, chy, chz)) return rc;
+    SCpml sc;
+    if (!packed_cpml(*cp, nx, ny, nzp, false, sc)) {
+        const int rc = mifdtd_update_h(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, chx, chy, chz, stream);
+        return rc ? rc : mifdtd_cpml_h(nx, ny, nzp, pad, cp, ex, ey, ez, hx, hy, hz, chx, chy, chz, stream);
+    }
+    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 4) ? cp->npml : 0, f, to_stream(stream));
+    w.cp = sc;
+    const float *const ch[3] = {chx, chy, chz};
+    return whole_h(w, no_aux(), nullptr, chx ? ch : nullptr);
 }
 
 int mifdtd_cpml_e(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp,
@@ -1069,6 +1123,22 @@ int mifdtd_gather(const float *f, const long long *offsets, int count, float *ou
     const unsigned g = (unsigned)((count + kBlock - 1) / kBlock);
     k_gather<<<g, kBlock, 0, to_stream(stream)>>>(f, offsets, count, out);
     MIFDTD_CHECK_LAUNCH("gather launch");
+    return 0;
+}
+
+int mifdtd_record(const float *const *at, int count, float *out, mifdtd_stream_t stream)
+{
+    if (count <= 0) return 0;
+    if (!at || !out) return fail(MIFDTD_ENULL, "record pointer is NULL");
+    for (int n = 0; n < count; n++)
+        if (!at[n]) return fail(MIFDTD_ENULL, "record pointer is NULL");
+    for (int n = 0; n < count; n += kRecord) {
+        RecordAt r{};
+        const int m = count - n < kRecord ? count - n : kRecord;
+        for (int q = 0; q < m; q++) r.p[q] = at[n + q];
+        k_record<<<1, kRecord, 0, to_stream(stream)>>>(r, m, out + n);
+        MIFDTD_CHECK_LAUNCH("record launch");
+    }
     return 0;
 }
 

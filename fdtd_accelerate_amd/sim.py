@@ -10,6 +10,8 @@ the in-place slab-ordered whole step (see ``fused.py``).
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -32,7 +34,6 @@ class YeeSim:
         self.cpml = Cpml(self.fields, npml, cpml_faces, m=cpml_m, R=cpml_R) if npml > 0 else None
         self.sources = []
         self.probe_points = []
-        self._probe_off = None
         self._series = []
         self.engine = engine
         self.tstep = 0
@@ -65,23 +66,15 @@ class YeeSim:
         if not (0 <= i < f.nx and 0 <= j < f.ny and 0 <= k < f.nz):
             raise ValueError(f"probe point {pt} outside the grid {f.ns}")
         self.probe_points.append((_NAMES.index(str_f), (int(i), int(j), int(k))))
-        self._probe_off = None
-
-    def _probe_offsets(self):
-        if self._probe_off is None and self.probe_points:
-            f = self.fields
-            offs = [(i * f.ny + j) * f.nz_pitch + k for _, (i, j, k) in self.probe_points]
-            self._probe_off = torch.tensor(offs, dtype=torch.int64, device=f.device)
-        return self._probe_off
 
     # -------------------------------------------------------------- stepping
     def _record(self, buf, t):
         """Gather every probe (insertion order) into row t of the device buffer."""
-        offs = self._probe_offsets()
         f = self.fields
-        for n, (c, _) in enumerate(self.probe_points):
-            _lib.call("mifdtd_gather", f.ehs[c].data_ptr(), offs[n:n + 1].data_ptr(), 1,
-                      buf[t, n:n + 1].data_ptr(), _lib.stream_handle(f.stream))
+        n = len(self.probe_points)
+        at = (ctypes.c_void_p * n)(*[f.ehs[c].data_ptr() + 4 * ((i * f.ny + j) * f.nz_pitch + k)
+                                     for c, (i, j, k) in self.probe_points])
+        _lib.call("mifdtd_record", at, n, buf.data_ptr() + 4 * t * buf.stride(0), _lib.stream_handle(f.stream))
 
     def set_savefields(self, str_f, pt0, pt1, tstep_range, dir_path, tag=0, max_tstep=None, **options):
         """Snapshot files of components of the box [pt0, pt1] at the steps ``tstep`` with

@@ -191,6 +191,23 @@ int mifdtd_cpml_h(int nx, int ny, int nz_pitch, int pad, const mifdtd_cpml_half 
                   const float *chx, const float *chy, const float *chz,
                   mifdtd_stream_t stream);
 
+/* The core update and the CPML of one half step together, as update_e (with the material
+ * indices where lut is given) followed by mifdtd_cpml_e, and update_h by mifdtd_cpml_h: one
+ * pass over the grid where the psi arrays are packed (MIFDTD_PSI_PACKED) with both faces of
+ * an axis or none, else those two calls.  No reference counterpart (there each face is a
+ * call of its own). */
+int mifdtd_half_e(int nx, int ny, int nz_pitch, int pad, const mifdtd_cpml_half *cp,
+                  float *ex, float *ey, float *ez,
+                  const float *hx, const float *hy, const float *hz,
+                  const float *cex, const float *cey, const float *cez,
+                  const unsigned char *mat_x, const unsigned char *mat_y,
+                  const unsigned char *mat_z, const float *lut, mifdtd_stream_t stream);
+int mifdtd_half_h(int nx, int ny, int nz_pitch, int pad, const mifdtd_cpml_half *cp,
+                  const float *ex, const float *ey, const float *ez,
+                  float *hx, float *hy, float *hz,
+                  const float *chx, const float *chy, const float *chz,
+                  mifdtd_stream_t stream);
+
 /* ---------------------------------------------------------------- sources ----
  * Replaces the IncidentDirect -> SetFields update of K7/cpu/incident_direct.py:75-77
  * and K7/cpu/get_set_fields.py:110-123 (and KU/gpu/core/source.cu:11-20):
@@ -247,6 +264,9 @@ int mifdtd_tfsf_faces(const mifdtd_tfsf_patches *p, float *const f[6], const flo
  *   out[n] = f[offsets[n]]  for n < count   (offsets: device int64 element offsets) */
 int mifdtd_gather(const float *f, const long long *offsets, int count, float *out,
                   mifdtd_stream_t stream);
+/* The probes of one step, of any components, in one launch: out[n] = *at[n], at: a HOST
+ * array of device addresses. */
+int mifdtd_record(const float *const *at, int count, float *out, mifdtd_stream_t stream);
 
 
 /* ------------------------------------------------------------- fused step ----
