@@ -113,15 +113,15 @@ int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *con
     return 0;
 }
 
-RowQuads grid_order(int nx, int ny, int nzp, int nz, int npml)
+RowQuads grid_order(int nx, int ny, int Q, int nz, int npml)
 {
     thread_local int key[5] = {0, 0, 0, 0, 0};
     thread_local RowQuads m;
-    const int want[5] = {nx, ny, nzp, nz, npml};
+    const int want[5] = {nx, ny, Q, nz, npml};
     bool same = true;
     for (int n = 0; n < 5; n++) same = same && key[n] == want[n];
     if (!same) {
-        m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)(nzp / 4), nz, npml);
+        m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, npml);
         for (int n = 0; n < 5; n++) key[n] = want[n];
     }
     return m;

@@ -28,7 +28,8 @@ inline SAux no_aux()
 int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf);
 int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *const *ch = nullptr);
 
-// row_quads of the whole grid; the last one a thread asked for is kept.
-RowQuads grid_order(int nx, int ny, int nzp, int nz, int npml);
+// row_quads of the whole grid of Q units of 16 bytes per row; the last one a thread asked for
+// is kept.
+RowQuads grid_order(int nx, int ny, int Q, int nz, int npml);
 
 }  // namespace mifdtd

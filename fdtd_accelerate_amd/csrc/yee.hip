@@ -207,7 +207,7 @@ static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_z, const f
     w.g.ny = ny;
     w.g.nzp = nzp;
     w.g.nz = nz;
-    w.g.m = grid_order(nx, ny, nzp, nz, npml_z);
+    w.g.m = grid_order(nx, ny, nzp / 4, nz, npml_z);
     for (int c = 0; c < 6; c++) w.F.e[c] = const_cast<float *>(f[c]);
     w.cem = kCeConst;
     w.st = st;
