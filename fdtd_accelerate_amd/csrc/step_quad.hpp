@@ -161,6 +161,35 @@ __device__ __forceinline__ unsigned tfsf_mask(const STfsf &t, int ia, int ib, in
     return m;
 }
 
+// Design box of the adjoint: the curl of H (the factor of CE in the core E update) of its
+// cells is stored component after component, C order, before the update changes E.
+struct SCurl {
+    int i0, j0, k0, di, dj, dk;
+    float *out;
+    __device__ __forceinline__ bool row_in(int i, int j) const
+    {
+        return i >= i0 && i < i0 + di && j >= j0 && j < j0 + dj;
+    }
+    __device__ __forceinline__ void store(int i, int j, int q0, const Q4 &x, const Q4 &y, const Q4 &z) const
+    {
+        const size_t s = (size_t)di * dj * dk;
+        float *p = out + ((size_t)(i - i0) * dj + (j - j0)) * dk + (q0 - k0);
+        if (q0 >= k0 && q0 + 4 <= k0 + dk && (((size_t)p | (s << 2)) & 15u) == 0) {
+            st4(p, x);
+            st4(p + s, y);
+            st4(p + 2 * s, z);
+            return;
+        }
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            if (q0 + l < k0 || q0 + l >= k0 + dk) continue;
+            p[l] = x.v[l];
+            p[l + s] = y.v[l];
+            p[l + 2 * s] = z.v[l];
+        }
+    }
+};
+
 struct SGeom {
     int nx, ny, nzp, nz;
     int i0;            // first plane of the slab
@@ -321,7 +350,7 @@ struct ZFace {
 // arrays cex.., 2 the uint8 material indices mx.. into tab ([3][256] floats, the same
 // values as the arrays, so the products are identical).  next: the next lane holds the
 // quad at k0+4 (else this lane loads its k0+4 neighbours itself).
-constexpr int kFeatDrude = 1, kFeatTfsf = 2;  // optional E-pass features (template bits)
+constexpr int kFeatDrude = 1, kFeatTfsf = 2, kFeatCurl = 4;  // optional E-pass features (template bits)
 
 template <int CM, bool PML, int FEAT = 0>
 __device__ __forceinline__ void e_quad_at(
@@ -331,7 +360,7 @@ __device__ __forceinline__ void e_quad_at(
     const SCpml &cp, const SAux &aux, const unsigned char *__restrict__ mx = nullptr,
     const unsigned char *__restrict__ my = nullptr, const unsigned char *__restrict__ mz = nullptr,
     const float *tab = nullptr, const SDrude *dr = nullptr, const STfsf *tf = nullptr, float *prow = nullptr,
-    const float *tv_row = nullptr, const int *tv = nullptr)
+    const float *tv_row = nullptr, const int *tv = nullptr, const SCurl *cu = nullptr)
 {
     constexpr bool DR = (FEAT & kFeatDrude) != 0;
     constexpr bool TF = (FEAT & kFeatTfsf) != 0;
@@ -407,6 +436,16 @@ __device__ __forceinline__ void e_quad_at(
     for (int l = 0; l < 4; ++l) {
         y1[l] = l < 3 ? hy0.v[l + 1] : hyn;
         x1[l] = l < 3 ? hx0.v[l + 1] : hxn;
+    }
+    if ((FEAT & kFeatCurl) && cu->row_in(i, j)) {
+        Q4 w0, w1, w2;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            w0.v[l] = (hzU.v[l] - hz0.v[l]) - (y1[l] - hy0.v[l]);
+            w1.v[l] = (x1[l] - hx0.v[l]) - (hzN.v[l] - hz0.v[l]);
+            w2.v[l] = (hyN.v[l] - hy0.v[l]) - (hxU.v[l] - hx0.v[l]);
+        }
+        cu->store(i, j, k0, w0, w1, w2);
     }
     if (jy) {
 #pragma unroll

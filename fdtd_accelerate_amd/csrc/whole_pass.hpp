@@ -23,9 +23,10 @@ inline SAux no_aux()
     return a;
 }
 
-// E pass, then H pass, each in place; dr / tf: null where the step has none; ch: the three
+// E pass, then H pass, each in place; dr / tf / cu: null where the step has none (cu goes
+// without the others); ch: the three
 // CH arrays, null for the constant 0.5 (which a step with tf has).
-int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf);
+int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf, const SCurl *cu = nullptr);
 int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *const *ch = nullptr);
 
 // row_quads of the whole grid of Q units of 16 bytes per row; the last one a thread asked for

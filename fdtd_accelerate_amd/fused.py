@@ -525,13 +525,19 @@ class SlabStepper(FusedStepper):
         torch.cuda.synchronize()
         return sum(a.elapsed_time(b) for a, b in evs) / max(nsteps, 1)
 
-    def _call(self, nsteps, buf, timed=False):
+    def _call(self, nsteps, buf, timed=False, design=None):
+        """``design``: (box, curls), to store the curl of H on the box before each step's E
+        update in the contiguous float32 tensor curls (nsteps, 3, di, dj, dk)."""
         sim = self.sim
         f = sim.fields
         if buf is None and sim.probe_points:
             buf = torch.zeros((nsteps, len(sim.probe_points)), dtype=torch.float32, device=f.device)
         d = self._desc()
         tv = self._tvals(nsteps)
+        if design is not None:
+            box, curls = design
+            d.design_box[:] = box
+            d.design_curl = curls.data_ptr()
         _lib.call("mifdtd_slab_run", ctypes.byref(d), self.S, nsteps, tv.ctypes.data,
                   None if buf is None else buf.data_ptr(), _lib.stream_handle(f.stream))
         for s in sim.sources:

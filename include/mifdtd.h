@@ -366,6 +366,11 @@ typedef struct {
      * e[], psiE and drude_j (the same values; *parity stays 0, sweep_ms brackets the two
      * passes) -- the faster form for grids that a sweep does not fill; not with e_mid */
     int whole_grid;
+    /* optional (mifdtd_slab_run): the curl of H on a design box (i0, j0, k0, di, dj, dk;
+     * i0 + di < nx and so on) before each step's E update, as mifdtd_design_curl gives it,
+     * into design_curl, DEVICE (nsteps, 3, di, dj, dk) */
+    int design_box[6];
+    float *design_curl;
 } mifdtd_fused_desc;
 #define MIFDTD_FUSED_MAX_CE_TRI 4096
 
