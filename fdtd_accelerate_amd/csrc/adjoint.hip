@@ -115,8 +115,7 @@ __device__ __forceinline__ size_t psi_at(const AGeom &g, int axis, int sd, int p
 // the curl and the CPML terms of all three axes; the psi of an axis is loaded only by the
 // rows and quads it reaches.  With a thread per cell the passes ran 7 scalar gathers per
 // component and re-derived every neighbour's validity: 160^3 cells, CPML 10, 75.5 + 110.6
-// us; now 41.0 + 61.0.  The bound is the traffic behind the L2s (84 B per cell and step and
-// the psi).
+// us; now 39.4 + 52.1 (84 B per cell and step and the psi, at 4.9-5.2 TB/s).
 __device__ __forceinline__ Q4 keep_cells(const Q4 &q, int k0, int lo, int hi)  // lanes lo <= k < hi, else 0
 {
     Q4 r;
@@ -199,8 +198,21 @@ __device__ __forceinline__ void add_diff(Q4 &v, const Q4 &p, const Q4 &m)
 
 __device__ __forceinline__ Q4 psi_ld(bool on, const float *lp, size_t o) { return on ? ld4u(lp + o) : splat4(0.f); }
 
+// psi1, psi2 and the table entry of a z-face cell (entry e; what e.t <= 0 loads is not used).
+// All cells' loads go ahead of the block's psi stores: a load that follows the previous
+// cell's store is a memory round trip of its own, and at 160 cells a row 2 of 5 waves are
+// z-slab waves (passes A + C 43.6 + 58.6 -> 39.4 + 52.1 us).  Pass A keeps 4 waves per SIMD
+// at 12 bytes of spill (130 VGPRs without).
+struct ZPsi {
+    float q1, q2, c;
+};
+__device__ __forceinline__ ZPsi z_psi(const Entry &e, const float *lp, const float *tab)
+{
+    return ZPsi{lp[e.o1], lp[e.o2], tab[e.t > 0 ? e.t : 0]};
+}
+
 // Pass A (and D of the later step) on one quad.
-__global__ __launch_bounds__(AB) void k_adj_a(AGeom g, RowQuads m, float *__restrict__ lex, float *__restrict__ ley,
+__global__ __launch_bounds__(AB) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_a(AGeom g, RowQuads m, float *__restrict__ lex, float *__restrict__ ley,
                                               float *__restrict__ lez, float *__restrict__ lhx,
                                               float *__restrict__ lhy, float *__restrict__ lhz,
                                               const float *__restrict__ lpH, const float *__restrict__ aH,
@@ -282,14 +294,21 @@ __global__ __launch_bounds__(AB) void k_adj_a(AGeom g, RowQuads m, float *__rest
     }
     if (nz_) {
         // D: psi1 ex (-), psi2 ey (+)
+        ZPsi zd[4], zt[5];
+#pragma unroll
+        for (int l = 0; l < 4; ++l) zd[l] = z_psi(entry<true>(g, 2, k0 + l, i, j, k0 + l), lpE, bE);
+#pragma unroll
+        for (int l = 0; l < 5; ++l) {
+            const int kk = k0 + l < g.nzp ? k0 + l : 0;
+            zt[l] = z_psi(entry<false>(g, 2, kk, i, j, kk), lpH, aH);
+        }
         const Q4 gx = scale4(cex, id, ex0), gy = scale4(cey, id, ey0);
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             const Entry d = entry<true>(g, 2, k0 + l, i, j, k0 + l);
             if (d.t > 0) {
-                const float b = bE[d.t];
-                if (jy) lpE[d.o1] = b * (lpE[d.o1] - gx.v[l]);
-                if (ix) lpE[d.o2] = b * (lpE[d.o2] + gy.v[l]);
+                if (jy) lpE[d.o1] = zd[l].c * (zd[l].q1 - gx.v[l]);
+                if (ix) lpE[d.o2] = zd[l].c * (zd[l].q2 + gy.v[l]);
             }
         }
         // a t of cells k0 .. k0+4: psi1 -> hx from ey (+), psi2 -> hy from ex (-)
@@ -301,9 +320,8 @@ __global__ __launch_bounds__(AB) void k_adj_a(AGeom g, RowQuads m, float *__rest
             const int kk = k < g.nzp ? k : 0;
             const Entry t = entry<false>(g, 2, kk, i, j, kk);
             if (k > 0 && k < nz && t.t > 0) {
-                const float a = aH[t.t];
-                if (jp) t1[l] = a * (lpH[t.o1] + 0.5f * (l < 4 ? hx0.v[l & 3] : hx4));
-                if (ip) t2[l] = a * (lpH[t.o2] - 0.5f * (l < 4 ? hy0.v[l & 3] : hy4));
+                if (jp) t1[l] = zt[l].c * (zt[l].q1 + 0.5f * (l < 4 ? hx0.v[l & 3] : hx4));
+                if (ip) t2[l] = zt[l].c * (zt[l].q2 - 0.5f * (l < 4 ? hy0.v[l & 3] : hy4));
             }
         }
 #pragma unroll
@@ -445,14 +463,21 @@ __global__ __launch_bounds__(AB) void k_adj_c(AGeom g, RowQuads m, float *__rest
     }
     if (nz_) {
         // B: psi1 hx (+), psi2 hy (-)
+        ZPsi zd[4], zt[5];
+#pragma unroll
+        for (int l = 0; l < 4; ++l) zd[l] = z_psi(entry<false>(g, 2, k0 + l, i, j, k0 + l), lpH, bH);
+#pragma unroll
+        for (int l = 0; l < 5; ++l) {
+            const int kk = k0 - 1 + l > 0 ? k0 - 1 + l : 0;
+            zt[l] = z_psi(entry<true>(g, 2, kk, i, j, kk), lpE, aE);
+        }
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             const int k = k0 + l;
             const Entry d = entry<false>(g, 2, k, i, j, k);
             if (d.t > 0 && k > 0) {
-                const float b = bH[d.t];
-                if (jp) lpH[d.o1] = b * (lpH[d.o1] + 0.5f * hx0.v[l]);
-                if (ip) lpH[d.o2] = b * (lpH[d.o2] - 0.5f * hy0.v[l]);
+                if (jp) lpH[d.o1] = zd[l].c * (zd[l].q1 + 0.5f * hx0.v[l]);
+                if (ip) lpH[d.o2] = zd[l].c * (zd[l].q2 - 0.5f * hy0.v[l]);
             }
         }
         // a t of cells k0-1 .. k0+3: psi1 -> ex from hy (-), psi2 -> ey from hx (+)
@@ -464,9 +489,8 @@ __global__ __launch_bounds__(AB) void k_adj_c(AGeom g, RowQuads m, float *__rest
             const int kk = k > 0 ? k : 0;
             const Entry t = entry<true>(g, 2, kk, i, j, kk);
             if (k >= 0 && k < nz - 1 && t.t > 0) {
-                const float a = aE[t.t];
-                if (jy) t1[l] = a * (lpE[t.o1] - (l > 0 ? gx0.v[(l + 3) & 3] : gxm));
-                if (ix) t2[l] = a * (lpE[t.o2] + (l > 0 ? gy0.v[(l + 3) & 3] : gym));
+                if (jy) t1[l] = zt[l].c * (zt[l].q1 - (l > 0 ? gx0.v[(l + 3) & 3] : gxm));
+                if (ix) t2[l] = zt[l].c * (zt[l].q2 + (l > 0 ? gy0.v[(l + 3) & 3] : gym));
             }
         }
 #pragma unroll
