@@ -216,11 +216,32 @@ __global__ __launch_bounds__(S4B) void k_s4_e(SAux, S4Geom g, S4Cpml cp, float d
                 dz2.v[l] = diff4(hxM.v[l], hx0.v[l], hxP.v[l], hxQ.v[l]);
             }
         }
-        // x faces: psi1 -> ey from hz (-), psi2 -> ez from hy (+)
-        if (i0 < p || i0 + 3 >= nx - 1 - p) {
-            S4FaceX fx;
+        // psi of all faces together, when the rows' and planes' registers are free: face after
+        // face, each one's loads wait for the stores before
+        S4FaceX fx;
+        const bool xf = i0 < p || i0 + 3 >= nx - 1 - p;
+        if (xf) {
             const int side = i0 + 3 >= nx - 1 - p;
             fx.load(cp, side, i0, side ? nx - 1 - p : 0, side ? p + 1 : 1, 1, nx - 2, (size_t)p * ((size_t)j + (size_t)ny * k));
+        }
+        float *py1 = nullptr, *py2 = nullptr, *pz1 = nullptr, *pz2 = nullptr;
+        Q4 sy1 = z4, sy2 = z4, sz1 = z4, sz2 = z4;
+        if (ty > 0 && (sdy ? cp.psi1[3] : cp.psi1[2])) {
+            const size_t n = (size_t)i0 + sy * ((size_t)qy + (size_t)p * k);
+            py1 = (sdy ? cp.psi1[3] : cp.psi1[2]) + n;
+            py2 = (sdy ? cp.psi2[3] : cp.psi2[2]) + n;
+            sy1 = ld4u(py1);
+            sy2 = ld4u(py2);
+        }
+        if (tz > 0 && (sdz ? cp.psi1[5] : cp.psi1[4])) {
+            const size_t n = (size_t)i0 + sy * ((size_t)j + (size_t)ny * qz);
+            pz1 = (sdz ? cp.psi1[5] : cp.psi1[4]) + n;
+            pz2 = (sdz ? cp.psi2[5] : cp.psi2[4]) + n;
+            sz1 = ld4u(pz1);
+            sz2 = ld4u(pz2);
+        }
+        // x faces: psi1 -> ey from hz (-), psi2 -> ez from hy (+)
+        if (xf) {
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 if (l < fx.lo || l >= fx.hi) continue;
@@ -236,38 +257,28 @@ __global__ __launch_bounds__(S4B) void k_s4_e(SAux, S4Geom g, S4Cpml cp, float d
             }
         }
         // y faces: psi1 -> ez from hx (-), psi2 -> ex from hz (+)
-        if (ty > 0) {
-            float *p1 = sdy ? cp.psi1[3] : cp.psi1[2], *p2 = sdy ? cp.psi2[3] : cp.psi2[2];
-            if (p1) {
-                const size_t n = (size_t)i0 + sy * ((size_t)qy + (size_t)p * k);
-                const S4Half h{dl, cp.b[ty], cp.a[ty]};
-                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+        if (py1) {
+            const S4Half h{dl, cp.b[ty], cp.a[ty]};
 #pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const int i = i0 + l;
-                    if (i > 0 && i < nx - 2) s4_psi_cell(h, s1.v[l], dy1.v[l], c2.v[l], e2.v[l], true);
-                    if (rx && i <= nx - 2) s4_psi_cell(h, s2.v[l], dy2.v[l], c0.v[l], e0.v[l], false);
-                }
-                st4u(p1 + n, s1);
-                st4u(p2 + n, s2);
+            for (int l = 0; l < 4; ++l) {
+                const int i = i0 + l;
+                if (i > 0 && i < nx - 2) s4_psi_cell(h, sy1.v[l], dy1.v[l], c2.v[l], e2.v[l], true);
+                if (rx && i <= nx - 2) s4_psi_cell(h, sy2.v[l], dy2.v[l], c0.v[l], e0.v[l], false);
             }
+            st4u(py1, sy1);
+            st4u(py2, sy2);
         }
         // z faces: psi1 -> ex from hy (-), psi2 -> ey from hx (+)
-        if (tz > 0) {
-            float *p1 = sdz ? cp.psi1[5] : cp.psi1[4], *p2 = sdz ? cp.psi2[5] : cp.psi2[4];
-            if (p1) {
-                const size_t n = (size_t)i0 + sy * ((size_t)j + (size_t)ny * qz);
-                const S4Half h{dl, cp.b[tz], cp.a[tz]};
-                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+        if (pz1) {
+            const S4Half h{dl, cp.b[tz], cp.a[tz]};
 #pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const int i = i0 + l;
-                    if (rx && i <= nx - 2) s4_psi_cell(h, s1.v[l], dz1.v[l], c0.v[l], e0.v[l], true);
-                    if (i > 0 && i < nx - 2) s4_psi_cell(h, s2.v[l], dz2.v[l], c1.v[l], e1.v[l], false);
-                }
-                st4u(p1 + n, s1);
-                st4u(p2 + n, s2);
+            for (int l = 0; l < 4; ++l) {
+                const int i = i0 + l;
+                if (rx && i <= nx - 2) s4_psi_cell(h, sz1.v[l], dz1.v[l], c0.v[l], e0.v[l], true);
+                if (i > 0 && i < nx - 2) s4_psi_cell(h, sz2.v[l], dz2.v[l], c1.v[l], e1.v[l], false);
             }
+            st4u(pz1, sz1);
+            st4u(pz2, sz2);
         }
     }
     const SAux &aux = first_kernel_arg<SAux>();
@@ -369,11 +380,32 @@ __global__ __launch_bounds__(S4B) void k_s4_h(SAux, S4Geom g, S4Cpml cp, float c
                 dz2.v[l] = diff4(exQ.v[l], exM.v[l], ex0.v[l], exP.v[l]);
             }
         }
-        // x faces: psi1 -> hy from ez (+), psi2 -> hz from ey (-)
-        if (i0 < p || i0 + 3 >= nx - p) {
-            S4FaceX fx;
+        // psi of all faces together, when the rows' and planes' registers are free: face after
+        // face, each one's loads wait for the stores before
+        S4FaceX fx;
+        const bool xf = i0 < p || i0 + 3 >= nx - p;
+        if (xf) {
             const int side = i0 + 3 >= nx - p;
             fx.load(cp, side, i0, side ? nx - p : 0, side ? p + 2 : 1, 2, nx - 1, (size_t)p * ((size_t)j + (size_t)ny * k));
+        }
+        float *py1 = nullptr, *py2 = nullptr, *pz1 = nullptr, *pz2 = nullptr;
+        Q4 sy1 = z4, sy2 = z4, sz1 = z4, sz2 = z4;
+        if (ty > 0 && (sdy ? cp.psi1[3] : cp.psi1[2])) {
+            const size_t n = (size_t)i0 + sy * ((size_t)qy + (size_t)p * k);
+            py1 = (sdy ? cp.psi1[3] : cp.psi1[2]) + n;
+            py2 = (sdy ? cp.psi2[3] : cp.psi2[2]) + n;
+            sy1 = ld4u(py1);
+            sy2 = ld4u(py2);
+        }
+        if (tz > 0 && (sdz ? cp.psi1[5] : cp.psi1[4])) {
+            const size_t n = (size_t)i0 + sy * ((size_t)j + (size_t)ny * qz);
+            pz1 = (sdz ? cp.psi1[5] : cp.psi1[4]) + n;
+            pz2 = (sdz ? cp.psi2[5] : cp.psi2[4]) + n;
+            sz1 = ld4u(pz1);
+            sz2 = ld4u(pz2);
+        }
+        // x faces: psi1 -> hy from ez (+), psi2 -> hz from ey (-)
+        if (xf) {
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 if (l < fx.lo || l >= fx.hi) continue;
@@ -389,38 +421,28 @@ __global__ __launch_bounds__(S4B) void k_s4_h(SAux, S4Geom g, S4Cpml cp, float c
             }
         }
         // y faces: psi1 -> hz from ex (+), psi2 -> hx from ez (-)
-        if (ty > 0) {
-            float *p1 = sdy ? cp.psi1[3] : cp.psi1[2], *p2 = sdy ? cp.psi2[3] : cp.psi2[2];
-            if (p1) {
-                const size_t n = (size_t)i0 + sy * ((size_t)qy + (size_t)p * k);
-                const S4Half h{cl, cp.b[ty], cp.a[ty]};
-                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+        if (py1) {
+            const S4Half h{cl, cp.b[ty], cp.a[ty]};
 #pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const int i = i0 + l;
-                    if (i > 1 && i <= nx - 2) s4_psi_cell(h, s1.v[l], dy1.v[l], c2.v[l], h2.v[l], false);
-                    if (rx && i <= nx - 2) s4_psi_cell(h, s2.v[l], dy2.v[l], c0.v[l], h0.v[l], true);
-                }
-                st4u(p1 + n, s1);
-                st4u(p2 + n, s2);
+            for (int l = 0; l < 4; ++l) {
+                const int i = i0 + l;
+                if (i > 1 && i <= nx - 2) s4_psi_cell(h, sy1.v[l], dy1.v[l], c2.v[l], h2.v[l], false);
+                if (rx && i <= nx - 2) s4_psi_cell(h, sy2.v[l], dy2.v[l], c0.v[l], h0.v[l], true);
             }
+            st4u(py1, sy1);
+            st4u(py2, sy2);
         }
         // z faces: psi1 -> hx from ey (+), psi2 -> hy from ex (-)
-        if (tz > 0) {
-            float *p1 = sdz ? cp.psi1[5] : cp.psi1[4], *p2 = sdz ? cp.psi2[5] : cp.psi2[4];
-            if (p1) {
-                const size_t n = (size_t)i0 + sy * ((size_t)j + (size_t)ny * qz);
-                const S4Half h{cl, cp.b[tz], cp.a[tz]};
-                Q4 s1 = ld4u(p1 + n), s2 = ld4u(p2 + n);
+        if (pz1) {
+            const S4Half h{cl, cp.b[tz], cp.a[tz]};
 #pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const int i = i0 + l;
-                    if (rx && i <= nx - 2) s4_psi_cell(h, s1.v[l], dz1.v[l], c0.v[l], h0.v[l], false);
-                    if (i > 1 && i <= nx - 2) s4_psi_cell(h, s2.v[l], dz2.v[l], c1.v[l], h1.v[l], true);
-                }
-                st4u(p1 + n, s1);
-                st4u(p2 + n, s2);
+            for (int l = 0; l < 4; ++l) {
+                const int i = i0 + l;
+                if (rx && i <= nx - 2) s4_psi_cell(h, sz1.v[l], dz1.v[l], c0.v[l], h0.v[l], false);
+                if (i > 1 && i <= nx - 2) s4_psi_cell(h, sz2.v[l], dz2.v[l], c1.v[l], h1.v[l], true);
             }
+            st4u(pz1, sz1);
+            st4u(pz2, sz2);
         }
     }
     const SAux &aux = first_kernel_arg<SAux>();
