@@ -174,7 +174,9 @@ def check(rc: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call a status-returning entry point and raise RuntimeError on failure."""
-    check(getattr(load(), name)(*args), name)
+    rc = getattr(_lib if _lib is not None else load(), name)(*args)
+    if rc:
+        check(rc, name)
 
 
 def stream_handle(stream=None):

@@ -13,6 +13,7 @@ from .build import KEMP_COEFFS, KEMP_PRECISIONS, kemp_program_path
 from .fields import Fields
 
 _programs = {}
+_NO_COEFF = (None, None, None)
 
 
 def program(precision_float="single", coeff_use="e", pad=0, split=False):
@@ -58,6 +59,7 @@ class Core:
         self.mainf = fields
         _lib.load()
         self._sfx = "" if fields.precision_float == "single" else "_f64"
+        self._update_e, self._update_h = "mifdtd_update_e" + self._sfx, "mifdtd_update_h" + self._sfx
         fields.append_instance(self)
 
     def update_e(self):
@@ -66,15 +68,13 @@ class Core:
             _lib.call("mifdtd_update_e_lut", f.nx, f.ny, f.nz_pitch, f.pad, *f.ptrs(f.ehs),
                       *[m.data_ptr() for m in f.ce_mat], f.ce_lut.data_ptr(), _lib.stream_handle(f.stream))
             return
-        ces = f.ces if f.ce_on else (None, None, None)
-        _lib.call("mifdtd_update_e" + self._sfx, f.nx, f.ny, f.nz_pitch, f.pad, *f.ptrs(f.ehs), *f.ptrs(ces),
-                  _lib.stream_handle(f.stream))
+        _lib.call(self._update_e, f.nx, f.ny, f.nz_pitch, f.pad, *[t.data_ptr() for t in f.ehs],
+                  *([t.data_ptr() for t in f.ces] if f.ce_on else _NO_COEFF), f.stream.cuda_stream)
 
     def update_h(self):
         f = self.mainf
-        chs = f.chs if f.ch_on else (None, None, None)
-        _lib.call("mifdtd_update_h" + self._sfx, f.nx, f.ny, f.nz_pitch, f.pad, *f.ptrs(f.ehs), *f.ptrs(chs),
-                  _lib.stream_handle(f.stream))
+        _lib.call(self._update_h, f.nx, f.ny, f.nz_pitch, f.pad, *[t.data_ptr() for t in f.ehs],
+                  *([t.data_ptr() for t in f.chs] if f.ch_on else _NO_COEFF), f.stream.cuda_stream)
 
 
 class CoreSplit(Core):

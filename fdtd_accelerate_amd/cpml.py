@@ -169,14 +169,14 @@ class Cpml:
         mats = (None,) * 4
         if f.ce_on and f.ce_mat is not None:
             mats = (*f.ptrs(f.ce_mat), f.ce_lut.data_ptr())
-        _lib.call("mifdtd_half_e", f.nx, f.ny, f.nz_pitch, f.pad, self._descE, *f.ptrs(f.ehs), *f.ptrs(ces), *mats,
-                  _lib.stream_handle(f.stream))
+        _lib.call("mifdtd_half_e", f.nx, f.ny, f.nz_pitch, f.pad, self._descE, *[t.data_ptr() for t in f.ehs],
+                  *f.ptrs(ces), *mats, f.stream.cuda_stream)
 
     def update_core_h(self):
         f = self.mainf
         chs = f.chs if f.ch_on else (None, None, None)
-        _lib.call("mifdtd_half_h", f.nx, f.ny, f.nz_pitch, f.pad, self._descH, *f.ptrs(f.ehs), *f.ptrs(chs),
-                  _lib.stream_handle(f.stream))
+        _lib.call("mifdtd_half_h", f.nx, f.ny, f.nz_pitch, f.pad, self._descH, *[t.data_ptr() for t in f.ehs],
+                  *f.ptrs(chs), f.stream.cuda_stream)
 
 
 # The update methods that a joined half step stands for (joins_core).

@@ -193,19 +193,19 @@ class Fields:
         return len(insts) > 1 and getattr(insts[1], "joins_core", None) is not None and insts[1].joins_core(insts[0])
 
     def update_e(self):
-        n = 0
+        insts = self.instance_list
         if self._joined():
-            self.instance_list[1].update_core_e()
-            n = 2
-        for inst in itertools.islice(self.instance_list, n, None):
+            insts[1].update_core_e()
+            insts = itertools.islice(insts, 2, None)
+        for inst in insts:
             inst.update_e()
 
     def update_h(self):
-        n = 0
+        insts = self.instance_list
         if self._joined():
-            self.instance_list[1].update_core_h()
-            n = 2
-        for inst in itertools.islice(self.instance_list, n, None):
+            insts[1].update_core_h()
+            insts = itertools.islice(insts, 2, None)
+        for inst in insts:
             inst.update_h()
 
     def enqueue_barrier(self):
