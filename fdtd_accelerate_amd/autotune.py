@@ -16,6 +16,8 @@ from __future__ import annotations
 import json
 import os
 
+from ._lib import MAX_CE_TRI
+
 _TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned_tiles.json")
 _table = None
 N_CU = 256
@@ -35,10 +37,10 @@ def _load():
 def lds_fits(T, CX, table, ntri=0, extra=0):
     """Whether the sweep's LDS (E and H row exchange 2 x 2 x T x 2 x 256 floats, the k-1
     carry (CX+1)(T+1)2 floats, the 3 x 256 CE table or ``ntri`` CE triples, ``extra``
-    more floats, ~0.4 KiB of source/probe tables) fits the 160 KiB of one gfx950
+    more floats, 1.25 KiB of source, probe and patch tables) fits the 160 KiB of one gfx950
     work-group."""
     tab = 4 * ((3 * ntri + 3) // 4) if ntri else (768 if table else 0)
-    return 4 * (tab + 2 * 2 * T * 2 * 256 + (CX + 1) * (T + 1) * 2 + extra) + 512 <= 160 * 1024
+    return 4 * (tab + 2 * 2 * T * 2 * 256 + (CX + 1) * (T + 1) * 2 + extra) + 1280 <= 160 * 1024
 
 
 def lds_fits_pairs(T, CX, table):
@@ -62,7 +64,7 @@ def _halved(nx, ny):
 
 def heuristic(nx, ny, nzp, npml, halved=False):
     """(T, CX): owned rows per block (one halo row each, T+1 waves) and planes per chunk
-    (one seed plane each).  One work-group runs per CU, so a sweep takes whole rounds of
+    (one seed plane each), of the tiles that leave room for the largest CE table.  One work-group runs per CU, so a sweep takes whole rounds of
     256 blocks: the tile with the least rounds * (CX + 2) * (T + 3), the planes and waves of
     a block with one plane for its start and two waves for the barrier.  Sweep against
     T = 9 and CX halved until 1024 blocks: 256^3 135 / 143 us, 384^3 563 / 651, 512^3
@@ -79,6 +81,8 @@ def heuristic(nx, ny, nzp, npml, halved=False):
         if T > max(1, by // 2):
             continue
         for CX in range(min(bx, 64), min(bx, 8) - 1, -1):
+            if not lds_fits(T, CX, True, MAX_CE_TRI):
+                continue
             rounds = -(-(-(-by // T) * -(-bx // CX)) // N_CU)
             c = rounds * (CX + 2) * (T + 3)
             if cost is None or c < cost:

@@ -17,6 +17,7 @@ def test_tile_rule(n, npml):
     from fdtd_accelerate_amd import _lib
     T, CX = autotune.heuristic(*n, npml)
     assert 1 <= T <= 13 and 1 <= CX <= min(64, n[0])
+    assert T == 1 or T <= n[1] // 2
     assert autotune.lds_fits(T, CX, True) and autotune.lds_fits(T, CX, True, _lib.MAX_CE_TRI)
 
 
