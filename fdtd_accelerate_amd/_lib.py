@@ -22,6 +22,11 @@ class CpmlHalf(ctypes.Structure):
     _fields_ = [("npml", _I), ("b", _P), ("a", _P), ("psi1", _P * 6), ("psi2", _P * 6)]
 
 
+class DrudeRegion(ctypes.Structure):
+    """``mifdtd_drude``: the region (i0, j0, k0, li, lj, lk), its currents and coefficients."""
+    _fields_ = [("region", _I * 6), ("j", _P * 3), ("cja", _P * 3), ("cjb", _P * 3)]
+
+
 MAX_SRC = 4
 MAX_PROBE = 8
 TFSF_MAX_PATCH = 12
@@ -106,7 +111,7 @@ _SIGS = {
     "mifdtd_cpml_face_z_h": (_I, [_I] * 6 + [_P] * 8 + [_P]),
     "mifdtd_cpml_e": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 9 + [_P]),
     "mifdtd_cpml_h": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 9 + [_P]),
-    "mifdtd_half_e": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 13 + [_P]),
+    "mifdtd_half_e": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 13 + [ctypes.POINTER(DrudeRegion), _P]),
     "mifdtd_half_h": (_I, [_I] * 4 + [ctypes.POINTER(CpmlHalf)] + [_P] * 9 + [_P]),
     "mifdtd_source": (_I, [_P] + [_I] * 9 + [_F, _P, _F, _I, _P]),
     "mifdtd_gather": (_I, [_P, _P, _I, _P, _P]),

@@ -18,6 +18,7 @@ import torch
 
 from . import _lib, util
 from .core import Core
+from .drude import Drude
 from .fields import Fields
 
 
@@ -155,22 +156,28 @@ class Cpml:
         _lib.call("mifdtd_cpml_h", f.nx, f.ny, f.nz_pitch, f.pad, self._descH, *f.ptrs(f.ehs),
                   *f.ptrs(chs), _lib.stream_handle(f.stream))
 
-    def joins_core(self, core):
-        """Whether ``update_core_e`` / ``update_core_h`` stand for the core's update followed by
-        this CPML's: both are of these classes themselves, on the same fields, with the
-        update methods as defined here (none replaced in a subclass, a class or an instance)."""
+    def joins(self, core, drude=None):
+        """Whether ``update_core_e`` / ``update_core_h`` stand for the core's update, the Drude
+        region's where one is given, then this CPML's: all are of these classes themselves, on
+        the same fields, with the update methods as defined here (none replaced in a subclass,
+        a class or an instance)."""
+        replaced = core.__dict__.keys() | self.__dict__.keys()
+        if drude is not None:
+            if type(drude) is not Drude or drude.mainf is not self.mainf:
+                return False
+            replaced |= drude.__dict__.keys()
         return (type(core) is Core and type(self) is Cpml and core.mainf is self.mainf
-                and not {"update_e", "update_h"} & (core.__dict__.keys() | self.__dict__.keys())
-                and (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h) == _OWN)
+                and not {"update_e", "update_h"} & replaced
+                and (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h, Drude.update_e, Drude.update_h) == _OWN)
 
-    def update_core_e(self):
+    def update_core_e(self, drude=None):
         f = self.mainf
         ces = f.ces if f.ce_on else (None, None, None)
         mats = (None,) * 4
         if f.ce_on and f.ce_mat is not None:
             mats = (*f.ptrs(f.ce_mat), f.ce_lut.data_ptr())
         _lib.call("mifdtd_half_e", f.nx, f.ny, f.nz_pitch, f.pad, self._descE, *[t.data_ptr() for t in f.ehs],
-                  *f.ptrs(ces), *mats, f.stream.cuda_stream)
+                  *f.ptrs(ces), *mats, None if drude is None else drude.region(), f.stream.cuda_stream)
 
     def update_core_h(self):
         f = self.mainf
@@ -179,8 +186,8 @@ class Cpml:
                   *f.ptrs(chs), f.stream.cuda_stream)
 
 
-# The update methods that a joined half step stands for (joins_core).
-_OWN = (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h)
+# The update methods that a joined half step stands for (joins).
+_OWN = (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h, Drude.update_e, Drude.update_h)
 
 _FACE_E = {0: ("ey", "ez", "hy", "hz", 1, 2), 1: ("ex", "ez", "hx", "hz", 0, 2), 2: ("ex", "ey", "hx", "hy", 0, 1)}
 

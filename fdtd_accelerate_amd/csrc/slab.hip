@@ -1,7 +1,7 @@
-// Slab-ordered step: per time step, for each slab of consecutive x planes, one E pass
-// (core E + CPML-E + E sources + E probes) then one H pass (core H + CPML-H + H sources
-// + H probes) over that slab, in place; by default the slab is the whole grid (two
-// launches per step).  Smaller slabs keep a slab's E/H planes in the last-level cache
+// The whole-grid passes (whole_pass.hpp) and the slab-ordered step: per time step, for each
+// slab of consecutive x planes, one E pass (core E + CPML-E + E sources + E probes) then one
+// H pass (core H + CPML-H + H sources + H probes) over that slab, in place; by default the
+// slab is the whole grid (two launches per step).  Smaller slabs keep a slab's E/H planes in the last-level cache
 // between its two passes, which on MI355X was measured to gain less than the extra
 // launches cost.
 //

@@ -259,10 +259,11 @@ __device__ __forceinline__ const T &first_kernel_arg()
     return *(const T *)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
-// Both passes issue the quad's core loads (fields, neighbours, CE) and the psi of its
-// first x or y face together, then compute; the psi of a second face (the edges along z)
-// and of the z faces follow after the core update.  That keeps the passes at 6 waves per
-// SIMD; holding all six psi quads across the update took 120 VGPRs, 4 waves per SIMD.
+// Both passes issue the quad's core loads (fields, neighbours, CE), the psi of its first x
+// or y face and the psi of its z-slab cells together, then compute; the psi of a second face
+// (the edges along z) follows after the core update.  92-104 and 96 VGPRs, 4 and 5 waves per
+// SIMD.  Holding all six psi quads across the update took 120 and spilled scalars; loading the
+// z faces after the update kept 6 waves and was slower (160^3 step 74 us against 64).
 
 // How CE reaches the E update: the constant 0.5, three float arrays, or three uint8
 // material-index arrays into a 3 x 256 float table (same float values, so the products

@@ -801,6 +801,17 @@ int mifdtd_update_h(int nx, int ny, int nz_pitch, int pad, const float *ex, cons
     return launch_core(false, nx, ny, nz_pitch, pad, {ex, ey, ez, hx, hy, hz}, chx, chy, chz, to_stream(stream));
 }
 
+static int check_drude(const mifdtd_drude &d, int nx, int ny, int nzp)
+{
+    for (int c = 0; c < 3; c++)
+        if (!d.j[c] || !d.cja[c] || !d.cjb[c]) return fail(MIFDTD_ENULL, "Drude array is NULL");
+    if (d.li < 1 || d.lj < 1 || d.lk < 1 || d.i0 < 0 || d.j0 < 0 || d.k0 < 0 || d.i0 + d.li > nx || d.j0 + d.lj > ny ||
+        d.k0 + d.lk > nzp)
+        return fail(MIFDTD_EINVAL, "Drude region outside the grid");
+    if ((unsigned long long)d.li * d.lj * d.lk >= (1ull << 32) - kBlock) return fail(MIFDTD_ERANGE, "Drude region too large");
+    return 0;
+}
+
 // The CPML of one half step for the whole-grid passes: psi packed (MIFDTD_PSI_PACKED: psi1 and
 // psi2 of each face in one buffer) with both faces of an axis or none.  False: not of this form.
 static bool packed_cpml(const mifdtd_cpml_half &h, int nx, int ny, int nzp, bool e_half, SCpml &cp)
@@ -840,7 +851,7 @@ static bool packed_cpml(const mifdtd_cpml_half &h, int nx, int ny, int nzp, bool
 int mifdtd_half_e(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, float *ex, float *ey, float *ez,
                   const float *hx, const float *hy, const float *hz, const float *cex, const float *cey,
                   const float *cez, const unsigned char *mat_x, const unsigned char *mat_y,
-                  const unsigned char *mat_z, const float *lut, mifdtd_stream_t stream)
+                  const unsigned char *mat_z, const float *lut, const mifdtd_drude *drude, mifdtd_stream_t stream)
 {
     if (!cp) return fail(MIFDTD_ENULL, "cpml descriptor is NULL");
     if (int rc = check_cpml(nx, ny, nzp, pad, cp->npml, cp->b, cp->a)) return rc;
@@ -851,14 +862,37 @@ int mifdtd_half_e(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, 
     const bool table = mat_x || mat_y || mat_z || lut;
     if (table)
         if (int rc = check_mats(mats, lut)) return rc;
+    const float *const ce[3] = {cex, cey, cez};
     SCpml sc;
-    if (!packed_cpml(*cp, nx, ny, nzp, true, sc)) {
-        const int rc = table ? mifdtd_update_e_lut(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, mat_x, mat_y, mat_z, lut, stream)
-                             : mifdtd_update_e(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, cex, cey, cez, stream);
+    SDrude dr{};
+    bool one = packed_cpml(*cp, nx, ny, nzp, true, sc);
+    if (drude) {
+        if (int rc = check_drude(*drude, nx, ny, nzp)) return rc;
+        dr.i0 = drude->i0;
+        dr.i1 = drude->i0 + drude->li - 1;
+        dr.j0 = drude->j0;
+        dr.j1 = drude->j0 + drude->lj - 1;
+        dr.k0 = drude->k0;
+        dr.k1 = drude->k0 + drude->lk - 1;
+        dr.lj = drude->lj;
+        dr.lk = drude->lk;
+        for (int c = 0; c < 3; c++) {
+            dr.jin[c] = dr.jout[c] = drude->j[c];
+            dr.a[c] = drude->cja[c];
+            dr.b[c] = drude->cjb[c];
+            one = one && aligned16(dr.jin[c]) && aligned16(dr.a[c]) && aligned16(dr.b[c]);
+        }
+    }
+    if (!one) {
+        int rc = table ? mifdtd_update_e_lut(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, mat_x, mat_y, mat_z, lut, stream)
+                       : mifdtd_update_e(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, cex, cey, cez, stream);
+        float *const e[3] = {ex, ey, ez};
+        if (!rc && drude)
+            rc = mifdtd_drude_e(e, ce, drude->j, drude->cja, drude->cjb, nx, ny, nzp, drude->i0, drude->j0, drude->k0,
+                                drude->li, drude->lj, drude->lk, stream);
         return rc ? rc : mifdtd_cpml_e(nx, ny, nzp, pad, cp, ex, ey, ez, hx, hy, hz, cex, cey, cez, stream);
     }
     WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 4) ? cp->npml : 0, f, to_stream(stream));
-    const float *const ce[3] = {cex, cey, cez};
     for (int c = 0; c < 3; c++) {
         w.F.ce[c] = ce[c];
         w.F.cm[c] = mats[c];
@@ -866,7 +900,7 @@ int mifdtd_half_e(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, 
     w.F.lut = lut;
     w.cem = table ? kCeTable : cex ? kCeArrays : kCeConst;
     w.cp = sc;
-    return whole_e(w, no_aux(), nullptr, nullptr);
+    return whole_e(w, no_aux(), drude ? &dr : nullptr, nullptr);
 }
 
 int mifdtd_half_h(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, const float *ex, const float *ey,
@@ -1040,11 +1074,10 @@ int mifdtd_drude_e(float *const e[3], const float *const ce[3], float *const j[3
 {
     if (!e || !j || !cja || !cjb) return fail(MIFDTD_ENULL, "Drude argument is NULL");
     for (int c = 0; c < 3; c++)
-        if (!e[c] || !j[c] || !cja[c] || !cjb[c]) return fail(MIFDTD_ENULL, "Drude array is NULL");
-    if (li < 1 || lj < 1 || lk < 1 || i0 < 0 || j0 < 0 || k0 < 0 || i0 + li > nx || j0 + lj > ny || k0 + lk > nz_pitch)
-        return fail(MIFDTD_EINVAL, "Drude region outside the grid");
+        if (!e[c]) return fail(MIFDTD_ENULL, "Drude array is NULL");
+    const mifdtd_drude d{i0, j0, k0, li, lj, lk, {j[0], j[1], j[2]}, {cja[0], cja[1], cja[2]}, {cjb[0], cjb[1], cjb[2]}};
+    if (int rc = check_drude(d, nx, ny, nz_pitch)) return rc;
     const unsigned long long tot = (unsigned long long)li * lj * lk;
-    if (tot >= (1ull << 32) - kBlock) return fail(MIFDTD_ERANGE, "Drude region too large");
     const float *c0 = ce ? ce[0] : nullptr, *c1 = ce ? ce[1] : nullptr, *c2 = ce ? ce[2] : nullptr;
     const unsigned g = (unsigned)((tot + kBlock - 1) / kBlock);
     k_drude_e<<<g, kBlock, 0, to_stream(stream)>>>(e[0], e[1], e[2], c0, c1, c2, j[0], j[1], j[2], cja[0], cja[1], cja[2],

@@ -56,6 +56,14 @@ class Drude:
         self.J = [torch.zeros(shape, dtype=torch.float32, device=dev) for _ in range(3)]
         fields.append_instance(self)
 
+    def region(self):
+        d = _lib.DrudeRegion()
+        d.region[:] = (*self.pt0, *self.shape)
+        d.j[:] = [t.data_ptr() for t in self.J]
+        d.cja[:] = [t.data_ptr() for t in self.cja]
+        d.cjb[:] = [t.data_ptr() for t in self.cjb]
+        return d
+
     def update_e(self):
         f = self.mainf
         P3 = ctypes.c_void_p * 3

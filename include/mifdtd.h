@@ -192,16 +192,23 @@ int mifdtd_cpml_h(int nx, int ny, int nz_pitch, int pad, const mifdtd_cpml_half 
                   mifdtd_stream_t stream);
 
 /* The core update and the CPML of one half step together, as update_e (with the material
- * indices where lut is given) followed by mifdtd_cpml_e, and update_h by mifdtd_cpml_h: one
- * pass over the grid where the psi arrays are packed (MIFDTD_PSI_PACKED) with both faces of
- * an axis or none, else those two calls.  No reference counterpart (there each face is a
- * call of its own). */
+ * indices where lut is given), mifdtd_drude_e where drude is given, then mifdtd_cpml_e, and
+ * update_h followed by mifdtd_cpml_h: one pass over the grid where the psi arrays are packed
+ * (MIFDTD_PSI_PACKED) with both faces of an axis or none (and the Drude arrays 16-byte
+ * aligned), else those calls.  No reference counterpart (there each face is a call of its
+ * own). */
+typedef struct {
+    int i0, j0, k0, li, lj, lk;    /* the region, as mifdtd_drude_e takes it */
+    float *j[3];
+    const float *cja[3], *cjb[3];
+} mifdtd_drude;
 int mifdtd_half_e(int nx, int ny, int nz_pitch, int pad, const mifdtd_cpml_half *cp,
                   float *ex, float *ey, float *ez,
                   const float *hx, const float *hy, const float *hz,
                   const float *cex, const float *cey, const float *cez,
                   const unsigned char *mat_x, const unsigned char *mat_y,
-                  const unsigned char *mat_z, const float *lut, mifdtd_stream_t stream);
+                  const unsigned char *mat_z, const float *lut, const mifdtd_drude *drude,
+                  mifdtd_stream_t stream);
 int mifdtd_half_h(int nx, int ny, int nz_pitch, int pad, const mifdtd_cpml_half *cp,
                   const float *ex, const float *ey, const float *ez,
                   float *hx, float *hy, float *hz,

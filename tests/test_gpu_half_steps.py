@@ -51,6 +51,31 @@ def test_half_steps_equal_separate_kernels(ns, npml, coeff, faces, index):
         assert torch.equal(ca.psiH_buf.view(torch.int32), cb.psiH_buf.view(torch.int32))
 
 
+@pytest.mark.parametrize("ns,npml,coeff,faces,index,box", [
+    ((18, 17, 33), 4, "", ALL, False, ((0, 0, 0), (17, 16, 32))),          # the whole grid, walls and slabs
+    ((21, 75, 61), 5, "eh", ALL, False, ((3, 2, 7), (19, 70, 50))),        # rows off the 16-byte lines
+    ((26, 130, 57), 12, "e", ALL, True, ((5, 60, 4), (6, 60, 55))),        # one row
+    ((19, 80, 48), 5, "e", ("", "", "fb"), False, ((2, 1, 8), (17, 78, 39))),
+    ((20, 26, 45), 5, "e", ("fb", "b", "fb"), False, ((4, 4, 5), (9, 20, 30))),  # separate calls
+])
+def test_half_steps_with_a_drude_region(ns, npml, coeff, faces, index, box):
+    from fdtd_accelerate_amd import Drude
+    out = []
+    for split in (False, True):
+        f, cp = _fields(ns, npml, coeff, faces, index, split)
+        d = Drude(f, *box, 0.5, 0.05)
+        rng = np.random.default_rng(8)
+        for t in d.J:
+            t.copy_(torch.from_numpy(rng.standard_normal(tuple(t.shape)).astype(np.float32)))
+        assert f._joined() == (0 if split else 3)
+        for _ in range(3):
+            f.update_e()
+            f.update_h()
+        out.append([*f.ehs, *d.J, cp.psiE_buf, cp.psiH_buf])
+    for x, y in zip(*out):
+        assert torch.equal(x.view(torch.int32), y.view(torch.int32))
+
+
 def test_replaced_updates_run_by_themselves():
     """An update method that a program replaces, on an instance or in a subclass, is called."""
     from fdtd_accelerate_amd import Core, Fields
