@@ -197,8 +197,8 @@ static int check_coeffs(const float *c0, const float *c1, const float *c2)
     return 0;
 }
 
-// The whole grid's half step.  In the whole-grid thread order (row_quads.hpp) the E + H core
-// of a cube ran, against a thread per quad in plain order: 160^3 67.6 -> 53.5 us, 192^3
+// The whole grid's half step in the thread order of row_quads.hpp.  The E + H core of a cube
+// against a thread per quad in memory order, from Python: 160^3 67.6 -> 53.5 us, 192^3
 // 111 -> 88, 256^3 269 -> 260.
 static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_z, const float *const (&f)[6], hipStream_t st)
 {
@@ -214,10 +214,29 @@ static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_z, const f
     return w;
 }
 
+static int launch_range(bool e_half, int nx, int ny, int nzp, int pad, const float *const (&f)[6], const float *c0,
+                        const float *c1, const float *c2, hipStream_t st, long long idx0, long long nmax);
+
+// Where the core alone runs in memory order: planes of too few rows for stripes, and planes of
+// a multiple of 8 blocks, whose rows fall to the same XCD in every plane by themselves.  E + H
+// on cold arrays, whole order / memory order: 100x70x200 24.8 / 23.9 us, 200x71x130 32.4 /
+// 30.5, 120x64x128 17.3 / 15.6, 400x40x400 87.3 / 86.1; 128^3 31.5 / 29.8, but 256^3 218.8 /
+// 224.3 (2^22 quads); 200x128x100 34.3 / 39.9.  Below 2^17 quads the launches bound, and the
+// whole-grid kernels' few structures are cheaper to pass than 18 arguments (64^3, from Python,
+// 14.8 / 17.0).
+static bool memory_order(int nx, int ny, int Q)
+{
+    const unsigned long long quads = (unsigned long long)nx * ny * Q;
+    if (quads < (1ull << 17)) return false;
+    return ny < (int)kStripeMinRows || (quads < (1ull << 21) && (long long)ny * Q % (8 * kBlock) == 0);
+}
+
 static int launch_core(bool e_half, int nx, int ny, int nzp, int pad, const float *const (&f)[6], const float *c0,
                        const float *c1, const float *c2, hipStream_t st)
 {
     if (int rc = check_grid(nx, ny, nzp, pad)) return rc;
+    if (memory_order(nx, ny, nzp / 4))
+        return launch_range(e_half, nx, ny, nzp, pad, f, c0, c1, c2, st, 0, (long long)nx * ny * nzp);
     if (int rc = check_fields(f)) return rc;
     if (int rc = check_coeffs(c0, c1, c2)) return rc;
     WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, 0, f, st);
