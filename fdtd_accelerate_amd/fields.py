@@ -188,7 +188,7 @@ class Fields:
     # A Cpml right behind the Core, or behind the Core and one Drude region, takes their update
     # into its own pass: a step of 128^3 cells with CPML 10 63 -> 40 us, 300 x 211 x 331 with
     # CPML 12 459 -> 364, 1024^3 17.4 -> 15.0 ms, 256^3 with CPML 10 and a Drude box of 128^3
-    # 416 -> 336 us, against the core, the region and one launch per axis of faces.
+    # 416 -> 341 us, against the core, the region and one launch per axis of faces.
     def _joined(self):
         """How many instances from the first on one pass takes: 0, 2 or 3."""
         insts = self.instance_list
