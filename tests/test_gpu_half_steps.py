@@ -33,7 +33,8 @@ def _fields(ns, npml, coeff, faces, index, split, seed=3):
 
 @pytest.mark.parametrize("ns,npml,coeff,faces,index", [
     ((2, 2, 3), 0, "", ALL, False), ((3, 72, 16), 0, "eh", ALL, False), ((5, 73, 61), 0, "h", ALL, False),
-    ((4, 100, 260), 0, "e", ALL, True), ((18, 17, 33), 4, "", ALL, False), ((21, 75, 61), 5, "eh", ALL, False),
+    ((4, 100, 260), 0, "e", ALL, True), ((60, 70, 127), 0, "eh", ALL, False), ((64, 128, 64), 0, "h", ALL, False),
+    ((18, 17, 33), 4, "", ALL, False), ((21, 75, 61), 5, "eh", ALL, False),
     ((26, 130, 57), 12, "e", ALL, True), ((20, 22, 64), 6, "h", ALL, False), ((19, 80, 48), 5, "e", ("", "", "fb"), False),
     ((17, 74, 131), 4, "e", ("fb", "", ""), True), ((24, 28, 50), 6, "eh", ("fb", "fb", ""), False),
     ((20, 76, 45), 5, "e", ("fb", "b", "fb"), True), ((20, 20, 40), 3, "", ("f", "", "b"), False),
