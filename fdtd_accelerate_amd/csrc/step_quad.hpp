@@ -20,7 +20,7 @@ struct SCpml {
     float *pe, *ph;          // packed psi E / psi H
     float *pe_out;           // where the E pass stores psi E (pe for in-place updates)
     size_t sX, sY, sZ;
-    __device__ __forceinline__ size_t off(int f, int c) const
+    __host__ __device__ __forceinline__ size_t off(int f, int c) const
     {
         const int ax = f >> 1, sd = f & 1;
         if (ax == 0) return (size_t)(2 * sd + c) * sX;
@@ -196,7 +196,7 @@ struct SGeom {
     RowQuads m;        // thread -> quad order over the slab's rows (whole-grid passes)
 };
 
-__device__ __forceinline__ int sslab_e(int q, int n_e, int npml, int &side, int &p)
+__host__ __device__ __forceinline__ int sslab_e(int q, int n_e, int npml, int &side, int &p)
 {
     side = 0;
     p = 0;
@@ -204,7 +204,7 @@ __device__ __forceinline__ int sslab_e(int q, int n_e, int npml, int &side, int 
     if (q >= n_e - 1 - npml && q < n_e - 1) { side = 1; p = q - (n_e - 1 - npml); return npml + 1 + p; }
     return -1;
 }
-__device__ __forceinline__ int sslab_h(int q, int n_e, int npml, int &side, int &p)
+__host__ __device__ __forceinline__ int sslab_h(int q, int n_e, int npml, int &side, int &p)
 {
     side = 0;
     p = 0;
@@ -328,15 +328,30 @@ inline void aux_box(SAux &a)
         aux_cover(a, a.prb.i[n], a.prb.i[n], a.prb.j[n], a.prb.j[n], a.prb.k[n], a.prb.k[n]);
 }
 
+// Table entry (t > 0: in a slab) and psi1 offset of cell k0+l of a z-slab quad; psi2 follows sZ
+// later.  A cell in no slab takes the first cell of the row in the slab that the quad meets:
+// its load, whose value is not used, stays inside the z faces, the only part of the buffer
+// that a caller with CPML on z alone has to provide.
+template <bool E>
+__host__ __device__ __forceinline__ int zface_at(const SCpml &cp, int i, int j, int k0, int l, int ny, int nz, size_t &o)
+{
+    int zs, zp, t = E ? sslab_e(k0 + l, nz, cp.npml, zs, zp) : sslab_h(k0 + l, nz, cp.npml, zs, zp);
+    if (!E && k0 + l == 0) t = -1;  // the wall
+    if (t <= 0) {
+        zs = k0 >= cp.npml;
+        zp = 0;
+    }
+    o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * cp.npml + zp;
+    return t;
+}
+
 // z-face psi and table entries of a quad's cells, loaded ahead of the update: loads that
 // follow the previous cell's psi store are four memory round trips in a row.
 struct ZFace {
     float q1[4], q2[4], b[4], a[4];
-    // cell l: psi1 at p (psi2 s2 after it) and table entry t, where the cell is in the slab (t > 0)
-    __device__ __forceinline__ void load(int l, int t, const float *psi, size_t off, size_t s2, const float *tb,
+    __device__ __forceinline__ void load(int l, int t, const float *psi, size_t o, size_t s2, const float *tb,
                                          const float *ta)
     {
-        const size_t o = t > 0 ? off : 0;
         const int e = t > 0 ? t : 0;
         q1[l] = psi[o];
         q2[l] = psi[o + s2];
@@ -413,9 +428,9 @@ __device__ __forceinline__ void e_quad_at(
         if (zq) {
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                int zs, zp;
-                const int t = sslab_e(k0 + l, nz, npml, zs, zp);
-                z.load(l, t, cp.pe, cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp, cp.sZ, cp.bE, cp.aE);
+                size_t o;
+                const int t = zface_at<true>(cp, i, j, k0, l, ny, nz, o);
+                z.load(l, t, cp.pe, o, cp.sZ, cp.bE, cp.aE);
             }
         }
     }
@@ -529,9 +544,8 @@ __device__ __forceinline__ void e_quad_at(
         if (zq) {  // psi1: ex, psi2: ey
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                int zs, zp;
-                const bool on = sslab_e(k0 + l, nz, npml, zs, zp) > 0;
-                const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
+                size_t o;
+                const bool on = zface_at<true>(cp, i, j, k0, l, ny, nz, o) > 0;
                 if (on && jy) {
                     const float tt = z.b[l] * z.q1[l] + z.a[l] * (y1[l] - hy0.v[l]);
                     cp.pe_out[o] = tt;
@@ -630,10 +644,9 @@ __device__ __forceinline__ void h_quad_at(
         if (zq) {
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                int zs, zp;
-                const int t = sslab_h(k0 + l, nz, npml, zs, zp);
-                z.load(l, k0 + l > 0 ? t : -1, cp.ph, cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp, cp.sZ, cp.bH,
-                       cp.aH);  // k = 0 is the wall
+                size_t o;
+                const int t = zface_at<false>(cp, i, j, k0, l, ny, nz, o);
+                z.load(l, t, cp.ph, o, cp.sZ, cp.bH, cp.aH);
             }
         }
     }
@@ -735,9 +748,8 @@ __device__ __forceinline__ void h_quad_at(
         if (zq) {  // psi1: hx, psi2: hy
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                int zs, zp;
-                const bool on = sslab_h(k0 + l, nz, npml, zs, zp) > 0 && k0 + l > 0;
-                const size_t o = cp.off(4 + zs, 0) + ((size_t)i * ny + j) * npml + zp;
+                size_t o;
+                const bool on = zface_at<false>(cp, i, j, k0, l, ny, nz, o) > 0;
                 if (on && jp) {
                     const float tt = z.b[l] * z.q1[l] + z.a[l] * (ey0.v[l] - ym[l]);
                     cp.ph[o] = tt;
