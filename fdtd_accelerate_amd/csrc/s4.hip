@@ -288,9 +288,10 @@ __global__ __launch_bounds__(S4B) void k_s4_e(SAux, S4Geom g, S4Cpml cp, float d
         sapply_src(aux.src, 1, k, j, i0, e1);
         sapply_src(aux.src, 2, k, j, i0, e2);
     }
-    st4(ex + id, e0);
-    st4(ey + id, e1);
-    st4(ez + id, e2);
+    // (rows that the stage does not write are left alone, as in the passes of step_quad.hpp)
+    if (rx || near) st4(ex + id, e0);
+    if (ry || near) st4(ey + id, e1);
+    if (rz || near) st4(ez + id, e2);
     if (near) {
         sprobe(aux.prb, 0, k, j, i0, e0);
         sprobe(aux.prb, 1, k, j, i0, e1);
@@ -447,9 +448,9 @@ __global__ __launch_bounds__(S4B) void k_s4_h(SAux, S4Geom g, S4Cpml cp, float c
     }
     const SAux &aux = first_kernel_arg<SAux>();
     const bool near = aux.near(k, j, i0);
-    st4(hx + id, h0);
-    st4(hy + id, h1);
-    st4(hz + id, h2);
+    if (rx) st4(hx + id, h0);
+    if (ry) st4(hy + id, h1);
+    if (rz) st4(hz + id, h2);
     if (near) {
         sprobe(aux.prb, 3, k, j, i0, h0);
         sprobe(aux.prb, 4, k, j, i0, h1);

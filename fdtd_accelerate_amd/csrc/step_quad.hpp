@@ -568,10 +568,12 @@ __device__ __forceinline__ void e_quad_at(
     if (TF) tfsf_quad(*tf, 0, i, j, k0, e0, e1, e2);
 
     // --------------------------------------------------------------- stores
-    // (unchanged lanes and wall rows store back the value they loaded)
-    st4(exo + id, e0);
-    st4(eyo + id, e1);
-    st4(ezo + id, e2);
+    // (unchanged lanes store back the value they loaded; in place, a row or plane that nothing
+    // updates is left alone, so that another stream may write it while the pass runs)
+    const bool all = exo != exi || near || drow || TF;
+    if (all || jy) st4(exo + id, e0);
+    if (all || ix) st4(eyo + id, e1);
+    if (all || (ix && jy)) st4(ezo + id, e2);
     if (drow) {
         drude_store(*dr, 0, i, j, k0, jn0);
         drude_store(*dr, 1, i, j, k0, jn1);
@@ -772,9 +774,10 @@ __device__ __forceinline__ void h_quad_at(
     if (tf) tfsf_quad(*tf, 3, i, j, k0, h0, h1, h2);
 
     // --------------------------------------------------------------- stores
-    st4(hxo + id, h0);
-    st4(hyo + id, h1);
-    st4(hzo + id, h2);
+    const bool all = hxo != hxi || near || tf;
+    if (all || jp) st4(hxo + id, h0);
+    if (all || ip) st4(hyo + id, h1);
+    if (all || (ip && jp)) st4(hzo + id, h2);
     if (near) {
         sprobe(aux.prb, 3, i, j, k0, h0, prow);
         sprobe(aux.prb, 4, i, j, k0, h1, prow);

@@ -58,3 +58,91 @@ def test_psi_of_the_z_faces_alone(ns, npml):
         out.append([*f.ehs, *psi])
     for x, y in zip(*out):
         assert torch.equal(x.view(torch.int32), y.view(torch.int32))
+
+
+def _shared(shape, first, second):
+    """Arrays first and second of one allocation, the last plane of the one the first plane of
+    the other."""
+    n, plane = shape[0], shape[1] * shape[2]
+    block = torch.empty((2 * n - 1) * plane, device="cuda")
+    a, b = block[:n * plane].view(shape), block[(n - 1) * plane:].view(shape)
+    a.copy_(first)
+    b.copy_(second)
+    return a, b
+
+
+def _check_shared(call, arrays, out, inner, written):
+    """``call`` on the six arrays, with the last plane of out[0] being the first plane of
+    out[1]: it leaves one of the two alone, so both orders of writing give the plane of the
+    array ``written``."""
+    want = [t.clone() for t in arrays]
+    call(want)
+    got = [t.clone() for t in arrays]
+    got[out[0]], got[out[1]] = _shared(arrays[0].shape, arrays[out[0]], arrays[out[1]])
+    keep = -1 if written == 0 else 0
+    if written == 0:  # the first array's last plane is the one that is updated
+        got[out[0]][-1].copy_(arrays[out[0]][-1])
+    call(got)
+    torch.cuda.synchronize()
+    same = lambda x, y: torch.equal(x.view(torch.int32), y.view(torch.int32))
+    assert same(got[out[written]][keep], want[out[written]][keep])
+    for c in inner:
+        x, y = got[c], want[c]
+        if c == out[0]:
+            x, y = x[:-1], y[:-1]
+        elif c == out[1]:
+            x, y = x[1:], y[1:]
+        assert same(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ns,npml", [((6, 80, 20), 0), ((8, 30, 64), 0), ((24, 75, 40), 5), ((300, 80, 256), 0)])
+def test_planes_not_updated_are_not_written(ns, npml):
+    """update_e leaves ey of the last plane alone and update_h hy of the first, also with the
+    CPML in the same pass: a plane that is such a one of one array and an updated one of
+    another ends as the update leaves it."""
+    from fdtd_accelerate_amd import Core, Fields, _lib
+    from fdtd_accelerate_amd.cpml import Cpml
+    f = Fields(*ns, coeff_use="")
+    Core(f)
+    cp = Cpml(f, npml) if npml else None
+    torch.manual_seed(4)
+    arrays = [torch.randn(tuple(f.ns_pitch), device=f.device) for _ in range(6)]
+    st, N, grid = torch.cuda.current_stream().cuda_stream, (None,) * 3, (*f.ns_pitch, f.pad)
+
+    def half(e):
+        def call(a):
+            p = [t.data_ptr() for t in a]
+            if cp is None:
+                _lib.call("mifdtd_update_e" if e else "mifdtd_update_h", *grid, *p, *N, st)
+            elif e:
+                cp.reset()
+                _lib.call("mifdtd_half_e", *grid, cp._descE, *p, *N, *N, None, None, st)
+            else:
+                cp.reset()
+                _lib.call("mifdtd_half_h", *grid, cp._descH, *p, *N, st)
+        return call
+
+    torch.cuda.synchronize()
+    _check_shared(half(True), arrays, (1, 0), (0, 1, 2), 1)   # ey's last plane, ex's first
+    _check_shared(half(False), arrays, (3, 4), (3, 4, 5), 0)  # hx's last plane, hy's first
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(40, 80, 12), (16, 20, 9)])
+def test_s4_rows_not_updated_are_not_written(n):
+    """The 4th-order stages leave the last z plane alone: the same with that of ex and the
+    first of ez, and of hx and hz."""
+    from fdtd_accelerate_amd import _lib
+    torch.manual_seed(5)
+    arrays = [torch.randn(n[2], n[1], n[0], device="cuda") for _ in range(6)]
+    st, N = torch.cuda.current_stream().cuda_stream, (None,) * 3
+
+    def stage(name):
+        def call(a):
+            _lib.call(name, *n, 0.3, *[t.data_ptr() for t in a], *N, 0.03, st)
+        return call
+
+    torch.cuda.synchronize()
+    _check_shared(stage("mifdtd_s4_update_e"), arrays, (0, 2), (0, 1, 2), 1)
+    _check_shared(stage("mifdtd_s4_update_h"), arrays, (3, 5), (3, 4, 5), 1)
