@@ -115,12 +115,18 @@ inline void stripe_rows(RowQuads &m, unsigned ny, int npml)
     while (x <= 8) m.jx[x++] = ny;
 }
 
+// Rows per plane of the largest stripe.
+inline unsigned long long stripe_max(const RowQuads &m)
+{
+    unsigned S = 0;
+    for (unsigned x = 0; x < m.ns; ++x) S = m.jx[x + 1] - m.jx[x] > S ? m.jx[x + 1] - m.jx[x] : S;
+    return S;
+}
+
 // Blocks of a pass (a multiple of the stripes; the stripes' own counts differ by a row a plane).
 inline unsigned long long row_quads_blocks(const RowQuads &m)
 {
-    unsigned long long S = 0;
-    for (unsigned x = 0; x < m.ns; ++x) S = m.jx[x + 1] - m.jx[x] > S ? m.jx[x + 1] - m.jx[x] : S;
-    return (m.planes * S + m.R - 1) / m.R * m.bpg * m.ns;
+    return (m.planes * stripe_max(m) + m.R - 1) / m.R * m.bpg * m.ns;
 }
 
 // The order for `planes` planes of ny rows of Q quads (nz cells, npml-cell z slabs; npml =
@@ -166,7 +172,8 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     m.m_b = reciprocal(row_quads_blocks(m) + kStripes, m.bpg);
     for (unsigned x = 0; x < 8; ++x) {
         const unsigned S = m.jx[x + 1] - m.jx[x];
-        m.m_s[x] = reciprocal((unsigned long long)planes * S + 64 * m.R, S);
+        // (the largest stripe's blocks: those past this stripe's rows divide by S too)
+        m.m_s[x] = reciprocal(planes * stripe_max(m) + 64 * m.R, S);
     }
     return m;
 }
