@@ -10,7 +10,8 @@ and the objective
 
 The gradient needs, of each step, the curl of H on the design box before it.
 ``forward(eps)`` runs the steps once and stores these curls for as many of the last steps
-as the memory set aside for them holds (``_curl_budget``); of the segments of ``ckpt``
+as there is memory for (``curl_bytes``: no more in all than checkpoints of every segment
+would take, or a share of the free memory); of the segments of ``ckpt``
 steps before those it keeps a checkpoint of the full state (fields and psi), and of the
 objective window the monitor-plane E.  ``backward()`` walks the segments in reverse: where
 the curls are not stored it restores a checkpoint and recomputes the segment with its
@@ -29,6 +30,19 @@ from . import _lib
 from .fused import SlabStepper
 from .sim import YeeSim
 from .sources import gaussian_pulse
+
+
+def curl_bytes(nsteps, ckpt, state, curl, room):
+    """Bytes of curls (``curl`` a step) to store for as many of the last steps as there is
+    memory for: whole segments of ``ckpt`` steps, such that the curls, the checkpoints
+    (``state`` each) of the segments before them and the buffer to recompute one of these take
+    no more than checkpoints of all segments with that buffer, or than ``room``."""
+    limit = max(-(-nsteps // ckpt) * state + ckpt * curl, room)
+    for kept in range(0, nsteps, ckpt):
+        curls = (nsteps - kept) * curl
+        if curls + kept // ckpt * state + (ckpt * curl if kept else 0) <= limit:
+            return curls
+    return 0
 
 
 class DesignProblem:
@@ -92,12 +106,16 @@ class DesignProblem:
         torch.stack([f.ehs[c][self.monitor] for c in range(3)], out=out)  # (3, ny, nzp)
 
     def _curl_budget(self):
-        """Bytes of curls that a forward run may hold: what the checkpoints of all segments
-        would take, or 1/32 of the GPU's memory (9 GB of 288) where that is more.  A run of
-        160^3 cells, 800 steps and a 64^3 box takes 2.5 GB of curls or 2.0 GB of checkpoints
-        and recomputes nothing: 193 -> 135 ms for forward and backward."""
-        state = sum(t.numel() * t.element_size() for t in self._state())
-        return max(-(-self.nsteps // self.ckpt) * state, torch.cuda.get_device_properties(self.dev).total_memory // 32)
+        """Bytes of curls that a forward run may hold (curl_bytes), with the room left on the
+        GPU beside what backward() allocates.  A run of 160^3 cells, 800 steps and a 64^3 box
+        takes 2.5 GB of curls or 2.0 GB of checkpoints and recomputes nothing: 193 -> 135 ms
+        for forward and backward."""
+        size = lambda ts: sum(t.numel() * t.element_size() for t in ts)
+        curl = 12 * int(np.prod(self.box[3:]))
+        free, total = torch.cuda.mem_get_info(self.dev)
+        free += torch.cuda.memory_reserved(self.dev) - torch.cuda.memory_allocated(self.dev)
+        state = size(self._state())
+        return curl_bytes(self.nsteps, self.ckpt, state, curl, min(total // 32, (free - state - 2 * curl) // 2))
 
     def _alloc_curls(self):
         """Curls of the steps after ``self.kept`` (a segment start), or None and no such step."""
@@ -117,13 +135,21 @@ class DesignProblem:
     def forward(self, eps):
         """Run the simulation for eps (design box values); returns J (float)."""
         self._set_eps(eps)
+        try:
+            return self._forward(True)
+        except torch.OutOfMemoryError:
+            if self.curls is None:
+                raise
+        return self._forward(False)
+
+    def _forward(self, keep_curls):
         self._reset()
         self.ckpts = {}
         nwin = self.nsteps - self.n0 + 1
         f = self.sim.fields
-        self.curls = None  # the last run's, before the new ones are allocated
+        self.planes = self.curls = None  # the last run's, before the new ones are allocated
         self.planes = torch.empty((nwin, 3, f.ny, f.nz_pitch), dtype=torch.float32, device=self.dev)
-        self.kept, self.curls = self._alloc_curls()
+        self.kept, self.curls = self._alloc_curls() if keep_curls else (self.nsteps, None)
         n = 0
         while n < self.nsteps:
             if n < self.kept and n % self.ckpt == 0:
@@ -144,6 +170,16 @@ class DesignProblem:
     # ------------------------------------------------------------------ backward
     def backward(self):
         """dJ/deps on the design box (float64 tensor, box shape) of the last forward."""
+        try:
+            return self._backward()
+        except torch.OutOfMemoryError:
+            if self.curls is None:
+                raise
+        self._set_eps(self._eps)
+        self._forward(False)  # the same run with checkpoints in place of the curls
+        return self._backward()
+
+    def _backward(self):
         f = self.sim.fields
         cp = self.sim.cpml
         i0, j0, k0, di, dj, dk = self.box
