@@ -161,28 +161,11 @@ __device__ __forceinline__ void h_pair(const GridF64 &g, const PairAt &r, const 
 }
 
 // Thread -> pair: the whole grid in the order of row_quads.hpp (a stripe of every plane per
-// XCD, so that the neighbour rows and planes are hits of its L2), or the pairs [p0, p1) in
-// memory order (the split form).
-struct OrderF64 {
-    RowQuads m;
-    unsigned p0, p1, P;
-};
-template <bool RANGE>
-__device__ __forceinline__ bool pair_at(const GridF64 &g, const OrderF64 &o, PairAt &r)
+// XCD, so that the neighbour rows and planes are hits of its L2).
+__device__ __forceinline__ bool pair_at(const RowQuads &m, PairAt &r)
 {
     const int lane = threadIdx.x & 63;
-    if (RANGE) {
-        const unsigned f = o.p0 + blockIdx.x * kBlockD + threadIdx.x;
-        if (f >= o.p1) return false;
-        const unsigned row = f / o.P;
-        r.k0 = (int)(f - row * o.P) * 2;
-        r.i = (int)(row / (unsigned)g.ny);
-        r.j = (int)row - r.i * g.ny;
-        r.next = lane < 63 && f + 1 < o.p1;
-        r.prev = lane > 0;
-        return true;
-    }
-    const QuadAt a = row_quad(o.m, blockIdx.x, threadIdx.x);
+    const QuadAt a = row_quad(m, blockIdx.x, threadIdx.x);
     r.i = a.i;
     r.j = a.j;
     r.k0 = 2 * a.q;
@@ -191,25 +174,143 @@ __device__ __forceinline__ bool pair_at(const GridF64 &g, const OrderF64 &o, Pai
     return a.active;
 }
 
-template <bool HC, bool RANGE>
-__global__ __launch_bounds__(kBlockD) void k_update_e_f64(GridF64 g, OrderF64 o, double *ex, double *ey, double *ez,
+template <bool HC>
+__global__ __launch_bounds__(kBlockD) void k_update_e_f64(GridF64 g, RowQuads m, double *ex, double *ey, double *ez,
                                                           const double *__restrict__ hx, const double *__restrict__ hy,
                                                           const double *__restrict__ hz, const double *__restrict__ cx,
                                                           const double *__restrict__ cy, const double *__restrict__ cz)
 {
     PairAt r;
-    if (pair_at<RANGE>(g, o, r)) e_pair<HC>(g, r, ex, ey, ez, hx, hy, hz, cx, cy, cz);
+    if (pair_at(m, r)) e_pair<HC>(g, r, ex, ey, ez, hx, hy, hz, cx, cy, cz);
 }
 
-template <bool HC, bool RANGE>
-__global__ __launch_bounds__(kBlockD) void k_update_h_f64(GridF64 g, OrderF64 o, const double *__restrict__ ex,
+template <bool HC>
+__global__ __launch_bounds__(kBlockD) void k_update_h_f64(GridF64 g, RowQuads m, const double *__restrict__ ex,
                                                           const double *__restrict__ ey, const double *__restrict__ ez,
                                                           double *hx, double *hy, double *hz,
                                                           const double *__restrict__ cx, const double *__restrict__ cy,
                                                           const double *__restrict__ cz)
 {
     PairAt r;
-    if (pair_at<RANGE>(g, o, r)) h_pair<HC>(g, r, ex, ey, ez, hx, hy, hz, cx, cy, cz);
+    if (pair_at(m, r)) h_pair<HC>(g, r, ex, ey, ez, hx, hy, hz, cx, cy, cz);
+}
+
+// Coefficients of the memory-order kernels: the arrays, or 0.5 where c is null.
+__device__ __forceinline__ D2 ldc_opt(const double *__restrict__ c, size_t id)
+{
+    return c ? ld2(c + id) : D2{{0.5, 0.5}};
+}
+
+// Memory order: the pairs [p0, p1), component after component (the split form, and the whole
+// grid where its planes have too few rows for stripes).  There the stripes' order gains no
+// cache hits, and holding a pair's 12 to 15 loads at once costs waves in flight: E + H, this /
+// e_pair and h_pair in the whole-grid order / in memory order, 62x42x250 with CE 20.1 / 23.8 /
+// 23.0 us, 120x64x128 23.8 / 26.0 / 25.4, 300x48x300 118 / 145 / 123; from 72 rows on the
+// whole-grid order wins: 72x72x72 12.8 / 9.8, 201x150x123 99 / 81, 320^3 873 / 844.
+__global__ __launch_bounds__(kBlockD) void k_range_e_f64(
+    int nx, int ny, int nzp, int nz, unsigned p0, unsigned p1, unsigned P,
+    double *__restrict__ ex, double *__restrict__ ey, double *__restrict__ ez,
+    const double *__restrict__ hx, const double *__restrict__ hy, const double *__restrict__ hz,
+    const double *__restrict__ cex, const double *__restrict__ cey, const double *__restrict__ cez)
+{
+    const unsigned f = p0 + blockIdx.x * kBlockD + threadIdx.x;  // pairs [p0, p1) of the grid
+    if (f >= p1) return;
+    const unsigned row = f / P;
+    const int k0 = (int)(f - row * P) * 2;
+    const int i = (int)(row / (unsigned)ny);
+    const int j = (int)row - i * ny;
+    const size_t id = (size_t)row * nzp + k0;
+    const size_t sx = (size_t)ny * nzp;
+
+    const D2 hx0 = ld2(hx + id), hy0 = ld2(hy + id), hz0 = ld2(hz + id);
+    if (j < ny - 1) {
+        const D2 e = ld2(ex + id), c = ldc_opt(cex, id), h1 = ld2(hz + id + nzp);
+        const double hyn = hy[id + 2];  // next row's first element on the last pair (row j+1 exists)
+        D2 r;
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            const double h2 = l < 1 ? hy0.v[l + 1] : hyn;
+            const double v = e.v[l] + c.v[l] * ((h1.v[l] - hz0.v[l]) - (h2 - hy0.v[l]));
+            r.v[l] = (k0 + l < nz - 1) ? v : v * 0.0;
+        }
+        st2(ex + id, r);
+    }
+    if (i < nx - 1) {
+        const D2 e = ld2(ey + id), c = ldc_opt(cey, id), h2 = ld2(hz + id + sx);
+        const double hxn = hx[id + 2];
+        D2 r;
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            const double h1 = l < 1 ? hx0.v[l + 1] : hxn;
+            const double v = e.v[l] + c.v[l] * ((h1 - hx0.v[l]) - (h2.v[l] - hz0.v[l]));
+            r.v[l] = (k0 + l < nz - 1) ? v : v * 0.0;
+        }
+        st2(ey + id, r);
+        if (j < ny - 1) {
+            const D2 e3 = ld2(ez + id), c3 = ldc_opt(cez, id), g1 = ld2(hy + id + sx), g2 = ld2(hx + id + nzp);
+            D2 r3;
+#pragma unroll
+            for (int l = 0; l < 2; l++) {
+                const double v = e3.v[l] + c3.v[l] * ((g1.v[l] - hy0.v[l]) - (g2.v[l] - hx0.v[l]));
+                r3.v[l] = (k0 + l < nz) ? v : v * 0.0;
+            }
+            st2(ez + id, r3);
+        }
+    }
+}
+
+__global__ __launch_bounds__(kBlockD) void k_range_h_f64(
+    int ny, int nzp, int nz, unsigned p0, unsigned p1, unsigned P,
+    const double *__restrict__ ex, const double *__restrict__ ey, const double *__restrict__ ez,
+    double *__restrict__ hx, double *__restrict__ hy, double *__restrict__ hz,
+    const double *__restrict__ chx, const double *__restrict__ chy, const double *__restrict__ chz)
+{
+    const unsigned f = p0 + blockIdx.x * kBlockD + threadIdx.x;  // pairs [p0, p1) of the grid
+    if (f >= p1) return;
+    const unsigned row = f / P;
+    const int k0 = (int)(f - row * P) * 2;
+    const int i = (int)(row / (unsigned)ny);
+    const int j = (int)row - i * ny;
+    const size_t id = (size_t)row * nzp + k0;
+    const size_t sx = (size_t)ny * nzp;
+
+    const D2 ex0 = ld2(ex + id), ey0 = ld2(ey + id), ez0 = ld2(ez + id);
+    if (j > 0) {
+        const D2 h = ld2(hx + id), c = ldc_opt(chx, id), e1 = ld2(ez + id - nzp);
+        const double eyp = ey[id - 1];  // previous row's last element when k0 == 0 (row j-1 exists)
+        D2 r;
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            const double e2 = l > 0 ? ey0.v[l - 1] : eyp;
+            const double v = h.v[l] - c.v[l] * ((ez0.v[l] - e1.v[l]) - (ey0.v[l] - e2));
+            const int k = k0 + l;
+            r.v[l] = (k > 0 && k < nz) ? v : v * 0.0;
+        }
+        st2(hx + id, r);
+    }
+    if (i > 0) {
+        const D2 h = ld2(hy + id), c = ldc_opt(chy, id), e2 = ld2(ez + id - sx);
+        const double exp_ = ex[id - 1];
+        D2 r;
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            const double e1 = l > 0 ? ex0.v[l - 1] : exp_;
+            const double v = h.v[l] - c.v[l] * ((ex0.v[l] - e1) - (ez0.v[l] - e2.v[l]));
+            const int k = k0 + l;
+            r.v[l] = (k > 0 && k < nz) ? v : v * 0.0;
+        }
+        st2(hy + id, r);
+        if (j > 0) {
+            const D2 h3 = ld2(hz + id), c3 = ldc_opt(chz, id), g1 = ld2(ey + id - sx), g2 = ld2(ex + id - nzp);
+            D2 r3;
+#pragma unroll
+            for (int l = 0; l < 2; l++) {
+                const double v = h3.v[l] - c3.v[l] * ((ey0.v[l] - g1.v[l]) - (ex0.v[l] - g2.v[l]));
+                r3.v[l] = (k0 + l < nz) ? v : v * 0.0;
+            }
+            st2(hz + id, r3);
+        }
+    }
 }
 
 int check_grid_f64(int nx, int ny, int nzp, int pad)
@@ -241,38 +342,34 @@ int launch_core_f64(bool e_half, int nx, int ny, int nzp, int pad, double *ex, d
     const unsigned npairs = (unsigned)nx * ny * P;
     const int nz = nzp - pad;
     const GridF64 g{nx, ny, nzp, nz};
-    const bool range = nmax >= 0, hc = c0 != nullptr;
-    OrderF64 o{};
-    o.P = P;
-    unsigned grid;
-    if (range) {  // the split form's element range, a pair per 2-element vector
+    const bool hc = c0 != nullptr;
+    unsigned p0 = 0, p1 = npairs;
+    if (nmax >= 0) {  // the split form's element range, a pair per 2-element vector
         const long long n = 2ll * npairs;
         if (idx0 < 0 || idx0 > nmax || nmax > n)
             return fail(MIFDTD_EINVAL, "element range [%lld, %lld) outside the grid's %lld", idx0, nmax, n);
         if (idx0 % 2) return fail(MIFDTD_EALIGN, "idx0 %lld does not start a 2-element vector", idx0);
-        o.p0 = (unsigned)(idx0 / 2);
-        o.p1 = (unsigned)((nmax + 1) / 2);
-        if (o.p1 == o.p0) return 0;
-        grid = (o.p1 - o.p0 + kBlockD - 1) / kBlockD;
-    } else {
-        o.m = grid_order(nx, ny, (int)P, nz, 0);
-        grid = (unsigned)row_quads_blocks(o.m);
+        p0 = (unsigned)(idx0 / 2);
+        p1 = (unsigned)((nmax + 1) / 2);
+        if (p1 == p0) return 0;
     }
-#define MIFDTD_F64_LAUNCH(K)                                                                             \
-    do {                                                                                                 \
-        if (hc && range) K<true, true><<<grid, kBlockD, 0, st>>>(g, o, ex, ey, ez, hx, hy, hz, c0, c1, c2);   \
-        else if (hc) K<true, false><<<grid, kBlockD, 0, st>>>(g, o, ex, ey, ez, hx, hy, hz, c0, c1, c2);      \
-        else if (range) K<false, true><<<grid, kBlockD, 0, st>>>(g, o, ex, ey, ez, hx, hy, hz, c0, c1, c2);   \
-        else K<false, false><<<grid, kBlockD, 0, st>>>(g, o, ex, ey, ez, hx, hy, hz, c0, c1, c2);             \
-    } while (0)
+    if (nmax >= 0 || ny < (int)kStripeMinRows) {
+        const unsigned grid = (p1 - p0 + kBlockD - 1) / kBlockD;
+        if (e_half) k_range_e_f64<<<grid, kBlockD, 0, st>>>(nx, ny, nzp, nz, p0, p1, P, ex, ey, ez, hx, hy, hz, c0, c1, c2);
+        else k_range_h_f64<<<grid, kBlockD, 0, st>>>(ny, nzp, nz, p0, p1, P, ex, ey, ez, hx, hy, hz, c0, c1, c2);
+        MIFDTD_CHECK_LAUNCH("update (double, memory order) launch");
+        return 0;
+    }
+    const RowQuads m = grid_order(nx, ny, (int)P, nz, 0);
+    const unsigned grid = (unsigned)row_quads_blocks(m);
     if (e_half) {
-        MIFDTD_F64_LAUNCH(k_update_e_f64);
-        MIFDTD_CHECK_LAUNCH("update_e (double) launch");
+        if (hc) k_update_e_f64<true><<<grid, kBlockD, 0, st>>>(g, m, ex, ey, ez, hx, hy, hz, c0, c1, c2);
+        else k_update_e_f64<false><<<grid, kBlockD, 0, st>>>(g, m, ex, ey, ez, hx, hy, hz, c0, c1, c2);
     } else {
-        MIFDTD_F64_LAUNCH(k_update_h_f64);
-        MIFDTD_CHECK_LAUNCH("update_h (double) launch");
+        if (hc) k_update_h_f64<true><<<grid, kBlockD, 0, st>>>(g, m, ex, ey, ez, hx, hy, hz, c0, c1, c2);
+        else k_update_h_f64<false><<<grid, kBlockD, 0, st>>>(g, m, ex, ey, ez, hx, hy, hz, c0, c1, c2);
     }
-#undef MIFDTD_F64_LAUNCH
+    MIFDTD_CHECK_LAUNCH("update (double) launch");
     return 0;
 }
 
