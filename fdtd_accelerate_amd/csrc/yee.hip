@@ -116,6 +116,75 @@ __global__ __launch_bounds__(kBlock) void k_update_e(
     }
 }
 
+// update_e with the CE arrays held as per-component uint8 material indices into a
+// 3 x 256 float table (the exact float32 CE values; staged in LDS): 39 instead of 48
+// bytes per cell, same arithmetic and masks as k_update_e<true>.  Memory order, where
+// memory_order takes it: against the whole-grid pass 245x43x68 5.1 / 6.3 us, 135x102x74
+// 6.5 / 7.8, 204x55x153 12.8 / 14.6, 300x48x300 30.7 / 32.9.
+__global__ __launch_bounds__(kBlock) void k_update_e_lut(
+    int nx, int ny, int nzp, int nz, unsigned nquads, unsigned Q,
+    float *__restrict__ ex, float *__restrict__ ey, float *__restrict__ ez,
+    const float *__restrict__ hx, const float *__restrict__ hy, const float *__restrict__ hz,
+    const unsigned char *__restrict__ mx, const unsigned char *__restrict__ my, const unsigned char *__restrict__ mz,
+    const float *__restrict__ lut)
+{
+    __shared__ float tab[3 * 256];
+    for (int t = threadIdx.x; t < 3 * 256; t += kBlock) tab[t] = lut[t];
+    __syncthreads();
+    const unsigned f = blockIdx.x * kBlock + threadIdx.x;
+    if (f >= nquads) return;
+    const unsigned row = f / Q;
+    const int k0 = (int)(f - row * Q) * 4;
+    const int i = (int)(row / (unsigned)ny);
+    const int j = (int)row - i * ny;
+    const size_t id = (size_t)row * nzp + k0;
+    const size_t sx = (size_t)ny * nzp;
+
+    const Q4 hx0 = ld4(hx + id), hy0 = ld4(hy + id), hz0 = ld4(hz + id);
+
+    if (j < ny - 1) {
+        const Q4 e = ld4(ex + id);
+        const Q4 c = ce_from_table(mx + id, tab);
+        const Q4 h1 = ld4(hz + id + nzp);
+        const float hyn = hy[id + 4];
+        Q4 r;
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            const float h2 = l < 3 ? hy0.v[l + 1] : hyn;
+            const float v = e.v[l] + c.v[l] * ((h1.v[l] - hz0.v[l]) - (h2 - hy0.v[l]));
+            r.v[l] = (k0 + l < nz - 1) ? v : v * 0.f;
+        }
+        st4(ex + id, r);
+    }
+    if (i < nx - 1) {
+        const Q4 e = ld4(ey + id);
+        const Q4 c = ce_from_table(my + id, tab + 256);
+        const Q4 h2 = ld4(hz + id + sx);
+        const float hxn = hx[id + 4];
+        Q4 r;
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            const float h1 = l < 3 ? hx0.v[l + 1] : hxn;
+            const float v = e.v[l] + c.v[l] * ((h1 - hx0.v[l]) - (h2.v[l] - hz0.v[l]));
+            r.v[l] = (k0 + l < nz - 1) ? v : v * 0.f;
+        }
+        st4(ey + id, r);
+        if (j < ny - 1) {
+            const Q4 e3 = ld4(ez + id);
+            const Q4 c3 = ce_from_table(mz + id, tab + 512);
+            const Q4 g1 = ld4(hy + id + sx);
+            const Q4 g2 = ld4(hx + id + nzp);
+            Q4 r3;
+#pragma unroll
+            for (int l = 0; l < 4; l++) {
+                const float v = e3.v[l] + c3.v[l] * ((g1.v[l] - hy0.v[l]) - (g2.v[l] - hx0.v[l]));
+                r3.v[l] = (k0 + l < nz) ? v : v * 0.f;
+            }
+            st4(ez + id, r3);
+        }
+    }
+}
+
 template <bool HAS_C>
 __global__ __launch_bounds__(kBlock) void k_update_h(
     int nx, int ny, int nzp, int nz, unsigned q0, unsigned q1, unsigned Q,
@@ -217,18 +286,22 @@ static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_z, const f
 static int launch_range(bool e_half, int nx, int ny, int nzp, int pad, const float *const (&f)[6], const float *c0,
                         const float *c1, const float *c2, hipStream_t st, long long idx0, long long nmax);
 
-// Where the core alone runs in memory order: planes of too few rows for stripes, and planes of
-// a multiple of 8 blocks, whose rows fall to the same XCD in every plane by themselves.  E + H
-// on cold arrays, whole order / memory order: 100x70x200 24.8 / 23.9 us, 200x71x130 32.4 /
-// 30.5, 120x64x128 17.3 / 15.6, 400x40x400 87.3 / 86.1; 128^3 31.5 / 29.8, but 256^3 218.8 /
-// 224.3 (2^22 quads); 200x128x100 34.3 / 39.9.  Below 2^17 quads the launches bound, and the
-// whole-grid kernels' few structures are cheaper to pass than 18 arguments (64^3, from Python,
-// 14.8 / 17.0).
+// Where the core alone runs in memory order: planes of too few rows for stripes, and planes
+// whose blocks are a multiple of 8, so that a row falls to the same XCD in every plane by
+// itself: exactly one (128^3 31.5 us in the whole order / 29.8 in memory order; 256^3, 2^22
+// quads, 218.8 / 224.3), or on grids of fewer than 2^19 quads nearly one (up to 112 quads off
+// a multiple of 2048: 129x171x48 13.0 / 11.0, 120x109x73 12.4 / 10.6, 64x138x116 13.8 / 11.8,
+// 83x121x203 26.5 / 25.1, E alone with CE indices 135x102x74 7.9 / 6.5; with more quads
+// 101x139x236 39.2 / 40.9, further off 96^3 11.3 / 12.9).  Planes of few rows: 100x70x200 24.8 / 23.9 on cold arrays, 200x71x130 32.4 / 30.5;
+// 200x128x100 34.3 / 39.9.  Below 2^17 quads the launches bound, and the whole-grid kernels'
+// few structures are cheaper to pass than 18 arguments (64^3, from Python, 14.8 / 17.0).
 static bool memory_order(int nx, int ny, int Q)
 {
     const unsigned long long quads = (unsigned long long)nx * ny * Q;
     if (quads < (1ull << 17)) return false;
-    return ny < (int)kStripeMinRows || (quads < (1ull << 21) && (long long)ny * Q % (8 * kBlock) == 0);
+    if (ny < (int)kStripeMinRows) return true;
+    const long long off = (long long)ny * Q % (8 * kBlock), near = off < 4 * kBlock ? off : 8 * kBlock - off;
+    return quads < (1ull << 19) ? near <= 112 : quads < (1ull << 21) && near == 0;
 }
 
 static int launch_core(bool e_half, int nx, int ny, int nzp, int pad, const float *const (&f)[6], const float *c0,
@@ -806,6 +879,13 @@ int mifdtd_update_e_lut(int nx, int ny, int nz_pitch, int pad, float *ex, float 
     if (int rc = check_fields(f)) return rc;
     const unsigned char *const mats[3] = {mat_x, mat_y, mat_z};
     if (int rc = check_mats(mats, lut)) return rc;
+    if (memory_order(nx, ny, nz_pitch / 4)) {
+        const unsigned Q = (unsigned)(nz_pitch / 4), nquads = (unsigned)nx * ny * Q;
+        k_update_e_lut<<<(nquads + kBlock - 1) / kBlock, kBlock, 0, to_stream(stream)>>>(
+            nx, ny, nz_pitch, nz_pitch - pad, nquads, Q, ex, ey, ez, hx, hy, hz, mat_x, mat_y, mat_z, lut);
+        MIFDTD_CHECK_LAUNCH("update_e_lut launch");
+        return 0;
+    }
     WholeGrid w = whole_grid(nx, ny, nz_pitch, nz_pitch - pad, 0, f, to_stream(stream));
     for (int c = 0; c < 3; c++) w.F.cm[c] = mats[c];
     w.F.lut = lut;
