@@ -21,15 +21,16 @@ struct SExtra {
     STfsf tf;
 };
 
-// CM: CeMode (kCeTable: CE from the material indices and the 3 x 256 table, staged in LDS:
-// E pass alone 208^3 60.2 -> 52.2 us, 433x380x56 60.2 -> 54.0, 266x169x245 81.5 -> 72.7
-// against table reads from global memory).  The sources and probes (first argument) are read
-// only by the waves near them.
-template <int CM, bool PML>
+// CM: CeMode (kCeTable: CE from the material indices and the 3 x 256 table).  The
+// sources and probes (first argument) are read only by the waves near them.  LDS: the table
+// staged in LDS, for the core alone on arrays of many materials (200 of them, E pass alone:
+// 208^3 60.2 -> 52.2 us, 433x380x56 60.2 -> 54.0, 266x169x245 81.5 -> 72.7); where most cells
+// are one material it costs 0-5% (192^3 40.9 -> 41.5), with the CPML in the pass 1-3.5%.
+template <int CM, bool PML, bool LDS = false>
 __global__ __launch_bounds__(SB) void k_slab_e(SAux, SGeom g, SFields F, SCpml cp)
 {
-    __shared__ float tab[CM == kCeTable ? 768 : 1];
-    if (CM == kCeTable) {
+    __shared__ float tab[LDS ? 768 : 1];
+    if (LDS) {
         for (int t = threadIdx.x; t < 768; t += SB) tab[t] = F.lut[t];
         __syncthreads();
     }
@@ -37,7 +38,7 @@ __global__ __launch_bounds__(SB) void k_slab_e(SAux, SGeom g, SFields F, SCpml c
     if (!slab_quad(g, blockIdx.x, r)) return;
     e_quad_at<CM, PML>(g, r.i, r.j, r.k0, r.next, F.e[0], F.e[1], F.e[2], F.e[0], F.e[1], F.e[2], F.e[3], F.e[4],
                        F.e[5], F.ce[0], F.ce[1], F.ce[2], cp, first_kernel_arg<SAux>(), F.cm[0], F.cm[1], F.cm[2],
-                       tab);
+                       LDS ? tab : F.lut);
 }
 
 // With a Drude box and / or TFSF patches (FEAT; a grid without CPML has cp.axes 0).
@@ -100,6 +101,7 @@ static void launch_e(const WholeGrid &w, unsigned grid, const SAux &a, const SDr
     }
     if (!dr && !tf) {
         if (w.cp.npml > 0) k_slab_e<CM, true><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
+        else if (CM == kCeTable && w.lds_table) k_slab_e<CM, false, CM == kCeTable><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
         else k_slab_e<CM, false><<<grid, SB, 0, w.st>>>(a, w.g, w.F, w.cp);
         return;
     }

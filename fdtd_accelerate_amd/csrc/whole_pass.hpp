@@ -12,6 +12,7 @@ struct WholeGrid {
     SFields F;
     SCpml cp;       // npml 0: none
     int cem;        // CeMode: constant, arrays or table
+    bool lds_table; // the table staged in LDS (E passes without CPML)
     hipStream_t st;
 };
 

@@ -890,6 +890,7 @@ int mifdtd_update_e_lut(int nx, int ny, int nz_pitch, int pad, float *ex, float 
     for (int c = 0; c < 3; c++) w.F.cm[c] = mats[c];
     w.F.lut = lut;
     w.cem = kCeTable;
+    w.lds_table = true;
     return whole_e(w, no_aux(), nullptr, nullptr);
 }
 
