@@ -133,8 +133,9 @@ inline unsigned long long row_quads_blocks(const RowQuads &m)
 // 0: none).  The E slabs are [0, npml) and [nz-1-npml, nz-1), the H slabs [0, npml) and
 // [nz-npml, nz): one order serves both.  front: cells at the front that count as slab cells
 // (the adjoint passes reach one cell further).  phase: quads from a 128-byte line to each
-// row's first quad.
-inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, int front = 0, unsigned phase = 0)
+// row's first quad.  max_rows: the most rows of a group.
+inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, int front = 0, unsigned phase = 0,
+                          unsigned max_rows = 64)
 {
     RowQuads m;
     m.Q = Q;
@@ -156,7 +157,7 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     // smallest R whose blocks leave at most 1 thread in 64 idle, else the R with the least
     unsigned best = 1;
     double waste = 2.0;
-    for (unsigned R = 1; R <= 64 && (R == 1 || R * Q <= 32768u); ++R) {
+    for (unsigned R = 1; R <= max_rows && (R == 1 || R * Q <= 32768u); ++R) {
         const unsigned n = R * Q, pad = (n + 255) / 256 * 256;
         const double w = (double)(pad - n) / pad;
         if (w < waste - 1e-9) {
@@ -176,6 +177,18 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
         m.m_s[x] = reciprocal(planes * stripe_max(m) + 64 * m.R, S);
     }
     return m;
+}
+
+// The order of a Yee E or H pass.  With CPML a group's z-slab runs follow the runs of all its
+// rows: at pitches off the lines a large group fetches the lines at the runs' ends twice.
+// E + H, CPML 10, groups of up to 64 / 8 / 2 rows: 341x240x258 424 / 379 / 383 us, 333x491x357
+// 1053 / 907 / 896, 448^3 1398 / 1298 / 1300, 352^3 673 / 641 / 645, 128^3 36.0 / 36.7 / 38.9,
+// 300x300x250 356 / 355 / 365.  The 4th-order stages and the adjoint passes keep 64 (8: 400 x
+// 300 x 200 2145 -> 2345 us a step, 160^3 128.9 -> 130.9 ms).
+constexpr unsigned kYeeRows = 8;
+inline RowQuads yee_order(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, unsigned phase = 0)
+{
+    return row_quads(planes, ny, Q, nz, npml, 0, phase, npml > 0 ? kYeeRows : 64);
 }
 
 }  // namespace mifdtd

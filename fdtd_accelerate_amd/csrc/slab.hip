@@ -154,7 +154,7 @@ RowQuads grid_order(int nx, int ny, int Q, int nz, int npml)
     bool same = true;
     for (int n = 0; n < 5; n++) same = same && key[n] == want[n];
     if (!same) {
-        m = row_quads((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, npml);
+        m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, npml);
         for (int n = 0; n < 5; n++) key[n] = want[n];
     }
     return m;
@@ -275,7 +275,7 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
         g.nzp = nzp;
         g.nz = nz;
         g.i0 = sl * S;
-        g.m = row_quads((unsigned)(nx - g.i0 < S ? nx - g.i0 : S), (unsigned)ny, Q, nz, pml ? d->npml : 0);
+        g.m = yee_order((unsigned)(nx - g.i0 < S ? nx - g.i0 : S), (unsigned)ny, Q, nz, pml ? d->npml : 0);
         return g;
     };
     auto tables = [&](const SProbe &P, int step, bool e_half) {

@@ -30,7 +30,7 @@ inline SAux no_aux()
 int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf, const SCurl *cu = nullptr);
 int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *const *ch = nullptr);
 
-// row_quads of the whole grid of Q units of 16 bytes per row; the last one a thread asked for
+// yee_order of the whole grid of Q units of 16 bytes per row; the last one a thread asked for
 // is kept.
 RowQuads grid_order(int nx, int ny, int Q, int nz, int npml);
 

@@ -1,6 +1,6 @@
 // Host-side checks of row_quads.hpp beyond tests/row_cover.cpp: the orders with slab cells
 // counted further at the front (the adjoint passes) and with rows off the 128-byte lines (the
-// fused engine's placed fields) take every quad once, with exact neighbour flags and no slab
+// fused engine's placed fields), and the Yee passes' own, take every quad once, with exact neighbour flags and no slab
 // cell in a plain run; and blocks past a stripe's rows find their row by an exact division.
 // Exit status 0 when all hold.
 #include "../fdtd_accelerate_amd/csrc/row_quads.hpp"
@@ -10,10 +10,11 @@
 
 using namespace mifdtd;
 
-static int cover(unsigned planes, unsigned ny, int nz, int nzp, int npml, int front, unsigned phase)
+static int cover(unsigned planes, unsigned ny, int nz, int nzp, int npml, int front, unsigned phase, bool yee = false)
 {
     const unsigned Q = (unsigned)nzp / 4;
-    const RowQuads m = row_quads(planes, ny, Q, nz, npml, front, phase);
+    const RowQuads m = yee ? yee_order(planes, ny, Q, nz, npml, phase) : row_quads(planes, ny, Q, nz, npml, front, phase);
+    if (yee && m.R > kYeeRows) { std::printf("a group of %u rows: %u x %d, npml %d\n", m.R, ny, nz, npml); return 1; }
     const unsigned nb = (unsigned)row_quads_blocks(m);
     std::vector<int> hits((size_t)planes * ny * Q, 0);
     for (unsigned b = 0; b < nb; ++b)
@@ -70,6 +71,7 @@ int main()
                 if (z[0] >= 2 * p + 2)
                     for (unsigned phase = 0; phase < 8; ++phase) {
                         if (cover(r[0], r[1], z[0], z[1], p, 0, phase)) return 1;
+                        if (cover(r[0], r[1], z[0], z[1], p, 0, phase, true)) return 1;
                         if (phase == 0 && cover(r[0], r[1], z[0], z[1], p, p + 1, 0)) return 1;
                     }
     if (idle(14861237, 144, 1, 4, 1) || idle(1651195, 414, 3, 10, 4) || idle(1651195, 414, 3, 12, 5)) return 1;
