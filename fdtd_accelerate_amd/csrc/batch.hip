@@ -130,7 +130,7 @@ static int build_batch(const mifdtd_instance *inst, int ninst, const float *bE, 
         B.g.nzp = nzp;
         B.g.nz = nz;
         B.g.i0 = 0;
-        B.g.m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)(nzp / 4), nz, d.npml);
+        B.g.m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)(nzp / 4), nz, d.npml, d.npml);
         for (int c = 0; c < 6; c++) B.F.e[c] = d.e[c];
         for (int c = 0; c < 3; c++) B.F.ce[c] = d.ce[c];
         if (tbl) {

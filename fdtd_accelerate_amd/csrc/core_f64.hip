@@ -360,7 +360,7 @@ int launch_core_f64(bool e_half, int nx, int ny, int nzp, int pad, double *ex, d
         MIFDTD_CHECK_LAUNCH("update (double, memory order) launch");
         return 0;
     }
-    const RowQuads m = grid_order(nx, ny, (int)P, nz, 0);
+    const RowQuads m = grid_order(nx, ny, (int)P, nz, 0, 0);
     const unsigned grid = (unsigned)row_quads_blocks(m);
     if (e_half) {
         if (hc) k_update_e_f64<true><<<grid, kBlockD, 0, st>>>(g, m, ex, ey, ez, hx, hy, hz, c0, c1, c2);

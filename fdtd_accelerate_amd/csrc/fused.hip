@@ -1458,9 +1458,9 @@ int mifdtd_fused_run_timed(const mifdtd_fused_desc *d, int nsteps, const float *
         if (pairs) return fail(MIFDTD_EINVAL, "whole-grid steps and step pairs exclude each other");
         WholeGrid w{};
         w.g = sg;
-        const int zp = (pml_axes & 4) ? d->npml : 0;
+        const int zp = (pml_axes & 4) ? d->npml : 0, yp = (pml_axes & 2) ? d->npml : 0;
         if ((unsigned long long)nx * ny * Q + SB >= (1ull << 31)) return fail(MIFDTD_ERANGE, "grid too large");
-        w.g.m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, zp, (unsigned)zph / 4);
+        w.g.m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, yp, zp, (unsigned)zph / 4);
         for (int q = 0; q < 6; q++) w.F.e[q] = d->e[q];
         for (int q = 0; q < 3; q++) {
             w.F.ce[q] = d->ce[q];

@@ -133,15 +133,16 @@ inline unsigned long long row_quads_blocks(const RowQuads &m)
 // 0: none).  The E slabs are [0, npml) and [nz-1-npml, nz-1), the H slabs [0, npml) and
 // [nz-npml, nz): one order serves both.  front: cells at the front that count as slab cells
 // (the adjoint passes reach one cell further).  phase: quads from a 128-byte line to each
-// row's first quad.  max_rows: the most rows of a group.
+// row's first quad.  max_rows: the most rows of a group.  npml_y: y slabs of another width
+// than the z slabs (a grid with CPML on one of the two axes); -1: the same.
 inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, int front = 0, unsigned phase = 0,
-                          unsigned max_rows = 64)
+                          unsigned max_rows = 64, int npml_y = -1)
 {
     RowQuads m;
     m.Q = Q;
     m.planes = planes;
     m.ns = ny >= kStripeMinRows ? kStripes : 1;
-    stripe_rows(m, ny, npml);
+    stripe_rows(m, ny, npml_y < 0 ? npml : npml_y);
     m.zf = npml > 0 ? (unsigned)(((front > npml ? front : npml) + 3) / 4) : 0u;
     m.zb = npml > 0 ? (unsigned)((nz - 1 - npml) / 4) : Q;
     if (npml > 0) {  // whole 128-byte lines (8 quads) on either side of a run's end
@@ -179,16 +180,16 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     return m;
 }
 
-// The order of a Yee E or H pass.  With CPML a group's z-slab runs follow the runs of all its
+// The order of a Yee E or H pass (npml_y, npml_z: 0 on an axis without CPML).  With CPML a group's z-slab runs follow the runs of all its
 // rows: at pitches off the lines a large group fetches the lines at the runs' ends twice.
 // E + H, CPML 10, groups of up to 64 / 8 / 2 rows: 341x240x258 424 / 379 / 383 us, 333x491x357
 // 1053 / 907 / 896, 448^3 1398 / 1298 / 1300, 352^3 673 / 641 / 645, 128^3 36.0 / 36.7 / 38.9,
 // 300x300x250 356 / 355 / 365.  The 4th-order stages and the adjoint passes keep 64 (8: 400 x
 // 300 x 200 2145 -> 2345 us a step, 160^3 128.9 -> 130.9 ms).
 constexpr unsigned kYeeRows = 8;
-inline RowQuads yee_order(unsigned planes, unsigned ny, unsigned Q, int nz, int npml, unsigned phase = 0)
+inline RowQuads yee_order(unsigned planes, unsigned ny, unsigned Q, int nz, int npml_y, int npml_z, unsigned phase = 0)
 {
-    return row_quads(planes, ny, Q, nz, npml, 0, phase, npml > 0 ? kYeeRows : 64);
+    return row_quads(planes, ny, Q, nz, npml_z, 0, phase, npml_z > 0 ? kYeeRows : 64, npml_y);
 }
 
 }  // namespace mifdtd

@@ -146,16 +146,16 @@ int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *con
     return 0;
 }
 
-RowQuads grid_order(int nx, int ny, int Q, int nz, int npml)
+RowQuads grid_order(int nx, int ny, int Q, int nz, int npml_y, int npml_z)
 {
-    thread_local int key[5] = {0, 0, 0, 0, 0};
+    thread_local int key[6] = {0, 0, 0, 0, 0, 0};
     thread_local RowQuads m;
-    const int want[5] = {nx, ny, Q, nz, npml};
+    const int want[6] = {nx, ny, Q, nz, npml_y, npml_z};
     bool same = true;
-    for (int n = 0; n < 5; n++) same = same && key[n] == want[n];
+    for (int n = 0; n < 6; n++) same = same && key[n] == want[n];
     if (!same) {
-        m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, npml);
-        for (int n = 0; n < 5; n++) key[n] = want[n];
+        m = yee_order((unsigned)nx, (unsigned)ny, (unsigned)Q, nz, npml_y, npml_z);
+        for (int n = 0; n < 6; n++) key[n] = want[n];
     }
     return m;
 }
@@ -275,7 +275,7 @@ int mifdtd_slab_run(const mifdtd_fused_desc *d, int slab_planes, int nsteps, con
         g.nzp = nzp;
         g.nz = nz;
         g.i0 = sl * S;
-        g.m = yee_order((unsigned)(nx - g.i0 < S ? nx - g.i0 : S), (unsigned)ny, Q, nz, pml ? d->npml : 0);
+        g.m = yee_order((unsigned)(nx - g.i0 < S ? nx - g.i0 : S), (unsigned)ny, Q, nz, pml ? d->npml : 0, pml ? d->npml : 0);
         return g;
     };
     auto tables = [&](const SProbe &P, int step, bool e_half) {

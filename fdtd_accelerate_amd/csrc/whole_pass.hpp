@@ -32,6 +32,6 @@ int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *con
 
 // yee_order of the whole grid of Q units of 16 bytes per row; the last one a thread asked for
 // is kept.
-RowQuads grid_order(int nx, int ny, int Q, int nz, int npml);
+RowQuads grid_order(int nx, int ny, int Q, int nz, int npml_y, int npml_z);
 
 }  // namespace mifdtd

@@ -269,14 +269,15 @@ static int check_coeffs(const float *c0, const float *c1, const float *c2)
 // The whole grid's half step in the thread order of row_quads.hpp.  The E + H core of a cube
 // against a thread per quad in memory order, from Python: 160^3 67.6 -> 53.5 us, 192^3
 // 111 -> 88, 256^3 269 -> 260.
-static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_z, const float *const (&f)[6], hipStream_t st)
+static WholeGrid whole_grid(int nx, int ny, int nzp, int nz, int npml_y, int npml_z, const float *const (&f)[6],
+                            hipStream_t st)
 {
     WholeGrid w{};
     w.g.nx = nx;
     w.g.ny = ny;
     w.g.nzp = nzp;
     w.g.nz = nz;
-    w.g.m = grid_order(nx, ny, nzp / 4, nz, npml_z);
+    w.g.m = grid_order(nx, ny, nzp / 4, nz, npml_y, npml_z);
     for (int c = 0; c < 6; c++) w.F.e[c] = const_cast<float *>(f[c]);
     w.cem = kCeConst;
     w.st = st;
@@ -312,7 +313,7 @@ static int launch_core(bool e_half, int nx, int ny, int nzp, int pad, const floa
         return launch_range(e_half, nx, ny, nzp, pad, f, c0, c1, c2, st, 0, (long long)nx * ny * nzp);
     if (int rc = check_fields(f)) return rc;
     if (int rc = check_coeffs(c0, c1, c2)) return rc;
-    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, 0, f, st);
+    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, 0, 0, f, st);
     const float *c[3] = {c0, c1, c2};
     if (!e_half) return whole_h(w, no_aux(), nullptr, c0 ? c : nullptr);
     for (int q = 0; q < 3; q++) w.F.ce[q] = c[q];
@@ -886,7 +887,7 @@ int mifdtd_update_e_lut(int nx, int ny, int nz_pitch, int pad, float *ex, float 
         MIFDTD_CHECK_LAUNCH("update_e_lut launch");
         return 0;
     }
-    WholeGrid w = whole_grid(nx, ny, nz_pitch, nz_pitch - pad, 0, f, to_stream(stream));
+    WholeGrid w = whole_grid(nx, ny, nz_pitch, nz_pitch - pad, 0, 0, f, to_stream(stream));
     for (int c = 0; c < 3; c++) w.F.cm[c] = mats[c];
     w.F.lut = lut;
     w.cem = kCeTable;
@@ -992,7 +993,8 @@ int mifdtd_half_e(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, 
                                 drude->li, drude->lj, drude->lk, stream);
         return rc ? rc : mifdtd_cpml_e(nx, ny, nzp, pad, cp, ex, ey, ez, hx, hy, hz, cex, cey, cez, stream);
     }
-    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 4) ? cp->npml : 0, f, to_stream(stream));
+    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 2) ? cp->npml : 0, (sc.axes & 4) ? cp->npml : 0, f,
+                             to_stream(stream));
     for (int c = 0; c < 3; c++) {
         w.F.ce[c] = ce[c];
         w.F.cm[c] = mats[c];
@@ -1017,7 +1019,8 @@ int mifdtd_half_h(int nx, int ny, int nzp, int pad, const mifdtd_cpml_half *cp, 
         const int rc = mifdtd_update_h(nx, ny, nzp, pad, ex, ey, ez, hx, hy, hz, chx, chy, chz, stream);
         return rc ? rc : mifdtd_cpml_h(nx, ny, nzp, pad, cp, ex, ey, ez, hx, hy, hz, chx, chy, chz, stream);
     }
-    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 4) ? cp->npml : 0, f, to_stream(stream));
+    WholeGrid w = whole_grid(nx, ny, nzp, nzp - pad, (sc.axes & 2) ? cp->npml : 0, (sc.axes & 4) ? cp->npml : 0, f,
+                             to_stream(stream));
     w.cp = sc;
     const float *const ch[3] = {chx, chy, chz};
     return whole_h(w, no_aux(), nullptr, chx ? ch : nullptr);

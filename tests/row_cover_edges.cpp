@@ -10,10 +10,11 @@
 
 using namespace mifdtd;
 
-static int cover(unsigned planes, unsigned ny, int nz, int nzp, int npml, int front, unsigned phase, bool yee = false)
+static int cover(unsigned planes, unsigned ny, int nz, int nzp, int npml, int front, unsigned phase, int yee_y = -1)
 {
     const unsigned Q = (unsigned)nzp / 4;
-    const RowQuads m = yee ? yee_order(planes, ny, Q, nz, npml, phase) : row_quads(planes, ny, Q, nz, npml, front, phase);
+    const bool yee = yee_y >= 0;
+    const RowQuads m = yee ? yee_order(planes, ny, Q, nz, yee_y, npml, phase) : row_quads(planes, ny, Q, nz, npml, front, phase);
     if (yee && m.R > kYeeRows) { std::printf("a group of %u rows: %u x %d, npml %d\n", m.R, ny, nz, npml); return 1; }
     const unsigned nb = (unsigned)row_quads_blocks(m);
     std::vector<int> hits((size_t)planes * ny * Q, 0);
@@ -61,6 +62,19 @@ static int idle(unsigned planes, unsigned ny, unsigned Q, int nz, int npml)
     return 0;
 }
 
+// Stripes: equal rows where the y axis has no slabs, whatever the z slabs, and smaller first and
+// last ones where it has.
+static int stripes(unsigned ny, int npml)
+{
+    const RowQuads a = yee_order(3, ny, 65, 258, 0, npml), b = yee_order(3, ny, 65, 258, npml, 0);
+    for (unsigned x = 0; x < 8; ++x) {
+        const unsigned S = a.jx[x + 1] - a.jx[x];
+        if (S != ny / 8 && S != (ny + 7) / 8) { std::printf("stripe %u of %u rows: %u\n", x, ny, S); return 1; }
+    }
+    if (b.jx[1] >= a.jx[1] || ny - b.jx[7] >= ny - a.jx[7]) { std::printf("y slabs of %u rows not weighted\n", ny); return 1; }
+    return 0;
+}
+
 int main()
 {
     const int nzs[][2] = {{26, 32}, {33, 36}, {64, 64}, {75, 76}, {123, 128}, {160, 160}, {258, 260}, {331, 336}, {1043, 1056}};
@@ -71,9 +85,11 @@ int main()
                 if (z[0] >= 2 * p + 2)
                     for (unsigned phase = 0; phase < 8; ++phase) {
                         if (cover(r[0], r[1], z[0], z[1], p, 0, phase)) return 1;
-                        if (cover(r[0], r[1], z[0], z[1], p, 0, phase, true)) return 1;
+                        if (cover(r[0], r[1], z[0], z[1], p, 0, phase, phase % 2 ? p : 0)) return 1;
                         if (phase == 0 && cover(r[0], r[1], z[0], z[1], p, p + 1, 0)) return 1;
                     }
+    for (unsigned ny : {200u, 240u, 333u, 491u})
+        if (stripes(ny, 12)) return 1;
     if (idle(14861237, 144, 1, 4, 1) || idle(1651195, 414, 3, 10, 4) || idle(1651195, 414, 3, 12, 5)) return 1;
     std::printf("row cover edges ok\n");
     return 0;
