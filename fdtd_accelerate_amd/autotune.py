@@ -62,29 +62,35 @@ def _halved(nx, ny):
     return T, max(1, cx)
 
 
-def heuristic(nx, ny, nzp, npml, halved=False):
+def tile_cost(T, CX, box):
+    """Planes times waves that the work-groups of a CU take one after the other: whole rounds of
+    256 blocks of CX planes and one for a block's start, T+1 waves and two for the barrier."""
+    rounds = -(-(-(-box[1] // T) * -(-box[0] // CX)) // N_CU)
+    return rounds * (CX + 2) * (T + 3)
+
+
+def heuristic(nx, ny, nzp, npml, halved=False, box=None, table=True):
     """(T, CX): owned rows per block (one halo row each, T+1 waves) and planes per chunk
-    (one seed plane each), of the tiles that leave room for the largest CE table.  One work-group runs per CU, so a sweep takes whole rounds of
-    256 blocks: the tile with the least rounds * (CX + 2) * (T + 3), the planes and waves of
-    a block with one plane for its start and two waves for the barrier.  Sweep against
-    T = 9 and CX halved until 1024 blocks: 256^3 135 / 143 us, 384^3 563 / 651, 512^3
-    1205-1230 / 1267, 350 x 420 x 500 641 / 694; within 3% of the best of 126 tiles
-    measured at five grids.  ``halved``: that older rule, which a Drude sweep (at most 7
-    rows, two blocks per CU) and a TFSF sweep (13 rows, its z-face rows cost more) keep, and
-    tiles of which the caller gives one number."""
+    (one seed plane each).  One work-group runs per CU, so a sweep takes whole rounds of 256
+    blocks: the tile with the least ``tile_cost`` for ``box``, the planes and rows that the
+    sweep updates (default: of a grid with CPML on x and y), of the tiles that leave room for
+    the largest CE table (``table``: the run has one).  Sweep against T = 9 and CX halved until
+    1024 blocks: 256^3 135 / 143 us, 384^3 563 / 651, 512^3 1205-1230 / 1267, 350 x 420 x 500
+    641 / 694; within 3% of the best of 126 tiles measured at five grids.  ``halved``: that
+    older rule, which a Drude sweep (at most 7 rows, two blocks per CU) and a TFSF sweep (13
+    rows, its z-face rows cost more) keep, and tiles of which the caller gives one number."""
     if halved:
         return _halved(nx, ny)
     edge = 2 * (npml + 1) if npml else 0
-    bx, by = max(1, nx - edge), max(1, ny - edge)
+    bx, by = (max(1, n) for n in (box or (nx - edge, ny - edge)))
     best, cost = None, None
     for T in (13, 11, 9, 8, 7, 6, 5, 4, 3, 2, 1):
         if T > max(1, by // 2):
             continue
         for CX in range(min(bx, 64), min(bx, 8) - 1, -1):
-            if not lds_fits(T, CX, True, MAX_CE_TRI):
+            if not lds_fits(T, CX, True, MAX_CE_TRI if table else 0):
                 continue
-            rounds = -(-(-(-by // T) * -(-bx // CX)) // N_CU)
-            c = rounds * (CX + 2) * (T + 3)
+            c = tile_cost(T, CX, (bx, by))
             if cost is None or c < cost:
                 best, cost = (T, CX), c
     return best
@@ -107,11 +113,11 @@ def fused_pairs(nx, ny, nzp, npml):
     return False
 
 
-def fused_tiles(nx, ny, nzp, npml, pairs=False, halved=False):
+def fused_tiles(nx, ny, nzp, npml, pairs=False, halved=False, box=None, table=True):
     if pairs:
         return heuristic_pairs(nx, ny, nzp, npml)
     t = _load().get((nx, ny, nzp, npml))
-    return t if t is not None else heuristic(nx, ny, nzp, npml, halved)
+    return t if t is not None else heuristic(nx, ny, nzp, npml, halved, box, table)
 
 
 def fused_tuned(nx, ny, nzp, npml):

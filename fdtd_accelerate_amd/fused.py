@@ -207,8 +207,9 @@ class FusedStepper:
                 f.ce_mat = [_offset_copy(m, (-kb) % 128) for m in f.ce_mat]
         table = f.ce_mat is not None
         asked = rows_per_thread is not None or planes_per_chunk is not None
+        xb, xe, yb, ye = self.sweep_box(pairs=False)[:4]
         T, CX = fused_tiles(f.nx, f.ny, f.nz_pitch, npml, self.pairs,
-                            asked or self.drude is not None or self.tfsf is not None)
+                            asked or self.drude is not None or self.tfsf is not None, (xe - xb, ye - yb), table)
         self.T = rows_per_thread or T
         self.CX = planes_per_chunk or CX
         if not lds_fits(self.T, self.CX, table):
