@@ -14,6 +14,7 @@ grid is too small, or fills the sweep's z segments too little, for a sweep at al
 from __future__ import annotations
 
 import json
+import math
 import os
 
 from ._lib import MAX_CE_TRI
@@ -125,23 +126,31 @@ def fused_tuned(nx, ny, nzp, npml):
     return (nx, ny, nzp, npml) in _load()
 
 
-def whole_grid_faster(cells, box_cells, fill, face_cells, ce_bytes, tri, drude, tfsf):
-    """Whether a step as two passes over the whole grid is faster than the sweep of the box
-    with its two shell passes.  A cell of the box costs 48 B + CE at 5 TB/s over the filled
-    part of the sweep's 256-cell z segments (a fifth to a quarter more with a plane wave or
-    a Drude box), a shell cell 72 B + CE at 2.9 TB/s, the sweep's launches 20 us more; a
-    cell of the whole-grid passes 72 B + CE, and 32 B of psi in the slabs, at 5.35 TB/s.
-    Measured, sweep / whole grid, CE as indices, CPML 12: 96^3 57 / 22 us, 160^3 85 / 63,
-    224^3 221 / 200, 256^3 277 / 279, 288^3 381 / 407, 320^3 623 / 529, 384^3 970 / 885,
-    448^3 1308 / 1462, 512^3 1707 / 2001; with a plane wave 384^3 1118 / 939, 512^3
-    2065 / 2077; with a Drude box 384^3 1355 / 1063, 512^3 2582 / 2428."""
-    sweep = box_cells * (48 + (2 if tri else ce_bytes)) / 5.0e6 / max(fill, 1e-3)
+def whole_grid_faster(cells, box, segments, tile, face_cells, ce_bytes, tri, drude, tfsf):
+    """Whether a step as two passes over the whole grid is faster than the sweep of the ``box``
+    (planes, rows, z cells) in ``segments`` z segments with its two shell passes.  Times in us:
+    a cell of the sweep costs 48 B + CE at 8.2 TB/s and the tile's rounds 0.22 us per plane and
+    wave of a segment (tile_cost), a seventh more with a plane wave and a third more with a
+    Drude box; a shell cell 72 B + CE at 2.7 TB/s.  A cell of the whole-grid passes (``cells``,
+    the pitch's too) costs 72 B + CE at 5.4 TB/s, up to 8.4 where the fields stay in the
+    last-level cache, and 9.4 us per million cells of the CPML faces.  Fitted to both forms of
+    477 runs of 40 to 512 cells an axis (CE none, float and indices, CPML 0-12 on all faces or on
+    z with periodic x and y, plane waves and Drude boxes): the form picked is within 2% of the
+    faster one in 454 of them and at most 13% off (172x117x170 without CPML: 45 us for 40).
+    Sweep / whole, CE as indices, CPML 12: 224^3 205 / 184 us, 288^3 382 / 399, 384^3 913 /
+    902, 448^3 1303 / 1398, 512^3 1733 / 1986; z CPML and periodic x, y, float CE: 300x300x250
+    351 / 400, 384^3 956 / 935, 448^3 1345 / 1472; with a plane wave 384^3 1077 / 948, 512^3
+    2018 / 2014; with a Drude box 384^3 1376 / 997, 512^3 2375 / 2259."""
+    if not box[0] * box[1] * box[2]:  # no interior: the shell passes would take the whole grid
+        return True
+    sweep = box[0] * box[1] * box[2] * (48 + (2 if tri else ce_bytes)) / 8.2e6 + 0.22 * segments * tile_cost(*tile, box)
     if tfsf:
-        sweep *= 1.22
+        sweep *= 1.145
     if drude:
-        sweep *= 1.25
-    sweep += (cells - box_cells) * (72 + ce_bytes) / 2.9e6 + 20.0
-    whole = (cells * (72 + ce_bytes) + 32 * face_cells) / 5.35e6 * (1.05 if tfsf else 1.0)
+        sweep *= 1.345
+    sweep += (cells - box[0] * box[1] * box[2]) * (72 + ce_bytes) / 2.7e6 + 8.0
+    rate = 5.4 + 3.0 * math.exp(-cells / 5.5e6)
+    whole = cells * (72 + ce_bytes) / (1e6 * rate) * (1.016 if tfsf else 1.0) + 9.4e-6 * face_cells + 10.0
     return whole < sweep
 
 

@@ -253,12 +253,12 @@ class FusedStepper:
         f, cp = self.sim.fields, self.sim.cpml
         xb, xe, yb, ye, kb, ke = self.sweep_box()
         zb0 = kb if self.z_phase and self.cpml_axes & 4 else 256 * (kb // 256)
-        fill = (ke - kb) / max(256 * (-(-(ke - zb0) // 256)), 1)
         cells = f.nx * f.ny * f.nz
         face = sum(2 * cp.npml * cells // f.ns[a] for a in range(3) if (self.cpml_axes >> a) & 1) if cp else 0
         ce = 0 if not f.ce_on else 12 if f.ce_mat is None else 3
-        return whole_grid_faster(cells, self.sweep_cells(), fill, face, ce, self.ce_tri is not None,
-                                 self.drude is not None, self.tfsf is not None)
+        return whole_grid_faster(f.nx * f.ny * f.nz_pitch, (xe - xb, ye - yb, ke - kb), -(-(ke - zb0) // 256),
+                                 (self.T, self.CX), face, ce, self.ce_tri is not None, self.drude is not None,
+                                 self.tfsf is not None)
 
     def _build_ce_triples(self):
         """One uint16 index per cell into the distinct (cex, cey, cez) triples of the
