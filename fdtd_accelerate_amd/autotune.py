@@ -121,22 +121,18 @@ def fused_tiles(nx, ny, nzp, npml, pairs=False, halved=False, box=None, table=Tr
     return t if t is not None else heuristic(nx, ny, nzp, npml, halved, box, table)
 
 
-def fused_tuned(nx, ny, nzp, npml):
-    """Whether ``tune_fused`` measured a tile for this grid."""
-    return (nx, ny, nzp, npml) in _load()
-
-
 def whole_grid_faster(cells, box, segments, tile, face_cells, ce_bytes, tri, drude, tfsf):
     """Whether a step as two passes over the whole grid is faster than the sweep of the ``box``
     (planes, rows, z cells) in ``segments`` z segments with its two shell passes.  Times in us:
     a cell of the sweep costs 48 B + CE at 8.2 TB/s and the tile's rounds 0.22 us per plane and
     wave of a segment (tile_cost), 4% more with a plane wave and 8% with a Drude box than these
-    add to the whole-grid passes; a shell cell 72 B + CE at 2.7 TB/s.  A cell of the whole-grid passes (``cells``,
-    the pitch's too) costs 72 B + CE at 5.4 TB/s, up to 8.4 where the fields stay in the
-    last-level cache, and 9.4 us per million cells of the CPML faces.  Fitted to both forms of
-    511 runs of 40 to 1024 cells an axis (CE none, float and indices, CPML 0-12 on all faces or
-    on z with periodic x and y, plane waves and Drude boxes): the form picked is within 2% of
-    the faster one in 486 of them and at most 13% off (172x117x170 without CPML: 45 us for 40).
+    add to the whole-grid passes; a shell cell 72 B + CE at 2.7 TB/s.  A cell of the whole-grid
+    passes (``cells``, the pitch's too) costs 72 B + CE at 5.4 TB/s, up to 8.4 where the fields
+    stay in the last-level cache, and 9.4 us per million cells of the CPML faces.  Fitted to
+    both forms of 511 runs of 40 to 1024 cells an axis (CE none, float and indices, CPML 0-12
+    on all faces or on z with periodic x and y, plane waves and Drude boxes): the form picked
+    is within 2% of the faster one in 486 of them and at most 13% off (172x117x170 without
+    CPML: 45 us for 40).
     Sweep / whole, CE as indices, CPML 12: 224^3 205 / 184 us, 288^3 382 / 399, 384^3 913 /
     902, 448^3 1303 / 1398, 512^3 1733 / 1986; z CPML and periodic x, y, float CE: 300x300x250
     351 / 400, 384^3 956 / 935, 448^3 1345 / 1472; with a plane wave 384^3 1077 / 948, 512^3

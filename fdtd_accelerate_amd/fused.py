@@ -20,8 +20,7 @@ import torch
 
 from . import _lib
 from . import fields as _fields
-from .autotune import (fused_pairs, fused_tiles, fused_tuned, lds_fits, lds_fits_pairs, slab_planes,
-                       whole_grid_faster)
+from .autotune import fused_pairs, fused_tiles, lds_fits, lds_fits_pairs, slab_planes, whole_grid_faster
 
 _COMP = {"ex": 0, "ey": 1, "ez": 2, "hx": 3, "hy": 4, "hz": 5}
 
@@ -242,12 +241,13 @@ class FusedStepper:
         self._tri_kb = kb if z_phase else 0
         self.ce_tri = self.ce_tri_lut = self._tri_src = None
         self._build_ce_triples()
-        # whole-grid steps instead of the sweep and its shell, unless a tile was asked for or
-        # measured (tune_fused); a run with sweep timing takes the sweep
+        # whole-grid steps instead of the sweep and its shell, unless a tile was asked for (one
+        # that tune_fused measured is the best of the sweep's, not faster than these steps); a
+        # run with sweep timing takes the sweep
         if whole_grid and self.pairs:
             raise ValueError("whole-grid steps and step pairs exclude each other")
         self.whole_grid = bool(whole_grid) if whole_grid is not None else \
-            not (asked or self.pairs or fused_tuned(f.nx, f.ny, f.nz_pitch, npml)) and self._whole_grid_faster()
+            not (asked or self.pairs) and self._whole_grid_faster()
 
     def _whole_grid_faster(self):
         f, cp = self.sim.fields, self.sim.cpml

@@ -42,3 +42,18 @@ _MEASURED = [
 @pytest.mark.parametrize("args,whole,sweep", _MEASURED)
 def test_the_faster_form_is_picked(args, whole, sweep):
     assert autotune.whole_grid_faster(*args) == (whole < sweep)
+
+
+@pytest.mark.gpu
+def test_a_tuned_tile_does_not_force_the_sweep():
+    """A tile that tune_fused measured is the sweep's; whether a step sweeps is the rule's."""
+    from fdtd_accelerate_amd.sim import YeeSim
+    key = (40, 44, 48, 6)
+    assert key not in autotune._load()
+    autotune._load()[key] = (3, 8)
+    try:
+        s = YeeSim(40, 44, 48, npml=6, coeff_use="", engine="fused")
+        s.run(1)
+        assert (s._fused.T, s._fused.CX) == (3, 8) and s._fused.whole_grid
+    finally:
+        del autotune._load()[key]
