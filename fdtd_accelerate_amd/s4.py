@@ -245,13 +245,14 @@ class S4Sim:
                 d.cpml_h[s] = self._half(self.psiH, *self._tabH[s])
         d.nsrc = len(self.sources)
         tv = np.zeros((max(nsteps, 1), 4, max(len(self.sources), 1)), np.float32)
-        for n, (c, p0, p1, tfunc, sv, svs) in enumerate(self.sources):
+        for n, (c, p0, p1, _, sv, svs) in enumerate(self.sources):
             d.src_comp[n] = c
             d.src_box[n][:] = (p0[0], p1[0], p0[1], p1[1], p0[2], p1[2])
             d.src_sv[n] = None if sv is None else sv.data_ptr()
             d.src_svs[n] = svs
-            for t in range(nsteps):
-                for s in range(4):
+        for t in range(nsteps):  # in the order of step(): functions may keep a state
+            for s in range(4):
+                for n, (_, _, _, tfunc, _, _) in enumerate(self.sources):
                     tv[t, s, n] = np.float32(tfunc(self.tstep + t + s / 5.0))
         if buf is not None:
             d.nprobe = len(self.probe_points)
