@@ -186,6 +186,7 @@ class Cpml:
                   *f.ptrs(chs), f.stream.cuda_stream)
 
 
+Fields._cpml = Cpml
 # The update methods that a joined half step stands for (joins).
 _OWN = (Core.update_e, Core.update_h, Cpml.update_e, Cpml.update_h, Drude.update_e, Drude.update_h)
 

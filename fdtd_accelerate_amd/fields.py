@@ -189,12 +189,13 @@ class Fields:
     # into its own pass: a step of 128^3 cells with CPML 10 63 -> 40 us, 300 x 211 x 331 with
     # CPML 12 459 -> 364, 1024^3 17.4 -> 15.0 ms, 256^3 with CPML 10 and a Drude box of 128^3
     # 416 -> 341 us, against the core, the region and one launch per axis of faces.
+    _cpml = None  # the class Cpml, set by its module
+
     def _joined(self):
         """How many instances from the first on one pass takes: 0, 2 or 3."""
         insts = self.instance_list
         for n in (1, 2):
-            joins = getattr(insts[n], "joins", None) if len(insts) > n else None
-            if joins is not None and joins(*insts[:n]):
+            if len(insts) > n and type(insts[n]) is self._cpml and insts[n].joins(*insts[:n]):
                 return n + 1
         return 0
 
