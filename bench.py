@@ -15,8 +15,8 @@ source + H update + CPML-H (+ probe gather).
                        instances in one batched step loop vs the same instances run
                        one after another)
     python bench.py --workload adjoint   (160^3 design problem: forward 800 steps with
-                       checkpoints every 50, adjoint gradient on the 64^3 box; reports
-                       backward / forward time)
+                       the design box's curls stored, adjoint gradient on the 64^3 box;
+                       reports backward / forward time)
     python bench.py --workload pbc   (the 1024^3 sphere workload with periodic x and y and
                        CPML on the z faces; steps timed without and with the periodic
                        boundaries)
@@ -57,22 +57,15 @@ HBM_PEAK_GBS = 8000.0
 
 # HBM bytes per launch of the dominant kernel (GB), from two rocprofv3 --pmc runs
 # (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0: the factors a plain 1 GiB copy gives), keyed by
-# (engine, n, npml, CE storage, --z-phase); profiles/update_e_yee_cpml12_1024cube_hbm_counters.txt,
-# profiles/update_e_lut_yee_cpml12_1024cube_hbm_counters.txt and
+# (engine, n, npml, CE storage, --z-phase); profiles/half_step_yee_cpml12_1024cube_hbm_counters.txt
+# (the in-place engine's E pass) and
 # profiles/k_fused_sweep_yee_cpml12_1024cube_hbm_counters.txt (the interior sweep; the
 # automatic line phase is 16 there, the sweep box z [16, 1008), CE read as uint16 triple
 # indices; at phase 0 the box is [32, 992) and the measurement predates the triple indices).
-MEASURED_TRAFFIC_GB = {("kemp", 1024, 12, "float32", None): 64.69,
-                       ("kemp", 1024, 12, "uint8 index + table", None): 53.24,
+MEASURED_TRAFFIC_GB = {("kemp", 1024, 12, "uint8 index + table", None): 49.17,
                        ("fused", 1024, 12, "uint8 index + table", None): 52.36,
                        ("fused", 1024, 12, "uint8 index + table", 16): 52.36,
                        ("fused", 1024, 12, "uint8 index + table", 0): 51.83}
-# The 4th-order E stage (k_s4_e_zm, CE as uint8 material indices), same method, keyed by
-# (n, npml); profiles/k_s4_zmarch_symplectic_cpml10_512cube_hbm_counters.txt.
-MEASURED_S4_TRAFFIC_GB = {(512, 10): 5.81}
-# The batched step (both launches of one step, all instances), same method, keyed by
-# (instances, cube edges drawn from); profiles/k_batch_uneven_64cubes_kernel_trace.txt.
-MEASURED_BATCH_TRAFFIC_GB = {(64, "64,96,128,160,192"): 16.86}
 
 
 def parse():
@@ -131,12 +124,13 @@ def build_sim(args):
 
 def time_kemp(sim, steps, warmup):
     """In-place engine, each half step through Fields.update_e / update_h; a second run of K
-    steps takes the instances one by one, with events around the core's update_e kernel (the
-    dominant launch) on the fields' stream."""
+    steps brackets, with events on the fields' stream, the E pass of the core (the dominant
+    launch) with the CPML and the Drude region that it takes into the pass."""
     import torch
     f = sim.fields
-    core = sim.core
-    others_e = [i for i in f.instance_list if i is not core]
+    joined = f._joined()
+    rest = f.instance_list[joined or 1:]
+    first = (lambda: f.instance_list[joined - 1].update_core_e(*f.instance_list[1:joined - 1])) if joined else sim.core.update_e
     for _ in range(warmup):
         f.update_e()
         f.update_h()
@@ -156,16 +150,21 @@ def time_kemp(sim, steps, warmup):
     ms = t0.elapsed_time(t1)
     for s in range(steps):
         evs[s][0].record(f.stream)
-        core.update_e()
+        first()
         evs[s][1].record(f.stream)
-        for inst in others_e:
+        for inst in rest:
             inst.update_e()
         f.update_h()
     torch.cuda.synchronize()
     kern_ms = sum(a.elapsed_time(b) for a, b in evs) / steps
-    if f.ce_mat is not None:
-        return ms / steps, wall, kern_ms, "update_e (CE as uint8 index + table)", 39.0
-    return ms / steps, wall, kern_ms, "update_e", 48.0
+    # E read and written, H and CE read, and in the CPML slabs two psi read and written
+    byts = 39.0 if f.ce_mat is not None else 48.0
+    name = "update_e" + (" (CE as uint8 index + table)" if f.ce_mat is not None else "")
+    if joined:
+        faces = sum(2 * sim.cpml.npml / f.ns[a] for a, d in enumerate(sim.cpml.apply_direction) if d)
+        byts += 16.0 * faces
+        name = name.replace("update_e", "k_slab_e, core and CPML of the E half step" + (", Drude region" if joined == 3 else ""))
+    return ms / steps, wall, kern_ms, name, byts
 
 
 def time_fused(sim, steps, warmup, pairs=False, z_phase=None):
@@ -188,9 +187,15 @@ def time_fused(sim, steps, warmup, pairs=False, z_phase=None):
     torch.cuda.synchronize()
     wall = time.perf_counter() - wall0
     ms = t0.elapsed_time(t1)
+    cells = sim.fields.nx * sim.fields.ny * sim.fields.nz
+    if st.whole_grid:
+        # small grids: an E and an H pass per step, no sweep; the two passes are the step.  60 B
+        # per cell of the plain step and two psi read and written per half in the CPML slabs
+        cp = sim.cpml
+        faces = sum(2 * cp.npml / sim.fields.ns[a] for a in range(3) if (st.cpml_axes >> a) & 1) if cp is not None else 0
+        return ms / steps, wall, ms / steps, "k_slab_e + k_slab_h (whole-grid steps, both passes)", 60.0 + 32.0 * faces
     # second pass of the same K steps with timing-only events around each sweep launch
     kern_ms = st.run(steps, None, time_kernel=True)
-    cells = sim.fields.nx * sim.fields.ny * sim.fields.nz
     sweep = st.sweep_cells()
     # algorithmic bytes on the per-cell basis of the plain Yee step: read 6 fields and 3 CE,
     # write 6 fields = 60 B (the sweep box holds no CPML cell); the kernel itself reads CE
@@ -241,24 +246,23 @@ def run_s4(args):
     sim.set_eps(geometry.eps_map_numpy((n, n, n), spheres))
     c = n // 2
     sim.add_source("ez", (c, c, c), (c, c, c), gaussian_pulse())
-    for _ in range(args.warmup):
-        sim.step()
+    sim.run(args.warmup)
     torch.cuda.synchronize()
-    evs = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(args.steps)]
     t0 = torch.cuda.Event(enable_timing=True)
     t1 = torch.cuda.Event(enable_timing=True)
     wall0 = time.perf_counter()
     t0.record(sim.stream)
-    for k in range(args.steps):
-        sim.step(events=evs[k])
+    sim.run(args.steps)
     t1.record(sim.stream)
     torch.cuda.synchronize()
     wall = time.perf_counter() - wall0
     ms = t0.elapsed_time(t1) / args.steps
-    kern_ms = sum(a.elapsed_time(b) for a, b in evs) / args.steps
     cells = n ** 3
-    step_bytes = 336.0 * cells + 32.0 * 4 * 6 * npml * n * n
-    achieved = 48.0 * cells / (kern_ms * 1e-3) / 1e9
+    # five H stages (E read, H read and written: 36 B) and four E stages (H read, CE read as 3 B
+    # of material indices, E read and written: 39 B), and two psi read and written per stage in
+    # the CPML slabs
+    step_bytes = 336.0 * cells + 16.0 * 9 * 6 * npml * n * n
+    achieved = step_bytes / (ms * 1e-3) / 1e9
     return {
         "metric": METRIC, "value": round(cells / (ms * 1e-3) / 1e9, 3), "unit": "Gcell/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 4), "higher_is_better": True,
@@ -266,11 +270,12 @@ def run_s4(args):
         "config": {"workload": f"4th-order symplectic FP32 {n}^3, {nsph} spheres, CPML {npml}, S=0.9*S_max={sim.S:.4f}, Ez point source",
                    "cells": cells},
         "hbm_frac_step": round(step_bytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-        "roofline": {"bound": "hbm", "kernel": "k_s4_e_zm (E stage)", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+        "roofline": {"bound": "hbm", "kernel": "k_s4_h + k_s4_e (the nine stages of a step, each with its CPML)", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": MEASURED_S4_TRAFFIC_GB.get((n, npml)), "traffic_unit": "GB per launch",
-                     "bytes_per_cell": 48.0, "bytes_basis": "read E, H, CE as float32, write E (the kernel reads CE as "
-                     "3 B of material indices: 39 B moved)", "avg_launch_ms": round(kern_ms, 4)},
+                     "traffic": None,
+                     "bytes_per_cell": round(step_bytes / cells, 1), "bytes_basis": "per step: 5 x 36 B and 4 x 39 B (CE as "
+                     "material indices) and 16 B per CPML face cell and stage",
+                     "avg_launch_ms": round(ms / 9, 4)},
         "wall_s": round(wall, 3), "device": torch.cuda.get_device_name(0),
     }
 
@@ -340,7 +345,7 @@ def run_batch(args):
         "roofline": {"bound": "hbm", "kernel": bt.kernel_name, "basis": "60 B per cell + 32 B per CPML face-slab cell per step",
                      "achieved": round(step_bytes / (ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(step_bytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                     "traffic": MEASURED_BATCH_TRAFFIC_GB.get((args.instances, args.sizes)), "traffic_unit": "GB per step",
+                     "traffic": None,
                      "algorithmic_gb": round(step_bytes / 1e9, 3), "ms_per_step": round(ms, 4)},
         "wall_s": round(wall, 3), "device": torch.cuda.get_device_name(0),
     }
@@ -550,8 +555,8 @@ ADJ_GOLD = os.path.join(ROOT, "tests", "golden", "adjoint_design160.npz")
 
 
 def run_adjoint(args):
-    """The 160^3 design problem: J(eps) forward (800 steps, checkpoints every 50) and dJ/deps on the
-    64^3 design box by the adjoint (recompute + adjoint kernels); GPU times of both.  With the
+    """The 160^3 design problem: J(eps) forward (800 steps, the design box's curls stored) and
+    dJ/deps on the 64^3 design box by the adjoint; GPU times of both.  With the
     committed float64 reference data, the gradient's error against the float64 central
     differences at its 32 voxels and against the float64 gradient over the box."""
     import numpy as np
