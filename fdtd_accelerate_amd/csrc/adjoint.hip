@@ -17,8 +17,8 @@
 //                t_E = lpsiE -/+ CE*lE on valid E slab cells;  grad_CE += lE * (K H_prev)
 //                on the design box;  lE = 0 on masked E lanes
 //   D:           lpsiE = b_E * t_E
-// A and C gather from neighbours (thread per cell), so every pass reads only values no
-// thread of the same pass writes.  B only touches the cell's own lH / lpsiH, so it runs
+// A and C gather from neighbours (a lane per quad of z cells), so every pass reads only
+// values no thread of the same pass writes.  B only touches the cell's own lH / lpsiH, so it runs
 // inside C (before C changes lH of that cell); D only touches the cell's own lE / lpsiE,
 // so it is deferred into A of the next (earlier) step, before A changes lE of that cell
 // (on the zero initial state it is a no-op).  Two launches per step.  Sources do not

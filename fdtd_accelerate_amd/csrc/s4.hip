@@ -25,11 +25,12 @@ constexpr int S4B = 256;
 // own).  One pass updates E (or H) of a stage with its CPML, sources and probes, so each
 // array is read and written once per stage; the y and z neighbour rows (three of each) are
 // L2 hits of the stripe.  The bound is the traffic behind the L2s.  Against a marching
-// work-group per 8 rows x 32 planes with separate CPML launches (which left most of the
-// chip idle on small grids: 36 work-groups at 132 x 90 x 75), per step with CPML 10: 64^3
-// 627 -> 68 us, 132 x 90 x 75 732 -> 115, 200^3 1081 -> 552, 400 x 300 x 200 2789 -> 2067,
-// 512^3 10.99 -> 10.86 ms.  The contiguous-axis faces cost most of what CPML costs (512^3:
-// none 10.2, y and z 10.3, x 11.0 ms).
+// work-group per 8 rows x 32 planes with separate CPML launches, called from Python (which
+// left most of the chip idle on small grids: 36 work-groups at 132 x 90 x 75), a run's step
+// with CPML 10: 64^3 620 -> 81 us, 132 x 90 x 75 726 -> 125, 200^3 971 -> 517, 400 x 300 x 200
+// 2719 -> 1980, 512^3 10.76 -> 10.77 ms; without CPML 128^3 626 -> 130 us, 200^3 698 -> 367,
+// 400^3 5542 -> 4294, 512^3 9.06 -> 8.78 ms; a bare stage H / E at 512^3 994 / 1035 -> 941 /
+// 965 us, at 768 x 768 x 512 2322 / 2379 -> 2302 / 2300 (float CE, E 2825 -> 2877).
 struct S4Geom {
     int nx, ny, nz;
     RowQuads m;

@@ -159,11 +159,11 @@ class Fields:
         self.ce_mat = self.ce_lut = None
 
     def compress_ce(self):
-        """Let the core E update read the CE arrays as uint8 material indices into a
+        """Let the E updates read the CE arrays as uint8 material indices into a
         3 x 256 table of their exact values (39 instead of 48 bytes per cell; results
         unchanged).  Possible when each component has at most 256 distinct values;
-        returns whether it was done.  The float arrays stay (the CPML kernels and host
-        access use them); call again after changing CE."""
+        returns whether it was done.  The float arrays stay (the CPML's and the Drude
+        regions' own launches and host access use them); call again after changing CE."""
         if not self.ce_on or self.precision_float != "single":
             return False
         lut = torch.zeros((3, 256), dtype=torch.float32, device=self.device)

@@ -8,9 +8,11 @@ hold S/(24 eps_r), and one step is
     H(c_4)
 
 (``100-base.py:124-141``; the closing H uses c_4 = c1 as the PyCUDA version does).
-The stage updates are ``mifdtd_s4_update_h/e`` (``S4/Python-C/dielectric.c``
-arithmetic); the optional CPML (``mifdtd_s4_cpml_h/e``, new: the reference has none)
-runs after each stage with the tables of that stage's time step w_s*S.
+The stage updates have ``S4/Python-C/dielectric.c``'s arithmetic; the optional CPML (new: the
+reference has none) follows each stage with the tables of that stage's time step w_s*S.
+``run`` takes its steps in one call (``mifdtd_s4_run``), each stage with its CPML, sources and
+probes in one pass; ``step`` takes the stages apart (``mifdtd_s4_update_h/e``,
+``mifdtd_s4_cpml_h/e``), with the same values.
 """
 from __future__ import annotations
 
@@ -137,7 +139,8 @@ class S4Sim:
     def set_ce(self, cex, cey, cez):
         """CE arrays; when each component holds at most 256 distinct values the E stages
         read them as uint8 material indices into an exact table (39 instead of 48 bytes
-        per cell, the same values; the CPML keeps the float arrays)."""
+        per cell, the same values; the CPML of ``step`` reads the float arrays, that of ``run``
+        the indices).  Call again after changing CE."""
         self.ces = [self._fortran(c) for c in (cex, cey, cez)]
         self.ce_mat = self.ce_lut = None
         lut = torch.zeros((3, 256), dtype=torch.float32, device=self.device)
