@@ -1,4 +1,4 @@
-// Thread -> quad order of the whole-grid passes (slab and batched engines), shared by the
+// Thread -> quad order of the whole-grid passes, shared by the
 // kernels and a host-side coverage check.
 //
 // Stripes: blocks are dealt round-robin to the 8 XCDs, each with its own L2.  Stripe x of
@@ -11,11 +11,12 @@
 // then those at the rows' ends with the z slabs.  A row of 64 to 256 cells is 16 to 64
 // quads, so with quads in plain row order every wave holds some z-slab lanes and issues the
 // z slab's psi loads, arithmetic and stores for a few lanes.  Runs cut within a line make
-// two waves fetch it: whole step at 256^3 / 320^3 / 448^3, CPML 10-12, cut at the slab 321 /
-// 557 / 1565 us, at lines 302 / 511 / 1455, plain row order 307 / 519 / 1360; 128^3 38.0 /
-// 37.1 / 39.2.  R is the smallest group that leaves next to no idle thread.  Quads next to
-// each other in a run are next to each other in memory too, so a lane finds its k+4 (k-1)
-// neighbour in the next (previous) lane except at a run's end.
+// two waves fetch it.  E + H, CPML 10, 128^3 / 256^3 / 320^3 / 448^3 / 512^3: cut at lines 37.1 /
+// 261 / 494 / 1297 / 1872 us, at the slab 38.3 / 278 / 528 / 1358 / 1970, plain row order 38.8 /
+// 266 / 510 / 1334 / 1892.  R is the smallest group that leaves next to no idle thread, within
+// the caller's limit (yee_order).  Quads next to each other in a run are next to each other in
+// memory too, so a lane finds its k+4 (k-1) neighbour in the next (previous) lane except at a
+// run's end.
 #pragma once
 
 #include "common.hpp"
@@ -97,9 +98,11 @@ constexpr unsigned kEqualRows = 512;
 
 // The stripes' rows: equal shares of the rows' cost, a row of a y slab (psi read and
 // written) costing 1.3 rows.  With equal row counts the first and the last XCD, which hold
-// the y slabs, end last: 160^3 / 192^3 / 256^3 cells, CPML 10, E + H pass 71.2 / 113.8 /
-// 318.9 us; with 1.3, 69.6 / 107.8 / 302.7.  Planes of kEqualRows rows and more take equal
-// stripes: the 4th-order step at 512^3 10.86 ms against 11.10 (256^3 1.47 / 1.44).
+// the y slabs, end last: E + H, CPML 10, equal rows / 1.3, 256^3 271 / 261 us, 300x288x300 427 /
+// 402, 448^3 1327 / 1300, 200x480x300 454 / 439.  Planes of kEqualRows rows and more take equal
+// stripes: the 4th-order step at 512^3 10.86 ms against 11.10 (256^3 1.47 / 1.44), the Yee passes
+// at 512^3 1870 us against 1890; flatter grids would still gain by 1.3 (200x512x300 481 / 469,
+// 150x600x256 354 / 352, 150x768x224 412 / 398).
 inline void stripe_rows(RowQuads &m, unsigned ny, int npml)
 {
     const unsigned slab = npml > 0 ? (unsigned)npml : 0u;
@@ -180,8 +183,9 @@ inline RowQuads row_quads(unsigned planes, unsigned ny, unsigned Q, int nz, int 
     return m;
 }
 
-// The order of a Yee E or H pass (npml_y, npml_z: 0 on an axis without CPML).  With CPML a group's z-slab runs follow the runs of all its
-// rows: at pitches off the lines a large group fetches the lines at the runs' ends twice.
+// The order of a Yee E or H pass (npml_y, npml_z: 0 on an axis without CPML).  With CPML a
+// group's z-slab runs follow the runs of all its rows: at pitches off the lines a large group
+// fetches the lines at the runs' ends twice.
 // E + H, CPML 10, groups of up to 64 / 8 / 2 rows: 341x240x258 424 / 379 / 383 us, 333x491x357
 // 1053 / 907 / 896, 448^3 1398 / 1298 / 1300, 352^3 673 / 641 / 645, 128^3 36.0 / 36.7 / 38.9,
 // 300x300x250 356 / 355 / 365.  The 4th-order stages and the adjoint passes keep 64 (8: 400 x

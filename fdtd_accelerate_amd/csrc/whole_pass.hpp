@@ -25,8 +25,8 @@ inline SAux no_aux()
 }
 
 // E pass, then H pass, each in place; dr / tf / cu: null where the step has none (cu goes
-// without the others); ch: the three
-// CH arrays, null for the constant 0.5 (which a step with tf has).
+// without the others); ch: the three CH arrays, null for the constant 0.5 (which a step with tf
+// has).
 int whole_e(const WholeGrid &w, const SAux &a, const SDrude *dr, const STfsf *tf, const SCurl *cu = nullptr);
 int whole_h(const WholeGrid &w, const SAux &a, const STfsf *tf, const float *const *ch = nullptr);
 

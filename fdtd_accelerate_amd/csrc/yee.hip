@@ -293,9 +293,10 @@ static int launch_range(bool e_half, int nx, int ny, int nzp, int pad, const flo
 // quads, 218.8 / 224.3), or on grids of fewer than 2^19 quads nearly one (up to 112 quads off
 // a multiple of 2048: 129x171x48 13.0 / 11.0, 120x109x73 12.4 / 10.6, 64x138x116 13.8 / 11.8,
 // 83x121x203 26.5 / 25.1, E alone with CE indices 135x102x74 7.9 / 6.5; with more quads
-// 101x139x236 39.2 / 40.9, further off 96^3 11.3 / 12.9).  Planes of few rows: 100x70x200 24.8 / 23.9 on cold arrays, 200x71x130 32.4 / 30.5;
-// 200x128x100 34.3 / 39.9.  Below 2^17 quads the launches bound, and the whole-grid kernels'
-// few structures are cheaper to pass than 18 arguments (64^3, from Python, 14.8 / 17.0).
+// 101x139x236 39.2 / 40.9, further off 96^3 11.3 / 12.9).  Planes of few rows: 100x70x200 24.8
+// / 23.9 on cold arrays, 200x71x130 32.4 / 30.5; 200x128x100 34.3 / 39.9.  Below 2^17 quads the
+// launches bound, and the whole-grid kernels' few structures are cheaper to pass than 18
+// arguments (64^3, from Python, 14.8 / 17.0).
 static bool memory_order(int nx, int ny, int Q)
 {
     const unsigned long long quads = (unsigned long long)nx * ny * Q;
